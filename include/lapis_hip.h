@@ -298,17 +298,16 @@ int lapis_hip_spmm_csr_f64_i32(int64_t nrows, int64_t ncols, int64_t k, const in
                                const int32_t *crd, const double *val, const double *B, int64_t ldb,
                                double *C, int64_t ldc, lapis_hip_stream_t stream);
 
-/* The same product with the plan's statistics deciding the kernel.
- *   group per row: matrices with short, even rows (mean <= 256, longest <= 4 x mean)
- *     whose columns stay local (the B rows a stretch of 1024 non-zeros touches fit the
- *     L2s: stencils, meshes).  64/LPR rows per wavefront at a time, one group of lanes
- *     per row, no cross-lane reduction: 1.25x-5.8x faster than the kernel below there.
- *   wavefront per row: everything else, and `plan == NULL` (the entry points above).
+/* The same product with the plan's statistics deciding how rows and columns are dealt to lanes.
+ *   several rows per wavefront ("spmm_group_row_kernel"): even rows (mean <= 256, longest <= 4 x mean), as many
+ *     as leave a group of lanes eight steps, fewer where the rows of B come from HBM.
+ *   wavefront per row ("spmm_wave_row_kernel"): everything else, and `plan == NULL` (the entry points above).
  *   LDS-staged row block: a workgroup stages the rows of B of its block's diagonal
  *     window in LDS with coalesced 128-bit loads and serves the non-zeros inside the
  *     window from LDS.  Built and kept selectable (LAPIS_HIP_SPMM_KERNEL=lds) but never
- *     chosen: on MI355X it measured 1.6x-2.4x slower than group per row on the
+ *     chosen: on MI355X it measured 2.5x-3x slower than the others on the
  *     stencil and FEM matrices it is meant for.
+ * k, ldb, ldc and the alignment of B and C are free: any of them takes the same kernels.
  * The reference chooses between its loop mappings by strategy name
  * (Pipelines/Passes.h:41-56), never by looking at the columns. */
 int lapis_hip_spmm_csr_f32_i32_plan(const lapis_hip_csr_plan *plan, int64_t nrows, int64_t ncols, int64_t k,

@@ -142,6 +142,15 @@ __device__ __forceinline__ unsigned xcd_contiguous_block(unsigned b, unsigned nb
   return xcd * q + (xcd < r ? xcd : r) + idx;
 }
 
+// The number of work-items along one dimension of a grid has to fit 32 bits: launches of more than 2^23
+// workgroups of 256 or 512 threads get a second dimension and number their workgroups with linear_block()
+// (numbers at or past the count asked for belong to nobody).
+inline dim3 grid_of(int64_t blocks) {
+  const int64_t x = blocks < (1 << 23) ? blocks : (1 << 23);
+  return dim3((unsigned)x, (unsigned)ceil_div(blocks, x));
+}
+__device__ __forceinline__ unsigned linear_block() { return blockIdx.y * gridDim.x + blockIdx.x; }
+
 // Orders LDS traffic between the lanes of ONE wavefront (no s_barrier): LDS
 // operations of a wave execute in issue order, the fences stop the compiler from
 // moving accesses across this point.

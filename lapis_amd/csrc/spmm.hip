@@ -12,212 +12,192 @@
 
 namespace lapis {
 
+// 16 bytes of a row of B or C.  Global memory takes 128-bit accesses at any address that is a multiple of
+// four, so the vectors only promise the alignment of their elements: any leading dimension, any base.
 template <typename T>
 struct RowVec;
 template <>
 struct RowVec<float> {
   typedef v4f type;
+  typedef float loose __attribute__((ext_vector_type(4), aligned(4)));
   static constexpr int width = 4;
 };
 template <>
 struct RowVec<double> {
   typedef v2d type;
+  typedef double loose __attribute__((ext_vector_type(2), aligned(8)));
   static constexpr int width = 2;
 };
 
-// One wavefront per row of A and per chunk of LPR * VW columns of B (blockIdx.y).  The
-// chunk of a B row is covered by LPR lanes with one 128-bit load each, so the 64 lanes
-// take G = 64/LPR non-zeros of the row per step: every gathered B row is one fully
-// coalesced read.  The row's crd/val are read once, 64 at a time and coalesced, then
-// handed to the lane groups by bpermute.  The G partial rows are added up with xor
-// shuffles.  VEC = false is the same kernel with element-wise guarded accesses, for k
-// that is no multiple of the vector width and for buffers that are not 16-byte aligned.
-template <typename T, int LPR, bool VEC, bool DEEP>
-__global__ __launch_bounds__(256) void spmm_wave_row_kernel(int nrows, int k, const int *__restrict__ pos,
-                                                            const int *__restrict__ crd,
-                                                            const T *__restrict__ val, const T *__restrict__ B,
-                                                            long long ldb, T *__restrict__ C, long long ldc) {
-  typedef typename RowVec<T>::type V;
-  constexpr int VW = RowVec<T>::width;
-  constexpr int G = 64 / LPR;
-  const int lane = threadIdx.x & 63;
-  const long long row = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= nrows) return;
-  const int g = lane / LPR;
-  const int l = lane % LPR;
-  const int col = (int)blockIdx.y * (LPR * VW) + l * VW;  // first of this lane's VW columns
-  const int start = pos[row];
-  const int end = pos[row + 1];
-  V acc = {};
-  for (int base = start; base < end; base += 64) {
-    const int cnt = min(64, end - base);
-    int c_l = 0;
-    T a_l = T(0);
-    if (lane < cnt) {
-      c_l = load_stream(crd + base + lane);
-      a_l = load_stream(val + base + lane);
+// How a launch deals B's columns and A's rows to lanes.
+//   Columns: chunk c holds the columns [chunk_first(c), chunk_first(c + 1)), a multiple of the vector width
+//   wide except the last, which takes what is left and is at least one vector wide.
+//   Rows: a group of lpr * par lanes takes one row of A; 64 / (lpr * par) groups to a wavefront.  In a group
+//   `lpr` lanes cover the chunk of a row of B, so the group takes `par` non-zeros of its row per step.
+struct SpmmShape {
+  int chunks;      // column chunks
+  int vectors;     // whole vectors in a row of B
+  int k;
+  int lpr, par;
+  int groups;      // 64 / (lpr * par)
+  int row_blocks;  // workgroups per chunk
+  int xcd_map;
+  template <int VW>
+  __device__ __forceinline__ int chunk_first(int c) const {
+    return c >= chunks ? k : VW * (int)(((long long)vectors * c) / chunks);
+  }
+};
+
+__device__ __forceinline__ int lane_get(int byte_of_lane, int v) { return __builtin_amdgcn_ds_bpermute(byte_of_lane, v); }
+__device__ __forceinline__ float lane_get(int byte_of_lane, float v) {
+  return __builtin_bit_cast(float, lane_get(byte_of_lane, __builtin_bit_cast(int, v)));
+}
+__device__ __forceinline__ double lane_get(int byte_of_lane, double v) {
+  v2i w = __builtin_bit_cast(v2i, v);
+  w.x = lane_get(byte_of_lane, w.x);
+  w.y = lane_get(byte_of_lane, w.y);
+  return __builtin_bit_cast(double, w);
+}
+
+// A wavefront owns `groups` consecutive rows; their entries are one contiguous stretch of crd/val, which it
+// stages in its own part of LDS with coalesced loads, all in flight together (window by window when the rows
+// hold more than kStaged entries), the column already turned into the byte offset of its row of B.  A lane of a
+// group holds one 128-bit vector (VW elements; VW = 1 for k smaller than a vector) of its group's row of
+// C and reads every par-th entry of the row from LDS.  A batch of up to DEPTH steps loads its rows of B first,
+// without any condition (past the row end a lane repeats the last non-zero's row), then adds them in order:
+// DEPTH gathered rows in flight per lane.  The `par` partial rows of a group are added with shuffles at the end.
+// A lane whose vector would pass the end of its chunk takes the chunk's last VW columns instead: it
+// computes (and stores) the same numbers as its neighbour, so no access needs a guard for a ragged k.
+//
+// What bounds short rows is the chain of dependent loads of a wavefront (positions, entries, rows of B, row of
+// C), not bandwidth: staging makes it one trip per wavefront instead of one per LPR entries, and the row of C
+// is asked for first.  Measured (us; entries handed round by bpermute, LPR or 64 per trip -> staged):
+//   7-point 97^3, fp64   k = 3: 316 -> 35   k = 10: 392 -> 72   k = 64: 409 -> 369
+//   27-point x 3, 30^3   k = 3 fp64: 48 -> 31   k = 10 fp32: 57 -> 34   k = 64 fp32: 82 -> 73
+//   random, 32 per row, 15 000 rows, k = 10 fp32: 9.9 -> 7.7; 1 M rows, k = 64 fp32 (rows of B from HBM): 1217 -> 1203
+// WIDE: B is 4 GB or more and the offsets take 64 bits.
+constexpr int kStaged = 512;  // entries per wavefront: 24 KB (fp64) per workgroup, six workgroups to a CU
+template <typename T, int VW, int DEPTH, bool WIDE>
+__device__ __forceinline__ void spmm_rows_body(int nrows, const SpmmShape &sh, const int *__restrict__ pos,
+                                               const int *__restrict__ crd, const T *__restrict__ val,
+                                               const T *__restrict__ B, long long ldb, T *__restrict__ C,
+                                               long long ldc) {
+  typedef typename std::conditional<VW == 1, T, typename RowVec<T>::loose>::type V;
+  __shared__ T s_val[4][kStaged];
+  __shared__ unsigned s_off[4][kStaged];
+  const unsigned nblocks = (unsigned)sh.row_blocks * (unsigned)sh.chunks, id = linear_block();
+  if (id >= nblocks) return;
+  unsigned block = sh.xcd_map ? xcd_contiguous_block(id, nblocks) : id;
+  int cfirst = 0, cend = sh.k;
+  if (sh.chunks > 1) {
+    const int chunk = (int)(block / (unsigned)sh.row_blocks);
+    block = block % (unsigned)sh.row_blocks;
+    cfirst = sh.chunk_first<VW>(chunk);
+    cend = sh.chunk_first<VW>(chunk + 1);
+  }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  T *wval = s_val[wave];
+  unsigned *woff = s_off[wave];
+  const int gs = sh.lpr * sh.par;
+  const int group = lane / gs, sub = lane - group * gs;
+  const int e = sub / sh.lpr, l = sub - e * sh.lpr;
+  const long long row0 = ((long long)block * 4 + wave) * sh.groups;
+  if (row0 >= nrows) return;
+  const int rows_here = (int)min((long long)sh.groups, nrows - row0);
+  const bool mine = group < rows_here;  // lanes past the last group of a wavefront have no row
+  const int ps = pos[row0 + min(group, rows_here)], pe = pos[row0 + min(group + 1, rows_here)];
+  // the row of C is asked for before anything that depends on the positions
+  const int col = min(cfirst + l * VW, cend - VW);
+  const bool writes = mine && e == 0 && cfirst + l * VW < cend;
+  T *cp = C + (row0 + group) * ldc + col;
+  V cin = {};
+  if (writes) cin = load_stream(reinterpret_cast<const V *>(cp));
+  const int first = __shfl(ps, 0, 64), end = __shfl(pe, 63, 64);
+  const unsigned col_bytes = (unsigned)(col * (int)sizeof(T));
+  T acc[VW];
+#pragma unroll
+  for (int i = 0; i < VW; ++i) acc[i] = T(0);
+  for (int w0 = first; w0 < end;) {
+    const int count = min(kStaged, end - w0);
+#pragma unroll
+    for (int i = 0; i < kStaged / 64; ++i) {
+      const int j = i * 64 + lane;
+      if (j < count) {
+        const unsigned c = (unsigned)load_stream(crd + w0 + j);
+        woff[j] = WIDE ? c : c * (unsigned)(ldb * sizeof(T));
+        wval[j] = load_stream(val + w0 + j);
+      }
     }
-    // Every lane runs every step (the bpermutes need their source lanes active).  With DEEP, steps go
-    // together in batches of 8, 4, 2 and 1: the B rows of a batch are loaded first, without any condition
-    // -- a lane group past the row end reads the row of a lane that holds column 0 and value 0, a lane
-    // past the last column of B reads column 0 -- and then added in order, so a lane keeps up to 8
-    // gathered rows in flight.  (Loads inside the `t < cnt` test are not unrolled by the compiler and
-    // are waited for one by one, which is what !DEEP does: better where B comes from HBM anyway.)
-    const int colc = col < k ? col : 0;
-    auto batch = [&](int t0, auto unr) {
+    wave_lds_sync();
+    int t = max(ps, w0) - w0;
+    const int hi = min(pe - w0, kStaged);
+    auto batch = [&](auto unr) {
       constexpr int UNR = decltype(unr)::value;
       T a[UNR];
-      if (VEC) {
-        V b[UNR];
+      V b[UNR];
 #pragma unroll
-        for (int u = 0; u < UNR; ++u) {
-          const int t = t0 + u * G + g;
-          const int cj = __shfl(c_l, t & 63, 64);
-          a[u] = __shfl(a_l, t & 63, 64);
-          b[u] = *reinterpret_cast<const V *>(B + (long long)cj * ldb + colc);
-        }
+      for (int u = 0; u < UNR; ++u) {
+        const int at = min(t + u * sh.par + e, hi - 1);
+        const unsigned o = woff[at];
+        a[u] = wval[at];
+        const char *bp = reinterpret_cast<const char *>(B);
+        if (WIDE)
+          b[u] = *reinterpret_cast<const V *>(bp + ((unsigned long long)o * (unsigned long long)ldb * sizeof(T) + col_bytes));
+        else
+          b[u] = *reinterpret_cast<const V *>(bp + (o + col_bytes));
+      }
 #pragma unroll
-        for (int u = 0; u < UNR; ++u) {
-          if (t0 + u * G + g < cnt && col < k) {
+      for (int u = 0; u < UNR; ++u) {
+        if (t + u * sh.par + e < hi) {
+          if constexpr (VW == 1) {
+            acc[0] = acc[0] + a[u] * b[u];
+          } else {
 #pragma unroll
-            for (int e = 0; e < VW; ++e) acc[e] = acc[e] + a[u] * b[u][e];
-          }
-        }
-      } else {
-        T b[UNR][VW];
-#pragma unroll
-        for (int u = 0; u < UNR; ++u) {
-          const int t = t0 + u * G + g;
-          const int cj = __shfl(c_l, t & 63, 64);
-          a[u] = __shfl(a_l, t & 63, 64);
-          const T *bp = B + (long long)cj * ldb;
-#pragma unroll
-          for (int e = 0; e < VW; ++e) b[u][e] = bp[col + e < k ? col + e : 0];
-        }
-#pragma unroll
-        for (int u = 0; u < UNR; ++u) {
-          if (t0 + u * G + g < cnt) {
-#pragma unroll
-            for (int e = 0; e < VW; ++e)
-              if (col + e < k) acc[e] = acc[e] + a[u] * b[u][e];
+            for (int i = 0; i < VW; ++i) acc[i] = acc[i] + a[u] * b[u][i];
           }
         }
       }
+      t += UNR * sh.par;
     };
-    int t0 = 0;
-    if (DEEP) {
-      for (; t0 + 7 * G < cnt; t0 += 8 * G) batch(t0, std::integral_constant<int, 8>());
-      if (t0 + 3 * G < cnt) {
-        batch(t0, std::integral_constant<int, 4>());
-        t0 += 4 * G;
-      }
-      if (t0 + G < cnt) {
-        batch(t0, std::integral_constant<int, 2>());
-        t0 += 2 * G;
-      }
-    }
-    for (; t0 < cnt; t0 += G) batch(t0, std::integral_constant<int, 1>());
+    if (DEPTH >= 4)
+      for (; hi - t > 2 * sh.par;) batch(std::integral_constant<int, 4>());
+    if (DEPTH >= 2)
+      for (; hi - t > sh.par;) batch(std::integral_constant<int, 2>());
+    for (; hi - t > 0;) batch(std::integral_constant<int, 1>());
+    if (end - w0 <= kStaged) break;
+    w0 += kStaged;
+    wave_lds_sync();  // the next window goes into the same LDS
   }
+  for (int o = sh.par >> 1; o > 0; o >>= 1) {  // lane e of the group adds lane e + o; the total ends in e = 0
+    const int src = min(lane + o * sh.lpr, 63) * 4;
 #pragma unroll
-  for (int o = LPR; o < 64; o <<= 1) {
-#pragma unroll
-    for (int e = 0; e < VW; ++e) acc[e] = acc[e] + __shfl_xor(acc[e], o, 64);
+    for (int i = 0; i < VW; ++i) acc[i] = acc[i] + lane_get(src, acc[i]);
   }
-  if (g == 0 && col < k) {
-    T *cp = C + row * ldc + col;
-    if (VEC) {
-      V cin = load_stream(reinterpret_cast<V *>(cp));
-#pragma unroll
-      for (int e = 0; e < VW; ++e) cin[e] = acc[e] + cin[e];
-      store_stream(reinterpret_cast<V *>(cp), cin);
+  if (writes) {
+    if constexpr (VW == 1) {
+      cin = acc[0] + cin;
     } else {
 #pragma unroll
-      for (int e = 0; e < VW; ++e)
-        if (col + e < k) cp[e] = acc[e] + cp[e];
+      for (int i = 0; i < VW; ++i) cin[i] = acc[i] + cin[i];
     }
+    store_stream(reinterpret_cast<V *>(cp), cin);
   }
 }
 
-// One group of LPR lanes per row of A: a wavefront works on G = 64/LPR rows at a time,
-// ROUNDS times over (once by default).  Each group walks its own row, LPR non-zeros per coalesced read of
-// crd/val, one B row (LPR 128-bit loads) per non-zero, and keeps the row of C in its own
-// registers: no reduction across lanes, G rows of loads in flight per instruction, and
-// the G rows of C a wavefront writes are neighbours.  For short, even rows (stencils,
-// meshes, fixed-degree graphs) this does the work of the kernel above with a quarter of
-// the wavefronts and none of its shuffles; one very long row would leave the other
-// groups of its wavefront idle, so skewed matrices stay with the kernel above.
-template <typename T, int LPR, int ROUNDS, bool XCD>
-__global__ __launch_bounds__(256) void spmm_group_row_kernel(int nrows, const int *__restrict__ pos,
-                                                             const int *__restrict__ crd,
-                                                             const T *__restrict__ val, const T *__restrict__ B,
-                                                             long long ldb, T *__restrict__ C, long long ldc) {
-  typedef typename RowVec<T>::type V;
-  constexpr int VW = RowVec<T>::width;
-  constexpr int G = 64 / LPR;
-  const int lane = threadIdx.x & 63;
-  const int g = lane / LPR;
-  const int l = lane % LPR;
-  // Workgroups go to the 8 XCDs round-robin; mapped like this each XCD works on one contiguous eighth of
-  // the rows, so with local columns its L2 fetches an eighth of B instead of all of it.
-  const unsigned block = XCD ? xcd_contiguous_block(blockIdx.x, gridDim.x) : blockIdx.x;
-  const long long wave_row0 = ((long long)block * 4 + (threadIdx.x >> 6)) * (G * ROUNDS);
-#pragma unroll 1
-  for (int r = 0; r < ROUNDS; ++r) {
-    const long long row = wave_row0 + r * G + g;
-    int start = 0, end = 0;
-    if (row < nrows) {
-      start = pos[row];
-      end = pos[row + 1];
-    }
-    V acc = {};
-    for (int base = start; base < end; base += LPR) {
-      const int cnt = min(LPR, end - base);
-      int c_l = 0;
-      T a_l = T(0);
-      if (l < cnt) {
-        c_l = load_stream(crd + base + l);
-        a_l = load_stream(val + base + l);
-      }
-      // Non-zeros go together in batches of 8, 4, 2 and 1: the B rows of a batch are loaded first, then
-      // added in order, so a lane keeps up to 8 gathered rows in flight (a loop that loads and adds one
-      // non-zero per trip is not unrolled by the compiler and waits for every row before it asks for the next)
-      auto batch = [&](int t0, auto unr) {
-        constexpr int UNR = decltype(unr)::value;
-        T a[UNR];
-        V b[UNR];
-#pragma unroll
-        for (int u = 0; u < UNR; ++u) {
-          const int src = g * LPR + t0 + u;  // a lane of this group: it runs the same trip
-          const int cj = __shfl(c_l, src, 64);
-          a[u] = __shfl(a_l, src, 64);
-          b[u] = *reinterpret_cast<const V *>(B + (long long)cj * ldb + l * VW);
-        }
-#pragma unroll
-        for (int u = 0; u < UNR; ++u) {
-#pragma unroll
-          for (int e = 0; e < VW; ++e) acc[e] = acc[e] + a[u] * b[u][e];
-        }
-      };
-      int t0 = 0;
-      for (; t0 + 8 <= cnt; t0 += 8) batch(t0, std::integral_constant<int, 8>());
-      if (t0 + 4 <= cnt) {
-        batch(t0, std::integral_constant<int, 4>());
-        t0 += 4;
-      }
-      if (t0 + 2 <= cnt) {
-        batch(t0, std::integral_constant<int, 2>());
-        t0 += 2;
-      }
-      if (t0 < cnt) batch(t0, std::integral_constant<int, 1>());
-    }
-    if (row < nrows) {
-      V *cp = reinterpret_cast<V *>(C + row * ldc + l * VW);
-      V cin = load_stream(cp);
-#pragma unroll
-      for (int e = 0; e < VW; ++e) cin[e] = acc[e] + cin[e];
-      store_stream(cp, cin);
-    }
-  }
+// Two names for the one body: profiles and lapis_hip_spmm_last_kernel tell the two regimes apart.
+template <typename T, int VW, int DEPTH, bool WIDE>
+__global__ __launch_bounds__(256) void spmm_wave_row_kernel(int nrows, SpmmShape shape, const int *__restrict__ pos,
+                                                            const int *__restrict__ crd, const T *__restrict__ val,
+                                                            const T *__restrict__ B, long long ldb, T *__restrict__ C,
+                                                            long long ldc) {
+  spmm_rows_body<T, VW, DEPTH, WIDE>(nrows, shape, pos, crd, val, B, ldb, C, ldc);
+}
+template <typename T, int VW, int DEPTH, bool WIDE>
+__global__ __launch_bounds__(256) void spmm_group_row_kernel(int nrows, SpmmShape shape, const int *__restrict__ pos,
+                                                             const int *__restrict__ crd, const T *__restrict__ val,
+                                                             const T *__restrict__ B, long long ldb, T *__restrict__ C,
+                                                             long long ldc) {
+  spmm_rows_body<T, VW, DEPTH, WIDE>(nrows, shape, pos, crd, val, B, ldb, C, ldc);
 }
 
 // LDS-staged row blocks, for matrices with a band around the diagonal.  A workgroup of
@@ -296,82 +276,178 @@ __global__ __launch_bounds__(1024) void spmm_rowblock_lds_kernel(int nrows, int 
 
 // Batched CSRV product of examples/bspmm.py:22-50: A is CSR over (n1, n2) and every
 // non-zero carries nh values (a trailing dense batch); out(i, d, h) += A(i, c, h) * V(c, d, h).
-// One wavefront per row; lanes walk the dh*nh values of an output row, so the read of
-// a V row is coalesced and the nh batch values of a non-zero are read contiguously.
-__global__ __launch_bounds__(256) void bspmm_csrv_kernel(int n1, int dh, int nh, const int *__restrict__ pos,
-                                                         const int *__restrict__ crd,
-                                                         const float *__restrict__ val,
-                                                         const float *__restrict__ V, float *__restrict__ out) {
-  const int lane = threadIdx.x & 63;
-  const long long row = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= n1) return;
-  const int start = pos[row], end = pos[row + 1];
-  const long long K = (long long)dh * nh;
-  for (long long j = lane; j < K; j += 64) {
-    const int h = (int)(j % nh);
-    float acc = out[row * K + j];
-    for (int e = start; e < end; ++e) {
-      const float prod = val[(long long)e * nh + h] * V[(long long)crd[e] * K + j];
+// A row of V is K = dh*nh consecutive floats, and column j of it is multiplied by value j % nh of the
+// non-zero.  A group of lpr lanes takes one row of A and one chunk of its columns, four per lane; the
+// chunk's sums start from `out` and take the non-zeros in order, one rounding per product and per sum,
+// as the reference's nest does.  A wavefront stages the coordinates and the values of its rows in LDS, `window`
+// entries of every row at a time; up to 4 rows of V are asked for before the first is added.
+// HV: nh is a multiple of 4, so a lane's four values are neighbours, one 128-bit LDS read.
+// Measured at 16384 rows of 32, dh = 32, nh = 8: 195 us with a wavefront per row that read each value and coordinate
+// from global memory for every 64 columns, 59 us now (7.3 TB/s of rows of V that miss L2); with twice the LDS 69.
+constexpr int kStagedBatched = 1024;        // values per wavefront and window
+constexpr int kStagedBatchedEntries = 256;  // non-zeros per wavefront and window at most
+constexpr int kBatchedGroups = 8;           // rows per wavefront at most: rows are long against narrow chunks
+template <bool HV, bool WIDE>
+__global__ __launch_bounds__(256) void bspmm_csrv_kernel(int n1, SpmmShape sh, int nh, int window_log2,
+                                                         const int *__restrict__ pos, const int *__restrict__ crd,
+                                                         const float *__restrict__ val, const float *__restrict__ V,
+                                                         float *__restrict__ out) {
+  typedef RowVec<float>::loose W;
+  __shared__ __align__(16) float s_val[4][kStagedBatched];
+  __shared__ unsigned s_off[4][kStagedBatchedEntries];
+  const unsigned nblocks = (unsigned)sh.row_blocks * (unsigned)sh.chunks, id = linear_block();
+  if (id >= nblocks) return;
+  unsigned block = xcd_contiguous_block(id, nblocks);
+  const int chunk = (int)(block / (unsigned)sh.row_blocks);
+  block = block % (unsigned)sh.row_blocks;
+  const int cfirst = sh.chunk_first<4>(chunk), cend = sh.chunk_first<4>(chunk + 1);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  unsigned *woff = s_off[wave];
+  float *wval = s_val[wave];
+  const int group = lane / sh.lpr, l = lane - group * sh.lpr;
+  const long long row0 = ((long long)block * 4 + wave) * sh.groups;
+  if (row0 >= n1) return;
+  const int rows_here = (int)min((long long)sh.groups, n1 - row0);
+  const int ps = pos[row0 + min(group, rows_here)], pe = pos[row0 + min(group + 1, rows_here)];
+  const long long K = sh.k;
+  const int col = min(cfirst + l * 4, cend - 4);
+  const bool writes = group < rows_here && cfirst + l * 4 < cend;
+  const int window = 1 << window_log2;
+  int h[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) h[i] = (col + i) % nh;
+  float *op = out + (row0 + group) * K + col;
+  W acc = {};
+  if (writes) acc = *reinterpret_cast<const W *>(op);
+  const int slots = sh.groups << window_log2;
+  int done = 0;                                      // entries of each row already taken
+  const int mine = group < rows_here ? pe - ps : 0;  // entries of this lane's row
+  while (__ballot(done < mine)) {
+    // slot j: entry done + j % window of row j / window (its first entry and length sit in that row's lanes)
+    // (all lanes run every trip: the shuffles need their source lanes active)
+    for (int j0 = 0; j0 < slots; j0 += 64) {
+      const int j = j0 + lane;
+      const int from = min((j >> window_log2) * sh.lpr, 63);
+      const int at = done + (j & (window - 1));
+      const int first = __shfl(ps, from, 64), count = __shfl(mine, from, 64);
+      if (j < slots && at < count) {
+        const unsigned c = (unsigned)load_stream(crd + first + at);
+        woff[j] = WIDE ? c : c * (unsigned)(K * 4);
+      }
+    }
+    for (int g = 0; g < sh.groups; ++g) {  // a row's values of a window are one contiguous stretch
+      const int first = __shfl(ps, g * sh.lpr, 64), count = min(__shfl(mine, g * sh.lpr, 64) - done, window);
+      const float *vp = val + ((long long)first + done) * nh;
+      for (int i = lane; i < count * nh; i += 64) wval[(g << window_log2) * nh + i] = vp[i];
+    }
+    wave_lds_sync();
+    const int hi = min(mine - done, window);
+    const unsigned *goff = woff + (group << window_log2);
+    const float *gval = wval + (group << window_log2) * nh;
+    int t = 0;
+    auto batch = [&](auto unr) {
+      constexpr int UNR = decltype(unr)::value;
+      W b[UNR];
+#pragma unroll
+      for (int u = 0; u < UNR; ++u) {
+        const unsigned o = goff[min(t + u, hi - 1)];
+        if (WIDE)
+          b[u] = *reinterpret_cast<const W *>(V + (long long)o * K + col);
+        else
+          b[u] = *reinterpret_cast<const W *>(reinterpret_cast<const char *>(V) + (o + (unsigned)(col * 4)));
+      }
+#pragma unroll
+      for (int u = 0; u < UNR; ++u) {
+        if (t + u < hi) {
+          const float *au = gval + (t + u) * nh;
+          v4f a;
+          if (HV) {
+            a = *reinterpret_cast<const v4f *>(au + h[0]);
+          } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) a[i] = au[h[i]];
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[i] = a[i] * b[u][i] + acc[i];
+        }
+      }
+      t += UNR;
+    };
+    for (; hi - t > 2;) batch(std::integral_constant<int, 4>());
+    for (; hi - t > 0;) batch(std::integral_constant<int, 2>());
+    done += window;
+    wave_lds_sync();  // the next window goes into the same LDS
+  }
+  if (writes) *reinterpret_cast<W *>(op) = acc;
+}
+
+// K smaller than a vector (or past int32): a lane per element of `out`.
+__global__ __launch_bounds__(256) void bspmm_csrv_scalar_kernel(long long n1, long long K, int nh,
+                                                                const int *__restrict__ pos,
+                                                                const int *__restrict__ crd,
+                                                                const float *__restrict__ val,
+                                                                const float *__restrict__ V, float *__restrict__ out) {
+  for (long long t = (long long)blockIdx.x * 256 + threadIdx.x; t < n1 * K; t += (long long)gridDim.x * 256) {
+    const long long row = t / K, j = t % K;
+    float acc = out[t];
+    for (int e = pos[row]; e < pos[row + 1]; ++e) {
+      const float prod = val[(long long)e * nh + j % nh] * V[(long long)crd[e] * K + j];
       acc = prod + acc;
     }
-    out[row * K + j] = acc;
+    out[t] = acc;
   }
 }
 
-template <typename T, int LPR, bool VEC>
-void launch_wave_row(int64_t nrows, int64_t k, const int *pos, const int *crd, const T *val, const T *B, int64_t ldb,
-                     T *C, int64_t ldc, hipStream_t st, bool deep) {
-  constexpr int VW = RowVec<T>::width;
-  const dim3 grid((unsigned)ceil_div(nrows, 4), (unsigned)ceil_div(k, LPR * VW));
-  if (deep)
-    launch_timed(spmm_wave_row_kernel<T, LPR, VEC, true>, grid, dim3(256), st, (int)nrows, (int)k, pos, crd, val, B,
-                 (long long)ldb, C, (long long)ldc);
+template <typename T>
+struct SpmmArgs {
+  int64_t nrows, k;
+  const int *pos, *crd;
+  const T *val, *B;
+  int64_t ldb;
+  T *C;
+  int64_t ldc;
+  hipStream_t st;
+};
+
+// Cuts k columns into chunks of at most `vectors_max` vectors of VW elements (a ragged rest counts as one
+// more) and deals `nrows` rows to groups of lanes per chunk, `par` non-zeros of a row at a time.
+inline SpmmShape make_shape(int64_t nrows, int64_t k, int vw, int vectors_max, int par, int xcd_map) {
+  SpmmShape s;
+  s.k = (int)k;
+  s.vectors = (int)(k / vw);
+  const int rest = k % vw != 0;
+  s.chunks = (int)ceil_div(s.vectors + rest, vectors_max);
+  while (ceil_div(s.vectors, s.chunks) + rest > vectors_max) ++s.chunks;
+  s.lpr = (int)ceil_div(s.vectors, s.chunks) + rest;
+  s.par = par;
+  while (s.par > 1 && s.lpr * s.par > 64) s.par /= 2;
+  s.groups = 64 / (s.lpr * s.par);
+  s.row_blocks = (int)ceil_div(nrows, 4 * s.groups);
+  s.xcd_map = xcd_map;
+  return s;
+}
+
+// smallest power of two >= n, at most 64
+inline int pow2_up(int64_t n) {
+  int p = 1;
+  while (p < 64 && p < n) p *= 2;
+  return p;
+}
+
+template <typename T, int VW, int DEPTH, bool WIDE>
+int launch_spmm_rows(const SpmmArgs<T> &a, const SpmmShape &shape) {
+  const int64_t blocks = (int64_t)shape.row_blocks * shape.chunks;
+  if (blocks > 0x7fffffffLL)
+    return set_error(LAPIS_HIP_ERR_INVALID_ARGUMENT, "spmm: %lld rows times %d column chunks exceed the grid limit",
+                     (long long)a.nrows, shape.chunks);
+  if (shape.groups == 1)
+    launch_timed(spmm_wave_row_kernel<T, VW, DEPTH, WIDE>, grid_of(blocks), dim3(256), a.st, (int)a.nrows, shape, a.pos,
+                 a.crd, a.val, a.B, (long long)a.ldb, a.C, (long long)a.ldc);
   else
-    launch_timed(spmm_wave_row_kernel<T, LPR, VEC, false>, grid, dim3(256), st, (int)nrows, (int)k, pos, crd, val, B,
-                 (long long)ldb, C, (long long)ldc);
-}
-
-template <typename T, bool VEC>
-void launch_wave_row_any(int64_t nrows, int64_t k, const int *pos, const int *crd, const T *val, const T *B, int64_t ldb,
-                         T *C, int64_t ldc, hipStream_t st, bool deep) {
-  constexpr int VW = RowVec<T>::width;
-  // lanes per chunk of a B row: the smallest power of two that covers k, at most a wavefront
-  int lpr = 1;
-  while (lpr < 64 && (int64_t)lpr * VW < k) lpr *= 2;
-  switch (lpr) {
-    case 1: launch_wave_row<T, 1, VEC>(nrows, k, pos, crd, val, B, ldb, C, ldc, st, deep); break;
-    case 2: launch_wave_row<T, 2, VEC>(nrows, k, pos, crd, val, B, ldb, C, ldc, st, deep); break;
-    case 4: launch_wave_row<T, 4, VEC>(nrows, k, pos, crd, val, B, ldb, C, ldc, st, deep); break;
-    case 8: launch_wave_row<T, 8, VEC>(nrows, k, pos, crd, val, B, ldb, C, ldc, st, deep); break;
-    case 16: launch_wave_row<T, 16, VEC>(nrows, k, pos, crd, val, B, ldb, C, ldc, st, deep); break;
-    case 32: launch_wave_row<T, 32, VEC>(nrows, k, pos, crd, val, B, ldb, C, ldc, st, deep); break;
-    default: launch_wave_row<T, 64, VEC>(nrows, k, pos, crd, val, B, ldb, C, ldc, st, deep); break;
-  }
-}
-
-template <typename T, int LPR, int ROUNDS>
-void launch_group_row_r(int64_t nrows, const int *pos, const int *crd, const T *val, const T *B, int64_t ldb, T *C,
-                        int64_t ldc, hipStream_t st) {
-  constexpr int rows_per_block = 4 * (64 / LPR) * ROUNDS;
-  const char *xcd = getenv("LAPIS_HIP_SPMM_XCD_MAP");
-  if (xcd && atoi(xcd) == 0)
-    launch_timed(spmm_group_row_kernel<T, LPR, ROUNDS, false>, dim3((unsigned)ceil_div(nrows, rows_per_block)), dim3(256),
-                 st, (int)nrows, pos, crd, val, B, (long long)ldb, C, (long long)ldc);
-  else
-    launch_timed(spmm_group_row_kernel<T, LPR, ROUNDS, true>, dim3((unsigned)ceil_div(nrows, rows_per_block)), dim3(256),
-                 st, (int)nrows, pos, crd, val, B, (long long)ldb, C, (long long)ldc);
-}
-
-template <typename T, int LPR>
-void launch_group_row(int64_t nrows, const int *pos, const int *crd, const T *val, const T *B, int64_t ldb, T *C,
-                      int64_t ldc, hipStream_t st) {
-  // Rounds of rows per wavefront.  One is fastest now that a lane keeps several B rows in flight (Laplace3D_100
-  // k = 64: 0.195 / 0.196 / 0.209 ms with 1 / 2 / 4 rounds; Elasticity3D_60: 0.606 / 0.623 / 0.649 ms): the fewer
-  // rows an XCD has in flight, the smaller the part of B its L2 has to hold.  LAPIS_HIP_SPMM_ROUNDS = 2, 4 for tuning.
-  const int rounds = getenv("LAPIS_HIP_SPMM_ROUNDS") ? atoi(getenv("LAPIS_HIP_SPMM_ROUNDS")) : 1;
-  if (rounds == 4) launch_group_row_r<T, LPR, 4>(nrows, pos, crd, val, B, ldb, C, ldc, st);
-  else if (rounds == 2) launch_group_row_r<T, LPR, 2>(nrows, pos, crd, val, B, ldb, C, ldc, st);
-  else launch_group_row_r<T, LPR, 1>(nrows, pos, crd, val, B, ldb, C, ldc, st);
+    launch_timed(spmm_group_row_kernel<T, VW, DEPTH, WIDE>, grid_of(blocks), dim3(256), a.st, (int)a.nrows, shape, a.pos,
+                 a.crd, a.val, a.B, (long long)a.ldb, a.C, (long long)a.ldc);
+  LAPIS_LAUNCH_CHECK();
+  return LAPIS_HIP_OK;
 }
 
 constexpr int kSpmmLdsBytes = 128 * 1024;  // staged rows of B per workgroup of the LDS kernel
@@ -432,75 +508,75 @@ int spmm_impl(const char *what, const lapis_hip_csr_plan *plan, int64_t nrows, i
   if (ncols == 0) return LAPIS_HIP_OK;  // a matrix without columns has no non-zeros
   hipStream_t st = as_stream(stream);
   constexpr int VW = RowVec<T>::width;
-  const bool vec = aligned16(B) && aligned16(C) && (ldb % VW == 0) && (ldc % VW == 0) && (k % VW == 0);
-  // The LDS-staged kernel: whole B rows of a power-of-two number of vectors, between 64 bytes and 1 KB,
-  // and at least three non-zeros per row inside the window it would stage.
-  const int64_t lpr = vec ? k / VW : 0;
-  const char *force = getenv("LAPIS_HIP_SPMM_KERNEL");  // "lds" / "wave": tuning and tests
-  bool use_lds = false;
-  int rb = 0, halo = 0, hi = 0;
-  if (vec && lpr >= 4 && lpr <= 64 && (lpr & (lpr - 1)) == 0) {
-    lds_block_shape(k * (int64_t)sizeof(T), &rb, &halo, &hi);
+  const char *force = getenv("LAPIS_HIP_SPMM_KERNEL");  // "lds" / "wave" / "group": tuning and tests
+  if (force && !strcmp(force, "lds")) {
     // Never chosen automatically: measured on MI355X it loses to the kernels below wherever it applies
-    // (7-point stencil 100^3, k = 64 fp32: 0.625 ms against 0.259 ms; 27-point x 3 unknowns 60^3: 1.55 against
-    // 0.94 ms).  The window a block stages is read from L2 once per block, halo included (twice B in
+    // (7-point stencil 100^3, k = 64 fp32: 0.625 ms against 0.195 ms; 27-point x 3 unknowns 60^3: 1.55 against
+    // 0.60 ms).  The window a block stages is read from L2 once per block, halo included (twice B in
     // all), the block cannot start on its rows before the window is in, and the reuse it serves -- a
     // B row used by neighbouring rows -- is reuse the 32 KB vector cache of the CU already catches.
-    if (force && !strcmp(force, "lds")) use_lds = true;
+    const bool vec = aligned16(B) && aligned16(C) && (ldb % VW == 0) && (ldc % VW == 0) && (k % VW == 0);
+    const int64_t lpr = vec ? k / VW : 0;
+    if (lpr >= 4 && lpr <= 64 && (lpr & (lpr - 1)) == 0) {
+      int rb = 0, halo = 0, hi = 0;
+      lds_block_shape(k * (int64_t)sizeof(T), &rb, &halo, &hi);
+      g_last_spmm_kernel = "spmm_rowblock_lds_kernel";
+      switch (lpr) {
+        case 4: return launch_rowblock_lds<T, 4>(nrows, ncols, rb, halo, pos, crd, val, B, ldb, C, ldc, st);
+        case 8: return launch_rowblock_lds<T, 8>(nrows, ncols, rb, halo, pos, crd, val, B, ldb, C, ldc, st);
+        case 16: return launch_rowblock_lds<T, 16>(nrows, ncols, rb, halo, pos, crd, val, B, ldb, C, ldc, st);
+        case 32: return launch_rowblock_lds<T, 32>(nrows, ncols, rb, halo, pos, crd, val, B, ldb, C, ldc, st);
+        default: return launch_rowblock_lds<T, 64>(nrows, ncols, rb, halo, pos, crd, val, B, ldb, C, ldc, st);
+      }
+    }
   }
-  if (force && !strcmp(force, "wave")) use_lds = false;
-  // Group-per-row: whole B rows of up to 32 vectors (a wavefront holds at least two rows), rows short and
-  // even enough that the groups of a wavefront finish together.
-  bool use_group = false;
-  if (vec && lpr >= 1 && lpr <= 32 && (lpr & (lpr - 1)) == 0 && plan) {
+
+  const int vw = k >= VW ? VW : 1;
+  const int vectors = (int)std::min<int64_t>(64, ceil_div(k, vw));  // lanes per row of B
+  const int wave_row = 64 / pow2_up(vectors);                       // par that gives a wavefront one row
+  int par = wave_row;
+  bool xcd = true;
+  int depth = 4;
+  if (plan && plan->stats.mean_row_len > 0.0) {
     const lapis_hip_csr_stats &ps = plan->stats;
-    // ... and the B rows a stretch of 1024 non-zeros touches fit the L2s (matrices with column locality:
-    // 7-point stencil, k = 64 fp32: 0.259 ms against 0.433 ms for the wavefront-per-row kernel, k = 16: 0.080
-    // against 0.310; 81 per row FEM: 0.94 against 1.01).  With columns all over B every gather goes to HBM
-    // and the wavefront-per-row kernel, which keeps more of them in flight, is 6-30 % faster.
-    use_group = ps.mean_row_len <= 256.0 && (double)ps.max_row_len <= 4.0 * std::max(ps.mean_row_len, 8.0) &&
-                ps.mean_chunk_col_span >= 0.0 && ps.mean_chunk_col_span * (double)(k * sizeof(T)) <= 32.0 * 1024 * 1024;
-  }
-  if (force) {
-    use_group = !strcmp(force, "group") && vec && lpr >= 1 && lpr <= 32 && (lpr & (lpr - 1)) == 0;
-    if (use_group) use_lds = false;
-  }
-  if (use_group && !use_lds) {
-    g_last_spmm_kernel = "spmm_group_row_kernel";
-    switch (lpr) {
-      case 1: launch_group_row<T, 1>(nrows, pos, crd, val, B, ldb, C, ldc, st); break;
-      case 2: launch_group_row<T, 2>(nrows, pos, crd, val, B, ldb, C, ldc, st); break;
-      case 4: launch_group_row<T, 4>(nrows, pos, crd, val, B, ldb, C, ldc, st); break;
-      case 8: launch_group_row<T, 8>(nrows, pos, crd, val, B, ldb, C, ldc, st); break;
-      case 16: launch_group_row<T, 16>(nrows, pos, crd, val, B, ldb, C, ldc, st); break;
-      default: launch_group_row<T, 32>(nrows, pos, crd, val, B, ldb, C, ldc, st); break;
+    const double mean = ps.mean_row_len;
+    const double span_bytes = ps.mean_chunk_col_span * (double)(k * sizeof(T));
+    const bool local = ps.mean_chunk_col_span >= 0.0 && span_bytes <= 32.0 * 1024 * 1024;
+    const bool even = mean <= 256.0 && (double)ps.max_row_len <= 4.0 * std::max(mean, 8.0);
+    if (even) {
+      // Several rows per wavefront, as many as leave their entries room in the staged window and a group at
+      // least 8 steps; where the rows of B come from HBM (columns of 1024 non-zeros spread over more than
+      // 32 MB of B) as few as the 8 steps allow (1 M rows of 32, k = 64 fp32: 1203 us against 1290 with 4 rows
+      // per wavefront); and in a matrix of few rows more lanes per row until there are wavefronts for the
+      // chip (15 000 rows of 32, k = 3 fp64: 7.0 us against 12.0).
+      auto groups = [&](int q) { return 64 / (vectors * q); };
+      par = 1;
+      while (par < wave_row && 2 * par * 8.0 <= mean && (!local || groups(par) * mean > kStaged)) par *= 2;
+      while (par < wave_row && 2 * par * 3.0 <= mean && ceil_div(nrows, groups(par)) < 2500) par *= 2;
     }
-    LAPIS_LAUNCH_CHECK();
-    return LAPIS_HIP_OK;
+    // Each XCD takes a contiguous part of the rows, so that neighbouring rows find each other's rows of B in its
+    // L2; not where they span more than that L2 holds anyway (7-point 97^3, k = 64 fp64: 391 us against 412).
+    xcd = !(local && span_bytes > 8.0 * 1024 * 1024);
+    // Rows of B in flight per lane: 4, but where the columns are all over a B that L2 does not hold more requests
+    // only lengthen each other's way, and the registers they take are wavefronts lost: 2 (50 000 rows of 60,
+    // k = 64 fp32: 55 us against 70), and 1 for rows of B of up to 16 vectors from HBM (1 M rows of 32, k = 64 fp32:
+    // 1209 us against 1242; k = 64 fp64, 32 vectors, would lose 10 %).
+    const bool scattered = ps.mean_chunk_col_span > 0.25 * (double)ncols;
+    if (scattered && span_bytes > 8.0 * 1024 * 1024) depth = !local && vectors <= 16 && mean >= 16.0 ? 1 : 2;
   }
-  if (use_lds) {
-    g_last_spmm_kernel = "spmm_rowblock_lds_kernel";
-    switch (lpr) {
-      case 4: return launch_rowblock_lds<T, 4>(nrows, ncols, rb, halo, pos, crd, val, B, ldb, C, ldc, st);
-      case 8: return launch_rowblock_lds<T, 8>(nrows, ncols, rb, halo, pos, crd, val, B, ldb, C, ldc, st);
-      case 16: return launch_rowblock_lds<T, 16>(nrows, ncols, rb, halo, pos, crd, val, B, ldb, C, ldc, st);
-      case 32: return launch_rowblock_lds<T, 32>(nrows, ncols, rb, halo, pos, crd, val, B, ldb, C, ldc, st);
-      default: return launch_rowblock_lds<T, 64>(nrows, ncols, rb, halo, pos, crd, val, B, ldb, C, ldc, st);
-    }
+  if (force) par = !strcmp(force, "group") && vectors <= 32 ? 1 : wave_row;
+  const SpmmShape shape = make_shape(nrows, k, vw, vectors, par, xcd);
+  g_last_spmm_kernel = shape.groups == 1 ? "spmm_wave_row_kernel" : "spmm_group_row_kernel";
+  const SpmmArgs<T> args{nrows, k, pos, crd, val, B, ldb, C, ldc, st};
+  const bool wide = (double)ncols * (double)ldb * sizeof(T) >= 4294967296.0;
+  if (vw == 1)
+    return wide ? launch_spmm_rows<T, 1, 4, true>(args, shape) : launch_spmm_rows<T, 1, 4, false>(args, shape);
+  if (wide) return launch_spmm_rows<T, VW, 2, true>(args, shape);
+  switch (depth) {
+    case 1: return launch_spmm_rows<T, VW, 1, false>(args, shape);
+    case 2: return launch_spmm_rows<T, VW, 2, false>(args, shape);
+    default: return launch_spmm_rows<T, VW, 4, false>(args, shape);
   }
-  g_last_spmm_kernel = "spmm_wave_row_kernel";
-  // Several gathered B rows in flight per lane pay where B rows come from L2 (columns of a chunk of A within
-  // 32 MB of B, or no plan to say otherwise); where every gather goes to HBM they only get in each other's way
-  // (config 4 of the benchmarks: 1.21 ms one at a time, 1.26 ms eight at a time).
-  bool deep = true;
-  if (plan) deep = plan->stats.mean_chunk_col_span * (double)k * sizeof(T) <= 32.0 * 1024 * 1024;
-  if (const char *d = getenv("LAPIS_HIP_SPMM_DEEP")) deep = atoi(d) != 0;
-  if (vec)
-    launch_wave_row_any<T, true>(nrows, k, pos, crd, val, B, ldb, C, ldc, st, deep);
-  else
-    launch_wave_row_any<T, false>(nrows, k, pos, crd, val, B, ldb, C, ldc, st, deep);
-  LAPIS_LAUNCH_CHECK();
-  return LAPIS_HIP_OK;
 }
 
 }  // namespace lapis
@@ -542,8 +618,38 @@ extern "C" int lapis_hip_bspmm_csrv_f32_i32(int64_t n1, int64_t n2, int64_t dh, 
   LAPIS_REQUIRE(pos && out, "bspmm_csrv: null positions or output");
   LAPIS_REQUIRE(n2 == 0 || (crd && val && V), "bspmm_csrv: null coordinates, values or V");
   if (n2 == 0) return LAPIS_HIP_OK;
-  hipLaunchKernelGGL(bspmm_csrv_kernel, dim3((unsigned)ceil_div(n1, 4)), dim3(256), 0, as_stream(stream), (int)n1,
-                     (int)dh, (int)nh, pos, crd, val, V, out);
+  hipStream_t st = as_stream(stream);
+  const int64_t K = dh * nh;
+  if (K < 4 || K > INT32_MAX || nh > kStagedBatched) {
+    const int64_t want = ceil_div(n1 * K, 256);
+    hipLaunchKernelGGL(bspmm_csrv_scalar_kernel, dim3((unsigned)std::min<int64_t>(want, 1 << 20)), dim3(256), 0, st,
+                       (long long)n1, (long long)K, (int)nh, pos, crd, val, V, out);
+    LAPIS_LAUNCH_CHECK();
+    return LAPIS_HIP_OK;
+  }
+  // As many columns of a row per group as there are (narrower chunks, whose part of V an XCD's L2 would hold,
+  // stage the same entries once per chunk: 117 us against 59 at 32 columns).
+  SpmmShape shape = make_shape(n1, K, 4, (int)std::min<int64_t>(64, ceil_div(K, 4)), 1, 1);
+  // at least 4 entries of every row per window
+  const int slots = (int)std::min<int64_t>(kStagedBatchedEntries, kStagedBatched / nh);
+  shape.groups = std::max(1, std::min({shape.groups, kBatchedGroups, slots / 4}));
+  shape.row_blocks = (int)ceil_div(n1, 4 * shape.groups);
+  int window_log2 = 0;
+  while ((2 << window_log2) * shape.groups <= slots) ++window_log2;
+  const int64_t blocks = (int64_t)shape.row_blocks * shape.chunks;
+  if (blocks > 0x7fffffffLL)
+    return set_error(LAPIS_HIP_ERR_INVALID_ARGUMENT, "bspmm_csrv: %lld rows of %lld elements exceed the grid limit",
+                     (long long)n1, (long long)K);
+  const bool wide = (double)n2 * (double)K * sizeof(float) >= 4294967296.0;
+#define LAPIS_BSPMM_LAUNCH(HV, WIDE)                                                                                  \
+  hipLaunchKernelGGL((bspmm_csrv_kernel<HV, WIDE>), grid_of(blocks), dim3(256), 0, st, (int)n1, shape, (int)nh,             \
+                     window_log2, pos, crd, val, V, out)
+  if (nh % 4 == 0) {
+    if (wide) LAPIS_BSPMM_LAUNCH(true, true); else LAPIS_BSPMM_LAUNCH(true, false);
+  } else {
+    if (wide) LAPIS_BSPMM_LAUNCH(false, true); else LAPIS_BSPMM_LAUNCH(false, false);
+  }
+#undef LAPIS_BSPMM_LAUNCH
   LAPIS_LAUNCH_CHECK();
   return LAPIS_HIP_OK;
 }

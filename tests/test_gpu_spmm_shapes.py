@@ -1,0 +1,65 @@
+"""SpMM and the batched CSRV product at the edges of their launch shapes: k around multiples of the vector width and
+of a wavefront's columns, rows longer than the staged window, rows of B at any address, every lanes-per-row split."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import dev, from_lengths
+from lapis_amd import generators as gen
+from test_gpu_spmm import _check
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 7, 10, 13, 31, 63, 127, 129, 255, 257, 259])
+def test_ragged_widths_on_short_and_long_rows(gpu, oracle, dtype, k):
+    rng = np.random.default_rng(k)
+    short = rng.integers(0, 12, 777)                                     # several rows per wavefront
+    long = np.concatenate([rng.integers(90, 240, 37), [0, 511, 512, 513, 0]])  # windows of 512 entries cut inside rows
+    for lengths, ncols in ((short, 500), (long, 3000)):
+        A = from_lengths(list(lengths), ncols, 7 + k, dtype)
+        B = gen.uniform_matrix(ncols, k, 8).astype(dtype)
+        C_in = gen.uniform_matrix(A.nrows, k, 9).astype(dtype)
+        for plan in (True, False):
+            _check(gpu, oracle, A, B, C_in, dtype, "rows of %d.., k=%d plan=%s" % (lengths[0], k, plan), plan=plan)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+def test_rows_of_B_and_C_at_any_address(gpu, oracle, dtype):
+    A = from_lengths([5] * 300, 200, 3, dtype)
+    for k, ldb, off in ((6, 7, 1), (16, 17, 3), (9, 9, 1)):
+        flat_b, flat_c = gen.uniform_matrix(1, 200 * ldb + off, 4)[0].astype(dtype), gen.uniform_matrix(1, 300 * ldb + off, 5)[0].astype(dtype)
+        view = lambda t, rows: torch.as_strided(t, (rows, k), (ldb, 1), off)
+        dB, dC = dev(flat_b), dev(flat_c)
+        B = np.lib.stride_tricks.as_strided(flat_b[off:], (200, k), (ldb * flat_b.itemsize, flat_b.itemsize)).copy()
+        want = np.lib.stride_tricks.as_strided(flat_c[off:], (300, k), (ldb * flat_c.itemsize, flat_c.itemsize)).copy()
+        oracle.spmm(A.pos, A.crd, A.val, B, want)
+        pos, crd = dev(A.pos), dev(A.crd)
+        plan = gpu.CsrPlan(A.nrows, A.ncols, pos, crd, value_bytes=np.dtype(dtype).itemsize)
+        gpu.spmm(A.nrows, A.ncols, pos, crd, dev(A.val), view(dB, 200), view(dC, 300), plan=plan)
+        got = dC.cpu().numpy()
+        assert np.allclose(view(dC, 300).cpu().numpy(), want, rtol=1e-5, atol=1e-5)
+        untouched = np.ones(got.size, bool)
+        untouched[(off + np.arange(300)[:, None] * ldb + np.arange(k)).ravel()] = False
+        assert np.array_equal(got[untouched], flat_c[untouched])
+
+
+@pytest.mark.parametrize("n,mean,k", [(70000, 4, 64), (140000, 16, 64), (140000, 16, 132)])
+def test_scattered_columns_over_a_B_larger_than_the_caches(gpu, oracle, n, mean, k):
+    A = gen.fixed_degree_random(n, mean, seed=5, dtype=np.float32)
+    B = gen.uniform_matrix(n, k, 6)
+    _check(gpu, oracle, A, B, np.zeros((n, k), np.float32), np.float32, "scattered n=%d k=%d" % (n, k), plan=True)
+
+
+@pytest.mark.parametrize("dh,nh", [(1, 1), (3, 1), (4, 1), (5, 1), (2, 3), (5, 7), (31, 8), (32, 8), (64, 4), (65, 4), (9, 300), (1, 1025)])
+def test_batched_csrv_product_shapes(gpu, oracle, dh, nh):
+    rng = np.random.default_rng(dh * 1000 + nh)
+    lengths = np.concatenate([rng.integers(0, 20, 61), [0, 300, 1, 257, 0, 33]])
+    A = from_lengths(list(lengths), 400, 17, np.float32)
+    values = rng.uniform(-1, 1, A.nnz * nh).astype(np.float32)
+    V = rng.uniform(-1, 1, (400, dh, nh)).astype(np.float32)
+    out = torch.zeros(A.nrows, dh, nh, dtype=torch.float32, device="cuda")
+    print("case", dh, nh, flush=True)
+    gpu.bspmm_csrv(A.nrows, 400, dev(A.pos), dev(A.crd), dev(values), dev(V), out)
+    assert np.array_equal(out.cpu().numpy(), oracle.bspmm_csrv(A.pos, A.crd, values, V, A.nrows))
