@@ -4,14 +4,17 @@ Outputs (in-tree, next to this package, so that they travel with a source snapsh
     lapis_amd/lib/liblapis_hip.so             the C-ABI kernel library (include/lapis_hip.h)
     lapis_amd/lib/liblapis_package_module.so  lapis_initialize / lapis_finalize / py_<func>
                                               (include/lapis_module.h), linked against the former
+    lapis_amd/lib/_lapis_calls.so             Python entry points of the device-resident calls (csrc/bindings.cpp)
     lapis_amd/bin/lapis_spmv_bench            MatrixMarket SpMV benchmark driver (csrc/spmv_bench_main.cpp)
 
 hipcc cross-compiles without a GPU.  Run ``python -m lapis_amd.build``.
 """
+import importlib.util
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -27,6 +30,7 @@ SHIM_SOURCES = ["module_shim.hip"]
 
 KERNEL_LIB = os.path.join(LIBDIR, "liblapis_hip.so")
 MODULE_LIB = os.path.join(LIBDIR, "liblapis_package_module.so")
+CALLS_LIB = os.path.join(LIBDIR, "_lapis_calls.so")
 BINDIR = os.path.join(HERE, "bin")
 BENCH_BIN = os.path.join(BINDIR, "lapis_spmv_bench")
 
@@ -67,6 +71,17 @@ def _compile(src):
     return obj
 
 
+def _bindings():
+    """csrc/bindings.cpp: host code against the headers of the interpreter and of torch (found, not imported)."""
+    torch = importlib.util.find_spec("torch").submodule_search_locations[0]
+    lib = os.path.join(torch, "lib")
+    _run([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          "-I", INCLUDE, "-I", sysconfig.get_paths()["include"], "-isystem", os.path.join(torch, "include"), "-isystem",
+          os.path.join(torch, "include", "torch", "csrc", "api", "include"), "-isystem", "/opt/rocm/include",
+          os.path.join(CSRC, "bindings.cpp"), "-L", LIBDIR, "-llapis_hip", "-L", lib, "-lc10", "-lc10_hip", "-ltorch_cpu",
+          "-ltorch_python", "-Wl,-rpath,$ORIGIN", "-o", CALLS_LIB])
+
+
 def build(verbose=False, jobs=8):
     """Compile every HIP source for gfx950 and link both shared libraries."""
     os.makedirs(LIBDIR, exist_ok=True)
@@ -77,6 +92,7 @@ def build(verbose=False, jobs=8):
     _run([_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", *kobjs, "-o", KERNEL_LIB])
     _run([_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", *sobjs, "-L", LIBDIR, "-llapis_hip",
           "-Wl,-rpath,$ORIGIN", "-o", MODULE_LIB])
+    _bindings()
     os.makedirs(BINDIR, exist_ok=True)
     _run([_hipcc(), "--offload-arch=gfx950", "-O2", "-std=c++17", "-I", INCLUDE,
           os.path.join(CSRC, "spmv_bench_main.cpp"), "-L", LIBDIR, "-llapis_hip", "-Wl,-rpath,$ORIGIN/../lib", "-o",
@@ -84,6 +100,7 @@ def build(verbose=False, jobs=8):
     if verbose:
         print("built", KERNEL_LIB)
         print("built", MODULE_LIB)
+        print("built", CALLS_LIB)
         print("built", BENCH_BIN)
     return KERNEL_LIB, MODULE_LIB
 

@@ -1,0 +1,399 @@
+// Python entry points of the device-resident calls, on the CPython and PyTorch C++ APIs.
+//
+// A call of a small matrix takes the GPU 4 us; checking its operands, looking up the stream and converting nine
+// arguments in Python and ctypes took 9 us.  The functions here do the same checks on the tensors themselves, take
+// torch's current stream and call the C ABI directly (include/lapis_hip.h).  lapis_amd/hip.py wraps them and
+// documents them; operands that are plain integers pass as raw device addresses, as they do there.
+#include <Python.h>
+
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cstdarg>
+
+#include "lapis_hip.h"
+
+namespace {
+
+PyObject *g_check = nullptr;  // lapis_amd.hip.check: raises LapisHipError for a status that is not OK
+PyObject *g_init = nullptr;   // lapis_amd.hip.init, called before the first call that reaches the device
+bool g_ready = false;
+
+// thrown once a Python error is set
+struct Raised {};
+
+[[noreturn]] void raise(PyObject *type, const char *fmt, ...) {
+  va_list ap;
+  va_start(ap, fmt);
+  PyErr_FormatV(type, fmt, ap);
+  va_end(ap);
+  throw Raised();
+}
+
+// An operand: a tensor, a raw address or None.
+struct Operand {
+  const at::Tensor *tensor = nullptr;
+  void *address = nullptr;
+};
+
+Operand operand(PyObject *o) {
+  Operand r;
+  if (o == Py_None) return r;
+  if (THPVariable_Check(o)) {
+    r.tensor = &THPVariable_Unpack(o);
+    r.address = r.tensor->data_ptr();
+    return r;
+  }
+  if (PyLong_Check(o)) {
+    r.address = PyLong_AsVoidPtr(o);
+    if (PyErr_Occurred()) throw Raised();
+    return r;
+  }
+  raise(PyExc_TypeError, "an operand is neither a tensor, a device address nor None but %s", Py_TYPE(o)->tp_name);
+}
+
+int64_t integer(PyObject *o) {
+  const long long v = PyLong_AsLongLong(o);
+  if (v == -1 && PyErr_Occurred()) {
+    // numpy integers and the like
+    PyErr_Clear();
+    PyObject *i = PyNumber_Index(o);
+    if (!i) throw Raised();
+    const long long w = PyLong_AsLongLong(i);
+    Py_DECREF(i);
+    if (w == -1 && PyErr_Occurred()) throw Raised();
+    return w;
+  }
+  return v;
+}
+
+double number(PyObject *o) {
+  const double v = PyFloat_AsDouble(o);
+  if (v == -1.0 && PyErr_Occurred()) throw Raised();
+  return v;
+}
+
+// Every call asks for its stream after its operands have passed their checks: malformed operands are refused
+// without a GPU too.
+lapis_hip_stream_t stream_of(PyObject *o) {
+  if (!g_ready) {
+    PyObject *r = PyObject_CallNoArgs(g_init);
+    if (!r) throw Raised();
+    Py_DECREF(r);
+    g_ready = true;
+  }
+  if (o == Py_None) return c10::hip::getCurrentHIPStream().stream();
+  if (PyLong_Check(o)) return PyLong_AsVoidPtr(o);
+  PyObject *raw = PyObject_GetAttrString(o, "cuda_stream");  // a torch.cuda.Stream
+  if (!raw) throw Raised();
+  void *p = PyLong_AsVoidPtr(raw);
+  Py_DECREF(raw);
+  if (PyErr_Occurred()) throw Raised();
+  return p;
+}
+
+lapis_hip_csr_plan *plan_of(PyObject *o) {
+  if (o == Py_None) return nullptr;
+  static PyObject *name = PyUnicode_InternFromString("address");
+  PyObject *a = PyObject_GetAttr(o, name);
+  if (!a) throw Raised();
+  void *p = a == Py_None ? nullptr : PyLong_AsVoidPtr(a);
+  Py_DECREF(a);
+  if (PyErr_Occurred()) throw Raised();
+  return static_cast<lapis_hip_csr_plan *>(p);
+}
+
+const char *type_name(at::ScalarType t) { return c10::toString(t); }
+
+// The C ABI takes pointers and counts: a tensor with fewer than `n` elements, of another element type than `like`
+// or with gaps between its elements would be read or written past its end on the device.
+void holds(const char *what, int64_t n, const Operand &o, const at::Tensor *like = nullptr) {
+  if (!o.tensor) return;
+  const at::Tensor &t = *o.tensor;
+  if (t.numel() < n)
+    raise(PyExc_ValueError, "%s: an operand of %lld elements where %lld are needed", what, (long long)t.numel(), (long long)n);
+  if (like && t.scalar_type() != like->scalar_type())
+    raise(PyExc_TypeError, "%s: operands of %s and %s", what, type_name(t.scalar_type()), type_name(like->scalar_type()));
+  if (!t.is_contiguous()) raise(PyExc_ValueError, "%s: an operand that is not contiguous", what);
+}
+
+void indices(const char *what, const Operand &o) {
+  if (o.tensor && o.tensor->scalar_type() != at::kInt)
+    raise(PyExc_TypeError, "%s: positions and coordinates are int32, got %s", what, type_name(o.tensor->scalar_type()));
+}
+
+// fp32 or fp64 by the element type of `o`
+bool is_f64(const Operand &o) {
+  if (!o.tensor) raise(PyExc_TypeError, "values must be a float32 or float64 tensor");
+  const auto t = o.tensor->scalar_type();
+  if (t != at::kDouble && t != at::kFloat) raise(PyExc_TypeError, "values must be float32 or float64, got %s", type_name(t));
+  return t == at::kDouble;
+}
+
+int64_t length(const char *what, const Operand &o) {
+  if (!o.tensor || o.tensor->dim() < 1) raise(PyExc_TypeError, "%s: an operand that is not a tensor of at least one dimension", what);
+  return o.tensor->size(0);
+}
+
+void check(int status) {
+  if (status == LAPIS_HIP_OK) return;
+  PyObject *r = PyObject_CallFunction(g_check, "i", status);
+  Py_XDECREF(r);
+  if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "lapis_hip call failed");
+  throw Raised();
+}
+
+PyObject *give(PyObject *o) {
+  Py_INCREF(o);
+  return o;
+}
+
+void arguments(const char *what, Py_ssize_t got, Py_ssize_t want) {
+  if (got != want) raise(PyExc_TypeError, "%s: %zd arguments, %zd expected", what, got, want);
+}
+
+template <typename F>
+PyObject *guarded(F f) {
+  try {
+    return f();
+  } catch (const Raised &) {
+    return nullptr;
+  } catch (const std::exception &e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+  }
+}
+
+#define LAPIS_PY(name) PyObject *name(PyObject *, PyObject *const *a, Py_ssize_t n)
+
+// (plan, nrows, ncols, pos, crd, val, x, y, stream)
+LAPIS_PY(py_spmv) {
+  return guarded([&] {
+    arguments("spmv", n, 9);
+    const int64_t nrows = integer(a[1]), ncols = integer(a[2]);
+    const Operand pos = operand(a[3]), crd = operand(a[4]), val = operand(a[5]), x = operand(a[6]), y = operand(a[7]);
+    indices("spmv", pos);
+    indices("spmv", crd);
+    holds("spmv", nrows + 1, pos);
+    holds("spmv", ncols, x, val.tensor);
+    holds("spmv", nrows, y, val.tensor);
+    if (crd.tensor) holds("spmv", crd.tensor->numel(), val);
+    lapis_hip_csr_plan *plan = plan_of(a[0]);
+    const auto p = static_cast<const int32_t *>(pos.address), c = static_cast<const int32_t *>(crd.address);
+    if (is_f64(val))
+      check(lapis_hip_spmv_csr_f64_i32(plan, nrows, ncols, p, c, (const double *)val.address, (const double *)x.address,
+                                       (double *)y.address, stream_of(a[8])));
+    else
+      check(lapis_hip_spmv_csr_f32_i32(plan, nrows, ncols, p, c, (const float *)val.address, (const float *)x.address,
+                                       (float *)y.address, stream_of(a[8])));
+    return give(a[7]);
+  });
+}
+
+// (nrows, ncols, pos, crd, val, B, C, stream, plan)
+LAPIS_PY(py_spmm) {
+  return guarded([&] {
+    arguments("spmm", n, 9);
+    const int64_t nrows = integer(a[0]), ncols = integer(a[1]);
+    const Operand pos = operand(a[2]), crd = operand(a[3]), val = operand(a[4]), B = operand(a[5]), C = operand(a[6]);
+    if (!B.tensor || !C.tensor || !crd.tensor || !val.tensor) raise(PyExc_TypeError, "spmm: crd, val, B and C are tensors");
+    indices("spmm", pos);
+    indices("spmm", crd);
+    holds("spmm", nrows + 1, pos);
+    holds("spmm", crd.tensor->numel(), val);
+    const at::Tensor &b = *B.tensor, &c = *C.tensor, &v = *val.tensor;
+    if (b.dim() != 2 || c.dim() != 2 || b.size(1) != c.size(1) || b.size(0) < ncols || c.size(0) < nrows ||
+        b.stride(1) != 1 || c.stride(1) != 1 || b.scalar_type() != v.scalar_type() || c.scalar_type() != v.scalar_type())
+      raise(PyExc_ValueError, "spmm: a %lld x %lld matrix of %s times B (%d dimensions, %lld elements) into C (%d, %lld)",
+            (long long)nrows, (long long)ncols, type_name(v.scalar_type()), (int)b.dim(), (long long)b.numel(), (int)c.dim(),
+            (long long)c.numel());
+    const int64_t k = c.size(1);
+    lapis_hip_csr_plan *plan = plan_of(a[8]);
+    const auto p = static_cast<const int32_t *>(pos.address), cr = static_cast<const int32_t *>(crd.address);
+    if (is_f64(val))
+      check(lapis_hip_spmm_csr_f64_i32_plan(plan, nrows, ncols, k, p, cr, (const double *)val.address, (const double *)B.address,
+                                            b.stride(0), (double *)C.address, c.stride(0), stream_of(a[7])));
+    else
+      check(lapis_hip_spmm_csr_f32_i32_plan(plan, nrows, ncols, k, p, cr, (const float *)val.address, (const float *)B.address,
+                                            b.stride(0), (float *)C.address, c.stride(0), stream_of(a[7])));
+    return give(a[6]);
+  });
+}
+
+// (n1, n2, pos, crd, val, V, out, stream)
+LAPIS_PY(py_bspmm_csrv) {
+  return guarded([&] {
+    arguments("bspmm_csrv", n, 8);
+    const int64_t n1 = integer(a[0]), n2 = integer(a[1]);
+    const Operand pos = operand(a[2]), crd = operand(a[3]), val = operand(a[4]), V = operand(a[5]), out = operand(a[6]);
+    if (!V.tensor || V.tensor->dim() != 3) raise(PyExc_IndexError, "bspmm_csrv: V has three dimensions");
+    check(lapis_hip_bspmm_csrv_f32_i32(n1, n2, V.tensor->size(1), V.tensor->size(2), (const int32_t *)pos.address,
+                                       (const int32_t *)crd.address, (const float *)val.address, (const float *)V.address,
+                                       (float *)out.address, stream_of(a[7])));
+    return give(a[6]);
+  });
+}
+
+// (x, y, result, init, stream)
+LAPIS_PY(py_dot) {
+  return guarded([&] {
+    arguments("dot", n, 5);
+    const Operand x = operand(a[0]), y = operand(a[1]), r = operand(a[2]);
+    const int64_t len = length("dot", x);
+    holds("dot", len, x, x.tensor);
+    holds("dot", len, y, x.tensor);
+    holds("dot", 1, r, x.tensor);
+    const double init = number(a[3]);
+    if (is_f64(x))
+      check(lapis_hip_dot_f64(len, (const double *)x.address, (const double *)y.address, init, (double *)r.address, stream_of(a[4])));
+    else
+      check(lapis_hip_dot_f32(len, (const float *)x.address, (const float *)y.address, (float)init, (float *)r.address,
+                              stream_of(a[4])));
+    return give(a[2]);
+  });
+}
+
+// (x, y, init, stream) -> float.  The call waits for the GPU: other Python threads run meanwhile.
+LAPIS_PY(py_dot_host) {
+  return guarded([&] {
+    arguments("dot", n, 4);
+    const Operand x = operand(a[0]), y = operand(a[1]);
+    const int64_t len = length("dot", x);
+    holds("dot", len, x, x.tensor);
+    holds("dot", len, y, x.tensor);
+    const double init = number(a[2]);
+    const lapis_hip_stream_t st = stream_of(a[3]);
+    double r64 = 0.0;
+    float r32 = 0.f;
+    const bool f64 = is_f64(x);
+    int status;
+    Py_BEGIN_ALLOW_THREADS;
+    status = f64 ? lapis_hip_dot_f64_host(len, (const double *)x.address, (const double *)y.address, init, &r64, st)
+                 : lapis_hip_dot_f32_host(len, (const float *)x.address, (const float *)y.address, (float)init, &r32, st);
+    Py_END_ALLOW_THREADS;
+    check(status);
+    return PyFloat_FromDouble(f64 ? r64 : (double)r32);
+  });
+}
+
+// (a, x, b, y, dst, stream): dst = a x + b y
+LAPIS_PY(py_axpby) {
+  return guarded([&] {
+    arguments("axpby", n, 6);
+    const double ca = number(a[0]), cb = number(a[2]);
+    const Operand x = operand(a[1]), y = operand(a[3]), d = operand(a[4]);
+    const int64_t len = length("axpby", x);
+    holds("axpby", len, x, x.tensor);
+    holds("axpby", len, y, x.tensor);
+    holds("axpby", len, d, x.tensor);
+    if (is_f64(x))
+      check(lapis_hip_axpby_f64(len, ca, (const double *)x.address, cb, (const double *)y.address, (double *)d.address, stream_of(a[5])));
+    else
+      check(lapis_hip_axpby_f32(len, (float)ca, (const float *)x.address, (float)cb, (const float *)y.address, (float *)d.address,
+                                stream_of(a[5])));
+    return give(a[4]);
+  });
+}
+
+// (x, y, dst, stream)
+template <int (*F64)(int64_t, const double *, const double *, double *, lapis_hip_stream_t),
+          int (*F32)(int64_t, const float *, const float *, float *, lapis_hip_stream_t)>
+PyObject *two_operands(const char *what, PyObject *const *a, Py_ssize_t n) {
+  return guarded([&] {
+    arguments(what, n, 4);
+    const Operand x = operand(a[0]), y = operand(a[1]), d = operand(a[2]);
+    const int64_t len = length(what, x);
+    holds(what, len, x, x.tensor);
+    holds(what, len, y, x.tensor);
+    holds(what, len, d, x.tensor);
+    if (is_f64(x))
+      check(F64(len, (const double *)x.address, (const double *)y.address, (double *)d.address, stream_of(a[3])));
+    else
+      check(F32(len, (const float *)x.address, (const float *)y.address, (float *)d.address, stream_of(a[3])));
+    return give(a[2]);
+  });
+}
+LAPIS_PY(py_mult) { return two_operands<lapis_hip_mult_f64, lapis_hip_mult_f32>("mult", a, n); }
+LAPIS_PY(py_div) { return two_operands<lapis_hip_div_f64, lapis_hip_div_f32>("div", a, n); }
+
+// (dst, value, stream)
+LAPIS_PY(py_fill) {
+  return guarded([&] {
+    arguments("fill", n, 3);
+    const Operand d = operand(a[0]);
+    const int64_t len = length("fill", d);
+    const double v = number(a[1]);
+    if (is_f64(d)) check(lapis_hip_fill_f64(len, v, (double *)d.address, stream_of(a[2])));
+    else check(lapis_hip_fill_f32(len, (float)v, (float *)d.address, stream_of(a[2])));
+    return give(a[0]);
+  });
+}
+
+// (src, dst, stream)
+LAPIS_PY(py_copy) {
+  return guarded([&] {
+    arguments("copy", n, 3);
+    const Operand s = operand(a[0]), d = operand(a[1]);
+    const int64_t len = length("copy", s);
+    holds("copy", len, s, s.tensor);
+    holds("copy", len, d, s.tensor);
+    if (is_f64(s)) check(lapis_hip_copy_f64(len, (const double *)s.address, (double *)d.address, stream_of(a[2])));
+    else check(lapis_hip_copy_f32(len, (const float *)s.address, (float *)d.address, stream_of(a[2])));
+    return give(a[1]);
+  });
+}
+
+// (plan, n, pos, crd, val, b, dinv, tol, maxiter, x, work, stream) -> (iterations, relative residual)
+LAPIS_PY(py_pcg) {
+  return guarded([&] {
+    arguments("pcg", n, 12);
+    const int64_t rows = integer(a[1]);
+    const Operand pos = operand(a[2]), crd = operand(a[3]), val = operand(a[4]), b = operand(a[5]), dinv = operand(a[6]),
+                  x = operand(a[9]), work = operand(a[10]);
+    indices("pcg", pos);
+    indices("pcg", crd);
+    holds("pcg", rows + 1, pos);
+    holds("pcg", rows, b, val.tensor);
+    holds("pcg", rows, dinv, val.tensor);
+    holds("pcg", rows, x, val.tensor);
+    holds("pcg", 4 * rows, work, val.tensor);
+    if (crd.tensor) holds("pcg", crd.tensor->numel(), val);
+    const double tol = number(a[7]);
+    const int64_t maxiter = integer(a[8]);
+    lapis_hip_csr_plan *plan = plan_of(a[0]);
+    const lapis_hip_stream_t st = stream_of(a[11]);
+    uint64_t iters = 0;
+    double relres = 0.0;
+    int status;
+    Py_BEGIN_ALLOW_THREADS;
+    status = lapis_hip_pcg_f64_i32(plan, rows, (const int32_t *)pos.address, (const int32_t *)crd.address,
+                                   (const double *)val.address, (const double *)b.address, (const double *)dinv.address, tol,
+                                   (uint64_t)maxiter, (double *)x.address, &iters, &relres, (double *)work.address, st);
+    Py_END_ALLOW_THREADS;
+    check(status);
+    return Py_BuildValue("(Kd)", (unsigned long long)iters, relres);
+  });
+}
+
+// setup(check, init)
+PyObject *py_setup(PyObject *, PyObject *args) {
+  PyObject *check_fn, *init_fn;
+  if (!PyArg_ParseTuple(args, "OO", &check_fn, &init_fn)) return nullptr;
+  Py_INCREF(check_fn);
+  Py_XSETREF(g_check, check_fn);
+  Py_INCREF(init_fn);
+  Py_XSETREF(g_init, init_fn);
+  Py_RETURN_NONE;
+}
+
+#define LAPIS_METHOD(name) {#name, (PyCFunction)(void (*)(void))py_##name, METH_FASTCALL, nullptr}
+PyMethodDef g_methods[] = {LAPIS_METHOD(spmv), LAPIS_METHOD(spmm), LAPIS_METHOD(bspmm_csrv), LAPIS_METHOD(dot),
+                           LAPIS_METHOD(dot_host), LAPIS_METHOD(axpby), LAPIS_METHOD(mult), LAPIS_METHOD(div),
+                           LAPIS_METHOD(fill), LAPIS_METHOD(copy), LAPIS_METHOD(pcg),
+                           {"setup", py_setup, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
+PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_lapis_calls", "Device-resident calls of the gfx950 kernel library.", -1,
+                        g_methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__lapis_calls(void) { return PyModule_Create(&g_module); }

@@ -1,15 +1,20 @@
-"""ctypes binding of the C-ABI kernel library (include/lapis_hip.h).
+"""Python binding of the C-ABI kernel library (include/lapis_hip.h).
 
-Pointers are DEVICE addresses: pass ``torch`` CUDA tensors (their ``data_ptr()`` is
+Plans, set-up and measurement go through ctypes; the calls a program makes over and over (spmv, spmm, bspmm_csrv,
+the vector operations, pcg) go through csrc/bindings.cpp, which checks their operands and calls the C ABI without
+ctypes (a planned spmv from Python: 9 us -> what its kernel takes).  Pointers are DEVICE addresses: pass ``torch`` CUDA tensors (their ``data_ptr()`` is
 taken), or plain integers.  ``stream`` is a ``torch.cuda.Stream``, a raw
 ``hipStream_t`` value, or None for torch's current stream.  The library has no CPU
 path: loading fails loudly when it has not been built.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "liblapis_hip.so")
+CALLS_PATH = os.path.join(_HERE, "lib", "_lapis_calls.so")
 
 SPMV_AUTO, SPMV_SUBWARP, SPMV_ROWBLOCK, SPMV_NNZSPLIT, SPMV_COLBLOCK = 0, 1, 2, 3, 4
 KERNEL_NAMES = {SPMV_AUTO: "auto", SPMV_SUBWARP: "subwarp", SPMV_ROWBLOCK: "rowblock", SPMV_NNZSPLIT: "nnzsplit",
@@ -157,6 +162,27 @@ def init():
     return lib
 
 
+class _Calls:
+    """Stands in for the extension module of csrc/bindings.cpp until the first call, which loads it."""
+
+    def __getattr__(self, name):
+        global _calls
+        import torch  # noqa: F401  (the extension's symbols come from torch's libraries)
+        load()
+        if not os.path.exists(CALLS_PATH):
+            raise FileNotFoundError("%s not found: build it first (python -m lapis_amd.build); "
+                                    "there is no CPU fallback" % CALLS_PATH)
+        loader = importlib.machinery.ExtensionFileLoader("_lapis_calls", CALLS_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_lapis_calls", loader))
+        loader.exec_module(module)
+        module.setup(check, init)
+        _calls = module
+        return getattr(module, name)
+
+
+_calls = _Calls()
+
+
 def _ptr(t):
     if t is None:
         return None
@@ -203,6 +229,7 @@ class CsrPlan:
             nnz = int(crd.shape[0])
         check(lib.lapis_hip_csr_plan_create(ctypes.byref(self._handle), nrows, ncols, nnz, _ptr(pos), _ptr(crd),
                                             value_bytes, _stream(stream)))
+        self.address = self._handle.value  # what the native calls take
 
     @property
     def handle(self):
@@ -258,6 +285,7 @@ class CsrPlan:
         if self._handle:
             self._lib.lapis_hip_csr_plan_destroy(self._handle)
             self._handle = _vp()
+            self.address = None
 
     def __del__(self):
         try:
@@ -299,39 +327,12 @@ def _indices(what, *tensors):
 
 def spmv(plan, nrows, ncols, pos, crd, val, x, y, stream=None):
     """y += A x.  ``plan`` may be None: the launch then follows the reference's own rule."""
-    _indices("spmv", pos, crd)
-    _holds("spmv", nrows + 1, pos)
-    _holds("spmv", ncols, x, like=val)
-    _holds("spmv", nrows, y, like=val)
-    if not isinstance(crd, int) and not isinstance(val, int) and crd is not None and val is not None:
-        _holds("spmv", crd.numel(), val)
-    lib = init()
-    fn = getattr(lib, "lapis_hip_spmv_csr_%s_i32" % _suffix(val))
-    check(fn(plan.handle if plan is not None else None, nrows, ncols, _ptr(pos), _ptr(crd), _ptr(val), _ptr(x),
-             _ptr(y), _stream(stream)))
-    return y
+    return _calls.spmv(plan, nrows, ncols, pos, crd, val, x, y, stream)
 
 
 def spmm(nrows, ncols, pos, crd, val, B, C, stream=None, plan=None):
     """C += A B with row-major B (ncols x k) and C (nrows x k); with a plan its statistics pick the kernel."""
-    k = int(C.shape[1])
-    _indices("spmm", pos, crd)
-    _holds("spmm", nrows + 1, pos)
-    _holds("spmm", crd.numel(), val)
-    if B.dim() != 2 or C.dim() != 2 or int(B.shape[1]) != k or B.shape[0] < ncols or C.shape[0] < nrows or \
-            B.stride(1) != 1 or C.stride(1) != 1 or B.dtype != val.dtype or C.dtype != val.dtype:
-        raise ValueError("spmm: a %d x %d matrix of %s times B %s into C %s" % (
-            nrows, ncols, val.dtype, tuple(B.shape), tuple(C.shape)))
-    lib = init()
-    if plan is not None:
-        fn = getattr(lib, "lapis_hip_spmm_csr_%s_i32_plan" % _suffix(val))
-        check(fn(plan.handle, nrows, ncols, k, _ptr(pos), _ptr(crd), _ptr(val), _ptr(B), int(B.stride(0)), _ptr(C),
-                 int(C.stride(0)), _stream(stream)))
-        return C
-    fn = getattr(lib, "lapis_hip_spmm_csr_%s_i32" % _suffix(val))
-    check(fn(nrows, ncols, k, _ptr(pos), _ptr(crd), _ptr(val), _ptr(B), int(B.stride(0)), _ptr(C), int(C.stride(0)),
-             _stream(stream)))
-    return C
+    return _calls.spmm(nrows, ncols, pos, crd, val, B, C, stream, plan)
 
 
 def spmm_last_kernel():
@@ -341,12 +342,7 @@ def spmm_last_kernel():
 
 def dot(x, y, result, init_value=0.0, stream=None):
     """result[0] = init + x.y, with ``result`` a one-element device tensor (no host sync)."""
-    _holds("dot", int(x.shape[0]), x, y, like=x)
-    _holds("dot", 1, result, like=x)
-    lib = init()
-    fn = getattr(lib, "lapis_hip_dot_%s" % _suffix(x))
-    check(fn(int(x.shape[0]), _ptr(x), _ptr(y), init_value, _ptr(result), _stream(stream)))
-    return result
+    return _calls.dot(x, y, result, init_value, stream)
 
 
 def calibrate_gather(x, window_bytes, lanes_per_line, stream_buf, gathers, sink, stream=None):
@@ -379,12 +375,7 @@ def calibrate_mix(mode, x, window_bytes, stream_buf, stream_bytes, gathers, cu_c
 
 def dot_host(x, y, init_value=0.0, stream=None):
     """init + x . y as a Python float: the entry point that returns the scalar to the host (blocking)."""
-    _holds("dot", int(x.shape[0]), x, y, like=x)
-    lib = init()
-    out = (_dbl if x.element_size() == 8 else _flt)(0.0)
-    fn = getattr(lib, "lapis_hip_dot_%s_host" % _suffix(x))
-    check(fn(int(x.shape[0]), _ptr(x), _ptr(y), init_value, ctypes.byref(out), _stream(stream)))
-    return out.value
+    return _calls.dot_host(x, y, init_value, stream)
 
 
 def axpby_dot(a, x, b, y, dst, z, result, init_value=0.0, stream=None):
@@ -408,36 +399,23 @@ def dot_noalloc(x, y, result, init_value=0.0, stream=None):
 
 
 def axpby(a, x, b, y, dst, stream=None):
-    _holds("axpby", int(x.shape[0]), x, y, dst, like=x)
-    lib = init()
-    fn = getattr(lib, "lapis_hip_axpby_%s" % _suffix(x))
-    check(fn(int(x.shape[0]), a, _ptr(x), b, _ptr(y), _ptr(dst), _stream(stream)))
-    return dst
+    return _calls.axpby(a, x, b, y, dst, stream)
 
 
 def mult(x, y, dst, stream=None):
-    _holds("mult", int(x.shape[0]), x, y, dst, like=x)
-    check(getattr(init(), "lapis_hip_mult_%s" % _suffix(x))(int(x.shape[0]), _ptr(x), _ptr(y), _ptr(dst), _stream(stream)))
-    return dst
+    return _calls.mult(x, y, dst, stream)
 
 
 def div(x, y, dst, stream=None):
-    _holds("div", int(x.shape[0]), x, y, dst, like=x)
-    check(getattr(init(), "lapis_hip_div_%s" % _suffix(x))(int(x.shape[0]), _ptr(x), _ptr(y), _ptr(dst), _stream(stream)))
-    return dst
+    return _calls.div(x, y, dst, stream)
 
 
 def fill(dst, value, stream=None):
-    lib = init()
-    fn = getattr(lib, "lapis_hip_fill_%s" % _suffix(dst))
-    check(fn(int(dst.shape[0]), value, _ptr(dst), _stream(stream)))
-    return dst
+    return _calls.fill(dst, value, stream)
 
 
 def copy(src, dst, stream=None):
-    _holds("copy", int(src.shape[0]), src, dst, like=src)
-    check(getattr(init(), "lapis_hip_copy_%s" % _suffix(src))(int(src.shape[0]), _ptr(src), _ptr(dst), _stream(stream)))
-    return dst
+    return _calls.copy(src, dst, stream)
 
 
 def scale(alpha, val, stream=None):
@@ -447,18 +425,7 @@ def scale(alpha, val, stream=None):
 
 def pcg(plan, n, pos, crd, val, b, dinv, tol, maxiter, x, work=None, stream=None):
     """CG of examples/pcg_solve.py on device buffers -> (iters, relres); x is filled in place."""
-    _indices("pcg", pos, crd)
-    _holds("pcg", n + 1, pos)
-    _holds("pcg", n, b, dinv, x, like=val)
-    _holds("pcg", 4 * n, work, like=val)
-    if not isinstance(crd, int) and not isinstance(val, int):
-        _holds("pcg", crd.numel(), val)
-    lib = init()
-    iters, relres = _u64(0), _dbl(0.0)
-    check(lib.lapis_hip_pcg_f64_i32(plan.handle if plan is not None else None, n, _ptr(pos), _ptr(crd), _ptr(val),
-                                    _ptr(b), _ptr(dinv), tol, maxiter, _ptr(x), ctypes.byref(iters),
-                                    ctypes.byref(relres), _ptr(work), _stream(stream)))
-    return int(iters.value), relres.value
+    return _calls.pcg(plan, n, pos, crd, val, b, dinv, tol, maxiter, x, work, stream)
 
 
 def pcg_masked(plan, n, pos, crd, val, b, mask, d, tol, maxiter, x, work=None, stream=None):
@@ -490,7 +457,4 @@ def normalize_mom2(mom1, mom2, out, stream=None):
 
 def bspmm_csrv(n1, n2, pos, crd, val, V, out, stream=None):
     """out(n1,dh,nh) += A(n1,n2,nh) * V(n2,dh,nh) with CSRV A (examples/bspmm.py)."""
-    dh, nh = int(V.shape[1]), int(V.shape[2])
-    check(init().lapis_hip_bspmm_csrv_f32_i32(n1, n2, dh, nh, _ptr(pos), _ptr(crd), _ptr(val), _ptr(V), _ptr(out),
-                                              _stream(stream)))
-    return out
+    return _calls.bspmm_csrv(n1, n2, pos, crd, val, V, out, stream)
