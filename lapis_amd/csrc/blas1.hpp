@@ -19,5 +19,7 @@ int launch_dot(int64_t n, const T *x, const T *y, T init, T *result, T *partials
 // release of the allocated ring of partials the other dot entry points use.
 int dot_noalloc_setup();
 void dot_release_scratch();
+// Gives back the scratch of finished CG solves (cg.hip).
+void cg_release_scratch();
 
 }  // namespace lapis

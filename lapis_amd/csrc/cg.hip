@@ -25,6 +25,9 @@
 // three times.  The pass that decides to leave still adds its alpha p and leaves p alone.
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
+#include <mutex>
+#include <vector>
 
 #include "blas1.hpp"
 #include "common.hpp"
@@ -334,11 +337,387 @@ __global__ __launch_bounds__(256) void cg_init_scalar_kernel(int count, const do
   }
 }
 
+// ---- small systems: the whole solve in one launch -------------------------------------------------
+//
+// On a system of a few ten thousand rows an iteration of the kernels above is launches and gaps (6 launches,
+// 25 us per iteration at 16 384 rows, of which the data of an iteration is worth 1 us; 6.5 us here: a whole solve of 40
+// iterations 1.50 -> 0.27 ms, 490 000 rows 2.20 -> 0.68 ms).  Here one workgroup per
+// compute unit keeps a stretch of rows for the whole solve: their entries in LDS, their r, x, p and dinv in
+// registers.  What the others need goes through memory: z (r where there is no preconditioner) and p, and two
+// exchanges per iteration, each a sum over the workgroups and a barrier in one:
+//     p = z + beta p (own rows) ; Ap = A p, with p of the gathered columns made on the way from z and the previous p
+//   exchange p.Ap -> alpha
+//     x += alpha p ; r -= alpha Ap ; z = r dinv
+//   exchange r.r, r.z -> convergence test, beta
+// An exchange is one hop: workgroup g writes its partial sums, each half tagged with the exchange's number, into
+// its slot, and every workgroup reads all slots until all carry the number.  Slots alternate between two sets:
+// a set is written again only after every workgroup has been through the exchange between.  p alternates
+// between two buffers for the same reason.
+// Shared words are written and read with agent-scope accesses (past the L2s, which are not coherent across the
+// XCDs); a wavefront waits for its own stores before its workgroup's slot is written.  Every wait is bounded: a
+// workgroup whose wait runs out (the others were not resident) gives up, so do all, and the host takes the
+// kernels above instead.  A launch makes at most `budget` iterations; the host continues from what it left.
+constexpr int kSmallMaxBlocks = 256;
+constexpr int kSmallThreads = 512;
+constexpr int kSmallMaxRowsPerThread = 4;
+constexpr int kSmallLdsBytes = 150 * 1024;
+
+struct CgSmallResult {
+  unsigned long long done_iter;  // the reference's counter at exit, 0 when the budget ended first
+  double relres;
+  double rz, beta, initres;  // where the next launch goes on
+  unsigned fault;
+  unsigned pad;
+};
+
+struct CgSmallArgs {
+  int n, rows, blocks;  // rows per workgroup, workgroups
+  int entries;          // LDS room for entries of a workgroup
+  const int *pos, *crd;
+  const double *val, *b, *dinv;
+  double *x, *r, *z, *p0, *p1;
+  unsigned long long *slots;  // [2][kSmallMaxBlocks][4]
+  unsigned epoch;             // number of the first exchange
+  int resume;
+  unsigned long long iter0;  // iterations made by earlier launches
+  unsigned long long maxiter, budget;
+  double tol, rz, beta, initres;
+  int spins;           // polls of an exchange before it gives up
+  CgSmallResult *out;  // host memory
+};
+
+__device__ __forceinline__ double shared_load(const double *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void shared_store(double *p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Sums v0 and v1 over all threads of all workgroups, in a fixed order; false when the wait ran out.
+// lds: 2 * 8 + 2 * kSmallMaxBlocks doubles.
+template <int V>
+__device__ __forceinline__ bool small_exchange(const CgSmallArgs &a, unsigned epoch, double (&v)[V], double *lds) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  double *part = lds + 16;
+#pragma unroll
+  for (int i = 0; i < V; ++i) v[i] = group_sum<64>(v[i]);
+  if (lane == 0) {
+#pragma unroll
+    for (int i = 0; i < V; ++i) lds[i * 8 + wave] = v[i];
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's z and p are where the others read them
+  __syncthreads();
+  unsigned long long *set = a.slots + (size_t)(epoch & 1) * kSmallMaxBlocks * 4;
+  if (tid < 2 * V) {
+    double sum = 0.0;
+    for (int w = 0; w < kSmallThreads / 64; ++w) sum = sum + lds[(tid >> 1) * 8 + w];
+    const unsigned long long bits = __builtin_bit_cast(unsigned long long, sum);
+    const unsigned half = (unsigned)(tid & 1 ? bits >> 32 : bits);
+    __hip_atomic_store(set + (size_t)blockIdx.x * 4 + tid, ((unsigned long long)epoch << 32) | half, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  }
+  bool ok = true;
+  if (tid < a.blocks) {
+    unsigned long long w[2 * V] = {};
+    ok = false;
+    for (int spin = 0; spin < a.spins; ++spin) {
+      ok = true;
+#pragma unroll
+      for (int i = 0; i < 2 * V; ++i)
+        w[i] = __hip_atomic_load(set + (size_t)tid * 4 + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int i = 0; i < 2 * V; ++i) ok = ok && (unsigned)(w[i] >> 32) == epoch;
+      if (ok) break;
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+      part[i * kSmallMaxBlocks + tid] =
+          __builtin_bit_cast(double, (w[2 * i] & 0xffffffffull) | (w[2 * i + 1] << 32));
+  }
+  ok = __syncthreads_and(ok);
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    double sum = 0.0;
+    for (int g = lane; g < a.blocks; g += 64) sum = sum + part[i * kSmallMaxBlocks + g];
+    v[i] = group_sum<64>(sum);
+  }
+  __syncthreads();  // the next exchange writes the same LDS
+  return ok;
+}
+
+template <int RPT, bool PRE>
+__global__ __launch_bounds__(kSmallThreads) void cg_small_kernel(CgSmallArgs a) {
+  extern __shared__ __align__(16) unsigned char small_lds[];
+  __shared__ double xlds[16 + 2 * kSmallMaxBlocks];
+  double *lval = reinterpret_cast<double *>(small_lds);
+  int *lcrd = reinterpret_cast<int *>(lval + a.entries);
+  const int tid = threadIdx.x;
+  const int row0 = blockIdx.x * a.rows;
+  const int rows_here = min(a.rows, a.n - row0);
+  const int first = a.pos[row0], last = a.pos[row0 + rows_here];
+  for (int j = tid; j < last - first; j += kSmallThreads) {
+    lval[j] = a.val[first + j];
+    lcrd[j] = a.crd[first + j];
+  }
+  double r[RPT], x[RPT], p[RPT], z[RPT], d[RPT];
+  int lo[RPT], hi[RPT];
+  double sums[2] = {0.0, 0.0};
+#pragma unroll
+  for (int i = 0; i < RPT; ++i) {
+    const int k = tid + i * kSmallThreads;
+    const bool have = k < rows_here;
+    const int row = row0 + k;
+    lo[i] = have ? a.pos[row] - first : 0;
+    hi[i] = have ? a.pos[row + 1] - first : 0;
+    d[i] = have && PRE ? a.dinv[row] : 1.0;
+    p[i] = 0.0;
+    if (a.resume) {
+      r[i] = have ? a.r[row] : 0.0;
+      x[i] = have ? a.x[row] : 0.0;
+      z[i] = PRE ? r[i] * d[i] : r[i];
+      p[i] = have ? shared_load((a.iter0 & 1 ? a.p1 : a.p0) + row) : 0.0;
+    } else {
+      r[i] = have ? a.b[row] : 0.0;
+      x[i] = 0.0;
+      z[i] = PRE ? r[i] * d[i] : r[i];
+      if (have) shared_store(a.z + row, z[i]);
+      sums[0] = sums[0] + r[i] * r[i];
+      sums[1] = sums[1] + r[i] * z[i];
+    }
+  }
+  unsigned epoch = a.epoch;
+  double rz = a.rz, beta = a.beta, initres = a.initres;
+  bool ok = true;
+  if (a.resume) {
+    __syncthreads();  // the entries are in LDS
+  } else {
+    ok = small_exchange<2>(a, epoch++, sums, xlds);
+    initres = sqrt(sums[0]);
+    rz = sums[1];
+  }
+  double relres = 0.0;
+  unsigned long long iter = a.iter0, done = 0;
+  bool first_pass = !a.resume;
+  while (ok && iter - a.iter0 < a.budget) {
+    ++iter;  // the reference's counter of this pass
+    double *pnew = iter & 1 ? a.p1 : a.p0;
+    const double *pold = iter & 1 ? a.p0 : a.p1;
+    double Ap[RPT];
+    double pAp[1] = {0.0};
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) {
+      const int k = tid + i * kSmallThreads;
+      if (first_pass) {
+        p[i] = z[i];
+      } else {
+        const double pt = p[i] * beta;
+        p[i] = z[i] + pt;
+      }
+      if (k < rows_here) shared_store(pnew + row0 + k, p[i]);
+      double acc = 0.0;
+      for (int j = lo[i]; j < hi[i]; j += 4) {  // four entries' z and p in flight, summed in ascending order
+        double zj[4], pj[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int c = lcrd[min(j + u, hi[i] - 1)];
+          zj[u] = shared_load(a.z + c);
+          pj[u] = first_pass ? 0.0 : shared_load(pold + c);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if (j + u < hi[i]) {
+            const double pt = pj[u] * beta;
+            const double pv = first_pass ? zj[u] : zj[u] + pt;
+            acc = acc + lval[j + u] * pv;
+          }
+        }
+      }
+      Ap[i] = acc;
+      pAp[0] = pAp[0] + p[i] * acc;
+    }
+    if (!(ok = small_exchange<1>(a, epoch++, pAp, xlds))) break;
+    const double alpha = rz / pAp[0];
+    const double malpha = -alpha;
+    sums[0] = sums[1] = 0.0;
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) {
+      const int k = tid + i * kSmallThreads;
+      const double xt = p[i] * alpha;
+      x[i] = x[i] + xt;
+      const double rt = Ap[i] * malpha;
+      r[i] = r[i] + rt;
+      z[i] = PRE ? r[i] * d[i] : r[i];
+      if (k < rows_here) shared_store(a.z + row0 + k, z[i]);
+      sums[0] = sums[0] + r[i] * r[i];
+      sums[1] = sums[1] + r[i] * z[i];
+    }
+    if (!(ok = small_exchange<2>(a, epoch++, sums, xlds))) break;
+    relres = sqrt(sums[0]) / initres;
+    beta = sums[1] / rz;
+    rz = sums[1];
+    first_pass = false;
+    if (!(relres > a.tol) || iter == a.maxiter) {
+      done = iter;
+      break;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < RPT; ++i) {
+    const int k = tid + i * kSmallThreads;
+    if (ok && k < rows_here) {
+      a.x[row0 + k] = x[i];
+      if (!done) a.r[row0 + k] = r[i];
+    }
+  }
+  if (tid == 0 && (blockIdx.x == 0 || !ok)) {
+    if (!ok) {
+      __hip_atomic_store(&a.out->fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    } else {
+      a.out->done_iter = done;
+      a.out->relres = relres;
+      a.out->rz = rz;
+      a.out->beta = beta;
+      a.out->initres = initres;
+    }
+  }
+}
+
 }  // namespace lapis
 
 using namespace lapis;
 
 namespace {
+
+// Scratch of one solve: device memory for the scalars, partial sums and exchange slots, and a word of pinned
+// host memory the device reports to.  A solve takes one for its duration (it synchronises its stream before it
+// returns), so a scratch is never shared; at most kKeptScratch are kept, until lapis_hip_finalize.
+struct CgScratch {
+  int device = 0;
+  CgState *state = nullptr;
+  double *partials = nullptr;
+  unsigned long long *slots = nullptr;
+  unsigned epoch = 1;  // slots carry smaller numbers only
+  CgState *host_state = nullptr;
+  CgSmallResult *host_result = nullptr;
+  void *device_block = nullptr, *host_block = nullptr;
+};
+constexpr int kKeptScratch = 8;
+std::mutex g_cg_mutex;
+std::vector<CgScratch *> g_cg_scratch;
+
+constexpr size_t kSlotWords = 2 * (size_t)kSmallMaxBlocks * 4;
+
+void free_scratch(CgScratch *s) {
+  if (s->device_block) (void)hipFree(s->device_block);
+  if (s->host_block) (void)hipHostFree(s->host_block);
+  delete s;
+}
+
+hipError_t take_scratch(CgScratch **out, hipStream_t st) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  {
+    std::lock_guard<std::mutex> lock(g_cg_mutex);
+    for (size_t i = 0; i < g_cg_scratch.size(); ++i) {
+      if (g_cg_scratch[i]->device != dev) continue;
+      *out = g_cg_scratch[i];
+      g_cg_scratch.erase(g_cg_scratch.begin() + (ptrdiff_t)i);
+      return hipSuccess;
+    }
+  }
+  CgScratch *s = new CgScratch();
+  s->device = dev;
+  const size_t partial_bytes = sizeof(double) * 3 * kDotMaxBlocks;
+  e = hipMalloc(&s->device_block, 256 + partial_bytes + 8 * kSlotWords);
+  if (e == hipSuccess) e = hipHostMalloc(&s->host_block, 4096, hipHostMallocDefault);
+  if (e == hipSuccess) {
+    char *base = static_cast<char *>(s->device_block);
+    s->state = reinterpret_cast<CgState *>(base);
+    s->partials = reinterpret_cast<double *>(base + 256);
+    s->slots = reinterpret_cast<unsigned long long *>(base + 256 + partial_bytes);
+    s->host_state = static_cast<CgState *>(s->host_block);
+    s->host_result = reinterpret_cast<CgSmallResult *>(static_cast<char *>(s->host_block) + 512);
+    // no slot carries the number of an exchange before that exchange writes it
+    if (lapis_hip_fill_f64((int64_t)kSlotWords, 0.0, reinterpret_cast<double *>(s->slots), st) != LAPIS_HIP_OK)
+      e = hipErrorUnknown;
+  }
+  if (e != hipSuccess) {
+    free_scratch(s);
+    return e;
+  }
+  *out = s;
+  return hipSuccess;
+}
+
+void give_scratch(CgScratch *s) {
+  {
+    std::lock_guard<std::mutex> lock(g_cg_mutex);
+    if ((int)g_cg_scratch.size() < kKeptScratch) {
+      g_cg_scratch.push_back(s);
+      return;
+    }
+  }
+  free_scratch(s);
+}
+}  // namespace
+
+namespace lapis {
+void cg_release_scratch() {
+  std::lock_guard<std::mutex> lock(g_cg_mutex);
+  for (CgScratch *s : g_cg_scratch) free_scratch(s);
+  g_cg_scratch.clear();
+}
+}  // namespace lapis
+
+namespace {
+static_assert(sizeof(CgState) <= 256, "the state sits in the first 256 bytes of the scratch");
+
+// Rows per workgroup of the one-launch solve, 0 when the system is not for it: it has to fit the chip with a
+// workgroup per compute unit, every workgroup's entries its LDS, and rows are walked by one thread each.
+int small_rows(const lapis_hip_csr_plan *plan, int64_t n, int *entries) {
+  const lapis_hip_csr_stats &s = plan->stats;
+  if (n < 1 || s.nnz < 1 || s.max_row_len > 64) return 0;
+  const int cus = std::min(device_cu_count(), kSmallMaxBlocks);
+  // fewer workgroups make a cheaper exchange: 256^2 rows of 5 take 327 us (41 iterations) with 512 rows each, 425 with 256
+  const int64_t rows = std::max<int64_t>(kSmallThreads, ceil_div(n, cus));
+  if (rows > (int64_t)kSmallThreads * kSmallMaxRowsPerThread) return 0;
+  if (rows * s.max_row_len * 12 > kSmallLdsBytes) return 0;
+  *entries = (int)((rows * s.max_row_len + 1) & ~(int64_t)1);
+  return (int)rows;
+}
+
+template <int RPT>
+hipError_t launch_small_rpt(const CgSmallArgs &a, size_t lds, hipStream_t st) {
+  auto kernel = a.dinv ? cg_small_kernel<RPT, true> : cg_small_kernel<RPT, false>;
+  static std::once_flag once;
+  static hipError_t status = hipSuccess;
+  std::call_once(once, [] {
+    status = hipFuncSetAttribute(reinterpret_cast<const void *>(cg_small_kernel<RPT, true>),
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, kSmallLdsBytes);
+    if (status == hipSuccess)
+      status = hipFuncSetAttribute(reinterpret_cast<const void *>(cg_small_kernel<RPT, false>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, kSmallLdsBytes);
+  });
+  if (status != hipSuccess) return status;
+  // A cooperative launch: the workgroups of one solve are resident together whatever other streams run (8 us more
+  // per solve than a plain launch).
+  CgSmallArgs copy = a;
+  void *params[] = {&copy};
+  return hipLaunchCooperativeKernel(reinterpret_cast<const void *>(kernel), dim3(a.blocks), dim3(kSmallThreads), params,
+                                    (unsigned)lds, st);
+}
+
+hipError_t launch_small(const CgSmallArgs &a, hipStream_t st) {
+  const size_t lds = (size_t)a.entries * 12;
+  switch ((int)ceil_div(a.rows, kSmallThreads)) {
+    case 1: return launch_small_rpt<1>(a, lds, st);
+    case 2: return launch_small_rpt<2>(a, lds, st);
+    case 3: return launch_small_rpt<3>(a, lds, st);
+    default: return launch_small_rpt<4>(a, lds, st);
+  }
+}
+
 
 // What the solver applies as A and as the preconditioner.
 //   mask == nullptr: A p is the SpMV, z = r * prec (prec may be null: z = r)      examples/pcg_solve.py:52-101
@@ -363,8 +742,7 @@ int pcg_run(lapis_hip_csr_plan *plan, int64_t n, const int32_t *pos, const int32
   lapis_hip_csr_plan *own_plan = nullptr;
   double *own_work = nullptr;
   int64_t stride = n;  // distance between the four work vectors
-  CgState *state = nullptr;
-  double *partials = nullptr;
+  CgScratch *scratch = nullptr;
   double *chunk_pap = nullptr;  // per chunk of the row-split SpMV: p.Ap over the rows inside it
   bool finished = false;
 
@@ -372,8 +750,10 @@ int pcg_run(lapis_hip_csr_plan *plan, int64_t n, const int32_t *pos, const int32
   auto cleanup = [&]() {
     if (own_plan) lapis_hip_csr_plan_destroy(own_plan);
     if (own_work) (void)hipFree(own_work);
-    if (state) (void)hipFree(state);
-    if (partials) (void)hipFree(partials);
+    if (scratch) {
+      if (!finished) (void)hipStreamSynchronize(st);  // an error left work queued on the scratch
+      give_scratch(scratch);
+    }
     if (chunk_pap) (void)hipFree(chunk_pap);
   };
 #define PCG_TRY(expr)                                                                          \
@@ -412,14 +792,68 @@ int pcg_run(lapis_hip_csr_plan *plan, int64_t n, const int32_t *pos, const int32
   double *r = work, *z = dinv ? work + stride : work, *p = work + 2 * stride, *Ap = work + 3 * stride;
   double *tmp = mask ? work + 4 * stride : nullptr;
   const int divide = mask ? 1 : 0;
-  PCG_TRY(hipMalloc(&state, sizeof(CgState)));
-  PCG_TRY(hipMalloc(&partials, sizeof(double) * 3 * kDotMaxBlocks));
+  PCG_TRY(take_scratch(&scratch, st));
+  if (!mask && maxiter != 0) {
+    int entries = 0;
+    const int rows = small_rows(plan, n, &entries);
+    if (rows) {
+      CgSmallArgs a{};
+      a.n = (int)n;
+      a.rows = rows;
+      a.blocks = (int)ceil_div(n, rows);
+      a.entries = entries;
+      a.pos = pos;
+      a.crd = crd;
+      a.val = val;
+      a.b = b;
+      a.dinv = dinv;
+      a.x = x;
+      a.r = r;
+      a.z = work + stride;
+      a.p0 = work + 2 * stride;
+      a.p1 = work + 3 * stride;
+      a.slots = scratch->slots;
+      a.maxiter = maxiter;
+      a.budget = 4096;
+      a.tol = tol;
+      const char *spins = getenv("LAPIS_HIP_CG_SPINS");  // tests of what happens when a wait runs out
+      a.spins = spins ? atoi(spins) : 1 << 18;
+      a.out = scratch->host_result;
+      for (;;) {
+        if (scratch->epoch > 0xf0000000u) {  // start over before the numbers wrap
+          PCG_RC(lapis_hip_fill_f64((int64_t)kSlotWords, 0.0, reinterpret_cast<double *>(scratch->slots), stream));
+          scratch->epoch = 1;
+        }
+        a.epoch = scratch->epoch;
+        scratch->epoch += 2 * (unsigned)a.budget + 2;
+        scratch->host_result->fault = 0;
+        PCG_TRY(launch_small(a, st));
+        PCG_TRY(hipStreamSynchronize(st));
+        const CgSmallResult &got = *scratch->host_result;
+        if (got.fault) break;  // the workgroups were not resident together: the kernels below start from the beginning
+        if (got.done_iter != 0) {
+          *iters = got.done_iter;
+          *relres = got.relres;
+          finished = true;
+          cleanup();
+          return LAPIS_HIP_OK;
+        }
+        a.resume = 1;
+        a.iter0 += a.budget;
+        a.rz = got.rz;
+        a.beta = got.beta;
+        a.initres = got.initres;
+      }
+    }
+  }
+  CgState *state = scratch->state;
+  double *partials = scratch->partials;
   if (!mask && plan->stats.kernel == LAPIS_HIP_SPMV_NNZSPLIT && plan->nchunks > 1)
     PCG_TRY(hipMalloc(&chunk_pap, sizeof(double) * (size_t)plan->nchunks));
-  CgState h{};
-  h.maxiter = maxiter;
-  h.tol = tol;
-  PCG_TRY(hipMemcpyAsync(state, &h, sizeof(h), hipMemcpyHostToDevice, st));
+  *scratch->host_state = CgState{};
+  scratch->host_state->maxiter = maxiter;
+  scratch->host_state->tol = tol;
+  PCG_TRY(hipMemcpyAsync(state, scratch->host_state, sizeof(CgState), hipMemcpyHostToDevice, st));
 
   const int grid = dot_grid(n);
   const int pre = dinv ? 1 : 0;
@@ -491,9 +925,9 @@ int pcg_run(lapis_hip_csr_plan *plan, int64_t n, const int32_t *pos, const int32
       PCG_TRY(hipGetLastError());
     }
     launched += (uint64_t)todo;
-    CgState now;
-    PCG_TRY(hipMemcpyAsync(&now, state, sizeof(now), hipMemcpyDeviceToHost, st));
+    PCG_TRY(hipMemcpyAsync(scratch->host_state, state, sizeof(CgState), hipMemcpyDeviceToHost, st));
     PCG_TRY(hipStreamSynchronize(st));
+    const CgState &now = *scratch->host_state;
     if (now.done_iter != 0) {
       *iters = now.done_iter;
       *relres = now.relres;

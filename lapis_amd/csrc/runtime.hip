@@ -80,7 +80,10 @@ extern "C" int lapis_hip_finalize(void) {
   std::lock_guard<std::mutex> lock(g_mutex);
   if (g_refcount <= 0)
     return set_error(LAPIS_HIP_ERR_NOT_INITIALIZED, "lapis_hip_finalize: not initialized");
-  if (--g_refcount == 0) dot_release_scratch();
+  if (--g_refcount == 0) {
+    dot_release_scratch();
+    cg_release_scratch();
+  }
   return LAPIS_HIP_OK;
 }
 

@@ -1,0 +1,68 @@
+"""The one-launch CG of systems that fit the chip's LDS, at the edges of its rows per workgroup and per thread, against
+the oracle; a solve that outlives one launch; and the way back to the many-launch solve when a wait runs out."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+import torch
+
+from gpu_util import dev
+
+pytestmark = pytest.mark.gpu
+
+
+def _spd(n, per_row, seed):
+    rng = np.random.Generator(np.random.PCG64(seed))
+    k = max(1, min(n, per_row) // 2)
+    R = sp.csr_matrix((rng.random(n * k), rng.integers(0, n, n * k), np.arange(0, n * k + 1, k)), shape=(n, n))
+    S = R + R.T
+    A = sp.csr_matrix(S + sp.diags(np.asarray(abs(S).sum(axis=1)).ravel() + 0.5 + rng.random(n)))
+    A.sum_duplicates()
+    A.sort_indices()
+    return A, rng
+
+
+def _solve(gpu, A, b, dinv, tol, maxiter):
+    n = b.shape[0]
+    pos, crd = dev(A.indptr.astype(np.int32)), dev(A.indices.astype(np.int32))
+    plan = gpu.CsrPlan(n, n, pos, crd)
+    x = torch.full((n,), 7.0, dtype=torch.float64, device="cuda")
+    iters, relres = gpu.pcg(plan, n, pos, crd, dev(A.data), dev(b), None if dinv is None else dev(dinv), tol, maxiter, x)
+    return x.cpu().numpy(), iters, relres
+
+
+@pytest.mark.parametrize("preconditioned", [False, True])
+@pytest.mark.parametrize("n,per_row", [(1, 1), (2, 2), (63, 6), (511, 6), (512, 6), (513, 6), (1025, 20), (131072, 4), (131073, 4),
+                                       (262145, 4), (400000, 4)])
+def test_solves_at_the_edges_of_its_shapes(gpu, oracle, n, per_row, preconditioned):
+    A, rng = _spd(n, per_row, n)
+    b = rng.standard_normal(n)
+    dinv = 1.0 / A.diagonal() if preconditioned else None
+    print("case", n, per_row, preconditioned, "longest row", np.diff(A.indptr).max(), flush=True)
+    for tol, maxiter in ((1e-9, 300), (0.0, 3)):
+        xo, io, ro = oracle.pcg(A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data, b,
+                                np.ones(n) if dinv is None else dinv, tol, maxiter)
+        xg, ig, rg = _solve(gpu, A, b, dinv, tol, maxiter)
+        assert ig == io
+        assert np.allclose(xg, xo, rtol=1e-9, atol=1e-12 * np.abs(xo).max())
+        assert abs(rg - ro) <= 1e-6 * ro + 1e-16
+
+
+def test_a_solve_longer_than_one_launch(gpu):
+    n = 20000  # a 1-D Laplacian: CG needs about n iterations, so 5000 leave it in the middle
+    A = sp.csr_matrix(sp.diags([-1.0, 2.0, -1.0], [-1, 0, 1], shape=(n, n)))
+    b = np.random.Generator(np.random.PCG64(4)).standard_normal(n)
+    x, iters, relres = _solve(gpu, A, b, np.full(n, 0.5), 0.0, 5000)
+    assert iters == 5000
+    true = np.linalg.norm(b - A @ x) / np.linalg.norm(b)
+    assert abs(true - relres) <= 1e-7 * max(true, 1.0)
+    x1, i1, r1 = _solve(gpu, A, b, None, 0.0, 4097)
+    assert i1 == 4097 and abs(np.linalg.norm(b - A @ x1) / np.linalg.norm(b) - r1) <= 1e-7 * max(r1, 1.0)
+
+
+def test_a_wait_that_runs_out_falls_back_to_the_many_launch_solve(gpu, oracle, monkeypatch):
+    A, rng = _spd(3000, 8, 9)
+    b = rng.standard_normal(3000)
+    want = _solve(gpu, A, b, None, 1e-9, 200)
+    monkeypatch.setenv("LAPIS_HIP_CG_SPINS", "0")
+    got = _solve(gpu, A, b, None, 1e-9, 200)
+    assert got[1] == want[1] and np.allclose(got[0], want[0], rtol=1e-9, atol=1e-12)
