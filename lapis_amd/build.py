@@ -24,7 +24,7 @@ LIBDIR = os.path.join(HERE, "lib")
 OBJDIR = os.path.join(CSRC, "build")
 INCLUDE = os.path.join(ROOT, "include")
 
-KERNEL_SOURCES = ["runtime.hip", "spmv.hip", "colblock.hip", "colgroup.hip", "spmm.hip", "blas1.hip", "cg.hip",
+KERNEL_SOURCES = ["runtime.hip", "spmv.hip", "rowchunk.hip", "colblock.hip", "colgroup.hip", "spmm.hip", "blas1.hip", "cg.hip",
                   "calibrate.hip"]
 SHIM_SOURCES = ["module_shim.hip"]
 

@@ -20,9 +20,10 @@
 // both reads and replaces (r.z) are kept twice, indexed by iteration parity.
 //
 // x is needed by nobody until the solve ends, so x += alpha p is made by the kernel
-// that reads p anyway to replace it (p = z + beta p), not by the one that updates r:
-// p is then read twice per iteration (by the SpMV's gathers and by that kernel), not
-// three times.  The pass that decides to leave still adds its alpha p and leaves p alone.
+// that reads p anyway to replace it (p = z + beta p), not by the one that updates r, and
+// there for two iterations at once: odd iterations leave their p where it is (the next p
+// goes into a second buffer), even ones add the alpha p of both, x being read and written
+// half as often.  The pass that decides to leave adds what is owed and makes no new p.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -42,11 +43,18 @@ struct CgState {
   double rr;       // r . r after the update
   double initres;  // sqrt(r0 . r0)
   double relres;
-  double alpha;    // r.z / p.Ap of the iteration under way
+  double alpha[2]; // r.z / p.Ap of iteration i is alpha[i & 1]
   unsigned long long done_iter;  // 0 while iterating, then the reference's counter i at exit (it starts at 1)
   unsigned long long maxiter;
   double tol;
 };
+
+// What the device writes into pinned host memory.
+struct CgProgress {
+  unsigned long long iter;  // last iteration whose convergence test was made; kLeft is set when it left
+  double relres;            // of the iteration that left
+};
+constexpr unsigned long long kLeft = 1ull << 63;
 
 __device__ __forceinline__ double block_sum_256d(double v, double *lds4) {
   v = group_sum<64>(v);
@@ -85,19 +93,17 @@ __device__ __forceinline__ double ordered_total(const double *partials, int coun
 __device__ __forceinline__ v2d ld2(const double *p, long long i) { return reinterpret_cast<const v2d *>(p)[i]; }
 __device__ __forceinline__ void st2(double *p, long long i, v2d v) { reinterpret_cast<v2d *>(p)[i] = v; }
 
-// r0 = b, z0 = r0*dinv (or r0), p0 = z0, x0 = 0; block partials of r0.r0 and r0.z0.
+// r0 = b, p0 = r0*dinv (or r0), x0 = 0; block partials of r0.r0 and r0.z0.
 __global__ __launch_bounds__(256) void cg_init_kernel(long long n, const double *__restrict__ b,
                                                       const double *__restrict__ dinv, double *__restrict__ x,
-                                                      double *__restrict__ r, double *__restrict__ z,
-                                                      double *__restrict__ p, double *__restrict__ partials,
-                                                      int divide) {
+                                                      double *__restrict__ r, double *__restrict__ p,
+                                                      double *__restrict__ partials, int divide) {
   __shared__ double lds4[4];
   double rr = 0.0, rz = 0.0;
   CG_GRID_STRIDE(i, 0, n) {
     const double ri = b[i];
     const double zi = dinv ? (divide ? ri / dinv[i] : ri * dinv[i]) : ri;
     r[i] = ri;
-    if (dinv) z[i] = zi;
     p[i] = zi;
     x[i] = 0.0;
     rr = rr + ri * ri;
@@ -126,6 +132,17 @@ __global__ __launch_bounds__(256) void cg_pap_kernel(long long n, const double *
   CG_GRID_STRIDE(i, 2 * nv, n) acc = acc + p[i] * Ap[i];
   const double bsum = block_sum_256d(acc, lds4);
   if (threadIdx.x == 0) partials[blockIdx.x] = bsum;
+}
+
+// Sums of `count` partial sums in at most kReducedPartials parts, a part per block, each in a fixed order.
+constexpr int kReducedPartials = 64;
+__global__ __launch_bounds__(256) void cg_reduce_partials_kernel(int count, const double *__restrict__ in,
+                                                                 double *__restrict__ out) {
+  __shared__ double lds4[4];
+  const int per = (count + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int first = (int)blockIdx.x * per;
+  const double sum = ordered_total(in + first, min(per, count - first), lds4);
+  if (threadIdx.x == 0) out[blockIdx.x] = sum;
 }
 
 // The same partials when Ap came from the row-split SpMV kernel with its fix-up left out
@@ -163,15 +180,24 @@ __global__ __launch_bounds__(256) void cg_pap_fix_kernel(int nchunks, int chunks
   if (threadIdx.x == 0) partials[blockIdx.x] = bsum;
 }
 
-// r -= alpha Ap ; block partials of r.r.   alpha = r.z / p.Ap with p.Ap summed here from the
-// partials the p.Ap kernel left; block 0 keeps alpha for the kernel that updates x and p.
+// z = r dinv, r / dinv or r
+enum { kNoPrec = 0, kMultiply = 1, kDivide = 2 };
+template <int PREC>
+__device__ __forceinline__ double preconditioned(double r, double d) {
+  return PREC == kDivide ? r / d : PREC == kMultiply ? r * d : r;
+}
+
+// r -= alpha Ap ; block partials of r.r and, preconditioned, of r.z.   alpha = r.z / p.Ap with p.Ap summed here
+// from the partials the p.Ap kernel left; block 0 keeps alpha for the kernel that updates x and p.
 // Ap is read here for the last time: it goes through streaming accesses, so that it does not
 // push p, which the next SpMV gathers from, out of the caches.
+template <int PREC>
 __global__ __launch_bounds__(256) void cg_update_r_kernel(long long n, const double *__restrict__ Ap,
-                                                          double *__restrict__ r, CgState *st,
-                                                          unsigned long long iter, int count,
+                                                          double *__restrict__ r, const double *__restrict__ dinv,
+                                                          CgState *st, unsigned long long iter, int count,
                                                           const double *__restrict__ pap_partials,
-                                                          double *__restrict__ rr_partials, int vec) {
+                                                          double *__restrict__ rr_partials,
+                                                          double *__restrict__ rz_partials, int vec) {
   __shared__ double lds4[4];
   if (block_done_iter(st)) return;
   const double pAp = ordered_total(pap_partials, count, lds4);
@@ -179,73 +205,56 @@ __global__ __launch_bounds__(256) void cg_update_r_kernel(long long n, const dou
   const double malpha = -alpha;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     st->pAp = pAp;
-    st->alpha = alpha;
+    st->alpha[iter & 1] = alpha;
   }
-  double rr = 0.0;
+  double rr = 0.0, rz = 0.0;
   const long long nv = vec ? n / 2 : 0;
   CG_GRID_STRIDE(i, 0, nv) {
     const v2d av = load_stream(reinterpret_cast<const v2d *>(Ap) + i);
-    v2d rv = ld2(r, i);
+    v2d rv = ld2(r, i), dv = {0.0, 0.0};
+    if (PREC) dv = ld2(dinv, i);
     rv.x = rv.x + av.x * malpha;
     rv.y = rv.y + av.y * malpha;
     st2(r, i, rv);
     rr = rr + rv.x * rv.x;
     rr = rr + rv.y * rv.y;
+    if (PREC) {
+      rz = rz + rv.x * preconditioned<PREC>(rv.x, dv.x);
+      rz = rz + rv.y * preconditioned<PREC>(rv.y, dv.y);
+    }
   }
   CG_GRID_STRIDE(i, 2 * nv, n) {
     const double rt = Ap[i] * malpha;
     const double ri = r[i] + rt;
     r[i] = ri;
     rr = rr + ri * ri;
+    if (PREC) rz = rz + ri * preconditioned<PREC>(ri, dinv[i]);
   }
-  const double bsum = block_sum_256d(rr, lds4);
-  if (threadIdx.x == 0) rr_partials[blockIdx.x] = bsum;
+  const double brr = block_sum_256d(rr, lds4);
+  if (threadIdx.x == 0) rr_partials[blockIdx.x] = brr;
+  if (PREC) {
+    const double brz = block_sum_256d(rz, lds4);
+    if (threadIdx.x == 0) rz_partials[blockIdx.x] = brz;
+  }
 }
 
 // The convergence test of examples/pcg_solve.py:84-90, made by every block from the
-// r.r partials: leave when !(relres > tol) or i == maxiter.  Block 0 records the exit.
-__device__ __forceinline__ bool cg_continues(CgState *st, unsigned long long iter, double rr) {
+// r.r partials: leave when !(relres > tol) or i == maxiter.  Block 0 records the exit, and tells the host how far
+// the device is (relaxed stores to pinned memory: nothing waits for them, and the host reads relres after it has
+// waited for the stream).
+__device__ __forceinline__ bool cg_continues(CgState *st, CgProgress *host, unsigned long long iter, double rr) {
   const double relres = sqrt(rr) / st->initres;
   const bool go_on = (relres > st->tol) && (iter != st->maxiter);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     st->rr = rr;
     st->relres = relres;
-    if (!go_on) st->done_iter = iter;
+    if (!go_on) {
+      st->done_iter = iter;
+      host->relres = relres;
+    }
+    __hip_atomic_store(&host->iter, go_on ? iter : iter | kLeft, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
   return go_on;
-}
-
-// Convergence test, then z = r * dinv (or r / dinv) ; block partials of r.z     (preconditioned runs only)
-__global__ __launch_bounds__(256) void cg_precond_kernel(long long n, const double *__restrict__ r,
-                                                         const double *__restrict__ dinv, double *__restrict__ z,
-                                                         CgState *st, unsigned long long iter, int count,
-                                                         const double *__restrict__ rr_partials,
-                                                         double *__restrict__ rz_partials, int vec, int divide) {
-  __shared__ double lds4[4];
-  if (block_done_iter(st)) return;  // an earlier pass left, or block 0 of this kernel has just decided to
-  const double rr = ordered_total(rr_partials, count, lds4);
-  if (!cg_continues(st, iter, rr)) return;
-  double acc = 0.0;
-  const long long nv = vec ? n / 2 : 0;
-  CG_GRID_STRIDE(i, 0, nv) {
-    // r and the preconditioner are read here for the last time in this iteration
-    const v2d rv = load_stream(reinterpret_cast<const v2d *>(r) + i);
-    const v2d dv = load_stream(reinterpret_cast<const v2d *>(dinv) + i);
-    v2d zv;
-    zv.x = divide ? rv.x / dv.x : rv.x * dv.x;
-    zv.y = divide ? rv.y / dv.y : rv.y * dv.y;
-    st2(z, i, zv);
-    acc = acc + rv.x * zv.x;
-    acc = acc + rv.y * zv.y;
-  }
-  CG_GRID_STRIDE(i, 2 * nv, n) {
-    const double ri = r[i];
-    const double zi = divide ? ri / dinv[i] : ri * dinv[i];
-    z[i] = zi;
-    acc = acc + ri * zi;
-  }
-  const double bsum = block_sum_256d(acc, lds4);
-  if (threadIdx.x == 0) rz_partials[blockIdx.x] = bsum;
 }
 
 // Elementwise pieces of the masked operator and of the moment right-hand sides
@@ -270,63 +279,85 @@ __global__ __launch_bounds__(256) void normalize_mom2_kernel(long long n, const 
   }
 }
 
-// x += alpha p ; p = z + beta p with beta = (new r.z) / (old r.z).  Unpreconditioned, z is r
-// and the new r.z is r.r: this kernel then makes the convergence test itself; preconditioned,
-// the test was made by cg_precond_kernel and `partials` holds r.z.  The pass that leaves
-// (the exit mark names this very iteration) still owes x its alpha p and keeps p as it is;
-// passes queued behind it find an older mark and touch nothing.  x goes through streaming
-// accesses: it is touched once per iteration and must not push p out of the caches.
-__global__ __launch_bounds__(256) void cg_update_xp_kernel(long long n, const double *__restrict__ z,
-                                                           double *__restrict__ p, double *__restrict__ x,
-                                                           CgState *st, unsigned long long iter, int count,
-                                                           const double *__restrict__ partials, int preconditioned,
-                                                           int vec) {
+// Convergence test; p_next = z + beta p with beta = (new r.z) / (old r.z) and z made from r; in even iterations
+// x += alpha' p' + alpha p, with the p' and alpha' of the iteration before (p_next overwrites p').
+// Every block makes the test, from the r.r partials.  The pass that leaves (the exit mark may already name this very
+// iteration) adds to x what is owed to it and makes no p; passes queued behind it find an older mark and touch
+// nothing.  x and r go through streaming accesses: they are touched for the last time in this iteration and must not
+// push p out of the caches.
+template <int PREC, bool EVEN>
+__global__ __launch_bounds__(256) void cg_update_xp_kernel(long long n, const double *__restrict__ r,
+                                                           const double *__restrict__ dinv, const double *__restrict__ p,
+                                                           double *__restrict__ other, double *__restrict__ x, CgState *st,
+                                                           CgProgress *host, unsigned long long iter, int count,
+                                                           const double *__restrict__ rr_partials,
+                                                           const double *__restrict__ rz_partials, int vec) {
   __shared__ double lds4[4];
   const unsigned long long mark = block_done_iter(st);
   if (mark != 0 && mark != iter) return;
-  const double rz_new = ordered_total(partials, count, lds4);
-  const bool go_on = preconditioned ? mark == 0 : cg_continues(st, iter, rz_new);
-  const double alpha = st->alpha;
+  const double rr = ordered_total(rr_partials, count, lds4);
+  const double rz_new = PREC ? ordered_total(rz_partials, count, lds4) : rr;
+  const bool go_on = cg_continues(st, host, iter, rr);
+  const double alpha = st->alpha[iter & 1], alpha_before = st->alpha[(iter + 1) & 1];
   const long long nv = vec ? n / 2 : 0;
   if (!go_on) {
     CG_GRID_STRIDE(i, 0, nv) {
       const v2d pv = ld2(p, i);
       v2d xv = load_stream(reinterpret_cast<const v2d *>(x) + i);
+      if (EVEN) {
+        const v2d qv = ld2(other, i);
+        xv.x = xv.x + qv.x * alpha_before;
+        xv.y = xv.y + qv.y * alpha_before;
+      }
       xv.x = xv.x + pv.x * alpha;
       xv.y = xv.y + pv.y * alpha;
       store_stream(reinterpret_cast<v2d *>(x) + i, xv);
     }
     CG_GRID_STRIDE(i, 2 * nv, n) {
-      const double xt = p[i] * alpha;
-      x[i] = x[i] + xt;
+      double xi = x[i];
+      if (EVEN) xi = xi + other[i] * alpha_before;
+      x[i] = xi + p[i] * alpha;
     }
     return;
   }
   const double beta = rz_new / st->rz[iter & 1];
   if (blockIdx.x == 0 && threadIdx.x == 0) st->rz[(iter + 1) & 1] = rz_new;
   CG_GRID_STRIDE(i, 0, nv) {
-    const v2d zv = load_stream(reinterpret_cast<const v2d *>(z) + i);
-    v2d pv = ld2(p, i);
-    v2d xv = load_stream(reinterpret_cast<const v2d *>(x) + i);
-    xv.x = xv.x + pv.x * alpha;
-    xv.y = xv.y + pv.y * alpha;
-    store_stream(reinterpret_cast<v2d *>(x) + i, xv);
-    pv.x = zv.x + pv.x * beta;
-    pv.y = zv.y + pv.y * beta;
-    st2(p, i, pv);
+    v2d zv = load_stream(reinterpret_cast<const v2d *>(r) + i);
+    if (PREC) {
+      const v2d dv = load_stream(reinterpret_cast<const v2d *>(dinv) + i);
+      zv.x = preconditioned<PREC>(zv.x, dv.x);
+      zv.y = preconditioned<PREC>(zv.y, dv.y);
+    }
+    const v2d pv = ld2(p, i);
+    if (EVEN) {
+      const v2d qv = ld2(other, i);
+      v2d xv = load_stream(reinterpret_cast<const v2d *>(x) + i);
+      xv.x = xv.x + qv.x * alpha_before;
+      xv.y = xv.y + qv.y * alpha_before;
+      xv.x = xv.x + pv.x * alpha;
+      xv.y = xv.y + pv.y * alpha;
+      store_stream(reinterpret_cast<v2d *>(x) + i, xv);
+    }
+    v2d nv2;
+    nv2.x = zv.x + pv.x * beta;
+    nv2.y = zv.y + pv.y * beta;
+    st2(other, i, nv2);
   }
   CG_GRID_STRIDE(i, 2 * nv, n) {
+    const double zi = preconditioned<PREC>(r[i], PREC ? dinv[i] : 1.0);
     const double pi = p[i];
-    const double xt = pi * alpha;
-    x[i] = x[i] + xt;
-    const double pt = pi * beta;
-    p[i] = z[i] + pt;
+    if (EVEN) {
+      const double xi = x[i] + other[i] * alpha_before;
+      x[i] = xi + pi * alpha;
+    }
+    other[i] = zi + pi * beta;
   }
 }
 
 // One block, once per solve: the scalars of the initial residual.
 __global__ __launch_bounds__(256) void cg_init_scalar_kernel(int count, const double *__restrict__ partials,
-                                                             CgState *st) {
+                                                             CgState *st, unsigned long long maxiter, double tol) {
   __shared__ double lds4[4];
   const double trr = ordered_total(partials, count, lds4);
   const double trz = ordered_total(partials + kDotMaxBlocks, count, lds4);
@@ -334,6 +365,8 @@ __global__ __launch_bounds__(256) void cg_init_scalar_kernel(int count, const do
     st->initres = sqrt(trr);
     st->rz[1] = trz;  // the first iteration is i = 1
     st->done_iter = 0;
+    st->maxiter = maxiter;
+    st->tol = tol;
   }
 }
 
@@ -597,9 +630,11 @@ struct CgScratch {
   double *partials = nullptr;
   unsigned long long *slots = nullptr;
   unsigned epoch = 1;  // slots carry smaller numbers only
-  CgState *host_state = nullptr;
+  CgProgress *progress = nullptr;
   CgSmallResult *host_result = nullptr;
   void *device_block = nullptr, *host_block = nullptr;
+  double *parts = nullptr;  // p.Ap in more parts than every block can add up
+  size_t parts_capacity = 0;
 };
 constexpr int kKeptScratch = 8;
 std::mutex g_cg_mutex;
@@ -609,6 +644,7 @@ constexpr size_t kSlotWords = 2 * (size_t)kSmallMaxBlocks * 4;
 
 void free_scratch(CgScratch *s) {
   if (s->device_block) (void)hipFree(s->device_block);
+  if (s->parts) (void)hipFree(s->parts);
   if (s->host_block) (void)hipHostFree(s->host_block);
   delete s;
 }
@@ -636,7 +672,7 @@ hipError_t take_scratch(CgScratch **out, hipStream_t st) {
     s->state = reinterpret_cast<CgState *>(base);
     s->partials = reinterpret_cast<double *>(base + 256);
     s->slots = reinterpret_cast<unsigned long long *>(base + 256 + partial_bytes);
-    s->host_state = static_cast<CgState *>(s->host_block);
+    s->progress = static_cast<CgProgress *>(s->host_block);
     s->host_result = reinterpret_cast<CgSmallResult *>(static_cast<char *>(s->host_block) + 512);
     // no slot carries the number of an exchange before that exchange writes it
     if (lapis_hip_fill_f64((int64_t)kSlotWords, 0.0, reinterpret_cast<double *>(s->slots), st) != LAPIS_HIP_OK)
@@ -650,7 +686,27 @@ hipError_t take_scratch(CgScratch **out, hipStream_t st) {
   return hipSuccess;
 }
 
+constexpr size_t kKeptParts = (size_t)1 << 19;
+
+hipError_t parts_of(CgScratch *s, size_t count, double **out) {
+  if (s->parts_capacity < count) {
+    if (s->parts) (void)hipFree(s->parts);
+    s->parts = nullptr;
+    s->parts_capacity = 0;
+    const hipError_t e = hipMalloc(&s->parts, sizeof(double) * count);
+    if (e != hipSuccess) return e;
+    s->parts_capacity = count;
+  }
+  *out = s->parts;
+  return hipSuccess;
+}
+
 void give_scratch(CgScratch *s) {
+  if (s->parts_capacity > kKeptParts) {
+    (void)hipFree(s->parts);
+    s->parts = nullptr;
+    s->parts_capacity = 0;
+  }
   {
     std::lock_guard<std::mutex> lock(g_cg_mutex);
     if ((int)g_cg_scratch.size() < kKeptScratch) {
@@ -743,7 +799,7 @@ int pcg_run(lapis_hip_csr_plan *plan, int64_t n, const int32_t *pos, const int32
   double *own_work = nullptr;
   int64_t stride = n;  // distance between the four work vectors
   CgScratch *scratch = nullptr;
-  double *chunk_pap = nullptr;  // per chunk of the row-split SpMV: p.Ap over the rows inside it
+  double *chunk_pap = nullptr;  // p.Ap per chunk or per workgroup of the SpMV, where every block cannot add up that many
   bool finished = false;
 
   // one-exit cleanup
@@ -754,7 +810,6 @@ int pcg_run(lapis_hip_csr_plan *plan, int64_t n, const int32_t *pos, const int32
       if (!finished) (void)hipStreamSynchronize(st);  // an error left work queued on the scratch
       give_scratch(scratch);
     }
-    if (chunk_pap) (void)hipFree(chunk_pap);
   };
 #define PCG_TRY(expr)                                                                          \
   do {                                                                                         \
@@ -789,9 +844,8 @@ int pcg_run(lapis_hip_csr_plan *plan, int64_t n, const int32_t *pos, const int32
     PCG_TRY(hipMalloc(&own_work, sizeof(double) * (mask ? 5 : 4) * (size_t)stride));
     work = own_work;
   }
-  double *r = work, *z = dinv ? work + stride : work, *p = work + 2 * stride, *Ap = work + 3 * stride;
+  double *r = work, *p_odd = work + 2 * stride, *p_even = work + stride, *Ap = work + 3 * stride;  // p of odd, even iterations
   double *tmp = mask ? work + 4 * stride : nullptr;
-  const int divide = mask ? 1 : 0;
   PCG_TRY(take_scratch(&scratch, st));
   if (!mask && maxiter != 0) {
     int entries = 0;
@@ -848,41 +902,46 @@ int pcg_run(lapis_hip_csr_plan *plan, int64_t n, const int32_t *pos, const int32
   }
   CgState *state = scratch->state;
   double *partials = scratch->partials;
-  if (!mask && plan->stats.kernel == LAPIS_HIP_SPMV_NNZSPLIT && plan->nchunks > 1)
-    PCG_TRY(hipMalloc(&chunk_pap, sizeof(double) * (size_t)plan->nchunks));
-  *scratch->host_state = CgState{};
-  scratch->host_state->maxiter = maxiter;
-  scratch->host_state->tol = tol;
-  PCG_TRY(hipMemcpyAsync(state, scratch->host_state, sizeof(CgState), hipMemcpyHostToDevice, st));
+  const bool row_chunks = !mask && plan->runs_rowchunk();
+  const int xy_blocks = row_chunks ? rowchunk_xy_blocks(plan) : 0;
+  if (xy_blocks > kDotMaxBlocks) PCG_TRY(parts_of(scratch, (size_t)xy_blocks, &chunk_pap));
+  if (!mask && !row_chunks && plan->stats.kernel == LAPIS_HIP_SPMV_NNZSPLIT && plan->nchunks > 1)
+    PCG_TRY(parts_of(scratch, (size_t)plan->nchunks, &chunk_pap));
 
   const int grid = dot_grid(n);
-  const int pre = dinv ? 1 : 0;
-  const int vec = (aligned16(x) && aligned16(r) && aligned16(z) && aligned16(p) && aligned16(Ap) &&
-                   (!dinv || aligned16(dinv)))
-                      ? 1
-                      : 0;
-  hipLaunchKernelGGL(cg_init_kernel, dim3(grid), dim3(256), 0, st, (long long)n, b, dinv, x, r, z, p, partials,
-                     divide);
-  hipLaunchKernelGGL(cg_init_scalar_kernel, dim3(1), dim3(256), 0, st, grid, partials, state);
+  const int prec = !dinv ? kNoPrec : mask ? kDivide : kMultiply;
+  const int vec = (aligned16(x) && aligned16(r) && aligned16(p_odd) && aligned16(p_even) && aligned16(Ap) && (!dinv || aligned16(dinv))) ? 1 : 0;
+  volatile CgProgress *progress = scratch->progress;
+  progress->iter = 0;
+  progress->relres = 0.0;
+  hipLaunchKernelGGL(cg_init_kernel, dim3(grid), dim3(256), 0, st, (long long)n, b, dinv, x, r, p_odd, partials,
+                     mask ? 1 : 0);
+  hipLaunchKernelGGL(cg_init_scalar_kernel, dim3(1), dim3(256), 0, st, grid, partials, state,
+                     (unsigned long long)maxiter, tol);
   PCG_TRY(hipGetLastError());
   double *pap_partials = partials, *rr_partials = partials + kDotMaxBlocks, *rz_partials = partials + 2 * kDotMaxBlocks;
-  // The host looks at the device's exit mark after each batch of iterations; a
-  // batch queued past convergence costs launches only (its kernels return at once
-  // or touch scratch vectors only).
+  // The host stays a few iterations ahead of the device, which tells it how far it is: enough that the device never
+  // waits for a launch (about 100 us of work), few enough that little is left queued when it leaves -- such passes
+  // find the exit mark and return at once, the product of long-row kernels excepted.
+  const double iteration_us = ((double)plan->stats.nnz * 12.0 + (double)n * 100.0) / 5e6;
+  const uint64_t ahead = (uint64_t)std::min(32.0, 2.0 + 100.0 / (iteration_us + 4.0));
   uint64_t launched = 0;
-  int batch = 1;
   while (!finished) {
-    int todo = batch;
-    if (maxiter != 0) todo = (int)std::min<uint64_t>((uint64_t)todo, maxiter - launched);
-    if (todo <= 0) {
-      // iteration `maxiter` always raises the flag, so this is unreachable unless the state was corrupted
-      cleanup();
-      return set_error(LAPIS_HIP_ERR_RUNTIME, "pcg: %llu iterations queued and the device never reported an exit",
-                       (unsigned long long)launched);
-    }
-    for (int it = 0; it < todo; ++it) {
+    if (maxiter == 0 || launched < maxiter) {
+      const unsigned long long iter = ++launched;  // the reference's counter for this pass
+      double *p = iter & 1 ? p_odd : p_even, *other = iter & 1 ? p_even : p_odd;
+      int pap_count = grid;
       int deferred = 0;  // chunk length when the SpMV left its cut rows to the p.Ap kernel
-      if (mask) {
+      if (row_chunks) {
+        // Ap = A p and p.Ap in one pass
+        PCG_RC(launch_rowchunk_xy(plan, crd, val, p, Ap, st, chunk_pap ? chunk_pap : pap_partials, &pap_count,
+                                  &state->done_iter));
+        if (chunk_pap) {
+          hipLaunchKernelGGL(cg_reduce_partials_kernel, dim3(kReducedPartials), dim3(256), 0, st, pap_count, chunk_pap,
+                             pap_partials);
+          pap_count = kReducedPartials;
+        }
+      } else if (mask) {
         // plpt: tmp = mask*p ; Ap = A tmp ; Ap = (d*tmp - Ap)*mask
         PCG_RC(lapis_hip_mult_f64(n, p, mask, tmp, stream));
         PCG_RC(spmv_overwrite_f64(plan, n, n, pos, crd, val, tmp, Ap, stream));
@@ -892,8 +951,6 @@ int pcg_run(lapis_hip_csr_plan *plan, int64_t n, const int32_t *pos, const int32
         PCG_RC(spmv_overwrite_f64(plan, n, n, pos, crd, val, p, Ap, stream, chunk_pap ? &deferred : nullptr,
                                   chunk_pap));
       }
-      const unsigned long long iter = launched + (uint64_t)it + 1;  // the reference's counter for this pass
-      int pap_count = grid;
       if (deferred) {
         // one thread per chunk, at most kDotMaxBlocks blocks
         const int nchunks = plan->nchunks;
@@ -912,28 +969,57 @@ int pcg_run(lapis_hip_csr_plan *plan, int64_t n, const int32_t *pos, const int32
             return set_error(LAPIS_HIP_ERR_RUNTIME, "pcg: no p.Ap kernel for chunks of %d non-zeros", deferred);
         }
 #undef PCG_PAP_FIX
-      } else {
+      } else if (!row_chunks) {
         hipLaunchKernelGGL(cg_pap_kernel, dim3(grid), dim3(256), 0, st, (long long)n, p, Ap, pap_partials, vec);
       }
-      hipLaunchKernelGGL(cg_update_r_kernel, dim3(grid), dim3(256), 0, st, (long long)n, Ap, r, state, iter,
-                         pap_count, pap_partials, rr_partials, vec);
-      if (pre)
-        hipLaunchKernelGGL(cg_precond_kernel, dim3(grid), dim3(256), 0, st, (long long)n, r, dinv, z, state, iter,
-                           grid, rr_partials, rz_partials, vec, divide);
-      hipLaunchKernelGGL(cg_update_xp_kernel, dim3(grid), dim3(256), 0, st, (long long)n, z, p, x, state, iter,
-                         grid, pre ? rz_partials : rr_partials, pre, vec);
+#define PCG_UPDATES(PREC)                                                                                           \
+  hipLaunchKernelGGL(cg_update_r_kernel<PREC>, dim3(grid), dim3(256), 0, st, (long long)n, Ap, r, dinv, state, iter, \
+                     pap_count, pap_partials, rr_partials, rz_partials, vec);                                       \
+  hipLaunchKernelGGL((iter & 1 ? cg_update_xp_kernel<PREC, false> : cg_update_xp_kernel<PREC, true>), dim3(grid),    \
+                     dim3(256), 0, st, (long long)n, r, dinv, p, other, x, state, scratch->progress, iter, grid,     \
+                     rr_partials, rz_partials, vec)
+      if (prec == kNoPrec) {
+        PCG_UPDATES(kNoPrec);
+      } else if (prec == kMultiply) {
+        PCG_UPDATES(kMultiply);
+      } else {
+        PCG_UPDATES(kDivide);
+      }
+#undef PCG_UPDATES
       PCG_TRY(hipGetLastError());
     }
-    launched += (uint64_t)todo;
-    PCG_TRY(hipMemcpyAsync(scratch->host_state, state, sizeof(CgState), hipMemcpyDeviceToHost, st));
-    PCG_TRY(hipStreamSynchronize(st));
-    const CgState &now = *scratch->host_state;
-    if (now.done_iter != 0) {
-      *iters = now.done_iter;
-      *relres = now.relres;
-      finished = true;
+    // wait until no more than `ahead` iterations are queued, or, past the last one, until all are done
+    const bool last = maxiter != 0 && launched == maxiter;
+    const uint64_t want = last ? launched : launched > ahead ? launched - ahead : 0;
+    bool drained = false;
+    for (unsigned spin = 1;; ++spin) {
+      const unsigned long long at = progress->iter;
+      finished = (at & kLeft) != 0;
+      if (finished || at >= want || drained) break;
+      __builtin_ia32_pause();
+      if (spin % 65536 == 0) {  // a stream that failed, or ended without a word, ends the wait
+        const hipError_t e = hipStreamQuery(st);
+        if (e == hipErrorNotReady)
+          (void)hipGetLastError();
+        else
+          PCG_TRY(e);
+        drained = e == hipSuccess;
+      }
     }
-    batch = std::min(batch * 2, 32);
+    if (finished || last || drained) {
+      PCG_TRY(hipStreamSynchronize(st));
+      const unsigned long long at = progress->iter;
+      if (!(at & kLeft)) {
+        // iteration `maxiter` always raises the flag, so this is unreachable unless the state was corrupted
+        finished = true;
+        cleanup();
+        return set_error(LAPIS_HIP_ERR_RUNTIME, "pcg: %llu iterations queued and the device never reported an exit",
+                         (unsigned long long)launched);
+      }
+      finished = true;
+      *iters = at & ~kLeft;
+      *relres = progress->relres;
+    }
   }
   cleanup();
 #undef PCG_TRY

@@ -19,6 +19,13 @@ struct lapis_hip_csr_plan {
   int *chunk_row;    // device, int[nchunks+1]
   void *part_first;  // device, 8 bytes * nchunks
   void *part_last;   // device, 8 bytes * nchunks
+  // chunks of whole rows (rowchunk.hip); rowchunk_cap = 0: not for this matrix
+  int rowchunk_cap;          // entries per chunk at most
+  int rowchunk_weight;       // rows + entries per chunk
+  int rowchunk_n;            // chunks
+  void *rowchunk_desc;       // device, int2[n + 1]: first row and first entry of a chunk
+  bool rowchunk_contiguous;  // neighbouring chunks on one XCD
+  bool rowchunk_use;         // the choice of kernel is the plan's own: ROWBLOCK and NNZSPLIT run as row chunks
   // column-blocked (COLBLOCK) copy of the matrix, built on request
   bool colblock_built;
   int colblock_value_bytes;
@@ -51,6 +58,11 @@ struct lapis_hip_csr_plan {
   unsigned colblock_pace_fp; // clock ticks per entry (16.16 fixed point) of the time-triggered pacing, 0 = off
   double colblock_free_ms;   // calibration: kernel time without pacing
   double colblock_paced_ms;  // calibration: kernel time at the chosen pace
+
+  // Chunks of whole rows replace the row-block and the row-split kernel wherever the plan itself chose one of these.
+  bool runs_rowchunk() const {
+    return rowchunk_use && (stats.kernel == LAPIS_HIP_SPMV_ROWBLOCK || stats.kernel == LAPIS_HIP_SPMV_NNZSPLIT);
+  }
 };
 
 namespace lapis {
@@ -62,6 +74,20 @@ inline int bits_for(int64_t n) {
   while (b < 62 && (1LL << b) < n) ++b;
   return b;
 }
+
+// Chunks of whole rows; defined in rowchunk.hip.
+constexpr int kRowchunkLongestRow = 256;  // a quarter of the largest chunk
+int build_rowchunk(lapis_hip_csr_plan *plan, int value_bytes, hipStream_t st);
+void free_rowchunk(lapis_hip_csr_plan *plan);
+// y += A x, or y = A x with accumulate = 0
+template <typename T>
+int launch_rowchunk(const lapis_hip_csr_plan *plan, const int *crd, const T *val, const T *x, T *y, hipStream_t st,
+                    int accumulate);
+// y = A x for a square A, and x . y in rowchunk_xy_blocks(plan) partial sums, one per workgroup; *count becomes their
+// number.  The whole launch returns at once when *skip (device memory) is not 0.
+int rowchunk_xy_blocks(const lapis_hip_csr_plan *plan);
+int launch_rowchunk_xy(const lapis_hip_csr_plan *plan, const int *crd, const double *val, const double *x, double *y,
+                       hipStream_t st, double *xy_partials, int *count, const unsigned long long *skip);
 
 // Workgroup-blocked layout; defined in colgroup.hip.
 template <typename T>

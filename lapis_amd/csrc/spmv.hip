@@ -610,6 +610,7 @@ int spmv_impl(lapis_hip_csr_plan *plan, int64_t nrows, int64_t ncols, const int3
                      (long long)ncols, (const void *)pos);
   if (s.nnz == 0) return LAPIS_HIP_OK;
   LAPIS_REQUIRE(x && crd && val, "spmv: null coordinates, values or x with %lld non-zeros", (long long)s.nnz);
+  if (plan->runs_rowchunk()) return launch_rowchunk<T>(plan, crd, val, x, y, st, 1);
   const bool vec = aligned16(crd) && aligned16(val);
   const bool nt = plan->nontemporal;
   switch (s.kernel) {
@@ -660,6 +661,11 @@ int spmv_overwrite_f64(lapis_hip_csr_plan *plan, int64_t nrows, int64_t ncols, c
                        const int32_t *crd, const double *val, const double *x, double *y,
                        lapis_hip_stream_t stream, int *deferred_chunk, double *xy_chunk) {
   if (deferred_chunk) *deferred_chunk = 0;
+  if (plan && plan->runs_rowchunk() && plan->stats.nnz > 0 && plan->stats.nrows == nrows && plan->stats.ncols == ncols &&
+      plan->pos == pos && crd && val && x) {
+    LAPIS_CHECK_INIT();
+    return launch_rowchunk<double>(plan, crd, val, x, y, as_stream(stream), 0);
+  }
   if (plan && plan->stats.kernel == LAPIS_HIP_SPMV_NNZSPLIT && plan->stats.empty_rows == 0 && plan->stats.nnz > 0 &&
       plan->stats.nrows == nrows && plan->stats.ncols == ncols && plan->pos == pos && aligned16(crd) &&
       aligned16(val)) {
@@ -687,6 +693,27 @@ void free_plan_buffers(lapis_hip_csr_plan *p) {
   p->chunk_row = nullptr;
   p->part_first = p->part_last = nullptr;
   free_colblock(p);
+  free_rowchunk(p);
+}
+
+// What the row-split kernel needs beside the matrix; made when a plan first comes to launch that kernel.
+int build_rowsplit(lapis_hip_csr_plan *p, hipStream_t st) {
+  if (p->chunk_row || p->nchunks == 0) return LAPIS_HIP_OK;
+  const int64_t nrows = p->stats.nrows;
+  if (!p->part_first) LAPIS_HIP_TRY(hipMalloc(&p->part_first, 8 * (size_t)p->nchunks));
+  if (!p->part_last) LAPIS_HIP_TRY(hipMalloc(&p->part_last, 8 * (size_t)p->nchunks));
+  int *rows = nullptr;
+  LAPIS_HIP_TRY(hipMalloc(&rows, sizeof(int) * ((size_t)p->nchunks + 1)));
+  p->chunk_row = rows;
+  const dim3 g((unsigned)ceil_div(nrows, 256));
+  if (p->chunk == 512)
+    hipLaunchKernelGGL((chunk_row_kernel<512>), g, dim3(256), 0, st, (int)nrows, p->nchunks, p->pos, rows);
+  else if (p->chunk == 2048)
+    hipLaunchKernelGGL((chunk_row_kernel<2048>), g, dim3(256), 0, st, (int)nrows, p->nchunks, p->pos, rows);
+  else
+    hipLaunchKernelGGL((chunk_row_kernel<1024>), g, dim3(256), 0, st, (int)nrows, p->nchunks, p->pos, rows);
+  LAPIS_LAUNCH_CHECK();
+  return LAPIS_HIP_OK;
 }
 
 }  // namespace
@@ -781,28 +808,17 @@ extern "C" int lapis_hip_csr_plan_create(lapis_hip_csr_plan **out, int64_t nrows
   p->nchunks = (int)ceil_div(nnz, p->chunk);
   choose_kernel(p);
 
-  // Row-split metadata is built whatever the choice, so that set_kernel can switch to it.
-  if (p->nchunks > 0) {
-    hipError_t e = hipMalloc(&p->chunk_row, sizeof(int) * ((size_t)p->nchunks + 1));
-    if (e == hipSuccess) e = hipMalloc(&p->part_first, 8 * (size_t)p->nchunks);
-    if (e == hipSuccess) e = hipMalloc(&p->part_last, 8 * (size_t)p->nchunks);
-    if (e == hipSuccess) {
-      const dim3 g((unsigned)ceil_div(nrows, 256));
-      if (p->chunk == 512)
-        hipLaunchKernelGGL((chunk_row_kernel<512>), g, dim3(256), 0, st, (int)nrows, p->nchunks, pos, p->chunk_row);
-      else if (p->chunk == 2048)
-        hipLaunchKernelGGL((chunk_row_kernel<2048>), g, dim3(256), 0, st, (int)nrows, p->nchunks, pos, p->chunk_row);
-      else
-        hipLaunchKernelGGL((chunk_row_kernel<1024>), g, dim3(256), 0, st, (int)nrows, p->nchunks, pos, p->chunk_row);
-      e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e != hipSuccess) {
-      free_plan_buffers(p);
-      delete p;
-      return set_error(LAPIS_HIP_ERR_RUNTIME, "csr_plan_create: building row-split metadata failed: %s",
-                       hipGetErrorString(e));
-    }
+  int rc = build_rowchunk(p, value_bytes, st);
+  p->rowchunk_use = p->rowchunk_cap > 0;
+  if (rc == LAPIS_HIP_OK && s.kernel == LAPIS_HIP_SPMV_NNZSPLIT && !p->runs_rowchunk()) rc = build_rowsplit(p, st);
+  if (rc == LAPIS_HIP_OK) {
+    const hipError_t e = hipStreamSynchronize(st);
+    if (e != hipSuccess) rc = set_error(LAPIS_HIP_ERR_RUNTIME, "csr_plan_create: %s", hipGetErrorString(e));
+  }
+  if (rc != LAPIS_HIP_OK) {
+    free_plan_buffers(p);
+    delete p;
+    return rc;
   }
   *out = p;
   return LAPIS_HIP_OK;
@@ -810,6 +826,7 @@ extern "C" int lapis_hip_csr_plan_create(lapis_hip_csr_plan **out, int64_t nrows
 
 extern "C" const char *lapis_hip_csr_plan_kernel_name(const lapis_hip_csr_plan *plan) {
   if (!plan) return "";
+  if (plan->runs_rowchunk()) return "spmv_rowchunk_kernel";
   switch (plan->stats.kernel) {
     case LAPIS_HIP_SPMV_SUBWARP: return "spmv_subwarp_kernel";
     case LAPIS_HIP_SPMV_ROWBLOCK: return "spmv_rowblock_kernel";
@@ -834,6 +851,7 @@ extern "C" int lapis_hip_csr_plan_set_kernel(lapis_hip_csr_plan *plan, int kerne
   switch (kernel) {
     case LAPIS_HIP_SPMV_AUTO:
       choose_kernel(plan);
+      plan->rowchunk_use = plan->rowchunk_cap > 0;
       return LAPIS_HIP_OK;
     case LAPIS_HIP_SPMV_SUBWARP: {
       const int w = width == 0 ? s.reference_vector_length : width;
@@ -848,12 +866,21 @@ extern "C" int lapis_hip_csr_plan_set_kernel(lapis_hip_csr_plan *plan, int kerne
       s.kernel = kernel;
       s.width = 0;
       s.chunk = 0;
+      plan->rowchunk_use = false;
       return LAPIS_HIP_OK;
-    case LAPIS_HIP_SPMV_NNZSPLIT:
+    case LAPIS_HIP_SPMV_NNZSPLIT: {
+      if (!plan->chunk_row && plan->nchunks > 0) {
+        LAPIS_CHECK_INIT();
+        const int rc = build_rowsplit(plan, nullptr);
+        if (rc != LAPIS_HIP_OK) return rc;
+        LAPIS_HIP_TRY(hipStreamSynchronize(nullptr));
+      }
       s.kernel = kernel;
       s.width = 0;
       s.chunk = plan->chunk;
+      plan->rowchunk_use = false;
       return LAPIS_HIP_OK;
+    }
     case LAPIS_HIP_SPMV_COLBLOCK:
       if (!plan->colblock_built)
         return set_error(LAPIS_HIP_ERR_INVALID_ARGUMENT,
