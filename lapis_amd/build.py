@@ -24,13 +24,14 @@ LIBDIR = os.path.join(HERE, "lib")
 OBJDIR = os.path.join(CSRC, "build")
 INCLUDE = os.path.join(ROOT, "include")
 
-KERNEL_SOURCES = ["runtime.hip", "spmv.hip", "rowchunk.hip", "colblock.hip", "colgroup.hip", "spmm.hip", "blas1.hip", "cg.hip",
-                  "calibrate.hip"]
+KERNEL_SOURCES = ["runtime.hip", "spmv.hip", "rowchunk.hip", "colblock.hip", "colgroup.hip", "spmm.hip", "blas1.hip",
+                  "cg.hip", "staging.hip", "calibrate.hip"]
 SHIM_SOURCES = ["module_shim.hip"]
 
 KERNEL_LIB = os.path.join(LIBDIR, "liblapis_hip.so")
 MODULE_LIB = os.path.join(LIBDIR, "liblapis_package_module.so")
 CALLS_LIB = os.path.join(LIBDIR, "_lapis_calls.so")
+MODULE_CALLS_LIB = os.path.join(LIBDIR, "_lapis_module_calls.so")
 BINDIR = os.path.join(HERE, "bin")
 BENCH_BIN = os.path.join(BINDIR, "lapis_spmv_bench")
 
@@ -82,6 +83,12 @@ def _bindings():
           "-ltorch_python", "-Wl,-rpath,$ORIGIN", "-o", CALLS_LIB])
 
 
+def _module_bindings():
+    """csrc/module_calls.cpp: host code against the interpreter's headers only."""
+    _run([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-I", INCLUDE, "-I",
+          sysconfig.get_paths()["include"], os.path.join(CSRC, "module_calls.cpp"), "-o", MODULE_CALLS_LIB])
+
+
 def build(verbose=False, jobs=8):
     """Compile every HIP source for gfx950 and link both shared libraries."""
     os.makedirs(LIBDIR, exist_ok=True)
@@ -93,6 +100,7 @@ def build(verbose=False, jobs=8):
     _run([_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", *sobjs, "-L", LIBDIR, "-llapis_hip",
           "-Wl,-rpath,$ORIGIN", "-o", MODULE_LIB])
     _bindings()
+    _module_bindings()
     os.makedirs(BINDIR, exist_ok=True)
     _run([_hipcc(), "--offload-arch=gfx950", "-O2", "-std=c++17", "-I", INCLUDE,
           os.path.join(CSRC, "spmv_bench_main.cpp"), "-L", LIBDIR, "-llapis_hip", "-Wl,-rpath,$ORIGIN/../lib", "-o",
@@ -101,6 +109,7 @@ def build(verbose=False, jobs=8):
         print("built", KERNEL_LIB)
         print("built", MODULE_LIB)
         print("built", CALLS_LIB)
+        print("built", MODULE_CALLS_LIB)
         print("built", BENCH_BIN)
     return KERNEL_LIB, MODULE_LIB
 

@@ -17,6 +17,7 @@
 
 #include "lapis_hip.h"
 #include "lapis_module.h"
+#include "staging.hpp"
 
 namespace {
 
@@ -73,28 +74,27 @@ auto *host_data(const M *m, int rank, const char *name) {
   return m->data + m->offset;
 }
 
-// The device half of a DualView built from a host view: allocated and filled from
-// the host buffer at construction ("modified_host" then syncDevice), copied back on
-// request (syncHost), freed at scope exit.
+using lapis::HostOperands;
+
+// The device halves of a call's DualViews: filled from the host buffers ("modified_host" then syncDevice), copied
+// back on request (syncHost), given back at scope exit.
 template <typename T>
-struct DeviceMirror {
-  T *dev = nullptr;
-  T *host = nullptr;
-  size_t count = 0;
-  DeviceMirror() = default;
-  DeviceMirror(T *h, size_t n, bool upload = true) : host(h), count(n) {
-    if (n == 0) return;
-    check_hip(hipMalloc(&dev, n * sizeof(T)), "hipMalloc");
-    if (upload) check_hip(hipMemcpy(dev, h, n * sizeof(T), hipMemcpyHostToDevice), "host-to-device copy");
+int add(HostOperands &ops, T *host, int64_t n) {
+  return ops.add(host, sizeof(T) * (size_t)n);
+}
+template <typename T>
+int add_device_only(HostOperands &ops, int64_t n) {
+  return ops.add(nullptr, sizeof(T) * (size_t)n);
+}
+void upload(HostOperands &ops) { check(ops.upload(), "host-to-device copy"); }
+void sync_host(HostOperands &ops, int index, void *host) { check(ops.download(index, host), "device-to-host copy"); }
+
+struct PlanHolder {
+  lapis_hip_csr_plan *plan = nullptr;
+  PlanHolder(HostOperands &ops, int pos, int crd, int value_bytes) {
+    check(ops.create_plan(pos, crd, value_bytes, &plan), "lapis_hip_csr_plan_create");
   }
-  DeviceMirror(const DeviceMirror &) = delete;
-  DeviceMirror &operator=(const DeviceMirror &) = delete;
-  ~DeviceMirror() {
-    if (dev) (void)hipFree(dev);
-  }
-  void sync_host() {
-    if (count) check_hip(hipMemcpy(host, dev, count * sizeof(T), hipMemcpyDeviceToHost), "device-to-host copy");
-  }
+  ~PlanHolder() { lapis_hip_csr_plan_destroy(plan); }
 };
 
 template <typename M, typename T>
@@ -143,22 +143,21 @@ void spmv_entry(MV **ret0, lapis_memref_1d_i32 *pos, lapis_memref_1d_i32 *crd, M
     if (y->sizes[0] < a.nrows) module_abort("y is shorter than the number of rows");
   }
   {
-    DeviceMirror<int32_t> dpos(hpos, (size_t)a.nrows + 1), dcrd(hcrd, (size_t)a.nnz);
-    DeviceMirror<T> dval(hval, (size_t)a.nnz), dx(hx, (size_t)a.ncols), dy(hy, (size_t)a.nrows);
-    lapis_hip_csr_plan *plan = nullptr;
-    check(lapis_hip_csr_plan_create(&plan, a.nrows, a.ncols, a.nnz, dpos.dev, dcrd.dev, (int)sizeof(T), nullptr),
-          "lapis_hip_csr_plan_create");
+    HostOperands ops;
+    const int pos_d = ops.add_positions(hpos, a.nrows, a.nnz), crd_d = ops.add_coordinates(hcrd, a.nnz, a.ncols);
+    const int val_d = add(ops, hval, a.nnz), x_d = add(ops, hx, a.ncols);
+    const int y_d = ops.add_direct(hy, sizeof(T) * (size_t)a.nrows);
+    upload(ops);
+    PlanHolder held(ops, pos_d, crd_d, (int)sizeof(T));
     int rc;
     if (sizeof(T) == 8)
-      rc = lapis_hip_spmv_csr_f64_i32(plan, a.nrows, a.ncols, dpos.dev, dcrd.dev, (const double *)dval.dev,
-                                      (const double *)dx.dev, (double *)dy.dev, nullptr);
+      rc = lapis_hip_spmv_csr_f64_i32(held.plan, a.nrows, a.ncols, ops.at<int32_t>(pos_d), ops.at<int32_t>(crd_d),
+                                      ops.at<double>(val_d), ops.at<double>(x_d), ops.at<double>(y_d), ops.abi_stream());
     else
-      rc = lapis_hip_spmv_csr_f32_i32(plan, a.nrows, a.ncols, dpos.dev, dcrd.dev, (const float *)dval.dev,
-                                      (const float *)dx.dev, (float *)dy.dev, nullptr);
+      rc = lapis_hip_spmv_csr_f32_i32(held.plan, a.nrows, a.ncols, ops.at<int32_t>(pos_d), ops.at<int32_t>(crd_d),
+                                      ops.at<float>(val_d), ops.at<float>(x_d), ops.at<float>(y_d), ops.abi_stream());
     check(rc, "lapis_hip_spmv_csr");
-    check(lapis_hip_stream_synchronize(nullptr), "stream synchronize");
-    lapis_hip_csr_plan_destroy(plan);
-    dy.sync_host();  // results.syncHost(): the caller's y (or the module's) now holds the result
+    sync_host(ops, y_d, hy);  // results.syncHost(): the caller's y (or the module's) now holds the result
   }
   set_result_1d(ret0, hy, a.nrows);
 }
@@ -176,23 +175,23 @@ void spmm_entry(MM **ret0, lapis_memref_1d_i32 *pos, lapis_memref_1d_i32 *crd, M
   if (B->sizes[0] < a.ncols || B->sizes[1] != k || C->sizes[0] < a.nrows)
     module_abort("SpMM operand shapes do not agree");
   {
-    DeviceMirror<int32_t> dpos(hpos, (size_t)a.nrows + 1), dcrd(hcrd, (size_t)a.nnz);
-    DeviceMirror<T> dval(hval, (size_t)a.nnz), dB(hB, (size_t)(a.ncols * k)), dC(hC, (size_t)(a.nrows * k));
+    HostOperands ops;
+    const int pos_d = ops.add_positions(hpos, a.nrows, a.nnz), crd_d = ops.add_coordinates(hcrd, a.nnz, a.ncols);
+    const int val_d = add(ops, hval, a.nnz), B_d = add(ops, hB, a.ncols * k), C_d = add(ops, hC, a.nrows * k);
+    upload(ops);
     // the plan checks the structure (a bad coordinate must not reach the kernel) and its statistics pick the kernel
-    lapis_hip_csr_plan *plan = nullptr;
-    check(lapis_hip_csr_plan_create(&plan, a.nrows, a.ncols, a.nnz, dpos.dev, dcrd.dev, (int)sizeof(T), nullptr),
-          "lapis_hip_csr_plan_create");
+    PlanHolder held(ops, pos_d, crd_d, (int)sizeof(T));
     int rc;
     if (sizeof(T) == 8)
-      rc = lapis_hip_spmm_csr_f64_i32_plan(plan, a.nrows, a.ncols, k, dpos.dev, dcrd.dev, (const double *)dval.dev,
-                                           (const double *)dB.dev, k, (double *)dC.dev, k, nullptr);
+      rc = lapis_hip_spmm_csr_f64_i32_plan(held.plan, a.nrows, a.ncols, k, ops.at<int32_t>(pos_d), ops.at<int32_t>(crd_d),
+                                           ops.at<double>(val_d), ops.at<double>(B_d), k, ops.at<double>(C_d), k,
+                                           ops.abi_stream());
     else
-      rc = lapis_hip_spmm_csr_f32_i32_plan(plan, a.nrows, a.ncols, k, dpos.dev, dcrd.dev, (const float *)dval.dev,
-                                           (const float *)dB.dev, k, (float *)dC.dev, k, nullptr);
+      rc = lapis_hip_spmm_csr_f32_i32_plan(held.plan, a.nrows, a.ncols, k, ops.at<int32_t>(pos_d), ops.at<int32_t>(crd_d),
+                                           ops.at<float>(val_d), ops.at<float>(B_d), k, ops.at<float>(C_d), k,
+                                           ops.abi_stream());
     check(rc, "lapis_hip_spmm_csr");
-    check(lapis_hip_stream_synchronize(nullptr), "stream synchronize");
-    lapis_hip_csr_plan_destroy(plan);
-    dC.sync_host();
+    sync_host(ops, C_d, hC);
   }
   (*ret0)->basePtr = hC;
   (*ret0)->data = hC;
@@ -457,18 +456,21 @@ extern "C" void py_pcg(lapis_memref_1d_f64 **ret0, size_t *ret1, double *ret2, l
   uint64_t iters = 0;
   double relres = 0.0;
   {
-    DeviceMirror<int32_t> dpos(hpos, (size_t)n + 1), dcrd(hcrd, (size_t)a.nnz);
-    DeviceMirror<double> dval(hval, (size_t)a.nnz), db(hb, (size_t)n), ddinv(hdinv, (size_t)n);
-    DeviceMirror<double> dx(hx, (size_t)n, false);
-    lapis_hip_csr_plan *plan = nullptr;
-    check(lapis_hip_csr_plan_create(&plan, n, n, a.nnz, dpos.dev, dcrd.dev, 8, nullptr), "lapis_hip_csr_plan_create");
+    HostOperands ops;
+    const int pos_d = ops.add_positions(hpos, n, a.nnz), crd_d = ops.add_coordinates(hcrd, a.nnz, n);
+    const int val_d = add(ops, hval, a.nnz), b_d = add(ops, hb, n), dinv_d = add(ops, hdinv, n);
+    const int x_d = add_device_only<double>(ops, n), work_d = add_device_only<double>(ops, 4 * n);
+    upload(ops);
+    PlanHolder held(ops, pos_d, crd_d, 8);
     // enough iterations for the column-blocked copy to pay back where the library recommends one
-    if (maxiter >= 64) check(lapis_hip_csr_plan_analyze(plan, dcrd.dev, dval.dev, 8, nullptr), "lapis_hip_csr_plan_analyze");
-    check(lapis_hip_pcg_f64_i32(plan, n, dpos.dev, dcrd.dev, dval.dev, db.dev, ddinv.dev, tol, (uint64_t)maxiter,
-                                dx.dev, &iters, &relres, nullptr, nullptr),
+    if (maxiter >= 64)
+      check(lapis_hip_csr_plan_analyze(held.plan, ops.at<int32_t>(crd_d), ops.at<double>(val_d), 8, ops.abi_stream()),
+            "lapis_hip_csr_plan_analyze");
+    check(lapis_hip_pcg_f64_i32(held.plan, n, ops.at<int32_t>(pos_d), ops.at<int32_t>(crd_d), ops.at<double>(val_d),
+                                ops.at<double>(b_d), ops.at<double>(dinv_d), tol, (uint64_t)maxiter, ops.at<double>(x_d),
+                                &iters, &relres, ops.at<double>(work_d), ops.abi_stream()),
           "lapis_hip_pcg_f64_i32");
-    lapis_hip_csr_plan_destroy(plan);
-    dx.sync_host();
+    sync_host(ops, x_d, hx);
   }
   set_result_1d(ret0, hx, n);
   *ret1 = (size_t)iters;
@@ -505,16 +507,16 @@ extern "C" void py_pte_local_bspmm(lapis_memref_3d_f32 **ret0, lapis_memref_1d_i
   float *hout = static_cast<float *>(keep_alive_alloc(sizeof(float) * out_count));
   memset(hout, 0, sizeof(float) * out_count);  // linalg.fill of the result (examples/bspmm.py:40-42)
   if (out_count > 0) {
-    DeviceMirror<int32_t> dpos(hpos, (size_t)n1 + 1), dcrd(hcrd, (size_t)nnz);
-    DeviceMirror<float> dval(hval, (size_t)(nnz * nh)), dB(hB, (size_t)(n2 * dh * nh)), dout(hout, out_count);
+    HostOperands ops;
+    const int pos_d = ops.add_positions(hpos, n1, nnz), crd_d = ops.add_coordinates(hcrd, nnz, n2);
+    const int val_d = add(ops, hval, nnz * nh), B_d = add(ops, hB, n2 * dh * nh), out_d = add(ops, hout, n1 * dh * nh);
+    upload(ops);
     // the plan is built only for its structure check: a bad coordinate must not reach the kernel
-    lapis_hip_csr_plan *plan = nullptr;
-    check(lapis_hip_csr_plan_create(&plan, n1, n2, nnz, dpos.dev, dcrd.dev, 4, nullptr), "lapis_hip_csr_plan_create");
-    lapis_hip_csr_plan_destroy(plan);
-    check(lapis_hip_bspmm_csrv_f32_i32(n1, n2, dh, nh, dpos.dev, dcrd.dev, dval.dev, dB.dev, dout.dev, nullptr),
+    PlanHolder held(ops, pos_d, crd_d, 4);
+    check(lapis_hip_bspmm_csrv_f32_i32(n1, n2, dh, nh, ops.at<int32_t>(pos_d), ops.at<int32_t>(crd_d), ops.at<float>(val_d),
+                                       ops.at<float>(B_d), ops.at<float>(out_d), ops.abi_stream()),
           "lapis_hip_bspmm_csrv_f32_i32");
-    check(lapis_hip_stream_synchronize(nullptr), "stream synchronize");
-    dout.sync_host();
+    sync_host(ops, out_d, hout);
   }
   (*ret0)->basePtr = hout;
   (*ret0)->data = hout;
@@ -536,14 +538,16 @@ extern "C" void py_plus_norm(lapis_memref_1d_f64 **ret0, double *ret1, lapis_mem
   double *hout = static_cast<double *>(keep_alive_alloc(sizeof(double) * (size_t)n));
   double sum = 0.0;
   {
-    DeviceMirror<double> dx(hx, (size_t)n), dy(hy, (size_t)n), dout(hout, (size_t)n, false);
-    double *dsum = nullptr;
-    check_hip(hipMalloc(&dsum, sizeof(double)), "hipMalloc");
-    check(lapis_hip_axpby_f64(n, 1.0, dx.dev, 1.0, dy.dev, dout.dev, nullptr), "lapis_hip_axpby_f64");
-    check(lapis_hip_dot_f64(n, dout.dev, dout.dev, 0.0, dsum, nullptr), "lapis_hip_dot_f64");
-    check_hip(hipMemcpy(&sum, dsum, sizeof(double), hipMemcpyDeviceToHost), "device-to-host copy");
-    (void)hipFree(dsum);
-    dout.sync_host();
+    HostOperands ops;
+    const int x_d = add(ops, hx, n), y_d = add(ops, hy, n);
+    const int out_d = add_device_only<double>(ops, n), sum_d = add_device_only<double>(ops, 1);
+    upload(ops);
+    check(lapis_hip_axpby_f64(n, 1.0, ops.at<double>(x_d), 1.0, ops.at<double>(y_d), ops.at<double>(out_d), ops.abi_stream()),
+          "lapis_hip_axpby_f64");
+    check(lapis_hip_dot_f64(n, ops.at<double>(out_d), ops.at<double>(out_d), 0.0, ops.at<double>(sum_d), ops.abi_stream()),
+          "lapis_hip_dot_f64");
+    sync_host(ops, sum_d, &sum);
+    sync_host(ops, out_d, hout);
   }
   set_result_1d(ret0, hout, n);
   *ret1 = sqrt(sum);
@@ -563,19 +567,22 @@ extern "C" void py_mht(lapis_memref_1d_f64 **ret0, lapis_memref_1d_f64 **ret1, l
   double *h1 = static_cast<double *>(keep_alive_alloc(sizeof(double) * (size_t)n));
   double *h2 = static_cast<double *>(keep_alive_alloc(sizeof(double) * (size_t)n));
   {
-    DeviceMirror<int32_t> dpos(hpos, (size_t)n + 1), dcrd(hcrd, (size_t)a.nnz);
-    DeviceMirror<double> dval(hval, (size_t)a.nnz), dmask(hmask, (size_t)n), dd(hd, (size_t)n);
-    DeviceMirror<double> d1(h1, (size_t)n, false), d2(h2, (size_t)n, false);
-    lapis_hip_csr_plan *plan = nullptr;
-    check(lapis_hip_csr_plan_create(&plan, n, n, a.nnz, dpos.dev, dcrd.dev, 8, nullptr), "lapis_hip_csr_plan_create");
+    HostOperands ops;
+    const int pos_d = ops.add_positions(hpos, n, a.nnz), crd_d = ops.add_coordinates(hcrd, a.nnz, n);
+    const int val_d = add(ops, hval, a.nnz), mask_d = add(ops, hmask, n), d_d = add(ops, hd, n);
+    const int d1 = add_device_only<double>(ops, n), d2 = add_device_only<double>(ops, n);
+    upload(ops);
+    PlanHolder held(ops, pos_d, crd_d, 8);
     // two solves of up to maxiter iterations each; mht refreshes the copy's values after it has scaled the matrix
-    if (maxiter >= 32) check(lapis_hip_csr_plan_analyze(plan, dcrd.dev, dval.dev, 8, nullptr), "lapis_hip_csr_plan_analyze");
-    check(lapis_hip_mht_f64_i32(plan, n, a.nnz, dpos.dev, dcrd.dev, dval.dev, dmask.dev, dd.dev, alpha, tol,
-                                (uint64_t)maxiter, d1.dev, d2.dev, nullptr),
+    if (maxiter >= 32)
+      check(lapis_hip_csr_plan_analyze(held.plan, ops.at<int32_t>(crd_d), ops.at<double>(val_d), 8, ops.abi_stream()),
+            "lapis_hip_csr_plan_analyze");
+    check(lapis_hip_mht_f64_i32(held.plan, n, a.nnz, ops.at<int32_t>(pos_d), ops.at<int32_t>(crd_d), ops.at<double>(val_d),
+                                ops.at<double>(mask_d), ops.at<double>(d_d), alpha, tol, (uint64_t)maxiter, ops.at<double>(d1),
+                                ops.at<double>(d2), ops.abi_stream()),
           "lapis_hip_mht_f64_i32");
-    lapis_hip_csr_plan_destroy(plan);
-    d1.sync_host();
-    d2.sync_host();
+    sync_host(ops, d1, h1);
+    sync_host(ops, d2, h2);
     // the scaled values stay on the device: they are no result of the function, and a
     // DualView built from host memory is not copied back unless it is one
   }
@@ -590,10 +597,12 @@ extern "C" void py_normalize_mom2(lapis_memref_1d_f64 **ret0, lapis_memref_1d_f6
   if (mom2->sizes[0] < n) module_abort("normalize_mom2: mom2 shorter than mom1");
   double *hout = static_cast<double *>(keep_alive_alloc(sizeof(double) * (size_t)n));
   {
-    DeviceMirror<double> d1(h1, (size_t)n), d2(h2, (size_t)n), dout(hout, (size_t)n, false);
-    check(lapis_hip_normalize_mom2_f64(n, d1.dev, d2.dev, dout.dev, nullptr), "lapis_hip_normalize_mom2_f64");
-    check(lapis_hip_stream_synchronize(nullptr), "stream synchronize");
-    dout.sync_host();
+    HostOperands ops;
+    const int d1 = add(ops, h1, n), d2 = add(ops, h2, n), out_d = add_device_only<double>(ops, n);
+    upload(ops);
+    check(lapis_hip_normalize_mom2_f64(n, ops.at<double>(d1), ops.at<double>(d2), ops.at<double>(out_d), ops.abi_stream()),
+          "lapis_hip_normalize_mom2_f64");
+    sync_host(ops, out_d, hout);
   }
   set_result_1d(ret0, hout, n);
 }

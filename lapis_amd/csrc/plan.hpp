@@ -66,6 +66,24 @@ struct lapis_hip_csr_plan {
 };
 
 namespace lapis {
+// What a pass over the structure finds; made by the kernels of spmv.hip, or by the host where the structure comes from
+// host memory (staging.hip).
+struct CsrCounts {
+  int min_len;
+  int max_len;
+  int bad;  // bit 0: positions decrease; bit 1: coordinate out of range
+  int pad;
+  unsigned long long empty_rows;
+  double sum_sq;
+  unsigned long long span_sum;  // sum over 1024-non-zero chunks of (max column - min column)
+  unsigned long long near[4];   // non-zeros with |column - row| <= 32, 64, 128, 256 (device counts only)
+};
+// A plan from counts made by the host, `first` and `last` being the first and the last position.  Nothing of the
+// device is waited for: the plan serves calls on `stream`.
+int create_counted_plan(lapis_hip_csr_plan **out, int64_t nrows, int64_t ncols, int64_t nnz, const int32_t *pos,
+                        const int32_t *crd, int value_bytes, const CsrCounts &counts, int32_t first, int32_t last,
+                        hipStream_t stream);
+
 constexpr int kColblockRowBits = 10;  // the per-wavefront layout keeps up to 1024 rows per wavefront
 
 // bits needed for values 0..n-1

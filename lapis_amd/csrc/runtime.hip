@@ -6,6 +6,7 @@
 
 #include "blas1.hpp"
 #include "common.hpp"
+#include "staging.hpp"
 
 namespace lapis {
 namespace {
@@ -83,6 +84,7 @@ extern "C" int lapis_hip_finalize(void) {
   if (--g_refcount == 0) {
     dot_release_scratch();
     cg_release_scratch();
+    release_staging();
   }
   return LAPIS_HIP_OK;
 }

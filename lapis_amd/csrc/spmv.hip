@@ -288,22 +288,11 @@ __global__ __launch_bounds__(256) void spmv_nnzsplit_fixup_kernel(
 // ------------------------------------------------------------------------------
 // Plan analysis kernels
 // ------------------------------------------------------------------------------
-struct DeviceStats {
-  int min_len;
-  int max_len;
-  int bad;  // bit 0: positions decrease; bit 1: coordinate out of range
-  int pad;
-  unsigned long long empty_rows;
-  double sum_sq;
-  unsigned long long span_sum;  // sum over 1024-non-zero chunks of (max column - min column)
-  unsigned long long near[4];   // non-zeros with |column - row| <= 32, 64, 128, 256
-};
-
-// Every statistic is first reduced over the block and reaches the one DeviceStats with one
+// Every statistic is first reduced over the block and reaches the one CsrCounts with one
 // atomic per block and field: tens of thousands of atomics on the same few words would take
 // longer than reading the matrix.
 __global__ __launch_bounds__(256) void row_stats_kernel(int nrows, const int *__restrict__ pos,
-                                                        DeviceStats *st) {
+                                                        CsrCounts *st) {
   __shared__ int s_mn[4], s_mx[4], s_bad[4];
   __shared__ unsigned long long s_empt[4];
   __shared__ double s_sq[4];
@@ -361,7 +350,7 @@ __global__ __launch_bounds__(256) void row_stats_kernel(int nrows, const int *__
 // row of a million entries costs what a million short rows cost.
 __global__ __launch_bounds__(256) void entry_stats_kernel(int nrows, long long nnz, int ncols,
                                                           const int *__restrict__ pos,
-                                                          const int *__restrict__ crd, DeviceStats *st) {
+                                                          const int *__restrict__ crd, CsrCounts *st) {
   __shared__ unsigned long long s_span[4], s_near[4][4];
   __shared__ int s_bad[4];
   __shared__ int s_rows[4][1024];
@@ -718,10 +707,9 @@ int build_rowsplit(lapis_hip_csr_plan *p, hipStream_t st) {
 
 }  // namespace
 
-extern "C" int lapis_hip_csr_plan_create(lapis_hip_csr_plan **out, int64_t nrows, int64_t ncols, int64_t nnz,
-                                         const int32_t *pos, const int32_t *crd, int value_bytes,
-                                         lapis_hip_stream_t stream) {
-  LAPIS_CHECK_INIT();
+namespace {
+int check_plan_arguments(lapis_hip_csr_plan **out, int64_t nrows, int64_t ncols, int64_t nnz, const int32_t *pos,
+                         int value_bytes) {
   LAPIS_REQUIRE(out, "csr_plan_create: null output");
   *out = nullptr;
   LAPIS_REQUIRE(nrows >= 0 && ncols >= 0 && nnz >= 0, "csr_plan_create: negative size");
@@ -729,41 +717,19 @@ extern "C" int lapis_hip_csr_plan_create(lapis_hip_csr_plan **out, int64_t nrows
                 "csr_plan_create: sizes exceed the int32 index range");
   LAPIS_REQUIRE(value_bytes == 4 || value_bytes == 8, "csr_plan_create: value_bytes must be 4 or 8");
   LAPIS_REQUIRE(pos, "csr_plan_create: null positions (a CSR matrix with n rows has n+1 positions)");
-  hipStream_t st = as_stream(stream);
+  return LAPIS_HIP_OK;
+}
 
-  int32_t ends[2] = {0, 0};
-  LAPIS_HIP_TRY(hipMemcpyAsync(&ends[0], pos, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-  LAPIS_HIP_TRY(hipMemcpyAsync(&ends[1], pos + nrows, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-  LAPIS_HIP_TRY(hipStreamSynchronize(st));
-  if (ends[0] != 0 || ends[1] != nnz)
+int check_ends(int32_t first, int32_t last, int64_t nnz) {
+  if (first != 0 || last != nnz)
     return set_error(LAPIS_HIP_ERR_BAD_CSR, "csr_plan_create: pos[0]=%d pos[n]=%d, expected 0 and nnz=%lld",
-                     ends[0], ends[1], (long long)nnz);
+                     first, last, (long long)nnz);
+  return LAPIS_HIP_OK;
+}
 
-  DeviceStats init{INT32_MAX, 0, 0, 0, 0ull, 0.0, 0ull, {0ull, 0ull, 0ull, 0ull}};
-  DeviceStats host = init;
-  if (nrows > 0) {
-    DeviceStats *dstats = nullptr;
-    LAPIS_HIP_TRY(hipMalloc(&dstats, sizeof(DeviceStats)));
-    hipError_t e = hipMemcpyAsync(dstats, &init, sizeof(init), hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) {
-      const int blocks = (int)std::min<int64_t>(ceil_div(nrows, 256), 1024);
-      hipLaunchKernelGGL(row_stats_kernel, dim3(blocks), dim3(256), 0, st, (int)nrows, pos, dstats);
-      e = hipGetLastError();
-    }
-    if (e == hipSuccess && crd && nnz > 0) {
-      const int blocks = (int)std::min<int64_t>(ceil_div(ceil_div(nnz, 1024), 4), 2048);
-      hipLaunchKernelGGL(entry_stats_kernel, dim3(blocks), dim3(256), 0, st, (int)nrows, (long long)nnz, (int)ncols,
-                         pos, crd, dstats);
-      e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipMemcpyAsync(&host, dstats, sizeof(host), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    (void)hipFree(dstats);
-    if (e != hipSuccess)
-      return set_error(LAPIS_HIP_ERR_RUNTIME, "csr_plan_create: analysis failed: %s", hipGetErrorString(e));
-  } else {
-    host.min_len = 0;
-  }
+// The plan of a structure whose counts are known; its own arrays are queued on `st` and not waited for.
+int make_plan(lapis_hip_csr_plan **out, int64_t nrows, int64_t ncols, int64_t nnz, const int32_t *pos, const int32_t *crd,
+              int value_bytes, const CsrCounts &host, bool near_known, hipStream_t st) {
   if (host.bad & 1) return set_error(LAPIS_HIP_ERR_BAD_CSR, "csr_plan_create: positions are not non-decreasing");
   if (host.bad & 2)
     return set_error(LAPIS_HIP_ERR_BAD_CSR, "csr_plan_create: a coordinate lies outside [0, %lld)", (long long)ncols);
@@ -780,12 +746,12 @@ extern "C" int lapis_hip_csr_plan_create(lapis_hip_csr_plan **out, int64_t nrows
   s.mean_row_len = nrows ? (double)nnz / (double)nrows : 0.0;
   s.var_row_len = nrows ? std::max(0.0, host.sum_sq / (double)nrows - s.mean_row_len * s.mean_row_len) : 0.0;
   s.mean_chunk_col_span = (crd && nnz > 0) ? (double)host.span_sum / (double)ceil_div(nnz, 1024) : -1.0;
-  for (int i = 0; i < 4; ++i) s.near_diagonal_fraction[i] = (crd && nnz > 0) ? (double)host.near[i] / (double)nnz : -1.0;
+  for (int i = 0; i < 4; ++i) s.near_diagonal_fraction[i] = (crd && nnz > 0 && near_known) ? (double)host.near[i] / (double)nnz : -1.0;
   // The column-blocked copy pays when the gathers of a chunk wander over more of x
   // than an XCD's L2 keeps (4 MB, shared with the streamed arrays) and the matrix is
   // large enough for the extra launch work not to matter.
   s.colblock_recommended = (s.mean_chunk_col_span * value_bytes > 2.0 * 1024 * 1024 && nnz >= (1 << 20)) ? 1 : 0;
-  s.reference_hint = reference_hint(nrows, ends[0], ends[1]);
+  s.reference_hint = reference_hint(nrows, 0, nnz);
   s.reference_vector_length = reference_vector_length(s.reference_hint);
   p->pos = pos;
   p->crd = crd;
@@ -811,16 +777,77 @@ extern "C" int lapis_hip_csr_plan_create(lapis_hip_csr_plan **out, int64_t nrows
   int rc = build_rowchunk(p, value_bytes, st);
   p->rowchunk_use = p->rowchunk_cap > 0;
   if (rc == LAPIS_HIP_OK && s.kernel == LAPIS_HIP_SPMV_NNZSPLIT && !p->runs_rowchunk()) rc = build_rowsplit(p, st);
-  if (rc == LAPIS_HIP_OK) {
-    const hipError_t e = hipStreamSynchronize(st);
-    if (e != hipSuccess) rc = set_error(LAPIS_HIP_ERR_RUNTIME, "csr_plan_create: %s", hipGetErrorString(e));
-  }
   if (rc != LAPIS_HIP_OK) {
     free_plan_buffers(p);
     delete p;
     return rc;
   }
   *out = p;
+  return LAPIS_HIP_OK;
+}
+}  // namespace
+
+namespace lapis {
+int create_counted_plan(lapis_hip_csr_plan **out, int64_t nrows, int64_t ncols, int64_t nnz, const int32_t *pos,
+                        const int32_t *crd, int value_bytes, const CsrCounts &counts, int32_t first, int32_t last,
+                        hipStream_t stream) {
+  LAPIS_CHECK_INIT();
+  int rc = check_plan_arguments(out, nrows, ncols, nnz, pos, value_bytes);
+  if (rc == LAPIS_HIP_OK) rc = check_ends(first, last, nnz);
+  if (rc != LAPIS_HIP_OK) return rc;
+  return make_plan(out, nrows, ncols, nnz, pos, crd, value_bytes, counts, false, stream);
+}
+}  // namespace lapis
+
+extern "C" int lapis_hip_csr_plan_create(lapis_hip_csr_plan **out, int64_t nrows, int64_t ncols, int64_t nnz,
+                                         const int32_t *pos, const int32_t *crd, int value_bytes,
+                                         lapis_hip_stream_t stream) {
+  LAPIS_CHECK_INIT();
+  int rc = check_plan_arguments(out, nrows, ncols, nnz, pos, value_bytes);
+  if (rc != LAPIS_HIP_OK) return rc;
+  hipStream_t st = as_stream(stream);
+
+  int32_t ends[2] = {0, 0};
+  LAPIS_HIP_TRY(hipMemcpyAsync(&ends[0], pos, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+  LAPIS_HIP_TRY(hipMemcpyAsync(&ends[1], pos + nrows, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+  LAPIS_HIP_TRY(hipStreamSynchronize(st));
+  rc = check_ends(ends[0], ends[1], nnz);
+  if (rc != LAPIS_HIP_OK) return rc;
+
+  CsrCounts init{INT32_MAX, 0, 0, 0, 0ull, 0.0, 0ull, {0ull, 0ull, 0ull, 0ull}};
+  CsrCounts host = init;
+  if (nrows > 0) {
+    CsrCounts *dstats = nullptr;
+    LAPIS_HIP_TRY(hipMalloc(&dstats, sizeof(CsrCounts)));
+    hipError_t e = hipMemcpyAsync(dstats, &init, sizeof(init), hipMemcpyHostToDevice, st);
+    if (e == hipSuccess) {
+      const int blocks = (int)std::min<int64_t>(ceil_div(nrows, 256), 1024);
+      hipLaunchKernelGGL(row_stats_kernel, dim3(blocks), dim3(256), 0, st, (int)nrows, pos, dstats);
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess && crd && nnz > 0) {
+      const int blocks = (int)std::min<int64_t>(ceil_div(ceil_div(nnz, 1024), 4), 2048);
+      hipLaunchKernelGGL(entry_stats_kernel, dim3(blocks), dim3(256), 0, st, (int)nrows, (long long)nnz, (int)ncols,
+                         pos, crd, dstats);
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpyAsync(&host, dstats, sizeof(host), hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    (void)hipFree(dstats);
+    if (e != hipSuccess)
+      return set_error(LAPIS_HIP_ERR_RUNTIME, "csr_plan_create: analysis failed: %s", hipGetErrorString(e));
+  } else {
+    host.min_len = 0;
+  }
+  lapis_hip_csr_plan *plan = nullptr;
+  rc = make_plan(&plan, nrows, ncols, nnz, pos, crd, value_bytes, host, true, st);
+  if (rc != LAPIS_HIP_OK) return rc;
+  const hipError_t e = hipStreamSynchronize(st);
+  if (e != hipSuccess) {
+    lapis_hip_csr_plan_destroy(plan);
+    return set_error(LAPIS_HIP_ERR_RUNTIME, "csr_plan_create: %s", hipGetErrorString(e));
+  }
+  *out = plan;
   return LAPIS_HIP_OK;
 }
 

@@ -12,6 +12,8 @@ as numpy arrays aliasing module-owned (or caller-owned, for in-place results)
 memory.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import numpy
@@ -19,7 +21,22 @@ import numpy
 from . import memref as rt
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
+_CALLS_PATH = os.path.join(_HERE, "lib", "_lapis_module_calls.so")
 DEFAULT_MODULE_PATH = os.path.join(_HERE, "lib", "liblapis_package_module.so")
+
+
+_calls = None
+
+
+def _load_calls():
+    """The extension that calls module functions on numpy arrays (csrc/module_calls.cpp)."""
+    global _calls
+    if _calls is None:
+        loader = importlib.machinery.ExtensionFileLoader("_lapis_module_calls", _CALLS_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_lapis_module_calls", loader))
+        loader.exec_module(module)
+        _calls = module
+    return _calls
 
 
 def _flatten_specifier(spec):
@@ -209,6 +226,8 @@ class LAPISModule:
         self.libHandle.lapis_resident_csr_pcg.restype = None
         self.libHandle.lapis_resident_csr_pcg.argtypes = [vp, vp, vp, ctypes.c_double, ctypes.c_size_t, vp,
                                                           ctypes.POINTER(ctypes.c_size_t), ctypes.POINTER(ctypes.c_double)]
+        self._call_spmv = _load_calls().spmv
+        self._spmv_entries = [ctypes.cast(fn, vp).value for fn in (self.libHandle.py_spmv, self.libHandle.py_spmv_f32)]
         self.libHandle.lapis_initialize()
 
     def __del__(self):
@@ -228,6 +247,9 @@ class LAPISModule:
 
     # func @spmv(A, x, y) -> y          (examples/spmv_noalloc.py:9, benchmarks/spmv/spmv.mlir)
     def spmv(self, param0, param1, param2, param3, param4, param5):
+        # arrays of the types the module takes go to its function as they are, anything else through the coercions below
+        if self._call_spmv(*self._spmv_entries, param0, param1, param2, param3, param4, param5):
+            return numpy.asarray(param5)[:param3[0][0]]
         val_dtype = numpy.float32 if numpy.asarray(param2).dtype == numpy.float32 else numpy.float64
         param0 = numpy.require(param0, dtype=numpy.int32, requirements=['C'])
         param1 = numpy.require(param1, dtype=numpy.int32, requirements=['C'])
@@ -245,7 +267,7 @@ class LAPISModule:
               param3.ctypes.data_as(ctypes.c_void_p),
               ctypes.pointer(rt.get_ranked_memref_descriptor(param4)),
               ctypes.pointer(rt.get_ranked_memref_descriptor(param5)))
-        return (rt.ranked_memref_to_numpy(ret0[0]))
+        return param5[:ret0[0][0].shape[0]]  # the caller's y, or the array it was coerced to
 
     # torch.mv export, entry `main` renamed lapis_main      (examples/spmv.py:47)
     def lapis_main(self, param0, param1, param2, param3, param4):
@@ -305,7 +327,7 @@ class LAPISModule:
               param3.ctypes.data_as(ctypes.c_void_p),
               ctypes.pointer(rt.get_ranked_memref_descriptor(param4)),
               ctypes.pointer(rt.get_ranked_memref_descriptor(param5)))
-        return (rt.ranked_memref_to_numpy(ret0[0]))
+        return param5[:]  # the caller's C, or the array it was coerced to
 
     # func @pte_local_bspmm(A: CSRV, B) -> out      (examples/bspmm.py:26-52, called at :103)
     def pte_local_bspmm(self, param0, param1, param2, param3, param4):
