@@ -85,36 +85,46 @@ def _run_by_operation(mod, ex, c, fname, decompose_tensors):
         params = list(params)
         args, written = [], []
         np_of = {"f64": numpy.float64, "f32": numpy.float32, "i32": numpy.int32, "i64": numpy.int64, "index": numpy.int64}
+        arrays, places = [], []  # host arrays, and what to do with the device tensor of each
 
-        def up(a, elem):
-            return torch.from_numpy(numpy.array(a, dtype=np_of[elem], order="C")).to(ex.device)
+        def up(a, elem, place):
+            arrays.append(numpy.ascontiguousarray(a, dtype=np_of[elem]))
+            places.append(place)
+
+        def argument():
+            args.append(None)
+            return len(args) - 1
 
         def take():
             if not params:
                 raise TypeError("@%s: too few arguments" % fname)
             return params.pop(0)
 
+        matrices = []  # (argument, index of its positions among the arrays, rows, columns)
         for kind, ty in zip(kinds, types):
             ty = ty.strip()
             if kind.startswith("csr:"):
                 if not decompose_tensors:
                     raise TypeError("@%s takes a sparse tensor: compile with decompose_tensors=True" % fname)
                 pos, crd, val, spec = take(), take(), take(), take()
-                args.append(_executor.Csr(up(pos, "i32"), up(crd, "i32"), up(val, kind[4:]), spec[0][0], spec[0][1]))
+                matrices.append((argument(), len(arrays), spec[0][0], spec[0][1]))
+                for a, elem in ((pos, "i32"), (crd, "i32"), (val, kind[4:])):
+                    up(a, elem, None)
             elif ty.startswith("tensor<"):
                 dims, elem = _executor._shape_spec(ty)
-                a = take()
-                args.append(up(a, elem) if dims else (numpy.float32(a) if elem == "f32" else float(a)))
+                a, at = take(), argument()
+                if dims:
+                    up(a, elem, (at, None))
+                else:
+                    args[at] = numpy.float32(a) if elem == "f32" else float(a)
             elif ty.startswith("memref<"):
                 dims, elem = _executor._shape_spec(ty)
-                a = take()
+                a, at = take(), argument()
                 if not dims:
-                    args.append(_executor.Cell(numpy.asarray(a).reshape(-1)[0]))
-                    written.append((a, args[-1]))
+                    args[at] = _executor.Cell(numpy.asarray(a).reshape(-1)[0])
+                    written.append((a, args[at]))
                 else:
-                    args.append(up(a, elem))
-                    if elem in ("f64", "f32"):
-                        written.append((a, args[-1]))
+                    up(a, elem, (at, a if elem in ("f64", "f32") else None))
             elif ty in ("f64", "f32"):
                 a = take()
                 args.append(numpy.float32(a) if ty == "f32" else float(a))
@@ -122,12 +132,29 @@ def _run_by_operation(mod, ex, c, fname, decompose_tensors):
                 args.append(int(take()))
         if params:
             raise TypeError("@%s: %d arguments too many" % (fname, len(params)))
+        hip = ex.hip
+        # the structure of the first matrix is counted on its way to the device, and its plan made from that
+        counted = None
+        if matrices:
+            _, i, rows, columns = matrices[0]
+            if arrays[i].shape == (rows + 1,) and columns >= 0 and arrays[i + 1].shape == arrays[i + 2].shape:
+                counted = (i, i + 1, rows, columns)
+        tensors, staged = hip.stage(arrays, counted)
+        for t, place in zip(tensors, places):
+            if place is not None:
+                args[place[0]] = t
+                if place[1] is not None:
+                    written.append((place[1], t))
+        for at, i, rows, columns in matrices:
+            A = args[at] = _executor.Csr(tensors[i], tensors[i + 1], tensors[i + 2], rows, columns)
+            if counted and i == counted[0]:
+                A.staged = lambda A=A, i=i: hip.staged_plan(staged, i, i + 1, A.pos, A.crd, A.val.element_size())
         try:
             results = ex.run(fname, args)
             out = []
             for r in results:
                 if isinstance(r, torch.Tensor):
-                    out.append(r.cpu().numpy())
+                    out.append(hip.fetch(r))
                 elif isinstance(r, _executor.Cell):
                     out.append(r.value)
                 else:
@@ -136,7 +163,7 @@ def _run_by_operation(mod, ex, c, fname, decompose_tensors):
                 if isinstance(dev, _executor.Cell):
                     numpy.asarray(host).reshape(-1)[0] = dev.value
                 elif isinstance(host, numpy.ndarray) and host.flags.writeable:
-                    numpy.copyto(host, dev.cpu().numpy().reshape(host.shape))
+                    numpy.copyto(host, hip.fetch(dev).reshape(host.shape))
         finally:
             for a in args:
                 if isinstance(a, _executor.Csr):

@@ -77,7 +77,7 @@ def _bindings():
     torch = importlib.util.find_spec("torch").submodule_search_locations[0]
     lib = os.path.join(torch, "lib")
     _run([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-          "-I", INCLUDE, "-I", sysconfig.get_paths()["include"], "-isystem", os.path.join(torch, "include"), "-isystem",
+          "-I", INCLUDE, "-I", CSRC, "-I", sysconfig.get_paths()["include"], "-isystem", os.path.join(torch, "include"), "-isystem",
           os.path.join(torch, "include", "torch", "csrc", "api", "include"), "-isystem", "/opt/rocm/include",
           os.path.join(CSRC, "bindings.cpp"), "-L", LIBDIR, "-llapis_hip", "-L", lib, "-lc10", "-lc10_hip", "-ltorch_cpu",
           "-ltorch_python", "-Wl,-rpath,$ORIGIN", "-o", CALLS_LIB])

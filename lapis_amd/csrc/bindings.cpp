@@ -6,12 +6,18 @@
 // documents them; operands that are plain integers pass as raw device addresses, as they do there.
 #include <Python.h>
 
+#include <ATen/ops/empty.h>
+#include <ATen/ops/from_blob.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstdarg>
+#include <memory>
+#include <vector>
 
+#include "blas1.hpp"
 #include "lapis_hip.h"
+#include "staging.hpp"
 
 namespace {
 
@@ -164,29 +170,91 @@ PyObject *guarded(F f) {
   }
 }
 
+// A dot product under way is a capsule: one that nobody finishes is waited for when it goes.
+constexpr const char *kSumName = "lapis_hip.dot";
+void abandon_sum(PyObject *capsule) {
+  lapis::dot_abandon(static_cast<lapis::HostSum *>(PyCapsule_GetPointer(capsule, kSumName)));
+}
+PyObject *sum_capsule(lapis::HostSum *sum) {
+  PyObject *c = PyCapsule_New(sum, kSumName, abandon_sum);
+  if (!c) {
+    lapis::dot_abandon(sum);
+    throw Raised();
+  }
+  return c;
+}
+
 #define LAPIS_PY(name) PyObject *name(PyObject *, PyObject *const *a, Py_ssize_t n)
+
+struct SpmvCall {
+  lapis_hip_csr_plan *plan;
+  int64_t nrows, ncols;
+  const int32_t *pos, *crd;
+  Operand val, x, y;
+  // a[0..7]: plan, nrows, ncols, pos, crd, val, x, y
+  explicit SpmvCall(PyObject *const *a) {
+    nrows = integer(a[1]);
+    ncols = integer(a[2]);
+    const Operand p = operand(a[3]), c = operand(a[4]);
+    val = operand(a[5]);
+    x = operand(a[6]);
+    y = operand(a[7]);
+    indices("spmv", p);
+    indices("spmv", c);
+    holds("spmv", nrows + 1, p);
+    holds("spmv", ncols, x, val.tensor);
+    holds("spmv", nrows, y, val.tensor);
+    if (c.tensor) holds("spmv", c.tensor->numel(), val);
+    plan = plan_of(a[0]);
+    pos = static_cast<const int32_t *>(p.address);
+    crd = static_cast<const int32_t *>(c.address);
+  }
+};
 
 // (plan, nrows, ncols, pos, crd, val, x, y, stream)
 LAPIS_PY(py_spmv) {
   return guarded([&] {
     arguments("spmv", n, 9);
-    const int64_t nrows = integer(a[1]), ncols = integer(a[2]);
-    const Operand pos = operand(a[3]), crd = operand(a[4]), val = operand(a[5]), x = operand(a[6]), y = operand(a[7]);
-    indices("spmv", pos);
-    indices("spmv", crd);
-    holds("spmv", nrows + 1, pos);
-    holds("spmv", ncols, x, val.tensor);
-    holds("spmv", nrows, y, val.tensor);
-    if (crd.tensor) holds("spmv", crd.tensor->numel(), val);
-    lapis_hip_csr_plan *plan = plan_of(a[0]);
-    const auto p = static_cast<const int32_t *>(pos.address), c = static_cast<const int32_t *>(crd.address);
-    if (is_f64(val))
-      check(lapis_hip_spmv_csr_f64_i32(plan, nrows, ncols, p, c, (const double *)val.address, (const double *)x.address,
-                                       (double *)y.address, stream_of(a[8])));
+    const SpmvCall c(a);
+    if (is_f64(c.val))
+      check(lapis_hip_spmv_csr_f64_i32(c.plan, c.nrows, c.ncols, c.pos, c.crd, (const double *)c.val.address,
+                                       (const double *)c.x.address, (double *)c.y.address, stream_of(a[8])));
     else
-      check(lapis_hip_spmv_csr_f32_i32(plan, nrows, ncols, p, c, (const float *)val.address, (const float *)x.address,
-                                       (float *)y.address, stream_of(a[8])));
+      check(lapis_hip_spmv_csr_f32_i32(c.plan, c.nrows, c.ncols, c.pos, c.crd, (const float *)c.val.address,
+                                       (const float *)c.x.address, (float *)c.y.address, stream_of(a[8])));
     return give(a[7]);
+  });
+}
+
+// (plan, nrows, ncols, pos, crd, val, x, y, stream): y = A x
+LAPIS_PY(py_spmv_overwrite) {
+  return guarded([&] {
+    arguments("spmv", n, 9);
+    const SpmvCall c(a);
+    if (is_f64(c.val))
+      check(lapis::spmv_overwrite<double>(c.plan, c.nrows, c.ncols, c.pos, c.crd, (const double *)c.val.address,
+                                          (const double *)c.x.address, (double *)c.y.address, stream_of(a[8])));
+    else
+      check(lapis::spmv_overwrite<float>(c.plan, c.nrows, c.ncols, c.pos, c.crd, (const float *)c.val.address,
+                                         (const float *)c.x.address, (float *)c.y.address, stream_of(a[8])));
+    return give(a[7]);
+  });
+}
+
+// (plan, nrows, ncols, pos, crd, val, x, y, init, stream) -> capsule of init + x . y: y = A x
+LAPIS_PY(py_spmv_dot_start) {
+  return guarded([&] {
+    arguments("spmv", n, 10);
+    const SpmvCall c(a);
+    const double init = number(a[8]);
+    lapis::HostSum *sum = nullptr;
+    if (is_f64(c.val))
+      check(lapis::spmv_dot_start<double>(c.plan, c.nrows, c.ncols, c.pos, c.crd, (const double *)c.val.address,
+                                          (const double *)c.x.address, (double *)c.y.address, init, stream_of(a[9]), &sum));
+    else
+      check(lapis::spmv_dot_start<float>(c.plan, c.nrows, c.ncols, c.pos, c.crd, (const float *)c.val.address,
+                                         (const float *)c.x.address, (float *)c.y.address, init, stream_of(a[9]), &sum));
+    return sum_capsule(sum);
   });
 }
 
@@ -273,6 +341,172 @@ LAPIS_PY(py_dot_host) {
     Py_END_ALLOW_THREADS;
     check(status);
     return PyFloat_FromDouble(f64 ? r64 : (double)r32);
+  });
+}
+
+// (x, y, init, stream) -> capsule of init + x . y
+LAPIS_PY(py_dot_start) {
+  return guarded([&] {
+    arguments("dot", n, 4);
+    const Operand x = operand(a[0]), y = operand(a[1]);
+    const int64_t len = length("dot", x);
+    holds("dot", len, x, x.tensor);
+    holds("dot", len, y, x.tensor);
+    const double init = number(a[2]);
+    const hipStream_t st = static_cast<hipStream_t>(stream_of(a[3]));
+    lapis::HostSum *sum = nullptr;
+    check(is_f64(x) ? lapis::dot_start<double>(len, (const double *)x.address, (const double *)y.address, init, st, &sum)
+                    : lapis::dot_start<float>(len, (const float *)x.address, (const float *)y.address, init, st, &sum));
+    return sum_capsule(sum);
+  });
+}
+
+// (a, x, b, y, dst, z or None, init, stream) -> capsule of init + dst . z (dst . dst without z): dst = a x + b y
+LAPIS_PY(py_axpby_dot_start) {
+  return guarded([&] {
+    arguments("axpby_dot", n, 8);
+    const double ca = number(a[0]), cb = number(a[2]);
+    const Operand x = operand(a[1]), y = operand(a[3]), d = operand(a[4]), z = operand(a[5]);
+    const int64_t len = length("axpby_dot", x);
+    holds("axpby_dot", len, x, x.tensor);
+    holds("axpby_dot", len, y, x.tensor);
+    holds("axpby_dot", len, d, x.tensor);
+    holds("axpby_dot", len, z, x.tensor);
+    const double init = number(a[6]);
+    const hipStream_t st = static_cast<hipStream_t>(stream_of(a[7]));
+    lapis::HostSum *sum = nullptr;
+    check(is_f64(x) ? lapis::axpby_dot_start<double>(len, ca, (const double *)x.address, cb, (const double *)y.address,
+                                                     (double *)d.address, (const double *)z.address, init, st, &sum)
+                    : lapis::axpby_dot_start<float>(len, (float)ca, (const float *)x.address, (float)cb, (const float *)y.address,
+                                                    (float *)d.address, (const float *)z.address, init, st, &sum));
+    return sum_capsule(sum);
+  });
+}
+
+// (capsule) -> float
+LAPIS_PY(py_dot_finish) {
+  return guarded([&] {
+    arguments("dot_finish", n, 1);
+    auto *sum = static_cast<lapis::HostSum *>(PyCapsule_GetPointer(a[0], kSumName));
+    if (!sum || PyCapsule_SetDestructor(a[0], nullptr) != 0 || PyCapsule_SetName(a[0], "lapis_hip.finished") != 0) throw Raised();
+    double total = 0.0;
+    int status;
+    Py_BEGIN_ALLOW_THREADS;
+    status = lapis::dot_finish(sum, &total);
+    Py_END_ALLOW_THREADS;
+    check(status);
+    return PyFloat_FromDouble(total);
+  });
+}
+
+// ---- host arrays on their way to the device and back (staging.hpp) ----
+
+struct HostArray {
+  Py_buffer view{};
+  bool held = false;
+  HostArray(PyObject *o, bool writable) {
+    if (PyObject_GetBuffer(o, &view, PyBUF_C_CONTIGUOUS | PyBUF_FORMAT | (writable ? PyBUF_WRITABLE : 0)) != 0) throw Raised();
+    held = true;
+  }
+  HostArray(HostArray &&other) noexcept : view(other.view), held(other.held) { other.held = false; }
+  ~HostArray() {
+    if (held) PyBuffer_Release(&view);
+  }
+  at::ScalarType type() const {
+    const char f = view.format ? view.format[0] : 0;
+    if (f == 'd') return at::kDouble;
+    if (f == 'f') return at::kFloat;
+    if (f == 'i') return at::kInt;
+    if (f == 'l' || f == 'q') return at::kLong;
+    raise(PyExc_TypeError, "an array of format %s", view.format ? view.format : "?");
+  }
+};
+
+constexpr const char *kStagedName = "lapis_hip.staged";
+typedef std::shared_ptr<lapis::HostOperands> Staged;
+void drop_staged(PyObject *capsule) { delete static_cast<Staged *>(PyCapsule_GetPointer(capsule, kStagedName)); }
+
+// (list of arrays, None or (index of positions, index of coordinates, rows, columns), stream)
+//   -> (list of tensors, capsule for staged_plan)
+LAPIS_PY(py_stage) {
+  return guarded([&] {
+    arguments("stage", n, 3);
+    PyObject *seq = PySequence_Fast(a[0], "stage: a sequence of arrays");
+    if (!seq) throw Raised();
+    std::unique_ptr<PyObject, void (*)(PyObject *)> seq_guard(seq, [](PyObject *o) { Py_DECREF(o); });
+    long long csr[4] = {-1, -1, 0, 0};
+    if (a[1] != Py_None && !PyArg_ParseTuple(a[1], "LLLL", &csr[0], &csr[1], &csr[2], &csr[3])) throw Raised();
+    std::vector<HostArray> arrays;
+    const Py_ssize_t count = PySequence_Fast_GET_SIZE(seq);
+    arrays.reserve((size_t)count);
+    for (Py_ssize_t i = 0; i < count; ++i) arrays.emplace_back(PySequence_Fast_GET_ITEM(seq, i), false);
+    const hipStream_t st = static_cast<hipStream_t>(stream_of(a[2]));
+    auto ops = std::make_shared<lapis::HostOperands>();
+    ops->use_stream(st);
+    if (csr[0] >= 0) {
+      if (csr[0] >= count || csr[1] < 0 || csr[1] >= count || arrays[(size_t)csr[0]].type() != at::kInt ||
+          arrays[(size_t)csr[1]].type() != at::kInt || arrays[(size_t)csr[0]].view.len != 4 * (csr[2] + 1) || csr[2] < 0 || csr[3] < 0)
+        raise(PyExc_ValueError, "stage: a CSR structure of %lld rows", csr[2]);
+    }
+    for (Py_ssize_t i = 0; i < count; ++i) {
+      const Py_buffer &v = arrays[(size_t)i].view;
+      if (i == csr[0])
+        ops->add_positions(static_cast<const int32_t *>(v.buf), csr[2], arrays[(size_t)csr[1]].view.len / 4);
+      else if (i == csr[1])
+        ops->add_coordinates(static_cast<const int32_t *>(v.buf), v.len / 4, csr[3]);
+      else
+        ops->add(v.buf, (size_t)v.len);
+    }
+    int status;
+    Py_BEGIN_ALLOW_THREADS;
+    status = ops->upload();
+    Py_END_ALLOW_THREADS;
+    check(status);
+    PyObject *tensors = PyList_New(count);
+    if (!tensors) throw Raised();
+    const at::Device device(at::kCUDA, c10::hip::getCurrentHIPStream().device_index());
+    for (Py_ssize_t i = 0; i < count; ++i) {
+      const HostArray &h = arrays[(size_t)i];
+      std::vector<int64_t> sizes(h.view.shape, h.view.shape + h.view.ndim);
+      const auto options = at::TensorOptions().dtype(h.type()).device(device);
+      at::Tensor t = h.view.len == 0 ? at::empty(sizes, options)
+                                     : at::from_blob(ops->at<void>((int)i), sizes, [ops](void *) {}, options, device);
+      PyList_SET_ITEM(tensors, i, THPVariable_Wrap(std::move(t)));
+    }
+    PyObject *capsule = PyCapsule_New(new Staged(ops), kStagedName, drop_staged);
+    return Py_BuildValue("(NN)", tensors, capsule);
+  });
+}
+
+// (capsule, index of positions, index of coordinates, bytes per value) -> address of a plan
+LAPIS_PY(py_staged_plan) {
+  return guarded([&] {
+    arguments("staged_plan", n, 4);
+    auto *staged = static_cast<Staged *>(PyCapsule_GetPointer(a[0], kStagedName));
+    if (!staged) throw Raised();
+    lapis_hip_csr_plan *plan = nullptr;
+    check((*staged)->create_plan((int)integer(a[1]), (int)integer(a[2]), (int)integer(a[3]), &plan));
+    return PyLong_FromVoidPtr(plan);
+  });
+}
+
+// (tensor, array, stream): the array gets the tensor's elements, after what is queued on the stream
+LAPIS_PY(py_fetch) {
+  return guarded([&] {
+    arguments("fetch", n, 3);
+    const Operand t = operand(a[0]);
+    HostArray to(a[1], true);
+    if (!t.tensor || !t.tensor->is_contiguous() || (int64_t)t.tensor->nbytes() != (int64_t)to.view.len)
+      raise(PyExc_ValueError, "fetch: %lld bytes of a contiguous tensor", (long long)to.view.len);
+    lapis::HostOperands ops;
+    ops.use_stream(static_cast<hipStream_t>(stream_of(a[2])));
+    int status;
+    Py_BEGIN_ALLOW_THREADS;
+    status = ops.upload();
+    if (status == LAPIS_HIP_OK) status = ops.download(t.address, (size_t)to.view.len, to.view.buf);
+    Py_END_ALLOW_THREADS;
+    check(status);
+    return give(a[1]);
   });
 }
 
@@ -389,7 +623,9 @@ PyObject *py_setup(PyObject *, PyObject *args) {
 #define LAPIS_METHOD(name) {#name, (PyCFunction)(void (*)(void))py_##name, METH_FASTCALL, nullptr}
 PyMethodDef g_methods[] = {LAPIS_METHOD(spmv), LAPIS_METHOD(spmm), LAPIS_METHOD(bspmm_csrv), LAPIS_METHOD(dot),
                            LAPIS_METHOD(dot_host), LAPIS_METHOD(axpby), LAPIS_METHOD(mult), LAPIS_METHOD(div),
-                           LAPIS_METHOD(fill), LAPIS_METHOD(copy), LAPIS_METHOD(pcg),
+                           LAPIS_METHOD(fill), LAPIS_METHOD(copy), LAPIS_METHOD(pcg), LAPIS_METHOD(spmv_overwrite),
+                           LAPIS_METHOD(spmv_dot_start), LAPIS_METHOD(dot_start), LAPIS_METHOD(axpby_dot_start),
+                           LAPIS_METHOD(dot_finish), LAPIS_METHOD(stage), LAPIS_METHOD(staged_plan), LAPIS_METHOD(fetch),
                            {"setup", py_setup, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_lapis_calls", "Device-resident calls of the gfx950 kernel library.", -1,
                         g_methods, nullptr, nullptr, nullptr, nullptr};

@@ -3,6 +3,8 @@
 // reference emits for the linalg.generic / linalg.dot ops of
 // examples/pcg_solve.py:22-47.
 #include <mutex>
+#include <vector>
+#include <cstring>
 
 #include "blas1.hpp"
 #include "common.hpp"
@@ -117,10 +119,18 @@ __device__ __forceinline__ T block_sum_256(T v, T *lds4) {
   return total;
 }
 
-template <typename T>
+// A block's partial sum: to device memory as a T, or to the host's as a double.
+template <typename T, bool HOST>
+__device__ __forceinline__ void leave_partial(void *partials, T v) {
+  if (HOST)
+    tell_host(static_cast<double *>(partials) + blockIdx.x, (double)v);
+  else
+    static_cast<T *>(partials)[blockIdx.x] = v;
+}
+
+template <typename T, bool HOST>
 __global__ __launch_bounds__(256) void dot_partial_kernel(long long n, const T *__restrict__ x,
-                                                          const T *__restrict__ y, T *__restrict__ partials,
-                                                          int vec) {
+                                                          const T *__restrict__ y, void *partials, int vec) {
   typedef typename VecOf<T>::type V;
   constexpr int VW = VecOf<T>::width;
   __shared__ T lds4[4];
@@ -134,7 +144,7 @@ __global__ __launch_bounds__(256) void dot_partial_kernel(long long n, const T *
   for (long long i = nv * VW + (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256)
     acc = acc + x[i] * y[i];
   const T total = block_sum_256(acc, lds4);
-  if (threadIdx.x == 0) partials[blockIdx.x] = total;
+  if (threadIdx.x == 0) leave_partial<T, HOST>(partials, total);
 }
 
 template <typename T>
@@ -151,9 +161,9 @@ __global__ __launch_bounds__(256) void dot_final_kernel(int count, const T *__re
 // dst = a*x + b*y and the partial sums of dst . z in one pass (z == nullptr: dst . dst).  Element order,
 // grid and the order of the additions are those of elementwise_kernel and dot_partial_kernel, so the pair
 // of results has the bits the two separate calls give.
-template <typename T>
+template <typename T, bool HOST>
 __global__ __launch_bounds__(256) void axpby_dot_partial_kernel(long long n, T a, const T *x, T b, const T *y, T *dst,
-                                                                const T *z, T *__restrict__ partials, int vec) {
+                                                                const T *z, void *partials, int vec) {
   typedef typename VecOf<T>::type V;
   constexpr int VW = VecOf<T>::width;
   __shared__ T lds4[4];
@@ -176,7 +186,7 @@ __global__ __launch_bounds__(256) void axpby_dot_partial_kernel(long long n, T a
     acc = acc + d * w;
   }
   const T total = block_sum_256(acc, lds4);
-  if (threadIdx.x == 0) partials[blockIdx.x] = total;
+  if (threadIdx.x == 0) leave_partial<T, HOST>(partials, total);
 }
 
 int dot_grid(int64_t n) {
@@ -188,7 +198,7 @@ int dot_grid(int64_t n) {
 template <typename T>
 int launch_dot(int64_t n, const T *x, const T *y, T init, T *result, T *partials, hipStream_t st) {
   const int grid = dot_grid(n);
-  hipLaunchKernelGGL((dot_partial_kernel<T>), dim3(grid), dim3(256), 0, st, (long long)n, x, y, partials,
+  hipLaunchKernelGGL((dot_partial_kernel<T, false>), dim3(grid), dim3(256), 0, st, (long long)n, x, y, (void *)partials,
                      (aligned16(x) && aligned16(y)) ? 1 : 0);
   hipLaunchKernelGGL((dot_final_kernel<T>), dim3(1), dim3(256), 0, st, grid, (const T *)partials, init, result);
   LAPIS_LAUNCH_CHECK();
@@ -205,7 +215,7 @@ constexpr int kSlots = 64;
 std::mutex g_scratch_mutex;
 char *g_scratch = nullptr;  // kSlots * kDotMaxBlocks * 8 bytes
 unsigned g_next_slot = 0;
-constexpr size_t kSlotBytes = ((size_t)kDotMaxBlocks + 2) * 8;  // the partials, then one result for the *_host entries
+constexpr size_t kSlotBytes = (size_t)kDotMaxBlocks * 8;
 
 int take_slot(void **partials) {
   std::lock_guard<std::mutex> lock(g_scratch_mutex);
@@ -251,6 +261,134 @@ int dot_entry(const char *what, int64_t n, const T *x, const T *y, T init, T *re
 }
 }  // namespace
 
+// ---- dot products whose value the host waits for -------------------------------------------------
+// The reference's parallel_reduce into a host scalar (TranslateToKokkosCpp.cpp:1696-1705,1838), blocking included.
+// A second kernel for the total, a copy of it and a wait for the stream took 24 us.  The parts go to pinned memory
+// instead, where the host has put a mark no sum has; it adds them up as the marks vanish, in the order the kernel would, 4 us after the
+// first kernel started on a short vector.
+namespace {
+constexpr unsigned long long kAwaited = 0x7ff46c617069732bull;  // a signalling NaN
+constexpr size_t kKeptSums = 16;
+std::mutex g_sums_mutex;
+std::vector<HostSum *> g_sums;
+
+// dot_final_kernel's order of additions: 256 strided sums, a binary tree over each 64 of them, the four in turn, init.
+template <typename T>
+double total_of(const double *lane, double init) {
+  T v[256];
+  for (int i = 0; i < 256; ++i) v[i] = (T)lane[i];
+  for (int width = 1; width < 64; width *= 2)
+    for (int i = 0; i < 256; i += 2 * width) v[i] = v[i] + v[i + width];
+  const T all = ((v[0] + v[64]) + v[128]) + v[192];
+  return (double)(all + (T)init);
+}
+
+void give_host_sum(HostSum *sum) {
+  {
+    std::lock_guard<std::mutex> lock(g_sums_mutex);
+    if (g_sums.size() < kKeptSums) {
+      g_sums.push_back(sum);
+      return;
+    }
+  }
+  (void)hipHostFree(sum->parts);
+  delete sum;
+}
+}  // namespace
+
+int take_host_sum(int count, double init, bool f32, hipStream_t st, HostSum **out) {
+  HostSum *sum = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(g_sums_mutex);
+    if (!g_sums.empty()) {
+      sum = g_sums.back();
+      g_sums.pop_back();
+    }
+  }
+  if (!sum) {
+    sum = new HostSum();
+    const hipError_t e = hipHostMalloc(&sum->parts, sizeof(double) * kDotMaxBlocks, hipHostMallocDefault);
+    if (e != hipSuccess) {
+      delete sum;
+      return set_error(LAPIS_HIP_ERR_RUNTIME, "dot: pinned memory: %s", hipGetErrorString(e));
+    }
+  }
+  sum->count = count;
+  sum->init = init;
+  sum->f32 = f32;
+  sum->stream = st;
+  volatile unsigned long long *word = reinterpret_cast<volatile unsigned long long *>(sum->parts);
+  for (int i = 0; i < count; ++i) word[i] = kAwaited;
+  *out = sum;
+  return LAPIS_HIP_OK;
+}
+
+int dot_finish(HostSum *sum, double *result) {
+  const volatile unsigned long long *word = reinterpret_cast<const volatile unsigned long long *>(sum->parts);
+  double lane[256] = {};
+  bool drained = false;
+  for (int i = 0; i < sum->count; ++i) {
+    unsigned long long w;
+    for (unsigned spin = 1; (w = word[i]) == kAwaited && !drained; ++spin) {
+      __builtin_ia32_pause();
+      if (spin % 16384 != 0) continue;
+      // a stream that failed, or that is done (the mark was a sum after all), ends the wait
+      const hipError_t e = hipStreamQuery(sum->stream);
+      if (e == hipErrorNotReady) {
+        (void)hipGetLastError();
+      } else if (e != hipSuccess) {
+        give_host_sum(sum);
+        return set_error(LAPIS_HIP_ERR_RUNTIME, "dot: %s", hipGetErrorString(e));
+      } else {
+        drained = true;
+      }
+    }
+    double part;
+    memcpy(&part, &w, sizeof(part));
+    lane[i & 255] = sum->f32 ? (double)((float)lane[i & 255] + (float)part) : lane[i & 255] + part;
+  }
+  *result = sum->f32 ? total_of<float>(lane, sum->init) : total_of<double>(lane, sum->init);
+  give_host_sum(sum);
+  return LAPIS_HIP_OK;
+}
+
+void dot_abandon(HostSum *sum) {
+  (void)hipStreamSynchronize(sum->stream);
+  give_host_sum(sum);
+}
+
+template <typename T>
+int dot_start(int64_t n, const T *x, const T *y, double init, hipStream_t st, HostSum **out) {
+  const int grid = dot_grid(n);
+  const int rc = take_host_sum(grid, init, sizeof(T) == 4, st, out);
+  if (rc != LAPIS_HIP_OK) return rc;
+  hipLaunchKernelGGL((dot_partial_kernel<T, true>), dim3(grid), dim3(256), 0, st, (long long)n, x, y, (void *)(*out)->parts,
+                     (aligned16(x) && aligned16(y)) ? 1 : 0);
+  const hipError_t e = hipGetLastError();
+  if (e == hipSuccess) return LAPIS_HIP_OK;
+  dot_abandon(*out);
+  return set_error(LAPIS_HIP_ERR_RUNTIME, "dot: %s", hipGetErrorString(e));
+}
+template int dot_start<double>(int64_t, const double *, const double *, double, hipStream_t, HostSum **);
+template int dot_start<float>(int64_t, const float *, const float *, double, hipStream_t, HostSum **);
+
+template <typename T>
+int axpby_dot_start(int64_t n, T a, const T *x, T b, const T *y, T *dst, const T *z, double init, hipStream_t st, HostSum **out) {
+  const int grid = dot_grid(n);
+  const int rc = take_host_sum(grid, init, sizeof(T) == 4, st, out);
+  if (rc != LAPIS_HIP_OK) return rc;
+  hipLaunchKernelGGL((axpby_dot_partial_kernel<T, true>), dim3(grid), dim3(256), 0, st, (long long)n, a, x, b, y, dst, z,
+                     (void *)(*out)->parts, (aligned16(x) && aligned16(y) && aligned16(dst) && (!z || aligned16(z))) ? 1 : 0);
+  const hipError_t e = hipGetLastError();
+  if (e == hipSuccess) return LAPIS_HIP_OK;
+  dot_abandon(*out);
+  return set_error(LAPIS_HIP_ERR_RUNTIME, "axpby_dot: %s", hipGetErrorString(e));
+}
+template int axpby_dot_start<double>(int64_t, double, const double *, double, const double *, double *, const double *, double,
+                                     hipStream_t, HostSum **);
+template int axpby_dot_start<float>(int64_t, float, const float *, float, const float *, float *, const float *, double,
+                                    hipStream_t, HostSum **);
+
 // Resolves the no-alloc scratch of the current device (called by lapis_hip_init, so that
 // the first lapis_hip_dot_f64_noalloc call does no set-up work either).
 int dot_noalloc_setup() {
@@ -264,6 +402,12 @@ void dot_release_scratch() {
   if (g_scratch) (void)hipFree(g_scratch);
   g_scratch = nullptr;
   g_next_slot = 0;
+  std::lock_guard<std::mutex> sums_lock(g_sums_mutex);
+  for (HostSum *sum : g_sums) {
+    (void)hipHostFree(sum->parts);
+    delete sum;
+  }
+  g_sums.clear();
 }
 
 }  // namespace lapis
@@ -289,24 +433,18 @@ extern "C" int lapis_hip_dot_f64_noalloc(int64_t n, const double *x, const doubl
 
 
 namespace {
-// dot with the result on the host: what the reference's parallel_reduce into a host scalar gives
-// (TranslateToKokkosCpp.cpp:1696-1705,1838), blocking included.
 template <typename T>
 int dot_host_entry(const char *what, int64_t n, const T *x, const T *y, T init, T *host_result, lapis_hip_stream_t stream) {
   LAPIS_CHECK_INIT();
   LAPIS_REQUIRE(n >= 0, "%s: negative length", what);
   LAPIS_REQUIRE(host_result, "%s: null result", what);
   LAPIS_REQUIRE(n == 0 || (x && y), "%s: null vector with n=%lld", what, (long long)n);
-  void *partials = nullptr;
-  int rc = take_slot(&partials);
-  if (rc != LAPIS_HIP_OK) return rc;
-  T *device_result = reinterpret_cast<T *>(static_cast<char *>(partials) + (size_t)kDotMaxBlocks * 8);
-  hipStream_t st = as_stream(stream);
-  rc = launch_dot<T>(n, x, y, init, device_result, static_cast<T *>(partials), st);
-  if (rc != LAPIS_HIP_OK) return rc;
-  LAPIS_HIP_TRY(hipMemcpyAsync(host_result, device_result, sizeof(T), hipMemcpyDeviceToHost, st));
-  LAPIS_HIP_TRY(hipStreamSynchronize(st));
-  return LAPIS_HIP_OK;
+  HostSum *sum = nullptr;
+  int rc = dot_start<T>(n, x, y, (double)init, as_stream(stream), &sum);
+  double total = 0.0;
+  if (rc == LAPIS_HIP_OK) rc = dot_finish(sum, &total);
+  if (rc == LAPIS_HIP_OK) *host_result = (T)total;
+  return rc;
 }
 
 template <typename T>
@@ -323,8 +461,8 @@ int axpby_dot_entry(const char *what, int64_t n, T a, const T *x, T b, const T *
   hipStream_t st = as_stream(stream);
   const int grid = dot_grid(n);
   const int vec = (aligned16(x) && aligned16(y) && aligned16(dst) && (!z || aligned16(z))) ? 1 : 0;
-  hipLaunchKernelGGL((axpby_dot_partial_kernel<T>), dim3(grid), dim3(256), 0, st, (long long)n, a, x, b, y, dst, z,
-                     partials, vec);
+  hipLaunchKernelGGL((axpby_dot_partial_kernel<T, false>), dim3(grid), dim3(256), 0, st, (long long)n, a, x, b, y, dst, z,
+                     (void *)partials, vec);
   hipLaunchKernelGGL((dot_final_kernel<T>), dim3(1), dim3(256), 0, st, grid, (const T *)partials, init, result);
   LAPIS_LAUNCH_CHECK();
   return LAPIS_HIP_OK;

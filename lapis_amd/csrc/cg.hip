@@ -934,8 +934,8 @@ int pcg_run(lapis_hip_csr_plan *plan, int64_t n, const int32_t *pos, const int32
       int deferred = 0;  // chunk length when the SpMV left its cut rows to the p.Ap kernel
       if (row_chunks) {
         // Ap = A p and p.Ap in one pass
-        PCG_RC(launch_rowchunk_xy(plan, crd, val, p, Ap, st, chunk_pap ? chunk_pap : pap_partials, &pap_count,
-                                  &state->done_iter));
+        PCG_RC(launch_rowchunk_xy<double>(plan, crd, val, p, Ap, st, chunk_pap ? chunk_pap : pap_partials, false, &pap_count,
+                                          &state->done_iter));
         if (chunk_pap) {
           hipLaunchKernelGGL(cg_reduce_partials_kernel, dim3(kReducedPartials), dim3(256), 0, st, pap_count, chunk_pap,
                              pap_partials);

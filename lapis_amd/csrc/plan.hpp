@@ -102,10 +102,20 @@ template <typename T>
 int launch_rowchunk(const lapis_hip_csr_plan *plan, const int *crd, const T *val, const T *x, T *y, hipStream_t st,
                     int accumulate);
 // y = A x for a square A, and x . y in rowchunk_xy_blocks(plan) partial sums, one per workgroup; *count becomes their
-// number.  The whole launch returns at once when *skip (device memory) is not 0.
+// number.  The sums may go to pinned host memory.  The whole launch returns at once when *skip (device memory) is not 0.
 int rowchunk_xy_blocks(const lapis_hip_csr_plan *plan);
-int launch_rowchunk_xy(const lapis_hip_csr_plan *plan, const int *crd, const double *val, const double *x, double *y,
-                       hipStream_t st, double *xy_partials, int *count, const unsigned long long *skip);
+template <typename T>
+int launch_rowchunk_xy(const lapis_hip_csr_plan *plan, const int *crd, const T *val, const T *x, T *y, hipStream_t st,
+                       double *xy_partials, bool to_host, int *count, const unsigned long long *skip);
+
+// y = A x with the checks of the SpMV entry points, and the same with the start of init + x . y (blas1.hpp).
+struct HostSum;
+template <typename T>
+int spmv_overwrite(lapis_hip_csr_plan *plan, int64_t nrows, int64_t ncols, const int32_t *pos, const int32_t *crd,
+                   const T *val, const T *x, T *y, lapis_hip_stream_t stream);
+template <typename T>
+int spmv_dot_start(lapis_hip_csr_plan *plan, int64_t nrows, int64_t ncols, const int32_t *pos, const int32_t *crd,
+                   const T *val, const T *x, T *y, double init, lapis_hip_stream_t stream, HostSum **out);
 
 // Workgroup-blocked layout; defined in colgroup.hip.
 template <typename T>

@@ -21,6 +21,7 @@
 // percent faster: not worth a second copy of the coordinates).
 #include <algorithm>
 
+#include "blas1.hpp"
 #include "common.hpp"
 #include "plan.hpp"
 
@@ -62,7 +63,7 @@ template <typename T, int CAP, int WAVES, bool NT>
 __global__ __launch_bounds__(64 * WAVES) void spmv_rowchunk_kernel(
     int nnz, int nchunks, const v2i *__restrict__ desc, const int *__restrict__ pos, const int *__restrict__ crd,
     const T *__restrict__ val, const T *__restrict__ x, T *__restrict__ y, int accumulate, int contiguous,
-    double *__restrict__ xy_partials, const unsigned long long *__restrict__ skip) {
+    double *__restrict__ xy_partials, int to_host, const unsigned long long *__restrict__ skip) {
   typedef Lanes<T> L;
   constexpr int PER = L::per;
   constexpr int STEPS = CAP / (64 * PER);
@@ -165,7 +166,10 @@ __global__ __launch_bounds__(64 * WAVES) void spmv_rowchunk_kernel(
     if (threadIdx.x == 0) {
       double s = wave_xy[0];
       for (int w = 1; w < WAVES; ++w) s = s + wave_xy[w];
-      xy_partials[blockIdx.x] = s;
+      if (to_host)
+        tell_host(xy_partials + blockIdx.x, s);
+      else
+        xy_partials[blockIdx.x] = s;
     }
   }
 }
@@ -229,41 +233,48 @@ int rowchunk_xy_blocks(const lapis_hip_csr_plan *p) {
 
 template <typename T, int CAP>
 int launch_rowchunk_cap(const lapis_hip_csr_plan *p, const int *crd, const T *val, const T *x, T *y, hipStream_t st,
-                        int accumulate, double *xy_partials, int *count, const unsigned long long *skip) {
+                        int accumulate, double *xy_partials, bool to_host, int *count,
+                        const unsigned long long *skip) {
   constexpr int kWaves = 4;
   int64_t blocks = ceil_div(p->rowchunk_n, kWaves);
   if (count) *count = (int)(blocks = rowchunk_xy_blocks(p));
   auto kernel = p->nontemporal ? spmv_rowchunk_kernel<T, CAP, kWaves, true> : spmv_rowchunk_kernel<T, CAP, kWaves, false>;
   launch_timed(kernel, dim3((unsigned)blocks), dim3(64 * kWaves), st, (int)p->stats.nnz, p->rowchunk_n,
                (const v2i *)p->rowchunk_desc, p->pos, crd, val, x, y, accumulate, (int)p->rowchunk_contiguous,
-               xy_partials, skip);
+               xy_partials, (int)to_host, skip);
   LAPIS_LAUNCH_CHECK();
   return LAPIS_HIP_OK;
 }
 
 template <typename T>
 int launch_rowchunk_any(const lapis_hip_csr_plan *p, const int *crd, const T *val, const T *x, T *y, hipStream_t st,
-                        int accumulate, double *xy_partials, int *count, const unsigned long long *skip) {
+                        int accumulate, double *xy_partials, bool to_host, int *count,
+                        const unsigned long long *skip) {
   switch (p->rowchunk_cap) {
-    case 256: return launch_rowchunk_cap<T, 256>(p, crd, val, x, y, st, accumulate, xy_partials, count, skip);
-    case 512: return launch_rowchunk_cap<T, 512>(p, crd, val, x, y, st, accumulate, xy_partials, count, skip);
-    default: return launch_rowchunk_cap<T, 1024>(p, crd, val, x, y, st, accumulate, xy_partials, count, skip);
+    case 256: return launch_rowchunk_cap<T, 256>(p, crd, val, x, y, st, accumulate, xy_partials, to_host, count, skip);
+    case 512: return launch_rowchunk_cap<T, 512>(p, crd, val, x, y, st, accumulate, xy_partials, to_host, count, skip);
+    default: return launch_rowchunk_cap<T, 1024>(p, crd, val, x, y, st, accumulate, xy_partials, to_host, count, skip);
   }
 }
 
 template <typename T>
 int launch_rowchunk(const lapis_hip_csr_plan *p, const int *crd, const T *val, const T *x, T *y, hipStream_t st,
                     int accumulate) {
-  return launch_rowchunk_any<T>(p, crd, val, x, y, st, accumulate, nullptr, nullptr, nullptr);
+  return launch_rowchunk_any<T>(p, crd, val, x, y, st, accumulate, nullptr, false, nullptr, nullptr);
 }
 template int launch_rowchunk<double>(const lapis_hip_csr_plan *, const int *, const double *, const double *, double *,
                                      hipStream_t, int);
 template int launch_rowchunk<float>(const lapis_hip_csr_plan *, const int *, const float *, const float *, float *,
                                     hipStream_t, int);
 
-int launch_rowchunk_xy(const lapis_hip_csr_plan *p, const int *crd, const double *val, const double *x, double *y,
-                       hipStream_t st, double *xy_partials, int *count, const unsigned long long *skip) {
-  return launch_rowchunk_any<double>(p, crd, val, x, y, st, 0, xy_partials, count, skip);
+template <typename T>
+int launch_rowchunk_xy(const lapis_hip_csr_plan *p, const int *crd, const T *val, const T *x, T *y, hipStream_t st,
+                       double *xy_partials, bool to_host, int *count, const unsigned long long *skip) {
+  return launch_rowchunk_any<T>(p, crd, val, x, y, st, 0, xy_partials, to_host, count, skip);
 }
+template int launch_rowchunk_xy<double>(const lapis_hip_csr_plan *, const int *, const double *, const double *, double *,
+                                        hipStream_t, double *, bool, int *, const unsigned long long *);
+template int launch_rowchunk_xy<float>(const lapis_hip_csr_plan *, const int *, const float *, const float *, float *,
+                                       hipStream_t, double *, bool, int *, const unsigned long long *);
 
 }  // namespace lapis

@@ -10,6 +10,7 @@
 #include <cstdlib>
 #include <cstring>
 
+#include "blas1.hpp"
 #include "common.hpp"
 #include "plan.hpp"
 #include "rowsplit_fix.hpp"
@@ -672,6 +673,52 @@ int spmv_overwrite_f64(lapis_hip_csr_plan *plan, int64_t nrows, int64_t ncols, c
   if (rc != LAPIS_HIP_OK) return rc;
   return lapis_hip_spmv_csr_f64_i32(plan, nrows, ncols, pos, crd, val, x, y, stream);
 }
+
+static bool as_row_chunks(const lapis_hip_csr_plan *plan, int64_t nrows, int64_t ncols, const int32_t *pos, const void *crd,
+                          const void *val, const void *x, const void *y) {
+  return plan && plan->runs_rowchunk() && plan->stats.nnz > 0 && plan->stats.nrows == nrows && plan->stats.ncols == ncols &&
+         plan->pos == pos && crd && val && x && y;
+}
+
+template <typename T>
+int spmv_overwrite(lapis_hip_csr_plan *plan, int64_t nrows, int64_t ncols, const int32_t *pos, const int32_t *crd,
+                   const T *val, const T *x, T *y, lapis_hip_stream_t stream) {
+  if constexpr (sizeof(T) == 8) {
+    return spmv_overwrite_f64(plan, nrows, ncols, pos, crd, val, x, y, stream);
+  } else {
+    LAPIS_CHECK_INIT();
+    if (as_row_chunks(plan, nrows, ncols, pos, crd, val, x, y))
+      return launch_rowchunk<float>(plan, crd, val, x, y, as_stream(stream), 0);
+    const int rc = lapis_hip_fill_f32(nrows, 0.f, y, stream);
+    return rc != LAPIS_HIP_OK ? rc : spmv_impl<float>(plan, nrows, ncols, pos, crd, val, x, y, stream);
+  }
+}
+template int spmv_overwrite<double>(lapis_hip_csr_plan *, int64_t, int64_t, const int32_t *, const int32_t *, const double *,
+                                    const double *, double *, lapis_hip_stream_t);
+template int spmv_overwrite<float>(lapis_hip_csr_plan *, int64_t, int64_t, const int32_t *, const int32_t *, const float *,
+                                   const float *, float *, lapis_hip_stream_t);
+
+template <typename T>
+int spmv_dot_start(lapis_hip_csr_plan *plan, int64_t nrows, int64_t ncols, const int32_t *pos, const int32_t *crd,
+                   const T *val, const T *x, T *y, double init, lapis_hip_stream_t stream, HostSum **out) {
+  LAPIS_CHECK_INIT();
+  LAPIS_REQUIRE(nrows == ncols, "spmv_dot: a %lld x %lld matrix", (long long)nrows, (long long)ncols);
+  hipStream_t st = as_stream(stream);
+  if (as_row_chunks(plan, nrows, ncols, pos, crd, val, x, y) && rowchunk_xy_blocks(plan) <= kDotMaxBlocks) {
+    int count = rowchunk_xy_blocks(plan);
+    int rc = take_host_sum(count, init, false, st, out);
+    if (rc != LAPIS_HIP_OK) return rc;
+    rc = launch_rowchunk_xy<T>(plan, crd, val, x, y, st, (*out)->parts, true, &count, nullptr);
+    if (rc != LAPIS_HIP_OK) dot_abandon(*out);
+    return rc;
+  }
+  const int rc = spmv_overwrite<T>(plan, nrows, ncols, pos, crd, val, x, y, stream);
+  return rc != LAPIS_HIP_OK ? rc : dot_start<T>(nrows, x, y, init, st, out);
+}
+template int spmv_dot_start<double>(lapis_hip_csr_plan *, int64_t, int64_t, const int32_t *, const int32_t *, const double *,
+                                    const double *, double *, double, lapis_hip_stream_t, HostSum **);
+template int spmv_dot_start<float>(lapis_hip_csr_plan *, int64_t, int64_t, const int32_t *, const int32_t *, const float *,
+                                   const float *, float *, double, lapis_hip_stream_t, HostSum **);
 }  // namespace lapis
 
 namespace {

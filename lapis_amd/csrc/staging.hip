@@ -334,11 +334,11 @@ Crew::Crew(HostOperands *owner, bool to_host, std::vector<HostOperands::Block> *
 }  // namespace
 
 void HostOperands::copy_block(const Block &b, bool to_host) {
-  const Operand &o = operands_[(size_t)b.operand];
   if (to_host) {
     memcpy(b.host, b.staged, b.bytes);
     return;
   }
+  const Operand &o = operands_[(size_t)b.operand];
   if (o.kind == kPlain || o.kind == kDirectly) {
     memcpy(b.staged, b.host, b.bytes);
     return;
@@ -378,7 +378,7 @@ HostOperands::~HostOperands() {
   if (!arena_) return;
   if (!idle_) {
     (void)hipStreamSynchronize(arena_->second);
-    (void)hipStreamSynchronize(arena_->stream);
+    (void)hipStreamSynchronize(primary_);
   }
   give_arena(arena_);
 }
@@ -402,7 +402,6 @@ int HostOperands::add_coordinates(const int32_t *host, int64_t nnz, int64_t ncol
   operands_.push_back({reinterpret_cast<const char *>(host), sizeof(int32_t) * (size_t)nnz, 0, kCoordinates});
   return (int)operands_.size() - 1;
 }
-hipStream_t HostOperands::stream() const { return arena_->stream; }
 void *HostOperands::device(int index) const {
   const Operand &o = operands_[(size_t)index];
   return !o.bytes ? nullptr : o.kind == kDirectly ? arena_->direct + o.at : arena_->memory + o.at;
@@ -425,6 +424,7 @@ int HostOperands::upload() {
   while (half < kHalf && half < bytes_) half *= 2;
   LAPIS_HIP_TRY(take_arena(&arena_, bytes_, half, direct_bytes));
   half = arena_->pinned_bytes;
+  if (own_stream_) primary_ = arena_->stream;
   counts_ = CsrCounts{};
   counts_.min_len = INT32_MAX;
 
@@ -455,7 +455,7 @@ int HostOperands::upload() {
   // (0.14 MB: 26 us a call against 31).  More goes in pieces of 4 MB after half a megabyte that gets the bus started, on
   // two streams in turn, so that a transfer is set up while another runs (27 MB: 0.70 ms a call against 0.85).
   const bool by_kernel = upload_bytes <= kByKernel;
-  const hipStream_t streams[2] = {arena_->stream, arena_->second};
+  const hipStream_t streams[2] = {primary_, arena_->second};
   size_t filled = 0, sent = 0, transfers = 0;
   for (size_t r = 0; r < rounds.size(); ++r) {
     if (r >= 2)
@@ -469,7 +469,7 @@ int HostOperands::upload() {
       if (upto > sent && (filled == rounds[r] || upto - sent >= worth)) {
         if (by_kernel) {
           const int n = (int)((upto + 15) / 16);
-          hipLaunchKernelGGL(staging_copy_kernel, dim3((unsigned)std::min(256, (n + 255) / 256)), dim3(256), 0, arena_->stream,
+          hipLaunchKernelGGL(staging_copy_kernel, dim3((unsigned)std::min(256, (n + 255) / 256)), dim3(256), 0, primary_,
                              n, reinterpret_cast<const v4i *>(arena_->pinned[0]), reinterpret_cast<v4i *>(arena_->memory));
           LAPIS_LAUNCH_CHECK();
         } else {
@@ -486,7 +486,7 @@ int HostOperands::upload() {
   }
   if (transfers > 1) {
     LAPIS_HIP_TRY(hipEventRecord(arena_->joined, arena_->second));
-    LAPIS_HIP_TRY(hipStreamWaitEvent(arena_->stream, arena_->joined, 0));
+    LAPIS_HIP_TRY(hipStreamWaitEvent(primary_, arena_->joined, 0));
   }
   q.limit.store((int)blocks.size(), std::memory_order_release);
   while (filled < blocks.size()) {
@@ -501,11 +501,11 @@ int HostOperands::create_plan(int positions, int coordinates, int value_bytes, l
   CsrCounts counts = counts_;
   if (nrows_ == 0) counts.min_len = 0;
   return create_counted_plan(plan, nrows_, ncols_, nnz_, at<int32_t>(positions), at<int32_t>(coordinates), value_bytes, counts,
-                             host[0], host[nrows_], arena_->stream);
+                             host[0], host[nrows_], primary_);
 }
 
 int HostOperands::synchronize() {
-  LAPIS_HIP_TRY(hipStreamSynchronize(arena_->stream));
+  LAPIS_HIP_TRY(hipStreamSynchronize(primary_));
   idle_ = true;
   return LAPIS_HIP_OK;
 }
@@ -528,17 +528,23 @@ int HostOperands::download(int index, void *host) {
         __builtin_ia32_pause();
     return LAPIS_HIP_OK;
   }
+  return download(arena_->memory + o.at, o.bytes, host);
+}
+
+int HostOperands::download(const void *from, size_t total, void *host) {
+  if (total == 0) return LAPIS_HIP_OK;
+  const char *source = static_cast<const char *>(from);
   const size_t half = arena_->pinned_bytes;
-  if (o.bytes <= half && o.bytes <= kAlone / 2) {
-    LAPIS_HIP_TRY(hipMemcpyAsync(arena_->pinned[0], arena_->memory + o.at, o.bytes, hipMemcpyDeviceToHost, arena_->stream));
+  if (total <= half && total <= kAlone / 2) {
+    LAPIS_HIP_TRY(hipMemcpyAsync(arena_->pinned[0], source, total, hipMemcpyDeviceToHost, primary_));
     const int rc = synchronize();
-    if (rc == LAPIS_HIP_OK) memcpy(host, arena_->pinned[0], o.bytes);
+    if (rc == LAPIS_HIP_OK) memcpy(host, arena_->pinned[0], total);
     return rc;
   }
   // pieces of up to 2 MB through the slots of both halves, copied out as they land
-  const size_t piece = std::min(half, std::max(kBlock, std::min((size_t)2 << 20, (o.bytes / 4 + kBlock - 1) / kBlock * kBlock)));
+  const size_t piece = std::min(half, std::max(kBlock, std::min((size_t)2 << 20, (total / 4 + kBlock - 1) / kBlock * kBlock)));
   const size_t per_half = half / piece, slots = std::min<size_t>(16, 2 * per_half);
-  const size_t pieces = (o.bytes + piece - 1) / piece;
+  const size_t pieces = (total + piece - 1) / piece;
   auto slot_of = [&](size_t p) {
     const size_t s = p % slots;
     return arena_->pinned[s / per_half] + (s % per_half) * piece;
@@ -546,21 +552,21 @@ int HostOperands::download(int index, void *host) {
   std::vector<Block> blocks;
   std::vector<size_t> last(pieces);  // one past the last block of each piece
   for (size_t p = 0; p < pieces; ++p) {
-    const size_t at = p * piece, bytes = std::min(piece, o.bytes - at);
+    const size_t at = p * piece, bytes = std::min(piece, total - at);
     for (size_t done = 0; done < bytes; done += kBlock)
-      blocks.push_back({slot_of(p) + done, static_cast<char *>(host) + at + done, std::min(kBlock, bytes - done), at + done, index, 0});
+      blocks.push_back({slot_of(p) + done, static_cast<char *>(host) + at + done, std::min(kBlock, bytes - done), at + done, 0, 0});
     last[p] = blocks.size();
   }
-  Crew crew(this, true, &blocks, o.bytes);
+  Crew crew(this, true, &blocks, total);
   BlockQueue &q = crew.queue;
   size_t queued = 0, landed = 0, emptied = 0, block = 0;
   idle_ = false;
   while (emptied < pieces) {
     while (queued < pieces && queued < emptied + slots) {
       const size_t at = queued * piece;
-      LAPIS_HIP_TRY(hipMemcpyAsync(slot_of(queued), arena_->memory + o.at + at, std::min(piece, o.bytes - at),
-                                   hipMemcpyDeviceToHost, arena_->stream));
-      LAPIS_HIP_TRY(hipEventRecord(arena_->landed[queued % slots], arena_->stream));
+      LAPIS_HIP_TRY(hipMemcpyAsync(slot_of(queued), source + at, std::min(piece, total - at),
+                                   hipMemcpyDeviceToHost, primary_));
+      LAPIS_HIP_TRY(hipEventRecord(arena_->landed[queued % slots], primary_));
       ++queued;
     }
     if (landed < queued) {

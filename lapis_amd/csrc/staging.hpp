@@ -27,6 +27,12 @@ class HostOperands {
   int add_positions(const int32_t *host, int64_t nrows, int64_t nnz);
   int add_coordinates(const int32_t *host, int64_t nnz, int64_t ncols);
 
+  // The copies and what follows are queued on this stream instead of one of the arena's own.
+  void use_stream(hipStream_t st) {
+    primary_ = st;
+    own_stream_ = false;
+  }
+
   int create_plan(int positions, int coordinates, int value_bytes, lapis_hip_csr_plan **plan);  // after upload()
 
   int upload();  // takes memory for all of them and queues their copies on stream()
@@ -34,11 +40,12 @@ class HostOperands {
   T *at(int index) const {
     return static_cast<T *>(device(index));
   }
-  hipStream_t stream() const;
+  hipStream_t stream() const { return primary_; }
   lapis_hip_stream_t abi_stream() const { return reinterpret_cast<lapis_hip_stream_t>(stream()); }
 
   // Brings an operand's device memory to `host`, after what is queued on stream(); returns when it is there.
   int download(int index, void *host);
+  int download(const void *from, size_t bytes, void *host);  // the same for any device memory
   int synchronize();
 
   struct Block {  // what one thread copies at a time
@@ -62,6 +69,8 @@ class HostOperands {
   std::vector<Operand> operands_;
   size_t bytes_ = 0;
   StagingArena *arena_ = nullptr;
+  hipStream_t primary_ = nullptr;
+  bool own_stream_ = true;
   bool idle_ = true;  // nothing is queued on the stream
   CsrCounts counts_{};  // of the CSR structure, after upload()
   int64_t nrows_ = 0, nnz_ = 0, ncols_ = 0;

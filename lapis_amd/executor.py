@@ -25,6 +25,7 @@ temporary this region made itself (tensor.empty, tensor.splat or the result of a
 that nothing mentions afterwards, otherwise the result gets a buffer of its own.  Memref operands are
 buffers and are always updated in place.
 """
+import math
 import re
 
 import numpy
@@ -32,6 +33,7 @@ import numpy
 from . import elementwise as _ew
 from . import loop_mapping as _lm
 from . import mlir_text as _mt
+from . import schedule as _sched
 
 
 class Refused(Exception):
@@ -39,10 +41,12 @@ class Refused(Exception):
 
 
 _NAME = r"%[\w.$-]+(?:#\d+)?"
-def _ieee(fn):
+def _ieee(fn, quick=None):
     """Host scalars follow IEEE 754 as the emitted C++ does: x/0 is an infinity or a NaN, not an exception,
     and the maximum of a NaN and a number is a NaN."""
     def apply(a, b):
+        if quick is not None and type(a) is float and type(b) is float and b:
+            return quick(a, b)
         f32 = isinstance(a, numpy.float32) and isinstance(b, numpy.float32)
         with numpy.errstate(all="ignore"):
             r = fn(numpy.float32(a) if f32 else numpy.float64(a), numpy.float32(b) if f32 else numpy.float64(b))
@@ -51,7 +55,7 @@ def _ieee(fn):
 
 
 _FLOAT_BIN = {"arith.addf": lambda a, b: a + b, "arith.subf": lambda a, b: a - b, "arith.mulf": lambda a, b: a * b,
-              "arith.divf": _ieee(numpy.divide), "arith.maximumf": _ieee(numpy.maximum),
+              "arith.divf": _ieee(numpy.divide, lambda a, b: a / b), "arith.maximumf": _ieee(numpy.maximum),
               "arith.minimumf": _ieee(numpy.minimum)}
 _INT_BIN = {"arith.addi": lambda a, b: a + b, "arith.subi": lambda a, b: a - b, "arith.muli": lambda a, b: a * b,
             "arith.divui": lambda a, b: a // b, "arith.divsi": lambda a, b: int(a / b) if b else 0,
@@ -74,6 +78,8 @@ _LINALG_NAMED = {"linalg.add": ("axpby", 1.0, 1.0), "linalg.sub": ("axpby", 1.0,
                  "linalg.div": ("div",)}
 _STRUCTURE = {"scf.while", "scf.for", "scf.if", "scf.condition", "scf.yield", "func.call", "call", "return",
               "func.return", "scf.parallel", "scf.reduce"}
+_OWNING = {"tensor.empty", "tensor.splat", "memref.alloc", "memref.alloca", "bufferization.alloc_tensor", "linalg.fill",
+           "linalg.copy", "linalg.matvec", "linalg.matmul", "linalg.generic"} | set(_LINALG_NAMED)  # results are buffers of this region
 _BUFFER_OPS = {"tensor.empty", "tensor.splat", "tensor.dim", "tensor.extract", "memref.alloc", "memref.alloca",
                "memref.dealloc", "memref.dim", "memref.load", "memref.store", "memref.copy", "linalg.fill",
                "linalg.copy", "linalg.dot", "linalg.matvec", "linalg.matmul", "linalg.generic",
@@ -95,11 +101,13 @@ class Csr:
             raise ValueError("a CSR operand with %d coordinates and %d values" % (self.nnz, int(val.shape[0])))
         self.plan = None
         self.products = 0
+        self.staged = None  # makes the plan where the pass that brought the buffers to the device has counted the structure
 
     def release(self):
         if self.plan is not None:
             self.plan.destroy()
             self.plan = None
+        self.staged = None
 
 
 class Cell:
@@ -168,12 +176,98 @@ def _group(head, keyword):
     return re.findall(_NAME, names), [t.strip() for t in _mt.split_top(types)] if types.strip() else []
 
 
-def _mentions(stmt, out):
-    out.update(re.findall(_NAME, stmt.head))
-    for _, sub in stmt.regions:
-        for s in sub:
-            _mentions(s, out)
-    return out
+def _flat(t):
+    return t if t.dim() == 1 else t.reshape(-1)
+
+
+def _constant(head):
+    left, ty = _split_colon(head)
+    tok, ty = left.strip(), ty.strip()
+    if tok in ("true", "false"):
+        return tok == "true"
+    if ty in ("f64", "f32"):
+        return numpy.float32(tok) if ty == "f32" else float(tok)
+    return int(float(tok)) if ty != "i1" else bool(int(tok))
+
+
+def _sqrt(v):
+    if type(v) is float and v >= 0.0:
+        return math.sqrt(v)
+    with numpy.errstate(all="ignore"):  # the root of a negative number is a NaN
+        return numpy.sqrt(v) if isinstance(v, numpy.floating) else float(numpy.sqrt(v))
+
+
+def _coefficient(expr):
+    """A function (values by name, destination) that gives the number a coefficient expression stands for."""
+    def general(env, d):
+        return float(_ew.evaluate(expr, env.__getitem__, numpy.float32 if d.element_size() == 4 else float))
+    if expr[0] == "const":
+        return general if float(numpy.float32(expr[1])) != expr[1] else (lambda env, d, v=expr[1]: v)
+    sign = 1.0
+    while expr[0] == "neg":
+        sign, expr = -sign, expr[1]
+    if expr[0] != "name":
+        if sign < 0.0:
+            expr = ("neg", expr)
+        return general
+    name = expr[1]
+
+    def value(env, d):
+        v = float(env[name])
+        return sign * (float(numpy.float32(v)) if d.element_size() == 4 else v)
+    return value
+
+
+def _raises(e):
+    def step(env):
+        raise e
+    return step
+
+
+def _giving(op, names, fn):
+    """A step that stores what `fn(values)` returns (a list, or None for no results) under `names`."""
+    def step(env):
+        results = fn(env)
+        if results is not None:
+            if len(results) != len(names):
+                raise RuntimeError("%s gave %d values for %d results" % (op, len(results), len(names)))
+            env.update(zip(names, results))
+    return step
+
+
+class _Block:
+    """The steps of a region, its constants, and the terminator with the names of the values it passes on."""
+
+    def __init__(self):
+        self.constants, self.steps, self.ops, self.end, self.names = {}, [], [], "end", []
+
+    def add(self, op, step):
+        self.ops.append(op)
+        self.steps.append(step)
+
+    def run(self, env):
+        env.update(self.constants)
+        at = 0
+        try:
+            for step in self.steps:
+                step(env)
+                at += 1
+            return self.end, [env[n] for n in self.names]
+        except KeyError as e:
+            name = e.args[0] if e.args else None
+            if isinstance(name, str) and name.startswith("%"):
+                raise RuntimeError("value %s is used before it is defined" % name)
+            self._wrong_type(at, e)
+        except ZeroDivisionError:
+            raise RuntimeError("%s: integer division by zero" % self.ops[at])
+        except (AttributeError, TypeError, IndexError) as e:
+            self._wrong_type(at, e)
+
+    def _wrong_type(self, at, e):
+        # an operand that is not what the operation's types say (a scalar where a tensor is named, ...):
+        # text MLIR's own verifier would not have let through
+        raise RuntimeError("%s: an operand does not have the type the operation declares (%s: %s)" % (
+            self.ops[at] if at < len(self.ops) else self.end, type(e).__name__, e))
 
 
 class Executor:
@@ -184,6 +278,7 @@ class Executor:
         self.c = canonicalizer
         self.aliases = canonicalizer.aliases
         self._parsed = {}
+        self._programs = {}
         self._torch = torch_module
         self._hip = hip_module
 
@@ -347,185 +442,223 @@ class Executor:
     # ---- running --------------------------------------------------------------------------------------
     def run(self, name, args):
         """Results of @name for `args` (device tensors, Csr operands, host scalars), as a list."""
-        f, stmts, nests = self._function(name)
-        env = {}
-        for (nm, _), v in zip(f.args, args):
-            env[nm] = v
-        kind, values = self._region(stmts, env, nests, owned=set())
+        names, block = self._program(name)
+        kind, values = block.run(dict(zip(names, args)))
         if kind != "return":
             raise RuntimeError("@%s ended without a return" % name)
         return values
 
-    def _val(self, env, name):
-        if name not in env:
-            raise RuntimeError("value %s is used before it is defined" % name)
-        return env[name]
+    def _program(self, name):
+        """(argument names, the function's statements as steps), made when a function is first run."""
+        if name not in self._programs:
+            f, stmts, nests = self._function(name)
+            if hasattr(self.hip, "dot_start") and not nests:
+                stmts = _sched.inline(stmts, self._inlinable, {name}, [0])
+            self._programs[name] = ([nm for nm, _ in f.args], self._block(stmts, nests, {}))
+        return self._programs[name]
 
-    def _region(self, stmts, env, nests, owned):
-        """Runs the statements; returns (terminator kind, its operand values)."""
-        later = [None] * len(stmts)
-        acc = set()
+    def _inlinable(self, name):
+        f, stmts, nests = self._function(name)
+        return None if nests else ([nm for nm, _ in f.args], stmts)
+
+    def _kind(self, s):
+        if s.op == "linalg.matvec":
+            return "product"
+        if s.op in ("linalg.add", "linalg.sub"):
+            return "axpby" if len(_group(s.head, "ins")[0]) == 2 else None
+        if s.op == "linalg.generic":
+            try:
+                plan = self._generic_plan(s)
+            except Refused:
+                return None
+            return "product" if plan == ("matvec",) else "axpby" if plan[0] == "elementwise" and plan[1][0] == "axpby" else None
+        return None
+
+    def _block(self, stmts, nests, constants):
+        constants = dict(constants)
+        for s in stmts:
+            if s.op == "arith.constant" and len(s.results) == 1:
+                try:
+                    constants[s.results[0]] = _constant(s.head)
+                except ValueError:
+                    pass
+        if hasattr(self.hip, "dot_start") and not nests:
+            stmts = _sched.rewrite(stmts, self._kind, constants)
+        later, acc = [None] * len(stmts), set()
         for k in range(len(stmts) - 1, -1, -1):
             later[k] = set(acc)
-            _mentions(stmts[k], acc)
-        defined_here = set()
+            _sched.mentions(stmts[k], acc)
+        block, owned, defined = _Block(), set(), set()
         for k, s in enumerate(stmts):
             op = s.op
             if op in ("return", "func.return", "scf.yield", "scf.condition"):
-                names = re.findall(_NAME, _split_colon(s.head)[0])
-                return op.split(".")[-1], [self._val(env, n) for n in names]
-            can_overwrite = lambda nm: nm in owned and nm in defined_here and nm not in later[k]
+                block.end, block.names = op.split(".")[-1], re.findall(_NAME, _split_colon(s.head)[0])
+                break
+            if op == "arith.constant" and s.results[0] in constants:
+                block.constants[s.results[0]] = constants[s.results[0]]
+                continue
+            can_overwrite = lambda nm, k=k: nm in owned and nm in defined and nm not in later[k]
             try:
-                results = self._statement(s, env, nests, owned, can_overwrite)
-            except ZeroDivisionError:
-                raise RuntimeError("%s: integer division by zero" % op)
-            except (AttributeError, TypeError, IndexError, KeyError) as e:
-                # an operand that is not what the operation's types say (a scalar where a tensor is named, ...):
-                # text MLIR's own verifier would not have let through
-                raise RuntimeError("%s: an operand does not have the type the operation declares (%s: %s)" % (
-                    op, type(e).__name__, e))
-            names = []
-            for r in s.results:
-                if ":" in r:
-                    base, cnt = r.split(":")
-                    names += ["%s#%d" % (base, j) for j in range(int(cnt))]
-                else:
-                    names.append(r)
-            if results is not None:
-                if len(results) != len(names):
-                    raise RuntimeError("%s gave %d values for %d results" % (op, len(results), len(names)))
-                for nm, v in zip(names, results):
-                    env[nm] = v
-                    defined_here.add(nm)
-        return "end", []
+                step = self._step(s, nests, can_overwrite, constants)
+            except (AttributeError, TypeError, IndexError, KeyError, ValueError) as e:
+                step = _raises(e)
+            block.add(op, step)
+            names = _sched.result_names(s)
+            defined.update(names)
+            if op in _OWNING and not isinstance(s, _sched.Fused) and s.results:
+                owned.add(s.results[0])
+            elif isinstance(s, _sched.Fused) and s.op != "lapis.dot_finish":
+                owned.update(s.results)
+        return block
 
-    # every handler returns the list of result values (or None for no results)
-    def _statement(self, s, env, nests, owned, can_overwrite):
+    # Every statement becomes a step: a function of the values by name that leaves its results among them.
+    def _step(self, s, nests, can_overwrite, constants):
         op, head = s.op, s.head
+        names = _sched.result_names(s)
         if op in _SCALAR_OPS:
-            return [self._scalar(op, head, env)]
+            return self._scalar_step(op, head, names[0])
+        if op.startswith("lapis."):
+            return self._fused_step(s, can_overwrite)
         if op == "scf.parallel":
-            return self._nest(s, nests[id(s)], env)
+            nest = nests[id(s)]
+            return _giving(op, names, lambda env: self._nest(s, nest, env))
         if op in ("func.call", "call"):
             callee = re.search(r"@([\w$.-]+)", head).group(1)
             i = head.index("(")
-            names = re.findall(_NAME, head[i:_mt._match(head, i)])
-            return self.run(callee, [self._val(env, n) for n in names])
+            given = re.findall(_NAME, head[i:_mt._match(head, i)])
+            return _giving(op, names, lambda env: self.run(callee, [env[n] for n in given]))
         if op == "scf.while":
-            return self._while(s, env, nests)
+            return _giving(op, names, self._while(s, nests, constants))
         if op == "scf.for":
-            return self._for(s, env, nests)
+            return _giving(op, names, self._for(s, nests, constants))
         if op == "scf.if":
-            cond = self._val(env, re.findall(_NAME, head)[0])
-            if len(s.regions) < 2 and not cond:
-                return None
-            bargs, sub = s.regions[0 if cond else 1]
-            kind, vals = self._region(sub, env, nests, set())
-            return vals if s.results else None
-        return self._buffer_op(s, env, owned, can_overwrite)
+            cond = re.findall(_NAME, head)[0]
+            blocks = [self._block(sub, nests, constants) for _, sub in s.regions]
 
-    def _scalar(self, op, head, env):
+            def branch(env):
+                if env[cond]:
+                    values = blocks[0].run(dict(env))[1]
+                elif len(blocks) > 1:
+                    values = blocks[1].run(dict(env))[1]
+                else:
+                    return None
+                return values if s.results else None
+            return _giving(op, names, branch)
+        return self._buffer_step(s, names, can_overwrite)
+
+    def _scalar_step(self, op, head, r):
         left, ty = _split_colon(head)
         ty = ty.strip()
         if op == "arith.constant":
-            tok = left.strip()
-            if tok in ("true", "false"):
-                return tok == "true"
-            if ty in ("f64", "f32"):
-                return numpy.float32(tok) if ty == "f32" else float(tok)
-            return int(float(tok)) if ty != "i1" else bool(int(tok))
-        names = re.findall(_NAME, left)
-        vals = [self._val(env, n) for n in names]
-        if op in _FLOAT_BIN:
-            return _FLOAT_BIN[op](vals[0], vals[1])
-        if op in _INT_BIN:
-            return _INT_BIN[op](vals[0], vals[1])
-        if op == "arith.negf":
-            return -vals[0]
-        if op == "math.sqrt":
-            with numpy.errstate(all="ignore"):  # the root of a negative number is a NaN
-                return numpy.sqrt(vals[0]) if isinstance(vals[0], numpy.floating) else float(numpy.sqrt(vals[0]))
-        if op == "math.absf":
-            return abs(vals[0])
+            v = _constant(head)
+
+            def step(env):
+                env[r] = v
+            return step
+        ops = re.findall(_NAME, left)
         if op in ("arith.cmpi", "arith.cmpf"):
-            pred = re.match(r"\s*(\w+)", left).group(1)
-            return (_CMPI if op == "arith.cmpi" else _CMPF)[pred](vals[0], vals[1])
+            fn = (_CMPI if op == "arith.cmpi" else _CMPF)[re.match(r"\s*(\w+)", left).group(1)]
+        else:
+            fn = _FLOAT_BIN.get(op) or _INT_BIN.get(op)
+        if fn is not None:
+            a, b = ops[0], ops[1]
+
+            def step(env):
+                env[r] = fn(env[a], env[b])
+            return step
         if op == "arith.select":
-            return vals[1] if vals[0] else vals[2]
-        if op in _CASTS:
+            c, a, b = ops[:3]
+
+            def step(env):
+                env[r] = env[a] if env[c] else env[b]
+            return step
+        if op == "arith.negf":
+            fn = lambda v: -v
+        elif op == "math.sqrt":
+            fn = _sqrt
+        elif op == "math.absf":
+            fn = abs
+        elif op in _CASTS:
             target = ty.split("to")[-1].strip()
-            if target == "f32":
-                return numpy.float32(vals[0])
-            if target == "f64":
-                return float(vals[0])
-            return int(vals[0])
-        raise Refused("the operation %s" % op)
+            fn = numpy.float32 if target == "f32" else float if target == "f64" else int
+        else:
+            raise Refused("the operation %s" % op)
+        a = ops[0]
+
+        def step(env):
+            env[r] = fn(env[a])
+        return step
 
     # ---- structured control flow -----------------------------------------------------------------------
-    def _while(self, s, env, nests):
+    def _while(self, s, nests, constants):
         head = s.head
         i = head.index("(")
         inits = [p.split("=") for p in _mt.split_top(head[i + 1:_mt._match(head, i) - 1]) if "=" in p]
         before_names = [a.strip() for a, _ in inits]
-        values = [self._val(env, b.strip()) for _, b in inits]
+        init_names = [b.strip() for _, b in inits]
         (_, before), (after_args, after) = s.regions
-        while True:
-            e = dict(env)
-            e.update(zip(before_names, values))
-            kind, out = self._region(before, e, nests, set())
-            if kind != "condition":
-                raise RuntimeError("the first region of scf.while does not end in scf.condition")
-            if not out[0]:
-                return out[1:]
-            e = dict(env)
-            e.update(zip(after_args, out[1:]))
-            kind, values = self._region(after, e, nests, set())
-            if kind != "yield":
-                raise RuntimeError("the second region of scf.while does not end in scf.yield")
+        before, after = self._block(before, nests, constants), self._block(after, nests, constants)
 
-    def _for(self, s, env, nests):
+        def loop(env):
+            values = [env[n] for n in init_names]
+            while True:
+                e = dict(env)
+                e.update(zip(before_names, values))
+                kind, out = before.run(e)
+                if kind != "condition":
+                    raise RuntimeError("the first region of scf.while does not end in scf.condition")
+                if not out[0]:
+                    return out[1:]
+                e = dict(env)
+                e.update(zip(after_args, out[1:]))
+                kind, values = after.run(e)
+                if kind != "yield":
+                    raise RuntimeError("the second region of scf.while does not end in scf.yield")
+        return loop
+
+    def _for(self, s, nests, constants):
         m = re.match(r"\s*(%s)\s*=\s*(%s)\s*to\s*(%s)\s*step\s*(%s)" % ((_NAME,) * 4), s.head)
         if not m:
             raise Refused("an scf.for that is not `%i = lo to hi step st`")
-        iv, lo, hi, st = m.group(1), self._val(env, m.group(2)), self._val(env, m.group(3)), self._val(env, m.group(4))
-        carried_names, values = [], []
+        iv, lo, hi, st = m.groups()
+        carried, inits = [], []
         im = re.search(r"iter_args\s*\(", s.head)
         if im:
             i = im.end() - 1
             for p in _mt.split_top(s.head[i + 1:_mt._match(s.head, i) - 1]):
                 a, b = p.split("=")
-                carried_names.append(a.strip())
-                values.append(self._val(env, b.strip()))
-        _, body = s.regions[0]
-        for k in range(lo, hi, st):
-            e = dict(env)
-            e[iv] = k
-            e.update(zip(carried_names, values))
-            kind, out = self._region(body, e, nests, set())
-            if carried_names:
-                values = out
-        return values if s.results else None
+                carried.append(a.strip())
+                inits.append(b.strip())
+        body = self._block(s.regions[0][1], nests, constants)
+
+        def loop(env):
+            values = [env[n] for n in inits]
+            for k in range(env[lo], env[hi], env[st]):
+                e = dict(env)
+                e[iv] = k
+                e.update(zip(carried, values))
+                kind, out = body.run(e)
+                if carried:
+                    values = out
+            return values if s.results else None
+        return loop
 
     # ---- tensors and memrefs ---------------------------------------------------------------------------
-    def _new(self, shape, elem):
-        torch = self.torch
-        return torch.empty(tuple(int(d) for d in shape), dtype=torch.float64 if elem == "f64" else
-                           torch.float32 if elem == "f32" else torch.int32, device=self.device)
-
-    def _sizes(self, ty, dynamic):
+    def _allocation(self, ty, names):
+        """A function of the values that allocates a tensor of the type, its dynamic sizes taken from `names`; None for
+        zero dimensions."""
         dims, elem = _shape_spec(ty)
-        dyn = iter(dynamic)
-        return [d if d is not None else int(next(dyn)) for d in dims], elem
+        if not dims:
+            return None
+        torch = self.torch
+        dtype = torch.float64 if elem == "f64" else torch.float32 if elem == "f32" else torch.int32
+        dyn = iter(names)
+        dims = [d if d is not None else next(dyn) for d in dims]
+        device = torch.device(self.device)
+        return lambda env: torch.empty([env[d] if isinstance(d, str) else d for d in dims], dtype=dtype, device=device)
 
-    def _dest(self, nm, env, can_overwrite, keep_contents):
-        """Buffer the result of a tensor operation goes to: the `outs` operand itself where that is allowed, else
-        a new buffer (a copy of the operand when the operation reads it)."""
-        t = self._val(env, nm)
-        if can_overwrite(nm):
-            return t
-        return t.clone() if keep_contents else self.torch.empty_like(t)
-
-    def _csr_product(self, A, x, y, k=None):
+    def _csr_product(self, A, x, y, k=None, overwrite=False, dot=None):
+        """y += A x, or with k columns Y += A X; overwrite: y = A x; dot: y = A x and the start of dot + x . y."""
         hip = self.hip
         if k is None:
             if x.numel() != A.ncols or y.numel() != A.nrows:
@@ -535,178 +668,287 @@ class Executor:
             raise ValueError("a %d x %d matrix times a %s matrix into a %s one" % (
                 A.nrows, A.ncols, "x".join(map(str, x.shape)), "x".join(map(str, y.shape))))
         if A.plan is None:
-            A.plan = hip.CsrPlan(A.nrows, A.ncols, A.pos, A.crd, value_bytes=A.val.element_size(), nnz=A.nnz)
+            A.plan = A.staged() if A.staged else \
+                hip.CsrPlan(A.nrows, A.ncols, A.pos, A.crd, value_bytes=A.val.element_size(), nnz=A.nnz)
         A.products += 1
-        if k is None:
-            if A.products == 6:  # a matrix multiplied with again and again: let the library decide on its blocked copy
-                A.plan.analyze(A.crd, A.val)
-            hip.spmv(A.plan, A.nrows, A.ncols, A.pos, A.crd, A.val, x, y)
-        else:
+        if k is not None:
             hip.spmm(A.nrows, A.ncols, A.pos, A.crd, A.val, x, y, plan=A.plan)
+            return y
+        if A.products == 6:  # a matrix multiplied with again and again: let the library decide on its blocked copy
+            A.plan.analyze(A.crd, A.val)
+        if dot is not None:
+            return y, hip.spmv_dot_start(A.plan, A.nrows, A.ncols, A.pos, A.crd, A.val, x, y, dot)
+        (hip.spmv_overwrite if overwrite else hip.spmv)(A.plan, A.nrows, A.ncols, A.pos, A.crd, A.val, x, y)
         return y
 
-    def _elementwise(self, call, operands, dst, scalars):
-        """dst = call(operands); `operands[k]` are flat device tensors, `scalars(name)` host values."""
-        hip = self.hip
-        f32 = dst.element_size() == 4
-        dtype = numpy.float32 if f32 else float
-        ev = lambda expr: float(_ew.evaluate(expr, scalars, dtype))
-        kind = call[0]
-        _same_size("an elementwise operation", dst, *operands)
-        if kind == "fill":
-            hip.fill(dst, ev(call[1]))
-        elif kind == "copy":
-            if operands[call[1]].data_ptr() != dst.data_ptr():
-                hip.copy(operands[call[1]], dst)
-        elif kind == "scale":
-            x = operands[call[2]]
-            hip.axpby(ev(call[1]), x, 0.0, x, dst)
-        elif kind == "mult":
-            hip.mult(operands[call[1]], operands[call[2]], dst)
-        elif kind == "axpby":
-            hip.axpby(ev(call[1]), operands[call[2]], ev(call[3]), operands[call[4]], dst)
-        else:
-            raise Refused("elementwise %s" % kind)
-        return dst
+    def _elementwise(self, call):
+        """A function (operands, dst, values by name) that computes dst = call(operands) on flat device tensors."""
+        hip, kind = self.hip, call[0]
+        coefficient = [_coefficient(c) if isinstance(c, tuple) else None for c in call]
 
-    def _buffer_op(self, s, env, owned, can_overwrite):
+        def checked(fn):
+            def go(operands, dst, env):
+                _same_size("an elementwise operation", dst, *operands)
+                fn([_flat(o) for o in operands], _flat(dst), env)
+                return dst
+            return go
+        if kind == "fill":
+            return checked(lambda o, d, env: hip.fill(d, coefficient[1](env, d)))
+        if kind == "copy":
+            return checked(lambda o, d, env: hip.copy(o[call[1]], d) if o[call[1]].data_ptr() != d.data_ptr() else None)
+        if kind == "scale":
+            return checked(lambda o, d, env: hip.axpby(coefficient[1](env, d), o[call[2]], 0.0, o[call[2]], d))
+        if kind == "mult":
+            return checked(lambda o, d, env: hip.mult(o[call[1]], o[call[2]], d))
+        if kind == "axpby":
+            return checked(lambda o, d, env: hip.axpby(coefficient[1](env, d), o[call[2]], coefficient[3](env, d), o[call[4]], d))
+        raise Refused("elementwise %s" % kind)
+
+    def _dest(self, nm, can_overwrite):
+        """A function of the values that gives the buffer a tensor operation's result goes to: the `outs` operand
+        itself where that is allowed, else a new one of its size.  What the operation reads of the operand it
+        reads from the operand."""
+        if can_overwrite(nm):
+            return lambda env: env[nm]
+        empty_like = self.torch.empty_like
+        return lambda env: empty_like(env[nm])
+
+    def _axpby_operands(self, s):
+        """(first coefficient, its operand, second coefficient, its operand, outs operand) of an a*x + b*y statement."""
+        ins, outs = _group(s.head, "ins")[0], _group(s.head, "outs")[0]
+        if s.op == "linalg.generic":
+            call = self._generic_plan(s)[1]
+            operands = ins + outs
+            return _coefficient(call[1]), operands[call[2]], _coefficient(call[3]), operands[call[4]], outs[0]
+        spec = _LINALG_NAMED[s.op]
+        return (lambda env, d: spec[1]), ins[0], (lambda env, d: spec[2]), ins[1], outs[0]
+
+    # what lapis_amd/schedule.py makes of several statements
+    def _fused_step(self, s, can_overwrite):
+        hip, op = self.hip, s.op
+        if op == "lapis.alias":
+            name, value = s.results[0], s.head.strip()
+
+            def step(env):
+                env[name] = env[value]
+            return step
+        if op == "lapis.product":
+            r = s.results[0]
+            A, x = _group(s.parts[0].head, "ins")[0]
+            dest = self._dest(s.outs, can_overwrite)
+
+            def step(env):
+                env[r] = self._csr_product(env[A], env[x], dest(env), overwrite=True)
+            return step
+        if op == "lapis.product_dot":
+            r, product = s.results[0], s.parts[0]
+            A, x = _group(product.parts[0].head, "ins")[0]
+            init = _group(s.parts[1].head, "outs")[0][0]
+            dest = self._dest(product.outs, can_overwrite)
+
+            def step(env):
+                d, x_ = dest(env), env[x]
+                _same_size("linalg.dot", x_, d)
+                env[r], env[id(s)] = self._csr_product(env[A], x_, d, dot=float(env[init]))
+            return step
+        if op == "lapis.elementwise_dot":
+            r, other = s.results[0], s.other
+            ca, a, cb, b, out = self._axpby_operands(s.parts[0])
+            init = _group(s.parts[1].head, "outs")[0][0]
+            dest = self._dest(out, can_overwrite)
+
+            def step(env):
+                d, va, vb = dest(env), env[a], env[b]
+                _same_size("an elementwise operation", d, va, vb)
+                z = None
+                if other is not None:
+                    z = env[other]
+                    _same_size("linalg.dot", d, z)
+                    z = _flat(z)
+                env[id(s)] = hip.axpby_dot_start(ca(env, d), _flat(va), cb(env, d), _flat(vb), _flat(d), z, float(env[init]))
+                env[r] = d
+            return step
+        if op == "lapis.dot_start":
+            a, b = _group(s.parts[0].head, "ins")[0]
+            init = _group(s.parts[0].head, "outs")[0][0]
+
+            def step(env):
+                va, vb = env[a], env[b]
+                _same_size("linalg.dot", va, vb)
+                env[id(s)] = hip.dot_start(_flat(va), _flat(vb), float(env[init]))
+            return step
+        if op == "lapis.dot_finish":
+            r, start = s.results[0], id(s.start)
+            f32 = re.search(r"f32\s*>\s*$", s.start.parts[-1].head) is not None
+
+            def step(env):
+                v = hip.dot_finish(env.pop(start))
+                env[r] = numpy.float32(v) if f32 else v
+            return step
+        raise Refused("the operation %s" % op)
+
+    def _buffer_step(self, s, names, can_overwrite):
         op, head = s.op, s.head
         torch, hip = self.torch, self.hip
-        result_is_tensor = bool(s.results)
-        own = lambda: owned.add(s.results[0]) if s.results else None
+        r = names[0] if names else None
         if op in ("tensor.empty", "memref.alloc", "memref.alloca", "bufferization.alloc_tensor"):
             left, ty = _rsplit_colon(head)
             i = left.index("(")
-            dyn = [self._val(env, n) for n in re.findall(_NAME, left[i:_mt._match(left, i)])]
-            dims, elem = self._sizes(ty, dyn)
-            own()
-            if not dims:
-                return [Cell(0.0)] if op.startswith("memref") else [0.0]
-            return [self._new(dims, elem)]
+            new = self._allocation(ty, re.findall(_NAME, left[i:_mt._match(left, i)]))
+            if new is None:
+                new = (lambda env: Cell(0.0)) if op.startswith("memref") else (lambda env: 0.0)
+
+            def step(env):
+                env[r] = new(env)
+            return step
         if op == "memref.dealloc":
-            return None
+            return lambda env: None
         if op == "tensor.splat":
             left, ty = _rsplit_colon(head)
-            names = re.findall(_NAME, left)
-            dims, elem = self._sizes(ty, [self._val(env, n) for n in names[1:]])
-            v = self._val(env, names[0])
-            own()
-            if not dims:
-                return [v]
-            t = self._new(dims, elem)
-            hip.fill(t.view(-1), float(v))
-            return [t]
-        if op in ("tensor.dim", "memref.dim"):
-            names = re.findall(_NAME, _split_colon(head)[0])
-            t, d = self._val(env, names[0]), self._val(env, names[1])
-            if isinstance(t, Csr):
-                return [(t.nrows, t.ncols)[d]]
-            return [int(t.shape[d])]
-        if op in ("tensor.extract", "memref.load"):
-            names = re.findall(_NAME, _split_colon(head)[0])
-            t = self._val(env, names[0])
-            idx = [self._val(env, n) for n in names[1:]]
-            if isinstance(t, Cell):
-                return [t.value]
-            if not isinstance(t, torch.Tensor):  # a zero-dimensional tensor is kept as a host scalar
-                return [t]
-            v = t[tuple(idx)].item()  # waits for the kernels that produce it
-            return [numpy.float32(v) if t.dtype == torch.float32 else v]
-        if op == "memref.store":
-            names = re.findall(_NAME, _split_colon(head)[0])
-            v, t = self._val(env, names[0]), self._val(env, names[1])
-            if isinstance(t, Cell):
-                t.value = v
-            else:
-                t[tuple(self._val(env, n) for n in names[2:])] = v
-            return None
-        if op == "memref.copy":
-            names = re.findall(_NAME, _split_colon(head)[0])
-            src, dst = self._val(env, names[0]), self._val(env, names[1])
-            if isinstance(dst, Cell):
-                dst.value = src.value
-            else:
-                dst.copy_(src)
-            return None
+            ops = re.findall(_NAME, left)
+            v, new = ops[0], self._allocation(ty, ops[1:])
 
-        ins, in_types = _group(head, "ins")
-        outs, out_types = _group(head, "outs")
+            def step(env):
+                if new is None:
+                    env[r] = env[v]
+                else:
+                    t = new(env)
+                    hip.fill(t.view(-1), float(env[v]))
+                    env[r] = t
+            return step
+        ops = re.findall(_NAME, _split_colon(head)[0])
+        if op in ("tensor.dim", "memref.dim"):
+            def step(env):
+                t, d = env[ops[0]], env[ops[1]]
+                env[r] = (t.nrows, t.ncols)[d] if isinstance(t, Csr) else int(t.shape[d])
+            return step
+        if op in ("tensor.extract", "memref.load"):
+            def step(env):
+                t = env[ops[0]]
+                if isinstance(t, Cell):
+                    env[r] = t.value
+                elif not isinstance(t, torch.Tensor):  # a zero-dimensional tensor is kept as a host scalar
+                    env[r] = t
+                else:
+                    v = t[tuple(env[n] for n in ops[1:])].item()  # waits for the kernels that produce it
+                    env[r] = numpy.float32(v) if t.dtype == torch.float32 else v
+            return step
+        if op == "memref.store":
+            def step(env):
+                v, t = env[ops[0]], env[ops[1]]
+                if isinstance(t, Cell):
+                    t.value = v
+                else:
+                    t[tuple(env[n] for n in ops[2:])] = v
+            return step
+        if op == "memref.copy":
+            def step(env):
+                src, dst = env[ops[0]], env[ops[1]]
+                if isinstance(dst, Cell):
+                    dst.value = src.value
+                else:
+                    dst.copy_(src)
+            return step
+
+        ins, _ = _group(head, "ins")
+        outs, _ = _group(head, "outs")
         if len(outs) != 1:
             raise Refused("%s with %d outputs" % (op, len(outs)))
         out_nm = outs[0]
-        out_v = self._val(env, out_nm)
-        scalar_out = not isinstance(out_v, torch.Tensor)  # a zero-dimensional tensor (host scalar) or a Cell
-        in_vals = [self._val(env, n) for n in ins]
-        in_place = not result_is_tensor  # memref semantics
-        flat = lambda t: t.reshape(-1)
+        is_tensor = lambda v: isinstance(v, torch.Tensor)  # otherwise a zero-dimensional tensor (host scalar) or a Cell
+        dest = self._dest(out_nm, can_overwrite) if r else (lambda env: env[out_nm])  # memrefs are updated in place
 
-        def dest(keep):
-            if in_place:
-                return out_v
-            own()
-            return self._dest(out_nm, env, can_overwrite, keep)
-
-        def give(t):
-            return [t] if result_is_tensor else None
+        def giving(compute):
+            """`compute(values, destination)` for an operation on tensors"""
+            def step(env):
+                d = dest(env)
+                compute(env, d)
+                if r:
+                    env[r] = d
+            return step
 
         if op == "linalg.fill":
-            if scalar_out:
-                if isinstance(out_v, Cell):
-                    out_v.value = in_vals[0]
-                    return None
-                return [in_vals[0]]
-            d = dest(False)
-            hip.fill(flat(d), float(in_vals[0]))
-            return give(d)
+            def fill(env, d):
+                hip.fill(_flat(d), float(env[ins[0]]))
+            on_tensors = giving(fill)
+
+            def step(env):
+                out = env[out_nm]
+                if is_tensor(out):
+                    on_tensors(env)
+                elif isinstance(out, Cell):
+                    out.value = env[ins[0]]
+                else:
+                    env[r] = env[ins[0]]
+            return step
         if op == "linalg.copy":
-            if scalar_out:
-                return [in_vals[0]]
-            d = dest(False)
-            if d.data_ptr() != in_vals[0].data_ptr():
-                _same_size("linalg.copy", in_vals[0], d)
-                hip.copy(flat(in_vals[0]), flat(d))
-            return give(d)
+            def copy(env, d):
+                v = env[ins[0]]
+                if d.data_ptr() != v.data_ptr():
+                    _same_size("linalg.copy", v, d)
+                    hip.copy(_flat(v), _flat(d))
+            on_tensors = giving(copy)
+
+            def step(env):
+                if is_tensor(env[out_nm]):
+                    on_tensors(env)
+                else:
+                    env[r] = env[ins[0]]
+            return step
         if op == "linalg.dot":
-            init = out_v.value if isinstance(out_v, Cell) else out_v
-            _same_size("linalg.dot", in_vals[0], in_vals[1])
-            r = hip.dot_host(flat(in_vals[0]), flat(in_vals[1]), float(init))
-            r = numpy.float32(r) if in_vals[0].element_size() == 4 else r
-            if isinstance(out_v, Cell):
-                out_v.value = r
-                return None
-            return [r]
+            a, b = ins[0], ins[1]
+
+            def step(env):
+                out, va, vb = env[out_nm], env[a], env[b]
+                _same_size("linalg.dot", va, vb)
+                v = hip.dot_host(_flat(va), _flat(vb), float(out.value if isinstance(out, Cell) else out))
+                v = numpy.float32(v) if va.element_size() == 4 else v
+                if isinstance(out, Cell):
+                    out.value = v
+                else:
+                    env[r] = v
+            return step
         plan = self._generic_plan(s) if op == "linalg.generic" else None
-        if op == "linalg.matvec" or plan == ("matvec",):
-            d = dest(True)
-            self._csr_product(in_vals[0], in_vals[1], d)
-            return give(d)
-        if op == "linalg.matmul" or plan == ("matmul",):
-            d = dest(True)
-            self._csr_product(in_vals[0], in_vals[1], d, k=int(in_vals[1].shape[1]))
-            return give(d)
+        if op in ("linalg.matvec", "linalg.matmul") or plan in (("matvec",), ("matmul",)):
+            wide = op == "linalg.matmul" or plan == ("matmul",)
+            in_place = r is None or can_overwrite(out_nm)
+
+            def step(env):
+                out, x = env[out_nm], env[ins[1]]
+                d = out if in_place else out.clone()
+                self._csr_product(env[ins[0]], x, d, k=int(x.shape[1]) if wide else None)
+                if r:
+                    env[r] = d
+            return step
         if op in _LINALG_NAMED:
             spec = _LINALG_NAMED[op]
-            d = dest(False)
-            a, b = flat(in_vals[0]), flat(in_vals[1])
-            _same_size(op, a, b, d)
-            if spec[0] == "axpby":
-                hip.axpby(spec[1], a, spec[2], b, flat(d))
-            elif spec[0] == "mult":
-                hip.mult(a, b, flat(d))
-            else:
-                hip.div(a, b, flat(d))
-            return give(d)
+
+            def named(env, d):
+                a, b = _flat(env[ins[0]]), _flat(env[ins[1]])
+                _same_size(op, a, b, d)
+                if spec[0] == "axpby":
+                    hip.axpby(spec[1], a, spec[2], b, _flat(d))
+                elif spec[0] == "mult":
+                    hip.mult(a, b, _flat(d))
+                else:
+                    hip.div(a, b, _flat(d))
+            return giving(named)
         if op == "linalg.generic":
             _, call, n_ins = plan
-            operands = in_vals + [out_v]
-            reads_out = any(isinstance(c, int) and c == n_ins for c in call[1:])
-            if scalar_out:
-                raise Refused("an elementwise linalg.generic over zero-dimensional tensors")
-            d = dest(reads_out)
-            if reads_out:
-                operands[n_ins] = d
-            self._elementwise(call, [flat(o) for o in operands], flat(d), lambda nm: self._val(env, nm))
-            return give(d)
+            apply = self._elementwise(call)
+            used = {c for c in call[1:] if isinstance(c, int)}
+
+            def generic(env, d):
+                operands = [env[n] for n in ins]
+                operands.append(env[out_nm] if n_ins in used else d)
+                apply(operands, d, env)
+            on_tensors = giving(generic)
+
+            def step(env):
+                if not is_tensor(env[out_nm]):
+                    raise Refused("an elementwise linalg.generic over zero-dimensional tensors")
+                on_tensors(env)
+            return step
         raise Refused("the operation %s" % op)
 
     # ---- loop nests the library has kernels for ----------------------------------------------------------
@@ -714,27 +956,27 @@ class Executor:
         hip = self.hip
         if n.csr_spmv:
             r = n.csr_spmv
-            y, pos, crd, val, x = (self._val(env, r[k]) for k in ("y", "pos", "crd", "val", "x"))
+            y, pos, crd, val, x = (env[r[k]] for k in ("y", "pos", "crd", "val", "x"))
             A = self._csr_for(pos, crd, val, int(y.shape[0]), int(x.shape[0]))
             self._csr_product(A, x, y)
             return None
         if n.csr_spmm:
             r = n.csr_spmm
-            C, pos, crd, val, B = (self._val(env, r[k]) for k in ("C", "pos", "crd", "val", "B"))
+            C, pos, crd, val, B = (env[r[k]] for k in ("C", "pos", "crd", "val", "B"))
             A = self._csr_for(pos, crd, val, int(C.shape[0]), int(B.shape[0]))
             self._csr_product(A, B, C, k=int(B.shape[1]))
             return None
         d = n.depth1
-        count = self._val(env, d["n"]) if d["n"] in env else int(d["n"])
-        if count < 0 or any(int(self._val(env, a).shape[0]) < count
+        count = env[d["n"]] if d["n"] in env else int(d["n"])
+        if count < 0 or any(int(env[a].shape[0]) < count
                             for a in ([d["x"], d["y"]] if d["kind"] == "dot" else list(d["arrays"]) + [d["dst"]])):
             raise ValueError("a loop over %d elements of a shorter buffer" % count)
         if d["kind"] == "dot":
-            x, y = self._val(env, d["x"])[:count], self._val(env, d["y"])[:count]
-            r = hip.dot_host(x, y, float(self._val(env, d["init"])))
+            x, y = env[d["x"]][:count], env[d["y"]][:count]
+            r = hip.dot_host(x, y, float(env[d["init"]]))
             return [numpy.float32(r) if x.element_size() == 4 else r]
-        arrays = [self._val(env, a)[:count] for a in d["arrays"]]
-        self._elementwise(d["call"], arrays, self._val(env, d["dst"])[:count], lambda nm: self._val(env, nm))
+        arrays = [env[a][:count] for a in d["arrays"]]
+        self._elementwise(d["call"])(arrays, env[d["dst"]][:count], env)
         return None
 
     def _csr_for(self, pos, crd, val, nrows, ncols):

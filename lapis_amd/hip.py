@@ -231,6 +231,13 @@ class CsrPlan:
                                             value_bytes, _stream(stream)))
         self.address = self._handle.value  # what the native calls take
 
+    @classmethod
+    def _adopt(cls, address, pos, crd):
+        """The plan object of a plan the library has made."""
+        self = cls.__new__(cls)
+        self._lib, self._handle, self.pos, self.crd, self.address = init(), _vp(address), pos, crd, address
+        return self
+
     @property
     def handle(self):
         return self._handle
@@ -396,6 +403,52 @@ def dot_noalloc(x, y, result, init_value=0.0, stream=None):
     lib = init()
     check(lib.lapis_hip_dot_f64_noalloc(int(x.shape[0]), _ptr(x), _ptr(y), init_value, _ptr(result), _stream(stream)))
     return result
+
+
+def spmv_overwrite(plan, nrows, ncols, pos, crd, val, x, y, stream=None):
+    """y = A x (y is not read)."""
+    return _calls.spmv_overwrite(plan, nrows, ncols, pos, crd, val, x, y, stream)
+
+
+# A dot product in two halves: the launch, and the wait for its value, between which other work can be launched.
+def dot_start(x, y, init_value=0.0, stream=None):
+    """The start of init + x . y, for ``dot_finish``."""
+    return _calls.dot_start(x, y, init_value, stream)
+
+
+def axpby_dot_start(a, x, b, y, dst, z, init_value=0.0, stream=None):
+    """dst = a*x + b*y and the start of init + dst . z (z None: dst . dst) in one launch."""
+    return _calls.axpby_dot_start(a, x, b, y, dst, z, init_value, stream)
+
+
+def spmv_dot_start(plan, nrows, ncols, pos, crd, val, x, y, init_value=0.0, stream=None):
+    """y = A x for a square A and the start of init + x . y, in one launch where the matrix has no long rows."""
+    return _calls.spmv_dot_start(plan, nrows, ncols, pos, crd, val, x, y, init_value, stream)
+
+
+def dot_finish(started):
+    """The value of a started dot product, as a Python float (blocking)."""
+    return _calls.dot_finish(started)
+
+
+def stage(arrays, csr=None, stream=None):
+    """Device tensors with the contents of C-contiguous numpy arrays, in memory of the library's own that is given back
+    when the last of them is gone.  ``csr`` = (index of positions, index of coordinates, rows, columns) names a matrix
+    whose structure is checked and counted on the way; -> (tensors, what ``staged_plan`` takes)."""
+    return _calls.stage(arrays, csr, stream)
+
+
+def staged_plan(staged, pos_index, crd_index, pos, crd, value_bytes):
+    """The plan of a matrix brought over by ``stage``."""
+    return CsrPlan._adopt(_calls.staged_plan(staged, pos_index, crd_index, value_bytes), pos, crd)
+
+
+def fetch(tensor, stream=None):
+    """A new numpy array with a device tensor's elements."""
+    import numpy
+    tensor = tensor.contiguous()
+    out = numpy.empty(tuple(tensor.shape), dtype=str(tensor.dtype).split(".")[-1])
+    return _calls.fetch(tensor, out, stream)
 
 
 def axpby(a, x, b, y, dst, stream=None):
