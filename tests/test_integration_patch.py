@@ -26,7 +26,7 @@ def _new_files(patch_text):
     return files
 
 
-@pytest.mark.skipif(not (os.path.isdir(REFERENCE) and shutil.which("patch")),
+@pytest.mark.skipif(not (os.path.isdir(os.path.join(REFERENCE, "mlir")) and shutil.which("patch")),
                     reason="needs the reference tree and the patch tool on this machine")
 def test_patch_applies_cleanly_to_the_reference_tree():
     proc = subprocess.run(["patch", "--dry-run", "-p1", "-d", REFERENCE, "-i", PATCH], capture_output=True, text=True)

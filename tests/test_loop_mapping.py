@@ -43,7 +43,7 @@ def test_own_worded_nests_map_as_the_reference_gold_says(name):
     assert hints == want["hints"]
 
 
-@pytest.mark.skipif(not os.path.isdir(REFERENCE), reason="the reference tree is not on this machine")
+@pytest.mark.skipif(not os.path.isdir(os.path.join(REFERENCE, "tests")), reason="the reference tree is not on this machine")
 @pytest.mark.parametrize("k", range(4))
 def test_reference_inputs_map_to_reference_golds(k):
     base = os.path.join(REFERENCE, "tests", "Dialect", "Kokkos", "loop_mapping_%d.mlir" % k)
