@@ -282,19 +282,25 @@ __global__ __launch_bounds__(1024) void spmm_rowblock_lds_kernel(int nrows, int 
 // as the reference's nest does.  A wavefront stages the coordinates and the values of its rows in LDS, `window`
 // entries of every row at a time; up to 4 rows of V are asked for before the first is added.
 // HV: nh is a multiple of 4, so a lane's four values are neighbours, one 128-bit LDS read.
+// All coordinates and values of a window are asked for at once, values four at a time; the stretches of two rows lie
+// kRowPad floats apart, since the lanes of all groups read the same entry of their row together, which without the
+// padding is the same bank; and seven wavefronts per SIMD (six where nh is no multiple of 4) keep enough rows of V in
+// flight (eight rows per lane instead of four: no faster, and twice as slow where they cost the wavefronts).
 // Measured at 16384 rows of 32, dh = 32, nh = 8: 195 us with a wavefront per row that read each value and coordinate
-// from global memory for every 64 columns, 59 us now (7.3 TB/s of rows of V that miss L2); with twice the LDS 69.
+// from global memory for every 64 columns, 47 us now (11.5 TB/s of rows of V, half of them from L2).
 constexpr int kStagedBatched = 1024;        // values per wavefront and window
 constexpr int kStagedBatchedEntries = 256;  // non-zeros per wavefront and window at most
+constexpr int kRowPad = 8;  // floats between the stretches of two rows
+constexpr int kCoords = kStagedBatchedEntries / 64, kVectors = kStagedBatched / 256;  // of a lane per window
 constexpr int kBatchedGroups = 8;           // rows per wavefront at most: rows are long against narrow chunks
 template <bool HV, bool WIDE>
-__global__ __launch_bounds__(256) void bspmm_csrv_kernel(int n1, SpmmShape sh, int nh, int window_log2,
+__global__ __launch_bounds__(256, HV ? 7 : 6) void bspmm_csrv_kernel(int n1, SpmmShape sh, int nh, int window_log2,
                                                          const int *__restrict__ pos, const int *__restrict__ crd,
                                                          const float *__restrict__ val, const float *__restrict__ V,
                                                          float *__restrict__ out) {
   typedef RowVec<float>::loose W;
-  __shared__ __align__(16) float s_val[4][kStagedBatched];
-  __shared__ unsigned s_off[4][kStagedBatchedEntries];
+  __shared__ __align__(16) float s_val[4][kStagedBatched + kBatchedGroups * kRowPad];
+  __shared__ unsigned s_off[4][kStagedBatchedEntries + kBatchedGroups];
   const unsigned nblocks = (unsigned)sh.row_blocks * (unsigned)sh.chunks, id = linear_block();
   if (id >= nblocks) return;
   unsigned block = xcd_contiguous_block(id, nblocks);
@@ -319,31 +325,56 @@ __global__ __launch_bounds__(256) void bspmm_csrv_kernel(int n1, SpmmShape sh, i
   float *op = out + (row0 + group) * K + col;
   W acc = {};
   if (writes) acc = *reinterpret_cast<const W *>(op);
-  const int slots = sh.groups << window_log2;
   int done = 0;                                      // entries of each row already taken
   const int mine = group < rows_here ? pe - ps : 0;  // entries of this lane's row
+  // What a lane stages of every window (all lanes run every trip: the shuffles need their source lanes active):
+  // coordinate slot j = entry done + j % window of row j / window, and four values at a time, vector q = floats 4 rest..
+  // of the stretch of row q / per_row.
+  const int slots = sh.groups << window_log2, per_row = ((nh << window_log2) + 3) >> 2;
+  const unsigned per_row_inv = (1u << 22) / (unsigned)per_row + 1;  // q * inv >> 22 == q / per_row for q, per_row <= 1024
   while (__ballot(done < mine)) {
-    // slot j: entry done + j % window of row j / window (its first entry and length sit in that row's lanes)
-    // (all lanes run every trip: the shuffles need their source lanes active)
-    for (int j0 = 0; j0 < slots; j0 += 64) {
-      const int j = j0 + lane;
-      const int from = min((j >> window_log2) * sh.lpr, 63);
-      const int at = done + (j & (window - 1));
+    // (every lane runs every step: the shuffles need their source lanes active)
+    unsigned c[kCoords];
+    W v[kVectors] = {};
+    int ln = lane;
+    asm volatile("" : "+v"(ln));  // the slots' numbers are worked out again in every window: kept, they cost 30 registers
+#pragma unroll
+    for (int i = 0; i < kCoords; ++i) {
+      const int j = i * 64 + ln, from = min((j >> window_log2) * sh.lpr, 63), at = done + (j & (window - 1));
       const int first = __shfl(ps, from, 64), count = __shfl(mine, from, 64);
-      if (j < slots && at < count) {
-        const unsigned c = (unsigned)load_stream(crd + first + at);
-        woff[j] = WIDE ? c : c * (unsigned)(K * 4);
+      c[i] = 0;
+      if (j < slots && at < count) c[i] = (unsigned)load_stream(crd + first + at);
+    }
+#pragma unroll
+    for (int i = 0; i < kVectors; ++i) {
+      const unsigned q = i * 64 + ln, row = (q * per_row_inv) >> 22;
+      const int rest = 4 * (int)(q - row * per_row), from = min((int)row * sh.lpr, 63);
+      const int first = __shfl(ps, from, 64), count = __shfl(mine, from, 64);
+      const int floats = min(count - done, window) * nh - rest;  // of the row's stretch from here on
+      const float *vp = val + ((long long)first + done) * nh + rest;
+      if ((int)row < sh.groups) {
+        if (HV || floats >= 4) {
+          if (floats > 0) v[i] = *reinterpret_cast<const W *>(vp);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 3; ++e) v[i][e] = e < floats ? vp[e] : 0.0f;
+        }
       }
     }
-    for (int g = 0; g < sh.groups; ++g) {  // a row's values of a window are one contiguous stretch
-      const int first = __shfl(ps, g * sh.lpr, 64), count = min(__shfl(mine, g * sh.lpr, 64) - done, window);
-      const float *vp = val + ((long long)first + done) * nh;
-      for (int i = lane; i < count * nh; i += 64) wval[(g << window_log2) * nh + i] = vp[i];
+#pragma unroll
+    for (int i = 0; i < kCoords; ++i) {
+      const int j = i * 64 + ln;
+      if (j < slots) woff[j + (j >> window_log2)] = WIDE ? c[i] : c[i] * (unsigned)(K * 4);
+    }
+#pragma unroll
+    for (int i = 0; i < kVectors; ++i) {
+      const unsigned q = i * 64 + ln, row = (q * per_row_inv) >> 22;
+      if ((int)row < sh.groups) *reinterpret_cast<v4f *>(wval + q * 4 + row * kRowPad) = v[i];
     }
     wave_lds_sync();
     const int hi = min(mine - done, window);
-    const unsigned *goff = woff + (group << window_log2);
-    const float *gval = wval + (group << window_log2) * nh;
+    const unsigned *goff = woff + (group << window_log2) + group;
+    const float *gval = wval + (group << window_log2) * nh + group * kRowPad;
     int t = 0;
     auto batch = [&](auto unr) {
       constexpr int UNR = decltype(unr)::value;
@@ -627,9 +658,22 @@ extern "C" int lapis_hip_bspmm_csrv_f32_i32(int64_t n1, int64_t n2, int64_t dh, 
     LAPIS_LAUNCH_CHECK();
     return LAPIS_HIP_OK;
   }
-  // As many columns of a row per group as there are (narrower chunks, whose part of V an XCD's L2 would hold,
-  // stage the same entries once per chunk: 117 us against 59 at 32 columns).
-  SpmmShape shape = make_shape(n1, K, 4, (int)std::min<int64_t>(64, ceil_div(K, 4)), 1, 1);
+  // As many columns of a row per group as there are, 256 at most, except where an XCD's 4 MB of L2 hold more of a part
+  // of V than of the whole: 512 bytes per part, 256 where the row is no multiple of 1024, so that the parts of the XCDs'
+  // rows still lie on every channel of L2.  us, 16 384 rows of 32, in 64 / 32 / 16 vectors per part:
+  //   K = 192, nh = 3: 45 / 42 / 33    K = 256, nh = 8: 56 / 47 / 53    K = 320, nh = 8: 69 / 65 / 59
+  //   K = 384, nh = 4: 82 / 65 / 60    K = 512, nh = 8: 110 / 83 / 92   K = 1024, nh = 8: 227 / 171 / 180
+  // Not for rows that are no multiple of 256 bytes (parts begin inside a line, which is fetched twice: K = 200: 58.0, in
+  // two 56.7), nor where a part is beyond 16 MB (60 000 rows of 6, K = 256: 67, in two 70) or the whole within 8 MB
+  // (6000 rows of 32, K = 320: 24, in five 29), nor where a window would hold fewer than 32 entries of a row.
+  int vectors = (int)std::min<int64_t>(64, ceil_div(K, 4));
+  const double v_bytes = (double)n2 * (double)K * sizeof(float);
+  if (K % 64 == 0 && K >= 192) {
+    const int part = K % 256 ? 16 : 32;
+    if (v_bytes > 8388608.0 && v_bytes * part <= 16777216.0 * (double)(K / 4) && nh * (64 / part) * 32 <= kStagedBatched)
+      vectors = part;
+  }
+  SpmmShape shape = make_shape(n1, K, 4, vectors, 1, 1);
   // at least 4 entries of every row per window
   const int slots = (int)std::min<int64_t>(kStagedBatchedEntries, kStagedBatched / nh);
   shape.groups = std::max(1, std::min({shape.groups, kBatchedGroups, slots / 4}));
@@ -640,7 +684,7 @@ extern "C" int lapis_hip_bspmm_csrv_f32_i32(int64_t n1, int64_t n2, int64_t dh, 
   if (blocks > 0x7fffffffLL)
     return set_error(LAPIS_HIP_ERR_INVALID_ARGUMENT, "bspmm_csrv: %lld rows of %lld elements exceed the grid limit",
                      (long long)n1, (long long)K);
-  const bool wide = (double)n2 * (double)K * sizeof(float) >= 4294967296.0;
+  const bool wide = v_bytes >= 4294967296.0;
 #define LAPIS_BSPMM_LAUNCH(HV, WIDE)                                                                                  \
   hipLaunchKernelGGL((bspmm_csrv_kernel<HV, WIDE>), grid_of(blocks), dim3(256), 0, st, (int)n1, shape, (int)nh,             \
                      window_log2, pos, crd, val, V, out)

@@ -63,3 +63,18 @@ def test_batched_csrv_product_shapes(gpu, oracle, dh, nh):
     print("case", dh, nh, flush=True)
     gpu.bspmm_csrv(A.nrows, 400, dev(A.pos), dev(A.crd), dev(values), dev(V), out)
     assert np.array_equal(out.cpu().numpy(), oracle.bspmm_csrv(A.pos, A.crd, values, V, A.nrows))
+
+
+@pytest.mark.parametrize("n2,dh,nh", [(11000, 64, 3), (11000, 12, 16), (8400, 32, 8), (8100, 32, 8), (7000, 40, 8), (7000, 40, 9),
+                                      (5000, 128, 4), (4200, 64, 9), (17000, 32, 8), (33000, 32, 8)])
+def test_batched_csrv_product_in_parts_of_a_row_of_V(gpu, oracle, n2, dh, nh):
+    # V on both sides of 8 MB and of 16 MB a part, rows of an even and an odd number of 256 bytes, windows of 32 and more
+    # entries and (too many heads) the general path; row lengths around the windows
+    rng = np.random.default_rng(n2 + nh)
+    A = from_lengths(list(np.concatenate([rng.integers(0, 70, 150), [0, 31, 32, 33, 63, 64, 65, 0, 300]])), n2, 18, np.float32)
+    values = rng.uniform(-1, 1, A.nnz * nh).astype(np.float32)
+    V = rng.uniform(-1, 1, (n2, dh, nh)).astype(np.float32)
+    out = torch.zeros(A.nrows, dh, nh, dtype=torch.float32, device="cuda")
+    print("case", n2, dh, nh, flush=True)
+    gpu.bspmm_csrv(A.nrows, n2, dev(A.pos), dev(A.crd), dev(values), dev(V), out)
+    assert np.array_equal(out.cpu().numpy(), oracle.bspmm_csrv(A.pos, A.crd, values, V, A.nrows))  # the order of the reference's nest: bit-exact
