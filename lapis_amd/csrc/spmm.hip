@@ -36,15 +36,16 @@ struct RowVec<double> {
 //   `lpr` lanes cover the chunk of a row of B, so the group takes `par` non-zeros of its row per step.
 struct SpmmShape {
   int chunks;      // column chunks
-  int vectors;     // whole vectors in a row of B
   int k;
+  int chunk_width, wider;  // vectors of a chunk, and how many of the first chunks have one more
   int lpr, par;
+  unsigned lpr_inv, group_inv;  // 65536 / lpr + 1, 65536 / (lpr * par) + 1: a lane's number divided without a division
   int groups;      // 64 / (lpr * par)
   int row_blocks;  // workgroups per chunk
   int xcd_map;
   template <int VW>
   __device__ __forceinline__ int chunk_first(int c) const {
-    return c >= chunks ? k : VW * (int)(((long long)vectors * c) / chunks);
+    return c >= chunks ? k : VW * (c * chunk_width + min(c, wider));
   }
 };
 
@@ -72,11 +73,15 @@ __device__ __forceinline__ double lane_get(int byte_of_lane, double v) {
 // What bounds short rows is the chain of dependent loads of a wavefront (positions, entries, rows of B, row of
 // C), not bandwidth: staging makes it one trip per wavefront instead of one per LPR entries, and the row of C
 // is asked for first.  Measured (us; entries handed round by bpermute, LPR or 64 per trip -> staged):
-//   7-point 97^3, fp64   k = 3: 316 -> 35   k = 10: 392 -> 72   k = 64: 409 -> 369
+//   7-point 97^3, fp64   k = 3: 316 -> 35   k = 10: 392 -> 68   k = 64: 409 -> 369
 //   27-point x 3, 30^3   k = 3 fp64: 48 -> 31   k = 10 fp32: 57 -> 34   k = 64 fp32: 82 -> 73
 //   random, 32 per row, 15 000 rows, k = 10 fp32: 9.9 -> 7.7; 1 M rows, k = 64 fp32 (rows of B from HBM): 1217 -> 1203
 // WIDE: B is 4 GB or more and the offsets take 64 bits.
-constexpr int kStaged = 512;  // entries per wavefront: 24 KB (fp64) per workgroup, six workgroups to a CU
+// Entries per wavefront and window: 384, 18 KB per workgroup in fp64, and registers for seven wavefronts per SIMD
+// (against 512 entries and 76 registers, six wavefronts: 7-point 97^3 fp64, k = 10: 75 us -> 68, k = 33: 228 -> 207;
+// 27-point x 3, 30^3, k = 10: 45 -> 38; scattered columns in an L2-sized B, 100 000 rows of 60, k = 33 fp64, pay 2 %:
+// 226 -> 232; registers for eight spill: 88 at the first).
+constexpr int kStaged = 384;
 template <typename T, int VW, int DEPTH, bool WIDE>
 __device__ __forceinline__ void spmm_rows_body(int nrows, const SpmmShape &sh, const int *__restrict__ pos,
                                                const int *__restrict__ crd, const T *__restrict__ val,
@@ -99,8 +104,8 @@ __device__ __forceinline__ void spmm_rows_body(int nrows, const SpmmShape &sh, c
   T *wval = s_val[wave];
   unsigned *woff = s_off[wave];
   const int gs = sh.lpr * sh.par;
-  const int group = lane / gs, sub = lane - group * gs;
-  const int e = sub / sh.lpr, l = sub - e * sh.lpr;
+  const int group = (lane * sh.group_inv) >> 16, sub = lane - group * gs;
+  const int e = (sub * sh.lpr_inv) >> 16, l = sub - e * sh.lpr;
   const long long row0 = ((long long)block * 4 + wave) * sh.groups;
   if (row0 >= nrows) return;
   const int rows_here = (int)min((long long)sh.groups, nrows - row0);
@@ -193,7 +198,7 @@ __global__ __launch_bounds__(256) void spmm_wave_row_kernel(int nrows, SpmmShape
   spmm_rows_body<T, VW, DEPTH, WIDE>(nrows, shape, pos, crd, val, B, ldb, C, ldc);
 }
 template <typename T, int VW, int DEPTH, bool WIDE>
-__global__ __launch_bounds__(256) void spmm_group_row_kernel(int nrows, SpmmShape shape, const int *__restrict__ pos,
+__global__ __launch_bounds__(256, 7) void spmm_group_row_kernel(int nrows, SpmmShape shape, const int *__restrict__ pos,
                                                              const int *__restrict__ crd, const T *__restrict__ val,
                                                              const T *__restrict__ B, long long ldb, T *__restrict__ C,
                                                              long long ldc) {
@@ -310,7 +315,7 @@ __global__ __launch_bounds__(256, HV ? 7 : 6) void bspmm_csrv_kernel(int n1, Spm
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   unsigned *woff = s_off[wave];
   float *wval = s_val[wave];
-  const int group = lane / sh.lpr, l = lane - group * sh.lpr;
+  const int group = (lane * sh.lpr_inv) >> 16, l = lane - group * sh.lpr;
   const long long row0 = ((long long)block * 4 + wave) * sh.groups;
   if (row0 >= n1) return;
   const int rows_here = (int)min((long long)sh.groups, n1 - row0);
@@ -445,14 +450,18 @@ struct SpmmArgs {
 inline SpmmShape make_shape(int64_t nrows, int64_t k, int vw, int vectors_max, int par, int xcd_map) {
   SpmmShape s;
   s.k = (int)k;
-  s.vectors = (int)(k / vw);
+  const int vectors = (int)(k / vw);
   const int rest = k % vw != 0;
-  s.chunks = (int)ceil_div(s.vectors + rest, vectors_max);
-  while (ceil_div(s.vectors, s.chunks) + rest > vectors_max) ++s.chunks;
-  s.lpr = (int)ceil_div(s.vectors, s.chunks) + rest;
+  s.chunks = (int)ceil_div(vectors + rest, vectors_max);
+  while (ceil_div(vectors, s.chunks) + rest > vectors_max) ++s.chunks;
+  s.lpr = (int)ceil_div(vectors, s.chunks) + rest;
+  s.chunk_width = vectors / s.chunks;
+  s.wider = vectors % s.chunks;
   s.par = par;
   while (s.par > 1 && s.lpr * s.par > 64) s.par /= 2;
   s.groups = 64 / (s.lpr * s.par);
+  s.lpr_inv = 65536 / s.lpr + 1;
+  s.group_inv = 65536 / (s.lpr * s.par) + 1;
   s.row_blocks = (int)ceil_div(nrows, 4 * s.groups);
   s.xcd_map = xcd_map;
   return s;

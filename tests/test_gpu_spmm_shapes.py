@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 def test_ragged_widths_on_short_and_long_rows(gpu, oracle, dtype, k):
     rng = np.random.default_rng(k)
     short = rng.integers(0, 12, 777)                                     # several rows per wavefront
-    long = np.concatenate([rng.integers(90, 240, 37), [0, 511, 512, 513, 0]])  # windows of 512 entries cut inside rows
+    long = np.concatenate([rng.integers(90, 240, 37), [0, 383, 384, 385, 0, 768]])  # windows of 384 entries cut inside rows
     for lengths, ncols in ((short, 500), (long, 3000)):
         A = from_lengths(list(lengths), ncols, 7 + k, dtype)
         B = gen.uniform_matrix(ncols, k, 8).astype(dtype)
