@@ -9,13 +9,16 @@
 // (first row, first entry) of chunk c: with it a wavefront asks for its positions, values, coordinates and
 // its part of y at once, then gathers x, then adds up -- three dependent latencies.
 //
-// Bound by memory: the matrix is streamed once.  Measured on MI355X, kernel time against the row-block and
-// row-split kernels it replaces, and the time of the bare bytes at the rate of a large copy (6.1 TB/s):
-//   5-point grid 1000^2    fp64  19.1 ->  14.9 us (14.4)    fp32  15.4 -> 10.4 us ( 9.2)
-//   7-point grid 100^3     fp64  24.1 ->  21.0 us (18.2)    fp32  19.3 -> 13.0 us (11.7)
-//   7-point grid 192^3     fp64   148 ->   142 us (130)     fp32   107 ->   97 us ( 83)
-//   27-node mesh of 20^3   fp64  27.9 ->   6.9 us ( 3.6)    fp32  26.1 ->  6.3 us ( 2.4)
-//   27-node mesh of 60^3   fp64   131 ->   120 us (103)     fp32   100 ->   88 us ( 68)
+// Bound by memory: the matrix is streamed once.  Measured on MI355X: the row-block and row-split kernels it replaces, then
+// with vectors of 16 bytes of entries per lane and guarded loads, then as it is (a lane takes every 64th entry, no load is
+// conditional), and the time of the bare bytes at the rate of a large copy (6.1 TB/s), us:
+//   5-point grid 1000^2    fp64  19.1  15.5  14.1 (14.4)
+//   7-point grid 100^3     fp64  24.1  18.6  17.3 (18.2)    fp32  19.3  13.9  13.6 (11.7)
+//   7-point grid 180^3     fp64         120   117 (107)     fp32         80    77 ( 68)
+//   27-node mesh of 35^3   fp64        23.7  19.4 (20.3)    fp32        21.1  14.7 (13.6)
+//   27-node mesh of 60^3   fp64   131   124   113 (103)     fp32   100   88    76 ( 68)
+// (below the bare bytes where the last-level cache holds the matrix from one call to the next).  With four neighbouring
+// entries in a lane the lanes of a gather are four entries apart and touch that many more lines.
 // Tried and not kept: staging columns and values in LDS and gathering x in the row phase (40 to 50 % slower: the
 // gathers have to be issued right behind the loads), and 16-bit coordinates per chunk (fp64 slower, fp32 a few
 // percent faster: not worth a second copy of the coordinates).
@@ -26,23 +29,6 @@
 #include "plan.hpp"
 
 namespace lapis {
-
-template <typename T>
-struct Lanes;  // entries a lane takes per step: 16 bytes of values
-template <>
-struct Lanes<double> {
-  static constexpr int per = 2;
-  typedef double vals __attribute__((ext_vector_type(2), aligned(8)));
-  typedef int cols __attribute__((ext_vector_type(2), aligned(4)));
-  typedef v2d lds;
-};
-template <>
-struct Lanes<float> {
-  static constexpr int per = 4;
-  typedef float vals __attribute__((ext_vector_type(4), aligned(4)));
-  typedef int cols __attribute__((ext_vector_type(4), aligned(4)));
-  typedef v4f lds;
-};
 
 // buf[lo..hi) with stride `step`, in ascending order, four reads in flight
 template <typename T>
@@ -61,12 +47,10 @@ __device__ __forceinline__ T sum_strided(const T *buf, int lo, int hi, int step)
 
 template <typename T, int CAP, int WAVES, bool NT>
 __global__ __launch_bounds__(64 * WAVES) void spmv_rowchunk_kernel(
-    int nnz, int nchunks, const v2i *__restrict__ desc, const int *__restrict__ pos, const int *__restrict__ crd,
+    int nchunks, const v2i *__restrict__ desc, const int *__restrict__ pos, const int *__restrict__ crd,
     const T *__restrict__ val, const T *__restrict__ x, T *__restrict__ y, int accumulate, int contiguous,
     double *__restrict__ xy_partials, int to_host, const unsigned long long *__restrict__ skip) {
-  typedef Lanes<T> L;
-  constexpr int PER = L::per;
-  constexpr int STEPS = CAP / (64 * PER);
+  constexpr int STEPS = CAP / 64;
   __shared__ __align__(16) T lds[WAVES * CAP];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -102,41 +86,20 @@ __global__ __launch_bounds__(64 * WAVES) void spmv_rowchunk_kernel(
       if (accumulate) yr = y[r];
       if (xy_partials) xr = x[r];
     }
-    // values and columns of the chunk
-    typename L::vals v[STEPS];
-    int col[STEPS][PER];
-    if ((long long)e0 + CAP <= nnz) {
-#pragma unroll
-      for (int s = 0; s < STEPS; ++s) {
-        const int k = (s * 64 + lane) * PER;
-        if (k < count) {
-          v[s] = ldv<NT>(reinterpret_cast<const typename L::vals *>(val + e0 + k));
-          const typename L::cols w = ldv<NT>(reinterpret_cast<const typename L::cols *>(crd + e0 + k));
-#pragma unroll
-          for (int i = 0; i < PER; ++i) col[s][i] = w[i];
-        }
-      }
-    } else {  // the arrays may end inside the last chunks
-#pragma unroll
-      for (int s = 0; s < STEPS; ++s) {
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-          const int k = (s * 64 + lane) * PER + i;
-          v[s][i] = k < count ? val[e0 + k] : T(0);
-          col[s][i] = k < count ? crd[e0 + k] : 0;
-        }
-      }
-    }
+    // Values and columns of the chunk, entry by entry: neighbouring lanes take neighbouring entries, whose x mostly share
+    // lines, and slots past the end repeat the last entry, so that no load waits behind a condition.  (A chunk of empty
+    // rows reads an entry of its neighbour's.)
+    const int eb = count > 0 ? e0 : max(e0 - 1, 0), kmax = max(count - 1, 0);
+    T v[STEPS];
+    int col[STEPS];
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) {
-      const int k = (s * 64 + lane) * PER;
-      if (k < count) {
-        typename L::lds pr;
-#pragma unroll
-        for (int i = 0; i < PER; ++i) pr[i] = v[s][i] * x[col[s][i]];
-        *reinterpret_cast<typename L::lds *>(buf + k) = pr;
-      }
+      const int k = min(s * 64 + lane, kmax);
+      v[s] = ldv<NT>(val + eb + k);
+      col[s] = ldv<NT>(crd + eb + k);
     }
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) buf[s * 64 + lane] = v[s] * x[col[s]];
     wave_lds_sync();
     for (int g = r0;;) {
       T acc = sum_strided(buf, ps - e0 + sub, pe - e0, 1 << shift);
@@ -203,32 +166,36 @@ int build_rowchunk(lapis_hip_csr_plan *p, int value_bytes, hipStream_t st) {
   // are left to the row-split kernel unless none is long (2425 power-law rows of up to 256: 16 us here, 5 there).
   if (s.nnz == 0 || s.max_row_len > kRowchunkLongestRow) return LAPIS_HIP_OK;
   if (s.max_row_len > 64 && s.max_row_len > 3.0 * s.mean_row_len) return LAPIS_HIP_OK;
-  // 256 entries per wavefront, 4 wavefronts per workgroup: the most loads in flight for the LDS they take (512:
-  // +2 to +7 %, 1024: +20 to +35 % in fp64).  Long rows in fp32 have half the bytes per entry and fewer rows per
-  // byte: 1024 gains 3 % on the large meshes and costs nothing on the small ones.  A chunk's rows fill it less
-  // well the longer they are, so the longest stays within a quarter of it.
-  int cap = value_bytes == 4 && s.mean_row_len >= 32.0 ? 1024 : 256;
+  // Entries per wavefront, 4 wavefronts per workgroup.  A matrix the 256 MB last-level cache holds: 256 in fp64 (512:
+  // +3 % in CG on 1024^2), 512 in fp32 (7-point 152^3: 39.1 us against 41.6).  From HBM more of it is asked for at once:
+  // 512 (7-point 180^3: 116.9 us against 118.4 in fp64, 76.5 against 79.2 in fp32), 1024 where rows are long (27-node
+  // mesh 60^3: 114 us against 125 in fp64, 77 against 80 in fp32; in cache, at 35^3, it loses: 21.2 against 19.3).
+  // A chunk's rows fill it less well the longer they are, so the longest stays within a quarter of it.
+  const bool cached = s.nnz * (value_bytes + 4) <= (256ll << 20);
+  int cap = !cached && s.mean_row_len >= 32.0 ? 1024 : cached && value_bytes == 8 ? 256 : 512;
   while (cap < 4 * s.max_row_len) cap *= 2;
   p->rowchunk_weight = (int)((int64_t)cap * (s.max_row_len + 1) / s.max_row_len - s.max_row_len);
   p->rowchunk_n = (int)((s.nnz + s.nrows) / p->rowchunk_weight + 1);
   LAPIS_HIP_TRY(hipMalloc(&p->rowchunk_desc, sizeof(v2i) * ((size_t)p->rowchunk_n + 1)));
   p->rowchunk_cap = cap;
-  // Every XCD a contiguous run of chunks while the matrix stays within half of the 256 MB last-level cache: the
-  // parts of x that neighbours share are read into one L2 instead of eight (-4 to -12 %).  A larger matrix comes
-  // from HBM, which eight distant streams suit less than one moving window (+6 to +10 %): round-robin there.
-  p->rowchunk_contiguous = s.nnz * (value_bytes + 4) <= (128ll << 20);
+  // Every XCD a contiguous run of chunks while the last-level cache holds the matrix: the parts of x that neighbours share
+  // are read into one L2 instead of eight (7-point 130^3 fp64, 184 MB: 33.7 us against 44.7; grid 1500^2 27.5 against
+  // 32.1).  A larger matrix comes from HBM, which eight distant streams suit less than one moving window (mesh 50^3
+  // fp64, 350 MB: 74.5 us against 72.8): round-robin there.
+  p->rowchunk_contiguous = cached;
   hipLaunchKernelGGL(rowchunk_desc_kernel, dim3((unsigned)ceil_div(s.nrows + 1, 256)), dim3(256), 0, st, (int)s.nrows,
                      p->rowchunk_weight, p->rowchunk_n, p->pos, static_cast<v2i *>(p->rowchunk_desc));
   LAPIS_LAUNCH_CHECK();
   return LAPIS_HIP_OK;
 }
 
-// Workgroups of a product that also sums x . y.  Up to 16 384 groups of chunks, 2048 workgroups take several in turn
-// (32 to 36 us at 120^3 either way); beyond, workgroups that stay drift apart and the front that moves through memory
-// frays (192^3: 161 us against 138 with a workgroup per group), and the caller adds up more partial sums instead.
+// Workgroups of a product that also sums x . y.  In cache, up to 16 384 groups of chunks, 2048 workgroups take several in
+// turn; beyond, and from HBM, workgroups that stay drift apart and the front that moves through memory frays (CG, 100
+// iterations: 140^3 8.87 ms against 8.37 with a workgroup per group, 164^3 14.6 against 13.6), and the caller adds up
+// more partial sums instead.
 int rowchunk_xy_blocks(const lapis_hip_csr_plan *p) {
   const int64_t groups = ceil_div(p->rowchunk_n, 4);
-  return (int)(groups <= 16384 ? std::min<int64_t>(groups, 2048) : groups);
+  return (int)(p->rowchunk_contiguous && groups <= 16384 ? std::min<int64_t>(groups, 2048) : groups);
 }
 
 template <typename T, int CAP>
@@ -239,7 +206,7 @@ int launch_rowchunk_cap(const lapis_hip_csr_plan *p, const int *crd, const T *va
   int64_t blocks = ceil_div(p->rowchunk_n, kWaves);
   if (count) *count = (int)(blocks = rowchunk_xy_blocks(p));
   auto kernel = p->nontemporal ? spmv_rowchunk_kernel<T, CAP, kWaves, true> : spmv_rowchunk_kernel<T, CAP, kWaves, false>;
-  launch_timed(kernel, dim3((unsigned)blocks), dim3(64 * kWaves), st, (int)p->stats.nnz, p->rowchunk_n,
+  launch_timed(kernel, dim3((unsigned)blocks), dim3(64 * kWaves), st, p->rowchunk_n,
                (const v2i *)p->rowchunk_desc, p->pos, crd, val, x, y, accumulate, (int)p->rowchunk_contiguous,
                xy_partials, (int)to_host, skip);
   LAPIS_LAUNCH_CHECK();

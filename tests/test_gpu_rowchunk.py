@@ -48,7 +48,7 @@ def test_chunks_of_whole_rows(gpu, oracle, name, dtype):
 
 
 def test_matrices_on_both_sides_of_the_last_level_cache_rule(gpu, oracle):
-    for n in (1200, 1600):  # 86 MB and 154 MB of matrix: contiguous chunks per XCD, then round-robin
+    for n in (1600, 2200):  # 154 MB and 290 MB of matrix: contiguous chunks per XCD, then round-robin
         A = gen.laplace2d(n)
         x = gen.uniform_vector(A.ncols, 3)
         want = np.zeros(A.nrows)
@@ -60,8 +60,8 @@ def test_matrices_on_both_sides_of_the_last_level_cache_rule(gpu, oracle):
         assert_rows_close(y.cpu().numpy(), want, scale, np.float64, "grid %d" % n)
 
 
-# more workgroups than partial sums every block adds up itself (1600^2), fewer (900), a single short chunk (3)
-@pytest.mark.parametrize("nx,iters", [(3, 2), (901, 1), (901, 2), (901, 3), (901, 4), (1600, 3)])
+# a workgroup per group of chunks (1900^2), workgroups that take several (1600, 901), a single short chunk (3)
+@pytest.mark.parametrize("nx,iters", [(3, 2), (901, 1), (901, 2), (901, 3), (901, 4), (1600, 3), (1900, 3)])
 @pytest.mark.parametrize("preconditioned", [False, True])
 def test_cg_leaves_after_odd_and_even_passes(gpu, oracle, monkeypatch, nx, iters, preconditioned):
     monkeypatch.setenv("LAPIS_HIP_CG_SPINS", "0")  # systems that would be solved in one launch take the passes too
