@@ -45,6 +45,8 @@ __device__ __forceinline__ T sum_strided(const T *buf, int lo, int hi, int step)
   return acc;
 }
 
+constexpr int kLongPart = 32;  // entries per lane from which the whole wavefront takes a row
+
 template <typename T, int CAP, int WAVES, bool NT>
 __global__ __launch_bounds__(64 * WAVES) void spmv_rowchunk_kernel(
     int nchunks, const v2i *__restrict__ desc, const int *__restrict__ pos, const int *__restrict__ crd,
@@ -102,8 +104,19 @@ __global__ __launch_bounds__(64 * WAVES) void spmv_rowchunk_kernel(
     for (int s = 0; s < STEPS; ++s) buf[s * 64 + lane] = v[s] * x[col[s]];
     wave_lds_sync();
     for (int g = r0;;) {
-      T acc = sum_strided(buf, ps - e0 + sub, pe - e0, 1 << shift);
+      const int lo = ps - e0, hi = pe - e0;
+      unsigned long long longs = __ballot((hi - lo) >> shift > kLongPart);
+      T acc = sum_strided(buf, lo + sub, (hi - lo) >> shift > kLongPart ? lo : hi, 1 << shift);
       for (int o = 1; o < (1 << shift); o <<= 1) acc = acc + __shfl_xor(acc, o, 64);
+      while (longs) {  // rows much longer than their lanes' share of the wavefront: all of it adds them up, row by row
+        const int src = __builtin_ctzll(longs);
+        longs &= ~(((1ull << (1 << shift)) - 1) << src);
+        const int lhi = __shfl(hi, src, 64);
+        T part = T(0);
+        for (int j = __shfl(lo, src, 64) + lane; j < lhi; j += 64) part = part + buf[j];
+        part = group_sum<64>(part);
+        if (lane >> shift == src >> shift) acc = part;
+      }
       if (r < r1 && sub == 0) {
         y[r] = accumulate ? acc + yr : acc;
         xy = xy + (double)xr * (double)acc;
@@ -162,10 +175,12 @@ void free_rowchunk(lapis_hip_csr_plan *p) {
 
 int build_rowchunk(lapis_hip_csr_plan *p, int value_bytes, hipStream_t st) {
   const lapis_hip_csr_stats &s = p->stats;
-  // One lane adds up a row where a chunk has 64 or more, so a chunk takes as long as its longest row: uneven rows
-  // are left to the row-split kernel unless none is long (2425 power-law rows of up to 256: 16 us here, 5 there).
   if (s.nnz == 0 || s.max_row_len > kRowchunkLongestRow) return LAPIS_HIP_OK;
-  if (s.max_row_len > 64 && s.max_row_len > 3.0 * s.mean_row_len) return LAPIS_HIP_OK;
+  // Short rows with a few long ones among them are left to the row-block kernel: the chunk has to hold four of the
+  // longest and is mostly rows (100 000 rows of 5, every 50th 250: 9.5 us here, 8.1 there; 500 000 of 3 and 100: 25.8 and
+  // 25.0).  From a mean of 16 the chunks win (2013 power-law rows of 31 on average, up to 201: 6.4 us against 11.5, the
+  // whole wavefront adding up a long row; 100 000 rows of 20, every tenth 100: 17.3 against 19.8).
+  if (s.max_row_len > 64 && s.max_row_len > 3.0 * s.mean_row_len && s.mean_row_len < 16.0) return LAPIS_HIP_OK;
   // Entries per wavefront, 4 wavefronts per workgroup.  A matrix the 256 MB last-level cache holds: 256 in fp64 (512:
   // +3 % in CG on 1024^2), 512 in fp32 (7-point 152^3: 39.1 us against 41.6).  From HBM more of it is asked for at once:
   // 512 (7-point 180^3: 116.9 us against 118.4 in fp64, 76.5 against 79.2 in fp32), 1024 where rows are long (27-node

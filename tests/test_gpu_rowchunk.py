@@ -20,6 +20,8 @@ LENGTHS = {
     "empties": [3] + [0] * 3000 + [5, 0, 64] + [0] * 700,
     "mostly_empty": ([0] * 9 + [1]) * 500,
     "mixed": list(np.random.default_rng(5).integers(0, 50, 5000)),
+    "uneven": [20, 19, 200, 0, 33, 65, 20, 1, 2, 256, 31, 32] * 60,
+    "uneven_ends": [256] + [17] * 300 + [255],
     "too_long": [257] + [2] * 300,
 }
 
