@@ -686,6 +686,10 @@ extern "C" int lapis_hip_bspmm_csrv_f32_i32(int64_t n1, int64_t n2, int64_t dh, 
   // at least 4 entries of every row per window
   const int slots = (int)std::min<int64_t>(kStagedBatchedEntries, kStagedBatched / nh);
   shape.groups = std::max(1, std::min({shape.groups, kBatchedGroups, slots / 4}));
+  // Two wavefronts per SIMD before a wavefront takes several rows: a few rows are bound by the trips of each wavefront
+  // (514 rows of 52, K = 56: 15.0 us -> 12.8; 4587 of 62, K = 36: 18.5 -> 14.7; 9811 of 31, K = 16: 11.1 -> 10.2, and
+  // 12.3 with four per SIMD).
+  while (shape.groups > 1 && ceil_div(n1, shape.groups) * shape.chunks < 2048) shape.groups = (shape.groups + 1) / 2;
   shape.row_blocks = (int)ceil_div(n1, 4 * shape.groups);
   int window_log2 = 0;
   while ((2 << window_log2) * shape.groups <= slots) ++window_log2;

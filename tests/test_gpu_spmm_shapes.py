@@ -78,3 +78,19 @@ def test_batched_csrv_product_in_parts_of_a_row_of_V(gpu, oracle, n2, dh, nh):
     print("case", n2, dh, nh, flush=True)
     gpu.bspmm_csrv(A.nrows, n2, dev(A.pos), dev(A.crd), dev(values), dev(V), out)
     assert np.array_equal(out.cpu().numpy(), oracle.bspmm_csrv(A.pos, A.crd, values, V, A.nrows))  # the order of the reference's nest: bit-exact
+
+
+@pytest.mark.parametrize("dh,nh", [(4, 1), (5, 1), (2, 3), (5, 7), (31, 1), (4, 12), (32, 4), (3, 100)])
+@pytest.mark.parametrize("rows", [2100, 4200, 17000])
+def test_batched_csrv_product_with_several_rows_per_wavefront(gpu, oracle, rows, dh, nh):
+    # from one row per wavefront to the most, by the number of rows
+    rng = np.random.default_rng(rows + dh * 1000 + nh)
+    lengths = rng.integers(0, 9, rows)
+    lengths[:: rows // 5] = rng.integers(60, 290, lengths[:: rows // 5].size)
+    A = from_lengths(list(lengths), 400, 19, np.float32)
+    values = rng.uniform(-1, 1, A.nnz * nh).astype(np.float32)
+    V = rng.uniform(-1, 1, (400, dh, nh)).astype(np.float32)
+    out = torch.zeros(A.nrows, dh, nh, dtype=torch.float32, device="cuda")
+    print("case", rows, dh, nh, flush=True)
+    gpu.bspmm_csrv(A.nrows, 400, dev(A.pos), dev(A.crd), dev(values), dev(V), out)
+    assert np.array_equal(out.cpu().numpy(), oracle.bspmm_csrv(A.pos, A.crd, values, V, A.nrows))
