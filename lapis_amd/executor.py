@@ -22,8 +22,9 @@ refuses what its pipeline cannot lower.
 
 Tensor values are immutable in MLIR; an operation's `outs` operand is overwritten in place only when it is a
 temporary this region made itself (tensor.empty, tensor.splat or the result of an earlier linalg operation)
-that nothing mentions afterwards, otherwise the result gets a buffer of its own.  Memref operands are
-buffers and are always updated in place.
+and no name that may stand for its buffer (its own, or that of a call's, a loop's or a branch's result that
+may have passed it through) is mentioned afterwards, otherwise the result gets a buffer of its own.  Memref
+operands are buffers and are always updated in place.
 """
 import math
 import re
@@ -80,6 +81,8 @@ _STRUCTURE = {"scf.while", "scf.for", "scf.if", "scf.condition", "scf.yield", "f
               "func.return", "scf.parallel", "scf.reduce"}
 _OWNING = {"tensor.empty", "tensor.splat", "memref.alloc", "memref.alloca", "bufferization.alloc_tensor", "linalg.fill",
            "linalg.copy", "linalg.matvec", "linalg.matmul", "linalg.generic"} | set(_LINALG_NAMED)  # results are buffers of this region
+_NO_BUFFERS = (_SCALAR_OPS - {"arith.select"}) | {"linalg.dot", "tensor.dim", "tensor.extract", "memref.dim", "memref.load",
+                                                  "lapis.dot_start", "lapis.dot_finish"}
 _BUFFER_OPS = {"tensor.empty", "tensor.splat", "tensor.dim", "tensor.extract", "memref.alloc", "memref.alloca",
                "memref.dealloc", "memref.dim", "memref.load", "memref.store", "memref.copy", "linalg.fill",
                "linalg.copy", "linalg.dot", "linalg.matvec", "linalg.matmul", "linalg.generic",
@@ -488,6 +491,9 @@ class Executor:
         for k in range(len(stmts) - 1, -1, -1):
             later[k] = set(acc)
             _sched.mentions(stmts[k], acc)
+        scalar = lambda s: s.op in _NO_BUFFERS or (s.op == "arith.select" and not re.search(r"\b(?:tensor|memref)\s*<", s.head))
+        fresh = lambda s: (s.op in _OWNING or isinstance(s, _sched.Fused)) and not scalar(s)
+        buffers = _sched.buffers(stmts, fresh, scalar)
         block, owned, defined = _Block(), set(), set()
         for k, s in enumerate(stmts):
             op = s.op
@@ -497,7 +503,8 @@ class Executor:
             if op == "arith.constant" and s.results[0] in constants:
                 block.constants[s.results[0]] = constants[s.results[0]]
                 continue
-            can_overwrite = lambda nm, k=k: nm in owned and nm in defined and nm not in later[k]
+            can_overwrite = lambda nm, k=k: nm in owned and nm in defined and \
+                not any(nm in buffers.get(other, (other,)) for other in later[k])
             try:
                 step = self._step(s, nests, can_overwrite, constants)
             except (AttributeError, TypeError, IndexError, KeyError, ValueError) as e:
@@ -505,10 +512,8 @@ class Executor:
             block.add(op, step)
             names = _sched.result_names(s)
             defined.update(names)
-            if op in _OWNING and not isinstance(s, _sched.Fused) and s.results:
-                owned.add(s.results[0])
-            elif isinstance(s, _sched.Fused) and s.op != "lapis.dot_finish":
-                owned.update(s.results)
+            if fresh(s):
+                owned.update(names[:1])
         return block
 
     # Every statement becomes a step: a function of the values by name that leaves its results among them.

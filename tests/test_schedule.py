@@ -109,3 +109,97 @@ def test_operands_that_a_delayed_operation_reads_are_kept():
     for hip in (fake_hip, _fused_hip()):
         (t, v, u), _ = _run(text, "f", lambda: [vec(_x), vec(_z)], hip)
         assert np.allclose(t.numpy(), _x) and np.allclose(u.numpy(), 2 * _x + _z) and np.isclose(v, np.sum((2 * _x + _z) ** 2))
+
+
+# Two names for one buffer: %a is a buffer of the function's own, %b another name for it that is read after an operation
+# whose `outs` is %a.  Each text computes 2x as %a and 3x as %c, and returns %b + %c.
+_SHARED = """
+    module {
+      func.func private @same(%%v: tensor<?xf64>) -> tensor<?xf64> {
+        return %%v : tensor<?xf64>
+      }
+      func.func private @plus(%%u: tensor<?xf64>, %%v: tensor<?xf64>) -> tensor<?xf64> {
+        %%s = linalg.add ins(%%u, %%v : tensor<?xf64>, tensor<?xf64>) outs(%%v : tensor<?xf64>) -> tensor<?xf64>
+        return %%s : tensor<?xf64>
+      }
+      func.func @f(%%x: tensor<?xf64>, %%n: index, %%yes: i1) -> tensor<?xf64> {
+        %%c0 = arith.constant 0 : index
+        %%c1 = arith.constant 1 : index
+        %%no = arith.constant false
+        %%m = tensor.dim %%x, %%c0 : tensor<?xf64>
+        %%e = tensor.empty(%%m) : tensor<?xf64>
+        %%a = linalg.add ins(%%x, %%x : tensor<?xf64>, tensor<?xf64>) outs(%%e : tensor<?xf64>) -> tensor<?xf64>
+        %(name)s
+        %(plus)s
+        %%g = tensor.empty(%%m) : tensor<?xf64>
+        %%d = linalg.add ins(%%b, %%c : tensor<?xf64>, tensor<?xf64>) outs(%%g : tensor<?xf64>) -> tensor<?xf64>
+        return %%d : tensor<?xf64>
+      }
+    }"""
+_ANOTHER_NAME = {
+    "call": "%b = func.call @same(%a) : (tensor<?xf64>) -> tensor<?xf64>",
+    "calls of calls": """%b0 = func.call @same(%a) : (tensor<?xf64>) -> tensor<?xf64>
+        %b = func.call @same(%b0) : (tensor<?xf64>) -> tensor<?xf64>""",
+    "for without trips": """%b = scf.for %i = %c0 to %n step %c1 iter_args(%w = %a) -> (tensor<?xf64>) {
+          %h = tensor.empty(%m) : tensor<?xf64>
+          %k = linalg.add ins(%w, %x : tensor<?xf64>, tensor<?xf64>) outs(%h : tensor<?xf64>) -> tensor<?xf64>
+          scf.yield %k : tensor<?xf64>
+        }""",
+    "for that yields its argument": """%b = scf.for %i = %c0 to %c1 step %c1 iter_args(%w = %a) -> (tensor<?xf64>) {
+          scf.yield %w : tensor<?xf64>
+        }""",
+    "if": """%b = scf.if %yes -> (tensor<?xf64>) {
+          scf.yield %a : tensor<?xf64>
+        } else {
+          scf.yield %x : tensor<?xf64>
+        }""",
+    "while": """%b = scf.while (%w = %a) : (tensor<?xf64>) -> (tensor<?xf64>) {
+          %go = arith.andi %no, %yes : i1
+          scf.condition(%go) %w : tensor<?xf64>
+        } do {
+        ^bb0(%w: tensor<?xf64>):
+          scf.yield %w : tensor<?xf64>
+        }""",
+    "select": "%b = arith.select %yes, %a, %x : tensor<?xf64>",
+}
+_PLUS = {
+    "direct": "%c = linalg.add ins(%x, %a : tensor<?xf64>, tensor<?xf64>) outs(%a : tensor<?xf64>) -> tensor<?xf64>",
+    "in a call": "%c = func.call @plus(%x, %a) : (tensor<?xf64>, tensor<?xf64>) -> tensor<?xf64>",
+}
+
+
+@pytest.mark.parametrize("plus", _PLUS)
+@pytest.mark.parametrize("name", _ANOTHER_NAME)
+def test_a_buffer_with_two_names_is_not_overwritten_while_one_is_read(name, plus):
+    text = _SHARED % {"name": _ANOTHER_NAME[name], "plus": _PLUS[plus]}
+    for hip in (fake_hip, _fused_hip()):
+        (d,), _ = _run(text, "f", lambda: [vec(_x), 0, True], hip)
+        assert np.array_equal(d.numpy(), 2 * _x + (_x + 2 * _x))
+
+
+def test_an_operation_moved_past_another_name_of_its_operand():
+    # %c = x + %a, into %a's buffer, is launched between the dot product's start and its end, behind the call that names
+    # %a once more
+    text = """
+    module {
+      func.func private @same(%v: tensor<?xf64>) -> tensor<?xf64> {
+        return %v : tensor<?xf64>
+      }
+      func.func @f(%x: tensor<?xf64>) -> (tensor<?xf64>, f64, tensor<?xf64>) {
+        %c0 = arith.constant 0 : index
+        %z = arith.constant 0.0 : f64
+        %m = tensor.dim %x, %c0 : tensor<?xf64>
+        %e = tensor.empty(%m) : tensor<?xf64>
+        %a = linalg.add ins(%x, %x : tensor<?xf64>, tensor<?xf64>) outs(%e : tensor<?xf64>) -> tensor<?xf64>
+        %c = linalg.add ins(%x, %a : tensor<?xf64>, tensor<?xf64>) outs(%a : tensor<?xf64>) -> tensor<?xf64>
+        %b = func.call @same(%a) : (tensor<?xf64>) -> tensor<?xf64>
+        %acc = tensor.splat %z[] : tensor<f64>
+        %d = linalg.dot ins(%b, %x : tensor<?xf64>, tensor<?xf64>) outs(%acc : tensor<f64>) -> tensor<f64>
+        %v = tensor.extract %d[] : tensor<f64>
+        return %c, %v, %b : tensor<?xf64>, f64, tensor<?xf64>
+      }
+    }"""
+    for hip in (fake_hip, _fused_hip()):
+        (c, v, b), calls = _run(text, "f", lambda: [vec(_x)], hip)
+        assert np.array_equal(c.numpy(), _x + 2 * _x) and np.array_equal(b.numpy(), 2 * _x) and np.isclose(v, 2 * np.sum(_x * _x))
+    assert calls.index("dot_start") < len(calls) - 1 - calls[::-1].index("axpby") < calls.index("dot_finish")
