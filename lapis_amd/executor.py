@@ -503,8 +503,9 @@ class Executor:
             if op == "arith.constant" and s.results[0] in constants:
                 block.constants[s.results[0]] = constants[s.results[0]]
                 continue
-            can_overwrite = lambda nm, k=k: nm in owned and nm in defined and \
-                not any(nm in buffers.get(other, (other,)) for other in later[k])
+            # `reads`: operands whose elements the operation still needs when it has written others
+            can_overwrite = lambda nm, *reads, k=k: nm in owned and nm in defined and \
+                not any(nm in buffers.get(other, (other,)) for other in later[k].union(reads))
             try:
                 step = self._step(s, nests, can_overwrite, constants)
             except (AttributeError, TypeError, IndexError, KeyError, ValueError) as e:
@@ -709,11 +710,11 @@ class Executor:
             return checked(lambda o, d, env: hip.axpby(coefficient[1](env, d), o[call[2]], coefficient[3](env, d), o[call[4]], d))
         raise Refused("elementwise %s" % kind)
 
-    def _dest(self, nm, can_overwrite):
+    def _dest(self, nm, can_overwrite, *reads):
         """A function of the values that gives the buffer a tensor operation's result goes to: the `outs` operand
         itself where that is allowed, else a new one of its size.  What the operation reads of the operand it
-        reads from the operand."""
-        if can_overwrite(nm):
+        reads from the operand; `reads` names what must not be the same buffer."""
+        if can_overwrite(nm, *reads):
             return lambda env: env[nm]
         empty_like = self.torch.empty_like
         return lambda env: empty_like(env[nm])
@@ -740,7 +741,7 @@ class Executor:
         if op == "lapis.product":
             r = s.results[0]
             A, x = _group(s.parts[0].head, "ins")[0]
-            dest = self._dest(s.outs, can_overwrite)
+            dest = self._dest(s.outs, can_overwrite, x)
 
             def step(env):
                 env[r] = self._csr_product(env[A], env[x], dest(env), overwrite=True)
@@ -749,7 +750,7 @@ class Executor:
             r, product = s.results[0], s.parts[0]
             A, x = _group(product.parts[0].head, "ins")[0]
             init = _group(s.parts[1].head, "outs")[0][0]
-            dest = self._dest(product.outs, can_overwrite)
+            dest = self._dest(product.outs, can_overwrite, x)
 
             def step(env):
                 d, x_ = dest(env), env[x]
@@ -760,7 +761,7 @@ class Executor:
             r, other = s.results[0], s.other
             ca, a, cb, b, out = self._axpby_operands(s.parts[0])
             init = _group(s.parts[1].head, "outs")[0][0]
-            dest = self._dest(out, can_overwrite)
+            dest = self._dest(out, can_overwrite, *([] if other is None else [other]))
 
             def step(env):
                 d, va, vb = dest(env), env[a], env[b]
@@ -916,7 +917,7 @@ class Executor:
         plan = self._generic_plan(s) if op == "linalg.generic" else None
         if op in ("linalg.matvec", "linalg.matmul") or plan in (("matvec",), ("matmul",)):
             wide = op == "linalg.matmul" or plan == ("matmul",)
-            in_place = r is None or can_overwrite(out_nm)
+            in_place = r is None or can_overwrite(out_nm, ins[1])
 
             def step(env):
                 out, x = env[out_nm], env[ins[1]]

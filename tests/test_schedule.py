@@ -203,3 +203,73 @@ def test_an_operation_moved_past_another_name_of_its_operand():
         (c, v, b), calls = _run(text, "f", lambda: [vec(_x)], hip)
         assert np.array_equal(c.numpy(), _x + 2 * _x) and np.array_equal(b.numpy(), 2 * _x) and np.isclose(v, 2 * np.sum(_x * _x))
     assert calls.index("dot_start") < len(calls) - 1 - calls[::-1].index("axpby") < calls.index("dot_finish")
+
+
+# The `outs` operand is a buffer of the function's own that nothing mentions afterwards, and the operation needs its old
+# elements when it has written new ones.
+_NEEDED = {
+    "product with its own output": """
+        %a = linalg.add ins(%x, %x : tensor<?xf64>, tensor<?xf64>) outs(%e : tensor<?xf64>) -> tensor<?xf64>
+        %p = linalg.matvec ins(%A, %a : tensor<?x?xf64, #CSR>, tensor<?xf64>) outs(%a : tensor<?xf64>) -> tensor<?xf64>
+        return %p, %z : tensor<?xf64>, f64""",
+    "product into zeros of another name's buffer": """
+        %a = linalg.add ins(%x, %x : tensor<?xf64>, tensor<?xf64>) outs(%e : tensor<?xf64>) -> tensor<?xf64>
+        %b = func.call @same(%a) : (tensor<?xf64>) -> tensor<?xf64>
+        %o = linalg.fill ins(%z : f64) outs(%a : tensor<?xf64>) -> tensor<?xf64>
+        %p = linalg.matvec ins(%A, %b : tensor<?x?xf64, #CSR>, tensor<?xf64>) outs(%o : tensor<?xf64>) -> tensor<?xf64>
+        return %p, %z : tensor<?xf64>, f64""",
+    "product and dot into zeros of another name's buffer": """
+        %a = linalg.add ins(%x, %x : tensor<?xf64>, tensor<?xf64>) outs(%e : tensor<?xf64>) -> tensor<?xf64>
+        %b = func.call @same(%a) : (tensor<?xf64>) -> tensor<?xf64>
+        %o = linalg.fill ins(%z : f64) outs(%a : tensor<?xf64>) -> tensor<?xf64>
+        %p = linalg.matvec ins(%A, %b : tensor<?x?xf64, #CSR>, tensor<?xf64>) outs(%o : tensor<?xf64>) -> tensor<?xf64>
+        %d = linalg.dot ins(%b, %p : tensor<?xf64>, tensor<?xf64>) outs(%acc : tensor<f64>) -> tensor<f64>
+        %v = tensor.extract %d[] : tensor<f64>
+        return %p, %v : tensor<?xf64>, f64""",
+    "sum and dot with what it overwrites": """
+        %a = linalg.add ins(%x, %x : tensor<?xf64>, tensor<?xf64>) outs(%e : tensor<?xf64>) -> tensor<?xf64>
+        %p = linalg.add ins(%a, %x : tensor<?xf64>, tensor<?xf64>) outs(%a : tensor<?xf64>) -> tensor<?xf64>
+        %d = linalg.dot ins(%p, %a : tensor<?xf64>, tensor<?xf64>) outs(%acc : tensor<f64>) -> tensor<f64>
+        %v = tensor.extract %d[] : tensor<f64>
+        return %p, %v : tensor<?xf64>, f64""",
+    "sum and dot with another name of what it overwrites": """
+        %a = linalg.add ins(%x, %x : tensor<?xf64>, tensor<?xf64>) outs(%e : tensor<?xf64>) -> tensor<?xf64>
+        %b = func.call @same(%a) : (tensor<?xf64>) -> tensor<?xf64>
+        %p = linalg.add ins(%a, %x : tensor<?xf64>, tensor<?xf64>) outs(%a : tensor<?xf64>) -> tensor<?xf64>
+        %d = linalg.dot ins(%b, %p : tensor<?xf64>, tensor<?xf64>) outs(%acc : tensor<f64>) -> tensor<f64>
+        %v = tensor.extract %d[] : tensor<f64>
+        return %p, %v : tensor<?xf64>, f64""",
+}
+
+
+@pytest.mark.parametrize("name", _NEEDED)
+def test_what_an_operation_needs_while_it_writes_is_not_its_output(name, monkeypatch):
+    text = """
+    #CSR = #sparse_tensor.encoding<{ map = (d0, d1) -> (d0 : dense, d1 : compressed), posWidth = 32, crdWidth = 32 }>
+    module {
+      func.func private @same(%%v: tensor<?xf64>) -> tensor<?xf64> {
+        return %%v : tensor<?xf64>
+      }
+      func.func @f(%%A: tensor<?x?xf64, #CSR>, %%x: tensor<?xf64>) -> (tensor<?xf64>, f64) {
+        %%c0 = arith.constant 0 : index
+        %%z = arith.constant 0.0 : f64
+        %%m = tensor.dim %%x, %%c0 : tensor<?xf64>
+        %%acc = tensor.splat %%z[] : tensor<f64>
+        %%e = tensor.empty(%%m) : tensor<?xf64>
+        %s
+      }
+    }""" % _NEEDED[name].strip()
+    a = 2 * _x
+    p = A @ a + a if name.endswith("its own output") else A @ a if name.startswith("product") else a + _x
+    v = np.dot(a, p) if "dot" in name else 0.0
+    for hip in (fake_hip, _fused_hip()):
+        written = []  # the stand-ins read all of x before they write y, which a kernel does not: no shared buffer
+        for fn in ("spmv", "spmv_overwrite", "spmv_dot_start"):
+            if hasattr(hip, fn):
+                def check(plan, nrows, ncols, pos, crd, val, x, y, *more, was=getattr(hip, fn)):
+                    written.append((x.data_ptr(), y.data_ptr()))
+                    return was(plan, nrows, ncols, pos, crd, val, x, y, *more)
+                monkeypatch.setattr(hip, fn, check)
+        (got, w), _ = _run(text, "f", lambda: [csr(A), vec(_x)], hip)
+        assert np.allclose(got.numpy(), p, rtol=1e-13) and np.isclose(w, v, rtol=1e-13)
+        assert all(x != y for x, y in written) and bool(written) == name.startswith("product")
