@@ -793,6 +793,7 @@ int pcg_run(lapis_hip_csr_plan *plan, int64_t n, const int32_t *pos, const int32
     return LAPIS_HIP_OK;
   }
   LAPIS_REQUIRE(pos && b && x, "pcg: null positions, right-hand side or solution");
+  const char *what = mask ? "pcg_masked" : "pcg";
 
   int rc = LAPIS_HIP_OK;
   lapis_hip_csr_plan *own_plan = nullptr;
@@ -834,9 +835,13 @@ int pcg_run(lapis_hip_csr_plan *plan, int64_t n, const int32_t *pos, const int32
     PCG_TRY(hipStreamSynchronize(st));
     PCG_RC(lapis_hip_csr_plan_create(&own_plan, n, n, nnz32, pos, crd, 8, stream));
     plan = own_plan;
+    PCG_RC(check_planned(what, plan, n, n, pos, crd, val, 8));
     // the column-blocked copy costs about as much as 40 SpMVs of such a matrix: build it
     // only when the iteration limit allows it to pay back
     if (maxiter >= 64) PCG_RC(lapis_hip_csr_plan_analyze(own_plan, crd, val, 8, stream));
+  } else {
+    // the kernels below size their LDS and their grids by the plan: refused before the first of them
+    PCG_RC(check_planned(what, plan, n, n, pos, crd, val, 8));
   }
   if (!work) {
     // own scratch: an even stride keeps all four vectors 16-byte aligned

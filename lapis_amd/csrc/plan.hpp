@@ -108,6 +108,11 @@ template <typename T>
 int launch_rowchunk_xy(const lapis_hip_csr_plan *plan, const int *crd, const T *val, const T *x, T *y, hipStream_t st,
                        double *xy_partials, bool to_host, int *count, const unsigned long long *skip);
 
+// May `plan` serve a product of this matrix?  The error the entry point `what` returns if not: a plan of other sizes or
+// positions, null entries, or a column-blocked copy (where the plan runs one) of other buffers.
+int check_planned(const char *what, const lapis_hip_csr_plan *plan, int64_t nrows, int64_t ncols, const int32_t *pos,
+                  const int32_t *crd, const void *val, int value_bytes);
+
 // y = A x with the checks of the SpMV entry points, and the same with the start of init + x . y (blas1.hpp).
 struct HostSum;
 template <typename T>

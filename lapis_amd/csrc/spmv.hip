@@ -566,6 +566,35 @@ int launch_nnzsplit(const lapis_hip_csr_plan *p, const int *pos, const int *crd,
   }
 }
 
+}  // namespace
+
+namespace lapis {
+int check_planned(const char *what, const lapis_hip_csr_plan *plan, int64_t nrows, int64_t ncols, const int32_t *pos,
+                  const int32_t *crd, const void *val, int value_bytes) {
+  const lapis_hip_csr_stats &s = plan->stats;
+  if (s.nrows != nrows || s.ncols != ncols || plan->pos != pos)
+    return set_error(LAPIS_HIP_ERR_PLAN_MISMATCH,
+                     "%s: plan was built for a %lld x %lld matrix at positions %p, called with %lld x %lld at %p", what,
+                     (long long)s.nrows, (long long)s.ncols, (const void *)plan->pos, (long long)nrows,
+                     (long long)ncols, (const void *)pos);
+  if (s.nnz == 0) return LAPIS_HIP_OK;
+  LAPIS_REQUIRE(crd && val, "%s: null coordinates or values with %lld non-zeros", what, (long long)s.nnz);
+  if (s.kernel != LAPIS_HIP_SPMV_COLBLOCK) return LAPIS_HIP_OK;
+  if (!plan->colblock_built || plan->colblock_value_bytes != value_bytes)
+    return set_error(LAPIS_HIP_ERR_PLAN_MISMATCH, "%s: the plan holds no column-blocked copy for %d-byte values", what,
+                     value_bytes);
+  // the copy stands in for crd/val: refuse buffers it was not made from (new values in the same
+  // buffer are brought in with lapis_hip_csr_plan_update_values)
+  if (crd != plan->colblock_src_crd || val != plan->colblock_src_val)
+    return set_error(LAPIS_HIP_ERR_PLAN_MISMATCH,
+                     "%s: the column-blocked copy was made from coordinates %p and values %p, called with %p and %p "
+                     "(lapis_hip_csr_plan_update_values takes new values)",
+                     what, plan->colblock_src_crd, plan->colblock_src_val, (const void *)crd, val);
+  return LAPIS_HIP_OK;
+}
+}  // namespace lapis
+
+namespace {
 template <typename T>
 int spmv_impl(lapis_hip_csr_plan *plan, int64_t nrows, int64_t ncols, const int32_t *pos, const int32_t *crd,
               const T *val, const T *x, T *y, lapis_hip_stream_t stream) {
@@ -592,14 +621,11 @@ int spmv_impl(lapis_hip_csr_plan *plan, int64_t nrows, int64_t ncols, const int3
     return launch_subwarp<T, true>(w, nrows, pos, crd, val, x, y, st);
   }
 
+  const int rc = check_planned("spmv", plan, nrows, ncols, pos, crd, val, (int)sizeof(T));
+  if (rc != LAPIS_HIP_OK) return rc;
   const lapis_hip_csr_stats &s = plan->stats;
-  if (s.nrows != nrows || s.ncols != ncols || plan->pos != pos)
-    return set_error(LAPIS_HIP_ERR_PLAN_MISMATCH,
-                     "spmv: plan was built for a %lld x %lld matrix at positions %p, called with %lld x %lld at %p",
-                     (long long)s.nrows, (long long)s.ncols, (const void *)plan->pos, (long long)nrows,
-                     (long long)ncols, (const void *)pos);
   if (s.nnz == 0) return LAPIS_HIP_OK;
-  LAPIS_REQUIRE(x && crd && val, "spmv: null coordinates, values or x with %lld non-zeros", (long long)s.nnz);
+  LAPIS_REQUIRE(x, "spmv: null x with %lld non-zeros", (long long)s.nnz);
   if (plan->runs_rowchunk()) return launch_rowchunk<T>(plan, crd, val, x, y, st, 1);
   const bool vec = aligned16(crd) && aligned16(val);
   const bool nt = plan->nontemporal;
@@ -618,16 +644,6 @@ int spmv_impl(lapis_hip_csr_plan *plan, int64_t nrows, int64_t ncols, const int3
                   : launch_nnzsplit<T, true, false>(plan, pos, crd, val, x, y, st);
       return launch_nnzsplit<T, false, true>(plan, pos, crd, val, x, y, st);
     case LAPIS_HIP_SPMV_COLBLOCK:
-      if (!plan->colblock_built || plan->colblock_value_bytes != (int)sizeof(T))
-        return set_error(LAPIS_HIP_ERR_PLAN_MISMATCH, "spmv: the plan holds no column-blocked copy for %d-byte values",
-                         (int)sizeof(T));
-      // the copy stands in for crd/val: refuse buffers it was not made from (new values in the same
-      // buffer are brought in with lapis_hip_csr_plan_update_values)
-      if (crd != plan->colblock_src_crd || val != plan->colblock_src_val)
-        return set_error(LAPIS_HIP_ERR_PLAN_MISMATCH,
-                         "spmv: the column-blocked copy was made from coordinates %p and values %p, called with %p and %p "
-                         "(lapis_hip_csr_plan_update_values takes new values)",
-                         plan->colblock_src_crd, plan->colblock_src_val, (const void *)crd, (const void *)val);
       return launch_colblock<T>(plan, pos, crd, val, x, y, st);
     default:
       return set_error(LAPIS_HIP_ERR_INVALID_ARGUMENT, "spmv: plan holds unknown kernel %d", s.kernel);
@@ -652,13 +668,13 @@ int spmv_overwrite_f64(lapis_hip_csr_plan *plan, int64_t nrows, int64_t ncols, c
                        lapis_hip_stream_t stream, int *deferred_chunk, double *xy_chunk) {
   if (deferred_chunk) *deferred_chunk = 0;
   if (plan && plan->runs_rowchunk() && plan->stats.nnz > 0 && plan->stats.nrows == nrows && plan->stats.ncols == ncols &&
-      plan->pos == pos && crd && val && x) {
+      plan->pos == pos && crd && val && x && y) {
     LAPIS_CHECK_INIT();
     return launch_rowchunk<double>(plan, crd, val, x, y, as_stream(stream), 0);
   }
   if (plan && plan->stats.kernel == LAPIS_HIP_SPMV_NNZSPLIT && plan->stats.empty_rows == 0 && plan->stats.nnz > 0 &&
-      plan->stats.nrows == nrows && plan->stats.ncols == ncols && plan->pos == pos && aligned16(crd) &&
-      aligned16(val)) {
+      plan->stats.nrows == nrows && plan->stats.ncols == ncols && plan->pos == pos && crd && val && x && y &&
+      aligned16(crd) && aligned16(val)) {
     LAPIS_CHECK_INIT();
     hipStream_t st = as_stream(stream);
     const bool defer = deferred_chunk && plan->nchunks > 1;

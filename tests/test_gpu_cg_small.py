@@ -66,3 +66,37 @@ def test_a_wait_that_runs_out_falls_back_to_the_many_launch_solve(gpu, oracle, m
     monkeypatch.setenv("LAPIS_HIP_CG_SPINS", "0")
     got = _solve(gpu, A, b, None, 1e-9, 200)
     assert got[1] == want[1] and np.allclose(got[0], want[0], rtol=1e-9, atol=1e-12)
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("n,per_row", [(900, 6), (3000, 90), (540000, 4)])  # one launch; chunks of rows, small and large
+def test_a_plan_or_entries_that_do_not_belong_to_the_system_are_refused(gpu, n, per_row, masked):
+    A, rng = _spd(n, per_row, n)
+    pos, crd, val = dev(A.indptr.astype(np.int32)), dev(A.indices.astype(np.int32)), dev(A.data)
+    b, ones = dev(rng.standard_normal(n)), torch.ones(n, dtype=torch.float64, device="cuda")
+    x = torch.full((n,), 7.0, dtype=torch.float64, device="cuda")
+    plan = gpu.CsrPlan(n, n, pos, crd)
+
+    def solve(plan, n=n, pos=pos, crd=crd, val=val):
+        if masked:
+            return gpu.pcg_masked(plan, n, pos, crd, val, b, ones, ones, 1e-9, 20, x)
+        return gpu.pcg(plan, n, pos, crd, val, b, None, 1e-9, 20, x)
+    wide = gpu.CsrPlan(n, n + 1, pos, crd)
+    other = gpu.CsrPlan(n, n, pos.clone(), crd)
+    for call in (lambda: solve(plan, n=n - 1), lambda: solve(wide), lambda: solve(other), lambda: solve(plan, pos=pos.clone())):
+        with pytest.raises(gpu.LapisHipError) as e:
+            call()
+        assert e.value.status_name == "LAPIS_HIP_ERR_PLAN_MISMATCH"
+    for p in (plan, None):
+        for call in (lambda: solve(p, crd=None), lambda: solve(p, val=None)):
+            with pytest.raises(gpu.LapisHipError) as e:
+                call()
+            assert e.value.status_name == "LAPIS_HIP_ERR_INVALID_ARGUMENT"
+    if n == 900:  # a column-blocked copy stands in for the buffers it was made from only
+        plan.build_colblock(crd, val)
+        with pytest.raises(gpu.LapisHipError) as e:
+            solve(plan, val=val.clone())
+        assert e.value.status_name == "LAPIS_HIP_ERR_PLAN_MISMATCH"
+    assert torch.equal(x, torch.full_like(x, 7.0))  # refused before anything was written
+    solve(plan)
+    assert not torch.equal(x, torch.full_like(x, 7.0))
