@@ -592,6 +592,9 @@ LAPIS_PY(py_pcg) {
     holds("pcg", rows, x, val.tensor);
     holds("pcg", 4 * rows, work, val.tensor);
     if (crd.tensor) holds("pcg", crd.tensor->numel(), val);
+    for (const Operand *o : {&val, &b, &dinv, &x, &work})
+      if (o->tensor && o->tensor->scalar_type() != at::kDouble)
+        raise(PyExc_TypeError, "pcg: operands are float64, got %s", type_name(o->tensor->scalar_type()));
     const double tol = number(a[7]);
     const int64_t maxiter = integer(a[8]);
     lapis_hip_csr_plan *plan = plan_of(a[0]);
