@@ -487,6 +487,8 @@ def pcg_masked(plan, n, pos, crd, val, b, mask, d, tol, maxiter, x, work=None, s
     _holds("pcg_masked", n + 1, pos)
     _holds("pcg_masked", n, b, mask, d, x, like=val)
     _holds("pcg_masked", 5 * n, work, like=val)
+    if not isinstance(val, int) and val is not None and val.element_size() != 8:
+        raise TypeError("pcg_masked: operands are float64, got %s" % val.dtype)
     lib = init()
     iters, relres = _u64(0), _dbl(0.0)
     check(lib.lapis_hip_pcg_masked_f64_i32(plan.handle if plan is not None else None, n, _ptr(pos), _ptr(crd),

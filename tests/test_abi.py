@@ -129,3 +129,14 @@ def test_the_python_binding_refuses_operands_the_kernels_would_overrun():
                  lambda: hip.spmv(None, 5, 5, i32(6), i32(9), f64(9), torch.ones(5), x5)):
         with pytest.raises(TypeError):
             call()
+
+
+def test_the_python_binding_refuses_float32_systems_for_the_float64_solvers():
+    import torch
+    from lapis_amd import hip
+    i32 = lambda n: torch.zeros(n, dtype=torch.int32)
+    v, x = torch.ones(9), torch.ones(5)
+    for call in (lambda: hip.pcg(None, 5, i32(6), i32(9), v, x, None, 0.0, 1, x),
+                 lambda: hip.pcg_masked(None, 5, i32(6), i32(9), v, x, x, x, 0.0, 1, x)):
+        with pytest.raises(TypeError, match="float64"):
+            call()

@@ -100,11 +100,3 @@ def test_a_plan_or_entries_that_do_not_belong_to_the_system_are_refused(gpu, n, 
     assert torch.equal(x, torch.full_like(x, 7.0))  # refused before anything was written
     solve(plan)
     assert not torch.equal(x, torch.full_like(x, 7.0))
-
-
-def test_single_precision_operands_are_refused(gpu):
-    A, rng = _spd(300, 6, 1)
-    pos, crd = dev(A.indptr.astype(np.int32)), dev(A.indices.astype(np.int32))
-    f32 = [dev(v.astype(np.float32)) for v in (A.data, np.ones(300), np.zeros(300))]
-    with pytest.raises(TypeError, match="float64"):
-        gpu.pcg(None, 300, pos, crd, f32[0], f32[1], None, 1e-9, 20, f32[2])
