@@ -635,6 +635,7 @@ struct CgScratch {
   void *device_block = nullptr, *host_block = nullptr;
   double *parts = nullptr;  // p.Ap in more parts than every block can add up
   size_t parts_capacity = 0;
+  unsigned lds_raised = 0;  // one-launch kernels (a bit per rows of a thread) that may take kSmallLdsBytes on this device
 };
 constexpr int kKeptScratch = 8;
 std::mutex g_cg_mutex;
@@ -744,36 +745,32 @@ int small_rows(const lapis_hip_csr_plan *plan, int64_t n, int *entries) {
 }
 
 template <int RPT>
-hipError_t launch_small_rpt(const CgSmallArgs &a, size_t lds, hipStream_t st) {
-  auto kernel = a.dinv ? cg_small_kernel<RPT, true> : cg_small_kernel<RPT, false>;
-  static std::once_flag once;
-  static hipError_t status = hipSuccess;
-  std::call_once(once, [] {
-    status = hipFuncSetAttribute(reinterpret_cast<const void *>(cg_small_kernel<RPT, true>),
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, kSmallLdsBytes);
-    if (status == hipSuccess)
-      status = hipFuncSetAttribute(reinterpret_cast<const void *>(cg_small_kernel<RPT, false>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, kSmallLdsBytes);
-  });
-  if (status != hipSuccess) return status;
+hipError_t launch_small_rpt(const CgSmallArgs &a, CgScratch *scratch, size_t lds, hipStream_t st) {
+  const void *kernel = reinterpret_cast<const void *>(a.dinv ? cg_small_kernel<RPT, true> : cg_small_kernel<RPT, false>);
+  const unsigned bit = 1u << (2 * RPT + (a.dinv ? 1 : 0));
+  if (!(scratch->lds_raised & bit)) {  // a setting of the device's, as the scratch is
+    const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kSmallLdsBytes);
+    if (e != hipSuccess) return e;
+    scratch->lds_raised |= bit;
+  }
   // A cooperative launch: the workgroups of one solve are resident together whatever other streams run (8 us more
   // per solve than a plain launch).
   CgSmallArgs copy = a;
   void *params[] = {&copy};
-  return hipLaunchCooperativeKernel(reinterpret_cast<const void *>(kernel), dim3(a.blocks), dim3(kSmallThreads), params,
-                                    (unsigned)lds, st);
+  return hipLaunchCooperativeKernel(kernel, dim3(a.blocks), dim3(kSmallThreads), params, (unsigned)lds, st);
 }
 
-hipError_t launch_small(const CgSmallArgs &a, hipStream_t st) {
+hipError_t launch_small(const CgSmallArgs &a, CgScratch *scratch, hipStream_t st) {
+  const char *off = getenv("LAPIS_HIP_CG_ONE_LAUNCH");  // "0": as on a device that refuses the launch
+  if (off && off[0] == '0') return hipErrorNotSupported;
   const size_t lds = (size_t)a.entries * 12;
   switch ((int)ceil_div(a.rows, kSmallThreads)) {
-    case 1: return launch_small_rpt<1>(a, lds, st);
-    case 2: return launch_small_rpt<2>(a, lds, st);
-    case 3: return launch_small_rpt<3>(a, lds, st);
-    default: return launch_small_rpt<4>(a, lds, st);
+    case 1: return launch_small_rpt<1>(a, scratch, lds, st);
+    case 2: return launch_small_rpt<2>(a, scratch, lds, st);
+    case 3: return launch_small_rpt<3>(a, scratch, lds, st);
+    default: return launch_small_rpt<4>(a, scratch, lds, st);
   }
 }
-
 
 // What the solver applies as A and as the preconditioner.
 //   mask == nullptr: A p is the SpMV, z = r * prec (prec may be null: z = r)      examples/pcg_solve.py:52-101
@@ -852,7 +849,7 @@ int pcg_run(lapis_hip_csr_plan *plan, int64_t n, const int32_t *pos, const int32
   double *r = work, *p_odd = work + 2 * stride, *p_even = work + stride, *Ap = work + 3 * stride;  // p of odd, even iterations
   double *tmp = mask ? work + 4 * stride : nullptr;
   PCG_TRY(take_scratch(&scratch, st));
-  if (!mask && maxiter != 0) {
+  if (!mask && maxiter != 0 && x != b) {  // x != b: what gives up after x is written starts again from b
     int entries = 0;
     const int rows = small_rows(plan, n, &entries);
     if (rows) {
@@ -886,10 +883,15 @@ int pcg_run(lapis_hip_csr_plan *plan, int64_t n, const int32_t *pos, const int32
         a.epoch = scratch->epoch;
         scratch->epoch += 2 * (unsigned)a.budget + 2;
         scratch->host_result->fault = 0;
-        PCG_TRY(launch_small(a, st));
+        // A launch that is refused (a device or a process that takes no cooperative launches, workgroups that do not
+        // fit) and workgroups that were not resident together: the kernels below start from the beginning.
+        if (launch_small(a, scratch, st) != hipSuccess) {
+          (void)hipGetLastError();
+          break;
+        }
         PCG_TRY(hipStreamSynchronize(st));
         const CgSmallResult &got = *scratch->host_result;
-        if (got.fault) break;  // the workgroups were not resident together: the kernels below start from the beginning
+        if (got.fault) break;
         if (got.done_iter != 0) {
           *iters = got.done_iter;
           *relres = got.relres;

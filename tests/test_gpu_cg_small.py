@@ -100,3 +100,37 @@ def test_a_plan_or_entries_that_do_not_belong_to_the_system_are_refused(gpu, n, 
     assert torch.equal(x, torch.full_like(x, 7.0))  # refused before anything was written
     solve(plan)
     assert not torch.equal(x, torch.full_like(x, 7.0))
+
+
+@pytest.mark.parametrize("preconditioned", [False, True])
+def test_a_launch_that_is_refused_falls_back_to_the_many_launch_solve(gpu, oracle, monkeypatch, preconditioned):
+    A, rng = _spd(3000, 8, 9)
+    b = rng.standard_normal(3000)
+    dinv = 1.0 / A.diagonal() if preconditioned else None
+
+    def solve():
+        gpu.kernel_timing_start(400)  # counts products launched on their own
+        result = _solve(gpu, A, b, dinv, 1e-9, 200)
+        return result, gpu.kernel_timing_stop()["count"]
+    want, products = solve()
+    assert products == 0
+    monkeypatch.setenv("LAPIS_HIP_CG_ONE_LAUNCH", "0")
+    got, products = solve()
+    assert products >= got[1] == want[1] and np.allclose(got[0], want[0], rtol=1e-9, atol=1e-12)
+    monkeypatch.delenv("LAPIS_HIP_CG_ONE_LAUNCH")
+    again, products = solve()
+    assert products == 0 and again[1] == want[1] and np.array_equal(again[0], want[0])
+
+
+def test_the_solution_in_the_right_hand_sides_buffer(gpu, monkeypatch):
+    A, rng = _spd(3000, 8, 9)
+    n, pos, crd, val = 3000, dev(A.indptr.astype(np.int32)), dev(A.indices.astype(np.int32)), dev(A.data)
+    b = rng.standard_normal(n)
+    want = _solve(gpu, A, b, None, 1e-9, 200)
+    plan = gpu.CsrPlan(n, n, pos, crd)
+    for spins in (None, "0"):  # as it comes, and through a one-launch solve that would give up
+        if spins:
+            monkeypatch.setenv("LAPIS_HIP_CG_SPINS", spins)
+        x = dev(b)
+        iters, _ = gpu.pcg(plan, n, pos, crd, val, x, None, 1e-9, 200, x)
+        assert iters == want[1] and np.allclose(x.cpu().numpy(), want[0], rtol=1e-9, atol=1e-12)
