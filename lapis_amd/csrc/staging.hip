@@ -14,8 +14,11 @@
 // A product on host arrays, fp64 7-point grids: 11^3 222 -> 26 us, 32^3 317 -> 130 us, 64^3 1.56 -> 0.70 ms,
 // 128^3 10.5 -> 5.1 ms.  Bound by the bus (55 GB/s) from 32^3 on, by four launches and a wait below.
 //
-// Kept between calls until the library shuts down: up to 4 arenas (a stream, pinned memory of up to 2 x 16 MB, device
-// memory of up to 1 GB) and the helper threads, which sleep.
+// Kept between calls until the library shuts down (lapis_hip_finalize): up to 4 arenas, each with two streams and pinned
+// memory of up to 2 x 16 MB and 4 MB, together with at most 256 MB of memory on a device; and the helper threads, which
+// sleep.  A call beyond that takes its memory and gives it back (hipMalloc 31 us, hipFree 236 us for 256 MB, where the
+// call itself takes 5 ms; 1 GB: 31 and 239).  Other allocators of the process cannot ask for what is kept; a call that
+// finds the device full gives back what the other arenas hold.
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
@@ -54,7 +57,7 @@ constexpr size_t kAlign = 4096;                 // operands start here: blocks a
 constexpr size_t kAlone = (size_t)1 << 20;      // up to here the caller's thread copies alone
 constexpr size_t kByKernel = (size_t)2 << 20;   // uploads up to here are one kernel's work
 constexpr size_t kDirect = (size_t)4 << 20;     // direct operands up to here stay in pinned memory
-constexpr size_t kKeptMemory = (size_t)1 << 30;
+constexpr size_t kKeptMemory = (size_t)256 << 20;  // device memory of all arenas at rest on a device
 constexpr int kKeptArenas = 4;
 constexpr int kHelpers = 3;
 
@@ -155,19 +158,25 @@ hipError_t take_arena(StagingArena **out, size_t bytes, size_t half, size_t dire
 }
 
 void give_arena(StagingArena *a) {
-  if (a->bytes > kKeptMemory) {
-    (void)hipFree(a->memory);
-    a->memory = nullptr;
-    a->bytes = 0;
-  }
+  char *surplus = nullptr;
+  bool kept = false;
   {
     std::lock_guard<std::mutex> lock(g_arena_mutex);
-    if ((int)g_arenas.size() < kKeptArenas) {
+    size_t bytes = a->bytes;
+    for (const StagingArena *other : g_arenas)
+      if (other->device == a->device) bytes += other->bytes;
+    kept = (int)g_arenas.size() < kKeptArenas;
+    if (kept) {
+      if (bytes > kKeptMemory) {
+        surplus = a->memory;
+        a->memory = nullptr;
+        a->bytes = 0;
+      }
       g_arenas.push_back(a);
-      return;
     }
   }
-  free_arena(a);
+  if (surplus) (void)hipFree(surplus);
+  if (!kept) free_arena(a);
 }
 
 // ---- copying passes -----------------------------------------------------------------------------------------

@@ -63,3 +63,18 @@ def test_several_threads(module):
     for t in threads:
         t.join()
     assert not errors
+
+
+def test_memory_kept_between_calls_is_bounded_for_all_of_them_together(gpu):
+    import torch
+    host = np.zeros(25_000_000)  # 200 MB: an arena of 256 MB each
+    free = lambda: torch.cuda.mem_get_info()[0]
+    torch.cuda.synchronize()
+    before = free()
+    held = [gpu.stage([host]) for _ in range(3)]
+    assert before - free() >= 512 << 20  # one of them may have been there
+    del held
+    torch.cuda.synchronize()
+    assert before - free() <= (256 << 20) + (32 << 20)
+    (t,), staged = gpu.stage([host[:1000] + 3.0])  # and the arenas still serve calls
+    assert torch.equal(t, torch.full_like(t, 3.0))
