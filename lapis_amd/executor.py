@@ -487,13 +487,15 @@ class Executor:
                     pass
         if hasattr(self.hip, "dot_start") and not nests:
             stmts = _sched.rewrite(stmts, self._kind, constants)
-        later, acc = [None] * len(stmts), set()
-        for k in range(len(stmts) - 1, -1, -1):
-            later[k] = set(acc)
-            _sched.mentions(stmts[k], acc)
+        said = [_sched.mentions(s) for s in stmts]
         scalar = lambda s: s.op in _NO_BUFFERS or (s.op == "arith.select" and not re.search(r"\b(?:tensor|memref)\s*<", s.head))
         fresh = lambda s: (s.op in _OWNING or isinstance(s, _sched.Fused)) and not scalar(s)
-        buffers = _sched.buffers(stmts, fresh, scalar)
+        buffers = _sched.buffers(zip(stmts, said), fresh, scalar)
+        last = {}  # the last statement that mentions a name of the buffer
+        for k, names in enumerate(said):
+            for n in names:
+                for nm in buffers.get(n, (n,)):
+                    last[nm] = k
         block, owned, defined = _Block(), set(), set()
         for k, s in enumerate(stmts):
             op = s.op
@@ -504,8 +506,8 @@ class Executor:
                 block.constants[s.results[0]] = constants[s.results[0]]
                 continue
             # `reads`: operands whose elements the operation still needs when it has written others
-            can_overwrite = lambda nm, *reads, k=k: nm in owned and nm in defined and \
-                not any(nm in buffers.get(other, (other,)) for other in later[k].union(reads))
+            can_overwrite = lambda nm, *reads, k=k: nm in owned and nm in defined and last.get(nm, k) <= k and \
+                not any(nm in buffers.get(other, (other,)) for other in reads)
             try:
                 step = self._step(s, nests, can_overwrite, constants)
             except (AttributeError, TypeError, IndexError, KeyError, ValueError) as e:

@@ -56,17 +56,15 @@ def result_names(s):
 
 
 def buffers(stmts, fresh, scalar):
-    """For every name the statements define, the names whose buffers it may be.  `fresh(statement)`: its results are
-    buffers of their own; `scalar(statement)`: its results hold no buffer.  What any other statement gives (a call, a
-    loop or branch that may pass an operand through, another name for a value) may be any buffer it mentions."""
+    """For every name that `stmts`, (statement, names it mentions) in order, define: the names whose buffers it may be.
+    `fresh(statement)`: its results are buffers of their own; `scalar(statement)`: its results hold no buffer.  What any
+    other statement gives (a call, a loop or branch that may pass an operand through, another name for a value) may be any
+    buffer it mentions."""
     of = {}
-    for s in stmts:
-        names = result_names(s)
-        shared = set()
-        if not (fresh(s) or scalar(s)):
-            for n in mentions(s):
-                shared |= of.get(n, {n})
-        of.update((n, shared | {n}) for n in names)
+    for s, said in stmts:
+        shared = set() if fresh(s) or scalar(s) else set().union(*(of.get(n, (n,)) for n in said))
+        for n in result_names(s):
+            of[n] = shared | {n}
     return of
 
 
