@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from gpu_util import dev, from_lengths
+from gpu_util import TOL, dev, from_lengths
 from lapis_amd import generators as gen
 from test_gpu_spmm import _check
 
@@ -94,3 +94,47 @@ def test_batched_csrv_product_with_several_rows_per_wavefront(gpu, oracle, rows,
     print("case", rows, dh, nh, flush=True)
     gpu.bspmm_csrv(A.nrows, 400, dev(A.pos), dev(A.crd), dev(values), dev(V), out)
     assert np.array_equal(out.cpu().numpy(), oracle.bspmm_csrv(A.pos, A.crd, values, V, A.nrows))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("rows_of_B", [(1 << 10) - 1, 1 << 10, 1500])
+def test_byte_offsets_into_B_around_two_to_the_32(gpu, oracle, dtype, rows_of_B):
+    # rows of B 4 MB apart: 32-bit byte offsets to the last below 4 GB, 64-bit ones from 4 GB on; vectors and single elements,
+    # one and several column chunks, even short rows (several per wavefront with a plan) and long ones
+    size = np.dtype(dtype).itemsize
+    ldb, rng = (1 << 22) // size, np.random.default_rng(rows_of_B)
+    whole = torch.empty((rows_of_B - 1) * ldb + 300, dtype=torch.float32 if size == 4 else torch.float64, device="cuda")
+    for lengths in ([7] * 150, list(rng.integers(0, 400, 40)) + [0, 385]):
+        A = from_lengths(lengths, rows_of_B, 23, dtype)
+        A.crd[A.pos[1:][np.diff(A.pos) > 0] - 1] = rows_of_B - 1  # the last row of B in every row of A
+        for k in (1, 3, 10, 64, 300):
+            B, C_in = rng.uniform(-1, 1, (rows_of_B, k)).astype(dtype), rng.uniform(-1, 1, (A.nrows, k)).astype(dtype)
+            view = torch.as_strided(whole, (rows_of_B, k), (ldb, 1))
+            view.copy_(dev(B))
+            want = C_in.copy()
+            oracle.spmm(A.pos, A.crd, A.val, B, want)
+            row_of = np.repeat(np.arange(A.nrows), np.diff(A.pos))
+            scale = np.abs(C_in) + np.bincount(row_of, np.abs(A.val), A.nrows)[:, None]  # |B| <= 1
+            pos, crd, val = dev(A.pos), dev(A.crd), dev(A.val)
+            for plan in (None, gpu.CsrPlan(A.nrows, rows_of_B, pos, crd, value_bytes=size)):
+                print("case", dtype.__name__, rows_of_B, lengths[0], k, plan is not None, flush=True)
+                C = dev(C_in)
+                gpu.spmm(A.nrows, rows_of_B, pos, crd, val, view, C, plan=plan)
+                assert np.all(np.abs(C.cpu().numpy().astype(np.float64) - want) <= TOL[np.dtype(dtype)] * scale)
+
+
+@pytest.mark.parametrize("n2,dh,nh", [((1 << 21) - 1, 64, 8), (1 << 21, 64, 8), ((1 << 21) + 5, 64, 8), (2093043, 171, 3), (2093042, 171, 3)])
+def test_byte_offsets_into_V_around_two_to_the_32(gpu, oracle, n2, dh, nh):
+    # V just below and from 4 GB on, heads in vectors and not; 300 of its rows are used, its first and last among them
+    rng = np.random.default_rng(n2)
+    used = np.unique(np.concatenate([[0, n2 - 1], rng.integers(0, n2, 298)]))
+    A = from_lengths(list(rng.integers(0, 40, 90)) + [0, 150], used.size, 29, np.float32)
+    A.crd[A.pos[1:][np.diff(A.pos) > 0] - 1] = used.size - 1
+    values = rng.uniform(-1, 1, A.nnz * nh).astype(np.float32)
+    small = rng.uniform(-1, 1, (used.size, dh, nh)).astype(np.float32)
+    V = torch.empty((n2, dh, nh), dtype=torch.float32, device="cuda")
+    V[torch.from_numpy(used).cuda()] = dev(small)
+    out = torch.zeros(A.nrows, dh, nh, dtype=torch.float32, device="cuda")
+    print("case", n2, dh, nh, flush=True)
+    gpu.bspmm_csrv(A.nrows, n2, dev(A.pos), dev(used[A.crd].astype(np.int32)), dev(values), V, out)
+    assert np.array_equal(out.cpu().numpy(), oracle.bspmm_csrv(A.pos, A.crd, values, small, A.nrows))
