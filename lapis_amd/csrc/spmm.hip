@@ -42,7 +42,6 @@ struct SpmmShape {
   unsigned lpr_inv, group_inv;  // 65536 / lpr + 1, 65536 / (lpr * par) + 1: a lane's number divided without a division
   int groups;      // 64 / (lpr * par)
   int row_blocks;  // workgroups per chunk
-  int xcd_map;
   template <int VW>
   __device__ __forceinline__ int chunk_first(int c) const {
     return c >= chunks ? k : VW * (c * chunk_width + min(c, wider));
@@ -76,6 +75,10 @@ __device__ __forceinline__ double lane_get(int byte_of_lane, double v) {
 //   7-point 97^3, fp64   k = 3: 316 -> 35   k = 10: 392 -> 68   k = 64: 409 -> 369
 //   27-point x 3, 30^3   k = 3 fp64: 48 -> 31   k = 10 fp32: 57 -> 34   k = 64 fp32: 82 -> 73
 //   random, 32 per row, 15 000 rows, k = 10 fp32: 9.9 -> 7.7; 1 M rows, k = 64 fp32 (rows of B from HBM): 1217 -> 1203
+// Each XCD takes a contiguous part of the rows, so that neighbouring rows find each other's rows of B in its L2.  Dealt
+// round-robin instead, us, 7-point grids in fp64, k = 64: 70^3 130 -> 153, 95^3 334 -> 325, 97^3 358 -> 352, 100^3
+// 393 -> 501, 115^3 595 -> 763; fp32, k = 64, 100^3: 181 -> 225; 27-point x 3, 45^3, fp64, k = 64: 423 -> 403, k = 100:
+// 764 -> 807.  (A rule that dealt round-robin where 1024 non-zeros span more than 8 MB of B rested on 97^3 alone.)
 // WIDE: B is 4 GB or more and the offsets take 64 bits.
 // Entries per wavefront and window: 384, 18 KB per workgroup in fp64, and registers for seven wavefronts per SIMD
 // (against 512 entries and 76 registers, six wavefronts: 7-point 97^3 fp64, k = 10: 75 us -> 68, k = 33: 228 -> 207;
@@ -92,7 +95,7 @@ __device__ __forceinline__ void spmm_rows_body(int nrows, const SpmmShape &sh, c
   __shared__ unsigned s_off[4][kStaged];
   const unsigned nblocks = (unsigned)sh.row_blocks * (unsigned)sh.chunks, id = linear_block();
   if (id >= nblocks) return;
-  unsigned block = sh.xcd_map ? xcd_contiguous_block(id, nblocks) : id;
+  unsigned block = xcd_contiguous_block(id, nblocks);
   int cfirst = 0, cend = sh.k;
   if (sh.chunks > 1) {
     const int chunk = (int)(block / (unsigned)sh.row_blocks);
@@ -447,7 +450,7 @@ struct SpmmArgs {
 
 // Cuts k columns into chunks of at most `vectors_max` vectors of VW elements (a ragged rest counts as one
 // more) and deals `nrows` rows to groups of lanes per chunk, `par` non-zeros of a row at a time.
-inline SpmmShape make_shape(int64_t nrows, int64_t k, int vw, int vectors_max, int par, int xcd_map) {
+inline SpmmShape make_shape(int64_t nrows, int64_t k, int vw, int vectors_max, int par) {
   SpmmShape s;
   s.k = (int)k;
   const int vectors = (int)(k / vw);
@@ -463,7 +466,6 @@ inline SpmmShape make_shape(int64_t nrows, int64_t k, int vw, int vectors_max, i
   s.lpr_inv = 65536 / s.lpr + 1;
   s.group_inv = 65536 / (s.lpr * s.par) + 1;
   s.row_blocks = (int)ceil_div(nrows, 4 * s.groups);
-  s.xcd_map = xcd_map;
   return s;
 }
 
@@ -575,7 +577,6 @@ int spmm_impl(const char *what, const lapis_hip_csr_plan *plan, int64_t nrows, i
   const int vectors = (int)std::min<int64_t>(64, ceil_div(k, vw));  // lanes per row of B
   const int wave_row = 64 / pow2_up(vectors);                       // par that gives a wavefront one row
   int par = wave_row;
-  bool xcd = true;
   int depth = 4;
   if (plan && plan->stats.mean_row_len > 0.0) {
     const lapis_hip_csr_stats &ps = plan->stats;
@@ -594,9 +595,6 @@ int spmm_impl(const char *what, const lapis_hip_csr_plan *plan, int64_t nrows, i
       while (par < wave_row && 2 * par * 8.0 <= mean && (!local || groups(par) * mean > kStaged)) par *= 2;
       while (par < wave_row && 2 * par * 3.0 <= mean && ceil_div(nrows, groups(par)) < 2500) par *= 2;
     }
-    // Each XCD takes a contiguous part of the rows, so that neighbouring rows find each other's rows of B in its
-    // L2; not where they span more than that L2 holds anyway (7-point 97^3, k = 64 fp64: 391 us against 412).
-    xcd = !(local && span_bytes > 8.0 * 1024 * 1024);
     // Rows of B in flight per lane: 4, but where the columns are all over a B that L2 does not hold more requests
     // only lengthen each other's way, and the registers they take are wavefronts lost: 2 (50 000 rows of 60,
     // k = 64 fp32: 55 us against 70), and 1 for rows of B of up to 16 vectors from HBM (1 M rows of 32, k = 64 fp32:
@@ -605,7 +603,7 @@ int spmm_impl(const char *what, const lapis_hip_csr_plan *plan, int64_t nrows, i
     if (scattered && span_bytes > 8.0 * 1024 * 1024) depth = !local && vectors <= 16 && mean >= 16.0 ? 1 : 2;
   }
   if (force) par = !strcmp(force, "group") && vectors <= 32 ? 1 : wave_row;
-  const SpmmShape shape = make_shape(nrows, k, vw, vectors, par, xcd);
+  const SpmmShape shape = make_shape(nrows, k, vw, vectors, par);
   g_last_spmm_kernel = shape.groups == 1 ? "spmm_wave_row_kernel" : "spmm_group_row_kernel";
   const SpmmArgs<T> args{nrows, k, pos, crd, val, B, ldb, C, ldc, st};
   const bool wide = (double)ncols * (double)ldb * sizeof(T) >= 4294967296.0;
@@ -682,7 +680,7 @@ extern "C" int lapis_hip_bspmm_csrv_f32_i32(int64_t n1, int64_t n2, int64_t dh, 
     if (v_bytes > 8388608.0 && v_bytes * part <= 16777216.0 * (double)(K / 4) && nh * (64 / part) * 32 <= kStagedBatched)
       vectors = part;
   }
-  SpmmShape shape = make_shape(n1, K, 4, vectors, 1, 1);
+  SpmmShape shape = make_shape(n1, K, 4, vectors, 1);
   // at least 4 entries of every row per window
   const int slots = (int)std::min<int64_t>(kStagedBatchedEntries, kStagedBatched / nh);
   shape.groups = std::max(1, std::min({shape.groups, kBatchedGroups, slots / 4}));
