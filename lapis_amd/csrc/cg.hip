@@ -373,8 +373,10 @@ __global__ __launch_bounds__(256) void cg_init_scalar_kernel(int count, const do
 // ---- small systems: the whole solve in one launch -------------------------------------------------
 //
 // On a system of a few ten thousand rows an iteration of the kernels above is launches and gaps (6 launches,
-// 25 us per iteration at 16 384 rows, of which the data of an iteration is worth 1 us; 6.5 us here: a whole solve of 40
-// iterations 1.50 -> 0.27 ms, 490 000 rows 2.20 -> 0.68 ms).  Here one workgroup per
+// 25 us per iteration at 16 384 rows, of which the data of an iteration is worth 1 us; 6.3 us here: a whole solve of 40
+// iterations 1.50 -> 0.27 ms, 490 000 rows 2.20 -> 0.68 ms).  What bounds it: two exchanges with the sums and barriers
+// around them, 2.5 us each across 32 workgroups, and a dependent trip past L2 for every four entries of a row, 0.6 us each
+// (16 384 rows of 3, 5, 7, 9 and 13 entries: 5.65, 6.25, 6.24, 6.79 and 7.34 us; one workgroup of 512 rows: 4.2 to 5.4).  Here one workgroup per
 // compute unit keeps a stretch of rows for the whole solve: their entries in LDS, their r, x, p and dinv in
 // registers.  What the others need goes through memory: z (r where there is no preconditioner) and p, and two
 // exchanges per iteration, each a sum over the workgroups and a barrier in one:

@@ -9,16 +9,18 @@
 // (first row, first entry) of chunk c: with it a wavefront asks for its positions, values, coordinates and
 // its part of y at once, then gathers x, then adds up -- three dependent latencies.
 //
-// Bound by memory: the matrix is streamed once.  Measured on MI355X: the row-block and row-split kernels it replaces, then
-// with vectors of 16 bytes of entries per lane and guarded loads, then as it is (a lane takes every 64th entry, no load is
-// conditional), and the time of the bare bytes at the rate of a large copy (6.1 TB/s), us:
-//   5-point grid 1000^2    fp64  19.1  15.5  14.1 (14.4)
-//   7-point grid 100^3     fp64  24.1  18.6  17.3 (18.2)    fp32  19.3  13.9  13.6 (11.7)
-//   7-point grid 180^3     fp64         120   117 (107)     fp32         80    77 ( 68)
-//   27-node mesh of 35^3   fp64        23.7  19.4 (20.3)    fp32        21.1  14.7 (13.6)
-//   27-node mesh of 60^3   fp64   131   124   113 (103)     fp32   100   88    76 ( 68)
-// (below the bare bytes where the last-level cache holds the matrix from one call to the next).  With four neighbouring
-// entries in a lane the lanes of a gather are four entries apart and touch that many more lines.
+// Bound by memory: the matrix is streamed once.  Measured on MI355X, us a product among others of the same matrix and
+// vectors, on one box: the row-block and row-split kernels it replaces, this one, and the time of the bare bytes at the rate
+// of a large copy (6.1 TB/s):
+//   5-point grid 1000^2    fp64  21.7  14.1 (14.4)
+//   7-point grid 100^3     fp64  25.7  17.3 (18.2)    fp32  21.8  13.8 (11.7)
+//   7-point grid 180^3     fp64   126   117 (107)     fp32    92    77 ( 68)
+//   27-node mesh of 35^3   fp64  32.1  19.7 (20.3)    fp32  27.9  14.8 (13.6)
+//   27-node mesh of 60^3   fp64   130   107 (103)     fp32    99    76 ( 68)
+// (below the bare bytes where the last-level cache holds the matrix from one product to the next; with another matrix every
+// time 100^3 takes 20.8 in fp64, and the mesh of 60^3, which no cache holds, 106.9).  With four neighbouring entries in a
+// lane instead of one, and guarded loads, the lanes of a gather are four entries apart and touch that many more lines:
+// 18.6 at 100^3 and 23.7 on the mesh of 35^3 in fp64.
 // Tried and not kept: staging columns and values in LDS and gathering x in the row phase (40 to 50 % slower: the
 // gathers have to be issued right behind the loads), and 16-bit coordinates per chunk (fp64 slower, fp32 a few
 // percent faster: not worth a second copy of the coordinates).

@@ -72,9 +72,9 @@ __device__ __forceinline__ double lane_get(int byte_of_lane, double v) {
 // What bounds short rows is the chain of dependent loads of a wavefront (positions, entries, rows of B, row of
 // C), not bandwidth: staging makes it one trip per wavefront instead of one per LPR entries, and the row of C
 // is asked for first.  Measured (us; entries handed round by bpermute, LPR or 64 per trip -> staged):
-//   7-point 97^3, fp64   k = 3: 316 -> 35   k = 10: 392 -> 68   k = 64: 409 -> 369
-//   27-point x 3, 30^3   k = 3 fp64: 48 -> 31   k = 10 fp32: 57 -> 34   k = 64 fp32: 82 -> 73
-//   random, 32 per row, 15 000 rows, k = 10 fp32: 9.9 -> 7.7; 1 M rows, k = 64 fp32 (rows of B from HBM): 1217 -> 1203
+//   7-point 97^3, fp64   k = 3: 342 -> 34   k = 10: 393 -> 66   k = 64: 387 -> 355
+//   27-point x 3, 30^3   k = 3 fp64: 47 -> 26   k = 10 fp32: 83 -> 30   k = 64 fp32: 77 -> 66
+//   random, 32 per row, 15 000 rows, k = 10 fp32: 9.9 -> 7.7; 1 M rows, k = 64 fp32 (rows of B from HBM): 1216 -> 1207
 // Each XCD takes a contiguous part of the rows, so that neighbouring rows find each other's rows of B in its L2.  Dealt
 // round-robin instead, us, 7-point grids in fp64, k = 64: 70^3 130 -> 153, 95^3 334 -> 325, 97^3 358 -> 352, 100^3
 // 393 -> 501, 115^3 595 -> 763; fp32, k = 64, 100^3: 181 -> 225; 27-point x 3, 45^3, fp64, k = 64: 423 -> 403, k = 100:
@@ -295,7 +295,8 @@ __global__ __launch_bounds__(1024) void spmm_rowblock_lds_kernel(int nrows, int 
 // padding is the same bank; and seven wavefronts per SIMD (six where nh is no multiple of 4) keep enough rows of V in
 // flight (eight rows per lane instead of four: no faster, and twice as slow where they cost the wavefronts).
 // Measured at 16384 rows of 32, dh = 32, nh = 8: 195 us with a wavefront per row that read each value and coordinate
-// from global memory for every 64 columns, 47 us now (11.5 TB/s of rows of V, half of them from L2).
+// from global memory for every 64 columns, 45.3 us now: 537 MB of rows of V at 11.8 TB/s, of which some 190 MB come from
+// beyond L2 (246 MB fetched in all, the entries of A read once per part of V among them; 58 % of L2's requests hit).
 constexpr int kStagedBatched = 1024;        // values per wavefront and window
 constexpr int kStagedBatchedEntries = 256;  // non-zeros per wavefront and window at most
 constexpr int kRowPad = 8;  // floats between the stretches of two rows
