@@ -22,7 +22,9 @@
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
+#include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <memory>
 #include <mutex>
 #include <thread>
@@ -282,15 +284,21 @@ struct StagingHelpers {
     }
   }
 
-  // false: another call has them
+  // false: another call has them, or there are none
   bool open(BlockQueue *q) {
     {
       std::lock_guard<std::mutex> lock(mutex);
       if (queue || inside) return false;
       if (threads.empty()) {
         stop = false;
-        const int n = std::min<int>(kHelpers, (int)std::thread::hardware_concurrency() / 2);
-        for (int i = 0; i < n; ++i) threads.emplace_back([this] { run(); });
+        const char *most = getenv("LAPIS_HIP_STAGING_HELPERS");
+        const int n = std::min<int>(most ? atoi(most) : kHelpers, (int)std::thread::hardware_concurrency() / 2);
+        try {
+          for (int i = 0; i < n; ++i) threads.emplace_back([this] { run(); });
+        } catch (const std::exception &) {
+          // a process at its limit of threads copies with those it got
+        }
+        if (threads.empty()) return false;
       }
       queue = q;
       ++serial;

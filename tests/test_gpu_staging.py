@@ -1,6 +1,9 @@
 """Calls on host arrays at the sizes where their way to the device changes: brought by a kernel, in one transfer, in pieces
 on two streams, in rounds of the pinned memory; results worked on in pinned memory or brought back in pieces; the counts
 the copying pass makes at the edges of its blocks; several threads at once."""
+import os
+import subprocess
+import sys
 import threading
 
 import numpy as np
@@ -78,3 +81,25 @@ def test_memory_kept_between_calls_is_bounded_for_all_of_them_together(gpu):
     assert before - free() <= (256 << 20) + (32 << 20)
     (t,), staged = gpu.stage([host[:1000] + 3.0])  # and the arenas still serve calls
     assert torch.equal(t, torch.full_like(t, 3.0))
+
+
+def test_a_process_that_gets_no_threads_copies_alone(gpu):
+    # a process of its own: the threads are started once
+    code = """
+import os
+os.environ["LAPIS_HIP_STAGING_HELPERS"] = "0"
+import numpy as np, scipy.sparse as sp
+from lapis_amd.module import LAPISModule
+n = 300001
+A = sp.csr_matrix(sp.diags([1.0, 2.0, 3.0], [-1, 0, 1], shape=(n, n)))
+x, y = np.arange(n) % 7 - 3.0, np.ones(n)
+pos, crd = A.indptr.astype(np.int32), A.indices.astype(np.int32)
+module = LAPISModule()
+for k in range(3):
+    module.spmv(pos, crd, A.data, ((n, n), (n + 1, len(crd), len(crd))), x, y)
+assert np.array_equal(y, 1.0 + 3.0 * (A @ x)), "wrong product"
+print("the same")
+"""
+    out = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                         capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0 and "the same" in out.stdout, out.stderr
